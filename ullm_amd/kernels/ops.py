@@ -955,8 +955,9 @@ def paged_attention_generic(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
         _p(q), _c_int(q.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(positions),
         _p(token_entry), _p(block_table), _c_int(block_table.stride(0)), _c_int(page_size), _c_int(T),
         _c_int(nq), _c_int(nkv), _c_int(hd), _c_float(scale), _c_int(window), _p(bias),
-        _c_int(_check_distance_bias(bias, nq)), _p(sink), _c_int(_dt(q)), _stream()),
-        "paged_attention_generic")
+        # as many block table rows as tokens: every request brings one
+        _c_int(_check_distance_bias(bias, nq)), _p(sink), _c_int(1 if T <= block_table.shape[0] else 0), _c_int(_dt(q)),
+        _stream()), "paged_attention_generic")
     return out
 
 
