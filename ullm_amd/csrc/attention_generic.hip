@@ -14,7 +14,7 @@
 // Two kernels: where the head size is a multiple of 16 up to 256 and a page holds a multiple of four tokens, the tiled one
 // on the 32-bit matrix instructions; else one block per (token, head).  Which one is a matter of the model's sizes alone,
 // never of the batch.
-#include "common.h"
+#include "mfma_f32.h"
 
 #define ATT_THREADS 128
 #define ATT_MAX_HD 1024
@@ -110,27 +110,21 @@ paged_attention_generic_kernel(const T* __restrict__ q, int q_stride, T* __restr
 
 // ------------------------------------------------------------------------------- tiles on the 32-bit matrix cores
 // A block of four waves takes 16 rows, a row being a (token, query head) pair of one kv head: `tp` consecutive tokens of the
-// batch times up to 16 heads of the group.  64 keys at a time (at multiples of 64 of the position): wave w makes the scores
-// of keys 16w .. 16w + 15 (A operand: keys, straight from the cache, B operand: the rows' queries, kept in registers), the
-// waves share the rows' maxima and the exponentials through shared memory, and wave w adds dims 16 (w + 4i) .. of the
+// batch times up to 16 heads of the group.  128 keys at a time (at multiples of 128 of the position): wave w makes the scores
+// of keys 16 w .. and 64 + 16 w .. (A operand: keys, straight from the cache, B operand: the rows' queries, kept in registers),
+// the waves share the rows' maxima and the exponentials through shared memory, and wave w adds dims 16 (w + 4 i) .. of the
 // values (A operand: values, transposed in the page, straight from the cache).  Every key and value is read once a block.
-// Lane (r, g) holds, of every 16 x 16 product, column r (a row of the block) and four consecutive keys or dims 4g + i;
-// v_mfma_f32_16x16x4_f32 is full 32-bit.  A row's sums never see another row: a key it does not see weighs exactly zero and
-// leaves its maximum alone, so how many rows share a tile changes no bit.  Tokens of several requests in one tile are taken
-// request by request.  A tile in which some row does not see every key and a value is not finite is added key by key by
-// ordinary arithmetic (zero times infinity must not reach a row that does not see the key).
-// What bounds it: 16 x 64 x hd products of 32-bit twice a tile (1.7 us of the matrix pipe for a block at hd = 128, shared by
-// the waves of the other blocks) and two barriers; the keys of the next tile are on their way while this one's exponentials
-// and values are worked.  500 tokens, 16 heads of 128 over 8 kv heads, 32-bit: 55 us; the kernel above, which reads every
+// Lane (r, g) holds, of every 16 x 16 product, column r (a row of the block) and four consecutive keys or dims 4 g + i;
+// v_mfma_f32_16x16x4_f32 is full 32-bit, and its operands lie so that scores and outputs are added in the order of channels
+// and keys (mfma_f32.h): without a window the results have the bits of the kernel above.  A row's sums never see another
+// row: a key it does not see weighs exactly zero and leaves its maximum alone, so how many rows share a tile changes no bit.
+// Tokens of several requests in one tile are taken request by request.  A half tile in which some row does not see every key
+// and a value is not finite is added key by key by ordinary arithmetic (zero times infinity must not reach a row that does
+// not see the key).
+// What bounds it: 16 x 128 x hd products of 32-bit twice a tile (3.4 us of the matrix pipe for a block at hd = 128, shared by
+// the waves of the other blocks) and two barriers; the keys of the next half tile are on their way while this one's values are
+// worked.  500 tokens, 16 heads of 128 over 8 kv heads, 32-bit: 63 us; the kernel above, which reads every
 // key once per query head with the lanes of a wave hd values apart, took 637.
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-__device__ __forceinline__ float4 ld4_f32(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 ld4_f32(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                     __uint_as_float(u.y & 0xffff0000u));
-}
-__device__ __forceinline__ float at4(const float4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
 __device__ __forceinline__ bool finite4(const float4& v) {
   return isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
 }
@@ -144,8 +138,8 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
                              int T_, int tp, int nq, int nkv, float scale, int window,
                              const float* __restrict__ bias, int bias_rows, const float* __restrict__ sink) {
   constexpr int HD = 16 * KC, NT = (KC + 3) / 4;
-  __shared__ float s_max[4][16], s_sum[4][16];
-  __shared__ __attribute__((aligned(16))) float s_p[16][68];
+  __shared__ float s_max[4][16];
+  __shared__ __attribute__((aligned(16))) float s_p[16][132];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
   const int group = nq / nkv, gh = group < 16 ? group : 16, chunks = (group + 15) / 16;
   const int kvh = blockIdx.y / chunks, h0 = blockIdx.y % chunks * 16;
@@ -157,12 +151,12 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
   const int t = t0 + (tt < n_tok ? tt : 0), h = kvh * group + (hh < group ? hh : 0);
   const int pos = positions[t], entry = token_entry[t];
   const int lo = first_seen_key(pos, window);
-  float4 qf[KC];
-  const T* qp = q + (size_t)t * q_stride + (size_t)h * HD + 4 * g;
+  f32x4_t qf[KC];                                        // [c][i]: channel 16 c + 4 i + g
+  const T* qp = q + (size_t)t * q_stride + (size_t)h * HD + g;
 #pragma unroll
   for (int c = 0; c < KC; ++c)
-    qf[c] = make_float4(ld_f32(qp + 16 * c) * scale, ld_f32(qp + 16 * c + 1) * scale, ld_f32(qp + 16 * c + 2) * scale,
-                        ld_f32(qp + 16 * c + 3) * scale);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qf[c][i] = ld_f32(qp + 16 * c + 4 * i) * scale;
   f32x4_t acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -183,131 +177,176 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
     first = end;
     const bool active = valid && entry == seg_entry;
     const int* bt = block_table + (size_t)seg_entry * bt_stride;
-    int base = low & ~63;
-    // pages of a tile: of this lane's key for the scores, of its four keys of every 16 for the values
-    int kpage, vpage[4];
-    auto pages_of = [&](int at, int& kp, int* vp) __attribute__((always_inline)) {
-      const int j = at + 16 * wave + r;
-      const int kv = bt[page_index(j <= hi ? j : hi)];
-      kp = j <= hi ? kv : -1;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int jv = at + 16 * c + 4 * g;
-        const int pv = bt[page_index(jv <= hi ? jv : hi)];
-        vp[c] = jv <= hi ? pv : -1;
-      }
+    // the page of key j, -1 past the last key
+    auto page_of = [&](int j) __attribute__((always_inline)) {
+      const int page = bt[page_index(j <= hi ? j : hi)];
+      return j <= hi ? page : -1;
     };
-    float4 kf[KC];
-    auto fetch_keys = [&](int at, int kp) __attribute__((always_inline)) {
+    // keys of both halves of a tile; up to hd = 128 registers hold them together, and the halves' products alternate
+    constexpr int KEY_SETS = KC <= 8 ? 2 : 1;
+    float4 kf[KEY_SETS][KC];
+    auto fetch_keys = [&](int set, int at, int page) __attribute__((always_inline)) {
       const int j = at + 16 * wave + r;
-      const T* src = k_pool + (((size_t)(kp < 0 ? 0 : kp) * nkv + kvh) * page_size + (kp < 0 ? 0 : j - page_index(j) * page_size)) * HD + 4 * g;
+      const T* src = k_pool + (((size_t)(page < 0 ? 0 : page) * nkv + kvh) * page_size + (page < 0 ? 0 : j - page_index(j) * page_size)) * HD + 4 * g;
 #pragma unroll
-      for (int c = 0; c < KC; ++c) kf[c] = ld4_f32(src + 16 * c);
+      for (int c = 0; c < KC; ++c) kf[set][c] = ld4_f32(src + 16 * c);
     };
-    pages_of(base, kpage, vpage);
-    fetch_keys(base, kpage);
-    for (; base <= hi; base += 64) {
-      const unsigned long long there = __ballot(kpage >= 0);            // bit r: key 16 wave + r has a page
-      float4 vf[NT][4];
+    // half a tile's values for this wave's dims, keys past the end and keys without a page zeroed
+    float4 vf[NT][4];
+    int vpage[4];
+    auto fetch_values = [&](int at) __attribute__((always_inline)) {
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int dim = 16 * (wave + 4 * n) + r;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const int jv = base + 16 * c + 4 * g;
+          const int jv = at + 16 * c + 4 * g;
           const bool have = vpage[c] >= 0;
           const size_t row = ((size_t)(have ? vpage[c] : 0) * nkv + kvh) * HD + (dim < HD ? dim : 0);
           vf[n][c] = ld4_f32(v_pool + row * page_size + (have ? jv - page_index(jv) * page_size : 0));
-          // keys past the end, or without a page, have no value
           if (!have) vf[n][c].x = 0.f;
           if (!have || jv + 1 > hi) vf[n][c].y = 0.f;
           if (!have || jv + 2 > hi) vf[n][c].z = 0.f;
           if (!have || jv + 3 > hi) vf[n][c].w = 0.f;
         }
       }
-      int vhave = 0;
+    };
+    auto value_pages = [&](int at) __attribute__((always_inline)) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) vhave |= (vpage[c] >= 0 ? 1 : 0) << c;
-      f32x4_t sc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < 4; ++c) vpage[c] = page_of(at + 16 * c + 4 * g);
+    };
+    int base = low & ~127;
+    int kpage[2];
 #pragma unroll
-      for (int c = 0; c < KC; ++c)
+    for (int half = 0; half < KEY_SETS; ++half) {
+      kpage[half] = page_of(base + 64 * half + 16 * wave + r);
+      fetch_keys(half, base + 64 * half, kpage[half]);
+    }
+    for (; base <= hi; base += 128) {
+      f32x4_t s[2];
+      unsigned long long there[2];                       // bit r: key 16 wave + r of the half has a page
+      bool ok[2][4];
+      float tile_max = -INFINITY;
+      if constexpr (KEY_SETS == 2) {
+        s[0] = s[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(kf[c], j), at4(qf[c], j), sc, 0, 0, 0);
-      pages_of(base + 64, kpage, vpage);                 // clamped to the last key's page past the end
-      fetch_keys(base + 64, kpage);
-      float s[4], tile_max = -INFINITY;
-      bool ok[4];
+        for (int c = 0; c < KC; ++c) {
+          const f32x4_t k0 = in_order(kf[0][c]), k1 = in_order(kf[1][c]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = base + 16 * wave + 4 * g + i;
-        ok[i] = active && j <= pos && j >= lo && ((there >> (4 * g + i)) & 1);
-        s[i] = sc[i];
-        if (bias && ok[i]) s[i] += bias[(size_t)h * bias_rows + (pos - j < bias_rows ? pos - j : bias_rows - 1)];
-        if (ok[i]) tile_max = fmaxf(tile_max, s[i]);
+          for (int i = 0; i < 4; ++i) {
+            s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0[i], qf[c][i], s[0], 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k1[i], qf[c][i], s[1], 0, 0, 0);
+          }
+        }
       }
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        constexpr bool both = KEY_SETS == 2;
+        const int at = base + 64 * half, set = both ? half : 0, next = both ? at + 128 : at + 64;
+        there[half] = __ballot(kpage[set] >= 0);
+        if constexpr (!both) {
+          s[half] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int c = 0; c < KC; ++c) {
+            const f32x4_t k = in_order(kf[0][c]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], qf[c][i], s[half], 0, 0, 0);
+          }
+        }
+        kpage[set] = page_of(next + 16 * wave + r);
+        fetch_keys(set, next, kpage[set]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = at + 16 * wave + 4 * g + i;
+          ok[half][i] = active && j <= pos && j >= lo && ((there[half] >> (4 * g + i)) & 1);
+          if (bias && ok[half][i]) s[half][i] += bias[(size_t)h * bias_rows + (pos - j < bias_rows ? pos - j : bias_rows - 1)];
+          if (ok[half][i]) tile_max = fmaxf(tile_max, s[half][i]);
+        }
+      }
+      value_pages(base);
       tile_max = max_with_lane_xor32(max_with_lane_xor16(tile_max));
       if (g == 0) s_max[wave][r] = tile_max;
       __syncthreads();
+      fetch_values(base);
       const float m_new = fmaxf(fmaxf(m, fmaxf(s_max[0][r], s_max[1][r])), fmaxf(s_max[2][r], s_max[3][r]));
       const float alpha = m_new == m ? 1.f : expf(m - m_new);
-      float p[4], sum = 0.f;
+      // the exponentials lie so that a reader of four neighbouring places has keys g, 4 + g, 8 + g, 12 + g of a chunk
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        p[i] = ok[i] ? expf(s[i] - m_new) : 0.f;
-        sum += p[i];
-      }
-      *reinterpret_cast<float4*>(&s_p[r][16 * wave + 4 * g]) = make_float4(p[0], p[1], p[2], p[3]);
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      if (g == 0) s_sum[wave][r] = sum;
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s_p[r][64 * half + 16 * wave + 4 * i + g] = ok[half][i] ? expf(s[half][i] - m_new) : 0.f;
       __syncthreads();
-      l = l * alpha + ((s_sum[0][r] + s_sum[1][r]) + (s_sum[2][r] + s_sum[3][r]));
       m = m_new;
 #pragma unroll
       for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[n][i] *= alpha;
-      // every row sees every key, or every value is finite
-      bool plain = alone && __all(!valid || (base >= lo && base + 63 <= pos));
-      if (!plain) {
-        bool fine = true;
+      float tile_sum = 0.f;
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
+      for (int half = 0; half < 2; ++half) {
+        const int at = base + 64 * half;
+        f32x4_t pf[4];
 #pragma unroll
-          for (int c = 0; c < 4; ++c) fine = fine && finite4(vf[n][c]);
-        plain = __all(fine);
-      }
-      if (plain) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float4 pf = *reinterpret_cast<const float4*>(&s_p[r][16 * c + 4 * g]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int n = 0; n < NT; ++n)
-              acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(vf[n][c], j), at4(pf, j), acc[n], 0, 0, 0);
+        for (int c = 0; c < 4; ++c) pf[c] = *reinterpret_cast<const f32x4_t*>(&s_p[r][64 * half + 16 * c + 4 * g]);
+        // the half's sum as a tree over the bits of the key's place, the highest first
+        {
+          const f32x4_t a = (pf[0] + pf[2]) + (pf[1] + pf[3]);          // [i]: places 4 i + g
+          float sum = (a[0] + a[2]) + (a[1] + a[3]);
+          sum += __shfl_xor(sum, 32, 64);
+          sum += __shfl_xor(sum, 16, 64);
+          tile_sum += sum;
         }
-      } else {
-        // lane (r, g) holds dims 4g + i of row r; the value of key 16c + 4o + j at dim 4g + i lies in lane (4g + i, o)
+        // every row sees every key, or every value is finite
+        bool plain = alone && __all(!valid || (at >= lo && at + 63 <= pos));
+        if (!plain) {
+          bool fine = true;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          for (int o = 0; o < 4; ++o) {
-            const int have = __shfl(vhave, 16 * o, 64);
+          for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int key = base + 16 * c + 4 * o + j;
-              const bool sees = active && key <= pos && key >= lo && ((have >> c) & 1);
-              const float w = s_p[r][16 * c + 4 * o + j];
+            for (int c = 0; c < 4; ++c) fine = fine && finite4(vf[n][c]);
+          plain = __all(fine);
+        }
+        int vhave = 0;
 #pragma unroll
-              for (int n = 0; n < NT; ++n)
+        for (int c = 0; c < 4; ++c) vhave |= (vpage[c] >= 0 ? 1 : 0) << c;
+        if (plain) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  const float v = __shfl(at4(vf[n][c], j), 16 * o + 4 * g + i, 64);
-                  if (sees) acc[n][i] += w * v;
-                }
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const f32x4_t v = in_order(vf[n][c]);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], pf[c][i], acc[n], 0, 0, 0);
             }
-          }
+        } else {
+          // lane (r, g) holds dims 4 g + i of row r; the value of key 16 c + 4 o + j at dim 4 g + i lies in lane (4 g + i, o)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            for (int o = 0; o < 4; ++o) {
+              const int have = __shfl(vhave, 16 * o, 64);
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int key = at + 16 * c + 4 * o + j;
+                const bool sees = active && key <= pos && key >= lo && ((have >> c) & 1);
+                const float w = s_p[r][64 * half + 16 * c + 4 * j + o];
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    const float mine = j == 0 ? vf[n][c].x : j == 1 ? vf[n][c].y : j == 2 ? vf[n][c].z : vf[n][c].w;
+                    const float v = __shfl(mine, 16 * o + 4 * g + i, 64);
+                    if (sees) acc[n][i] += w * v;
+                  }
+              }
+            }
+        }
+        if (half == 0) {
+          value_pages(at + 64);
+          fetch_values(at + 64);
+        }
       }
+      l = l * alpha + tile_sum;
     }
     __syncthreads();                                     // the next request's maxima are written only now
   }

@@ -1,36 +1,24 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) with 32-bit products and sums in a fixed K order, on the 32-bit matrix
 // instruction v_mfma_f32_16x16x4_f32 (whose products and sums are full 32-bit: no rounding of the inputs).
-// The product of row m never depends on M, on the other rows or on the tile it lies in: every variant below walks K in
-// chunks of 16 with the same four instructions a chunk (the j-th takes k = j, 4 + j, 8 + j, 12 + j of the chunk) into two
-// chains of sums per output, even chunks and odd ones, added at the end: a token's result is the same in every batch.  This is the matrix product of the float32
+// The product of row m never depends on M, on the other rows or on the tile it lies in: every variant below adds the products
+// in the order of K into one chain of sums per output (mfma_f32.h), so a token's result is the same in every batch, and the
+// bits are those of a plain loop of fma over K.  This is the matrix product of the float32
 // mode and the general fallback for bfloat16 operands (widened exactly on their way to shared memory).
 // Weights are [out, in] as the reference stores them for F.linear (ullm/layers/linear.py:165,268).
 //
 // What bounds it: the matrix pipe (157 TFLOP/s in 32-bit) where the tiles fill the chip, the chain over K where they do
 // not (a 16 x 16 tile adds 4 k in 32 cycles).  Hence the tile sizes: large ones read shared memory and the second-level
 // cache less per product, small ones make more blocks.  Against a 64 x 64 tile of scalar multiply-adds whose operands came
-// one value a load: 500 rows, 4096 outputs, K = 1024 117 -> 48 us (87 TFLOP/s), 1024 outputs, K = 3072 406 -> 45 us; 2048
-// rows, 4096 outputs 267 -> 178 us; one row of 151 936 outputs 436 -> 111 us (5.6 TB/s); two chains halve the error's square
-// (5.7e-7 -> 4.1e-7 of the result at K = 1024).
-#include "common.h"
-
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
-__device__ __forceinline__ float4 ld4_f32(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 ld4_f32(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                     __uint_as_float(u.y & 0xffff0000u));
-}
-
-__device__ __forceinline__ float at4(const float4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
+// one value a load: 500 rows, 4096 outputs, K = 1024 122 -> 49 us (85 TFLOP/s), 1024 outputs, K = 3072 407 -> 52 us; 2048
+// rows, 4096 outputs 272 -> 179 us; one row of 151 936 outputs 434 -> 115 us (5.4 TB/s).
+#include "mfma_f32.h"
 
 // A block of four waves takes BM rows of A against BN rows of W, WGM waves side by side along M.  A stage is BK values of
 // K: rows in shared memory whose 16-byte piece c of row r lies at piece c ^ ((r >> 1) & 7) (the 16 lanes the hardware
 // serves together then read different bank groups); two stages take turns, and a stage is fetched into registers two
 // stages before its products.  A stage costs about 600 cycles of writing, barrier and reading beside its products, so the
-// smallest tile takes 128 values a stage (32 x 32 at 64 rows, 1024 outputs, K = 2048: 23 us with 32).  Lane (r, g) of a wave reads k = 4g .. 4g + 3 of its row's chunk at once and
-// holds out[row r of A][columns 4g .. 4g + 3] of each 16 x 16 tile.  VEC: four values a load (K and the row lengths are
+// smaller tiles take 64 values a stage.  Lane (r, g) of a wave reads k = g, 4 + g, 8 + g, 12 + g of its row's chunk at
+// once (they are written side by side) and holds out[row r of A][columns 4g .. 4g + 3] of each 16 x 16 tile.  VEC: four values a load (K and the row lengths are
 // multiples of four values and the addresses of that alignment); else one by one.  No load stands under a condition: a
 // row past the end reads the last row, a piece past K the row's last piece (replaced by zeros); neither is stored.
 template <typename TA, typename TW, typename TC, int BM, int BN, int WGM, int BK, bool VEC>
@@ -51,18 +39,18 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
   const int pc = tid % PR, prow = tid / PR;
   const TA* asrc[AP];
   const TW* wsrc[WP];
-  int aput[AP], wput[WP];
+  int aput[AP], wput[WP], alow[AP], wlow[WP];
 #pragma unroll
   for (int i = 0; i < AP; ++i) {
     const int row = (prow + STEP * i) % BM;              // more threads than pieces: two fetch and write the same
     asrc[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda;
-    aput[i] = row * BK * 4 + ((pc ^ ((row >> 1) & 7)) << 4);
+    aput[i] = row * BK * 4 + (((pc & ~3) ^ ((row >> 1) & 4)) << 4) + 4 * (pc & 3), alow[i] = (row >> 1) & 3;
   }
 #pragma unroll
   for (int i = 0; i < WP; ++i) {
     const int row = (prow + STEP * i) % BN;
     wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw;
-    wput[i] = (BM + row) * BK * 4 + ((pc ^ ((row >> 1) & 7)) << 4);
+    wput[i] = (BM + row) * BK * 4 + (((pc & ~3) ^ ((row >> 1) & 4)) << 4) + 4 * (pc & 3), wlow[i] = (row >> 1) & 3;
   }
   float4 areg[2][AP], wreg[2][WP];
   auto fetch = [&](int set, int k0) __attribute__((always_inline)) {
@@ -96,46 +84,47 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
       for (int i = 0; i < WP; ++i) wreg[set][i] = one(wsrc[i]);
     }
   };
+  // value e of a piece goes to the chunk's piece e: a lane group's 16 bytes are then values g, 4 + g, 8 + g, 12 + g of the chunk
+  // (64 lanes write one value each to 64 different banks)
   auto put = [&](int set, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < AP; ++i) *reinterpret_cast<float4*>(stages[buf] + aput[i]) = areg[set][i];
+    for (int i = 0; i < AP; ++i) {
+      const float v[4] = {areg[set][i].x, areg[set][i].y, areg[set][i].z, areg[set][i].w};
 #pragma unroll
-    for (int i = 0; i < WP; ++i) *reinterpret_cast<float4*>(stages[buf] + wput[i]) = wreg[set][i];
+      for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(stages[buf] + aput[i] + ((e ^ alow[i]) << 4)) = v[e];
+    }
+#pragma unroll
+    for (int i = 0; i < WP; ++i) {
+      const float v[4] = {wreg[set][i].x, wreg[set][i].y, wreg[set][i].z, wreg[set][i].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(stages[buf] + wput[i] + ((e ^ wlow[i]) << 4)) = v[e];
+    }
   };
-  f32x4_t acc[2][TN][TM];
+  f32x4_t acc[TN][TM];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int n = 0; n < TN; ++n)
 #pragma unroll
-    for (int n = 0; n < TN; ++n)
-#pragma unroll
-      for (int m = 0; m < TM; ++m) acc[h][n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < TM; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto products = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c0 = 0; c0 < BK / 16; c0 += 2) {
-      float4 a[2][TM], w[2][TN];
+    for (int c = 0; c < BK / 16; ++c) {
+      f32x4_t a[TM], w[TN];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int c = c0 + h;
-#pragma unroll
-        for (int m = 0; m < TM; ++m) {
-          const int row = wm + 16 * m + r;
-          a[h][m] = *reinterpret_cast<const float4*>(stages[buf] + row * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
-        }
-#pragma unroll
-        for (int n = 0; n < TN; ++n) {
-          const int row = wn + 16 * n + r;
-          w[h][n] = *reinterpret_cast<const float4*>(stages[buf] + (BM + row) * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
-        }
+      for (int m = 0; m < TM; ++m) {
+        const int row = wm + 16 * m + r;
+        a[m] = *reinterpret_cast<const f32x4_t*>(stages[buf] + row * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int n = 0; n < TN; ++n) {
+        const int row = wn + 16 * n + r;
+        w[n] = *reinterpret_cast<const f32x4_t*>(stages[buf] + (BM + row) * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
+      }
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int n = 0; n < TN; ++n)
+        for (int n = 0; n < TN; ++n)
 #pragma unroll
-            for (int m = 0; m < TM; ++m)
-              acc[h][n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(w[h][n], j), at4(a[h][m], j), acc[h][n][m], 0, 0, 0);
+          for (int m = 0; m < TM; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n][i], a[m][i], acc[n][m], 0, 0, 0);
     }
   };
   fetch(0, 0);
@@ -165,7 +154,7 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
       float v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        v[i] = acc[0][n][m][i] + acc[1][n][m][i];
+        v[i] = acc[n][m][i];
         if (bias) v[i] += bias[gn + i < N ? gn + i : N - 1];
       }
       if (sizeof(TC) == 4 && gn + 3 < N && (ldc & 3) == 0 && !((uintptr_t)C & 15)) {
