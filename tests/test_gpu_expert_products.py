@@ -1,0 +1,53 @@
+"""The experts' products over large tiles: rows on both sides of a wave's 64 and a tile's edge, one to five stages of K,
+columns past the last block's, a gathered and a plain row order, against 64-bit results."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from ullm_amd.kernels import ops
+    return ops
+
+
+@pytest.mark.parametrize("tile_rows", [128, 256])
+@pytest.mark.parametrize("K,n_out", [(64, 130), (128, 256), (192, 64), (256, 388), (320, 260)])
+@pytest.mark.parametrize("limit", [0.0, 1.5])
+def test_experts_with_rows_at_every_edge(ops, tile_rows, K, n_out, limit):
+    g = torch.Generator().manual_seed(K + n_out + tile_rows)
+    counts = [1, 63, 64, 65, 0, 127, 128, 129, 255, 256, 257, 16]
+    experts, T = len(counts), sum(counts)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=g)].int()[:, None].contiguous().to(DEV)
+    wide = torch.randn(T, K + 8, generator=g).bfloat16().to(DEV)
+    x = wide[:, :K]                                                   # rows further apart than they are long
+    w_gu = (torch.randn(experts, 2 * n_out, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    w = (torch.randn(experts, n_out, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    slot, token, tiles, offsets = ops.moe_sort(ids, experts, tile_rows)
+    gated = ops.moe_rows(x, token, w_gu, tiles, tile_rows, T, gated=True, limit=limit, alpha=1.3)
+    by_slot = x[token.long()].contiguous()
+    plain = ops.moe_rows(by_slot, None, w, tiles, tile_rows, T, gated=False)
+    at = offsets.cpu().tolist()
+    for e, n in enumerate(counts):
+        rows = slice(at[e], at[e] + n)
+        assert at[e + 1] - at[e] == n
+        h = by_slot[rows].double()
+        size = h.abs() @ w[e].double().abs().T
+        assert ((plain[rows].double() - h @ w[e].double().T).abs() <= (K + 1) * 2.0 ** -24 * size).all()    # K 32-bit sums
+        gu = h @ w_gu[e].double().T
+        a, u = gu[:, :n_out], gu[:, n_out:]
+        if limit:
+            a, u = a.clamp(max=limit), u.clamp(-limit, limit)
+            want = a * torch.sigmoid(1.3 * a) * (u + 1)
+        else:
+            want = a * torch.sigmoid(a) * u
+        # the result's rounding to bfloat16, and of the 32-bit sums what the unit makes of it (its slopes are below 3 + |u|)
+        off = (K + 8) * 2.0 ** -24 * (h.abs() @ w_gu[e].double().abs().T).amax(-1, keepdim=True) * (4 + u.abs() + a.abs())
+        assert ((gated[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + off).all()
+    # a row's result does not depend on the rows beside it: 128 and 256 rows a tile add up the same way
+    other = 384 - tile_rows
+    slot2, token2, tiles2, _ = ops.moe_sort(ids, experts, other)
+    again = ops.moe_rows(x[token2.long()].contiguous(), None, w, tiles2, other, T, gated=False)
+    assert torch.equal(again[slot2.long()], plain[slot.long()])

@@ -19,6 +19,7 @@
 // window or chunk (a negative `window`: see first_seen_key), query head h reads kv head h / (nq / nkv) (ullm/layers/attention.py:76-104,271,298-309).
 #include "common.h"
 #include <type_traits>
+#include "lds_load.h"
 #include "no_alloc.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -1215,30 +1216,6 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __r
 // compiler's own whose wait could be off by the ones it does not see: the page ids lie in shared memory.
 #define DMA_TILES 4                       // tiles of shared memory that take turns
 #define DMA_TABLE_TILES 128               // tiles whose page ids shared memory holds at a time (and 4 more, for the loads ahead)
-
-// 16 bytes per lane from `src` to shared memory at lds_base + 16 * lane (lds_base the same in the whole wave).
-// The instruction takes the place in shared memory from M0, which the compiler keeps for itself and warns
-// about; nothing else in these kernels uses it.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load16_to_lds(const void* src, unsigned char* lds_base) {
-#ifdef __HIP_DEVICE_COMPILE__
-  typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
-  const unsigned at = (unsigned)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_byte_t*)lds_base);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(at) : "memory", "m0");
-#else
-  __builtin_amdgcn_global_load_lds(src, lds_base, 16, 0, 0);
-#endif
-}
-#pragma clang diagnostic pop
-// at most N of this wave's loads are still on their way
-template <int N>
-__device__ __forceinline__ void loads_left() {
-  static_assert(N >= 0 && N < 64, "the counter has six bits");
-#ifdef __HIP_DEVICE_COMPILE__
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-#endif
-}
 
 template <int NQK>
 struct DmaTile {

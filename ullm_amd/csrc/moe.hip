@@ -24,6 +24,7 @@
 // or for float32 and for shapes the tiles do not take a kernel with one wave per output value that sums K in a
 // fixed order.  Expert matrices are stacked: gate|up [experts, 2 ff, hidden], down [experts, hidden, ff].
 #include "common.h"
+#include "mfma_tiles.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
@@ -671,9 +672,88 @@ moe_tiles_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restri
   }
 }
 
+// The same products where K is a multiple of 64, by the loop of mfma_tiles.h: a block takes a tile of up to 64 WMW rows against
+// 256 rows of the expert's matrix (GATED: the gate rows and the up rows of 128 output columns, a wave the same 64 of each).
+// What bounds it: the experts' matrices from memory (268 MB of gate|up: 45 us) and, beside them, the matrix pipe, which the
+// loop keeps busy 57 % of the time where every operand lies in the second-level cache.  32 experts, top 4, width 2048, 1024
+// columns an expert, against the kernel above: gate|up at 2048 / 3000 / 8192 tokens 160 / 217 / 470 -> 117 / 140 / 279 us (590 /
+// 720 / 987 TFLOP/s), down 87 / 120 / 270 -> 73 / 87 / 206 us.  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a
+// stage ahead of its products took 127 to 150 us at 2048 tokens, whatever the number of stages; a wave of its own that asked
+// for the matrix's lines ahead of time made them slower (180 us).
+template <int WMW, int STAGES, bool GATED>
+__global__ void __launch_bounds__(128 * WMW)
+moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
+                    const bf16_t* __restrict__ w, const int* __restrict__ tiles, int n_tiles, int n_col_blocks,
+                    void* __restrict__ out_, int ldo, int n_out, int K, float limit, float alpha) {
+  using T = ProductTiles<WMW, STAGES>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char tile_stages[];
+  const int used = tiles[3 * n_tiles];                   // dies and tiles as above
+  const int total = used * n_col_blocks, per_die = (total + 7) / 8;
+  const int item = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_die || item >= total) return;
+  const int tile = item / n_col_blocks, col_block = item % n_col_blocks;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int e = tiles[3 * tile], slot0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  if (rows <= 0) return;
+  constexpr int COLS = GATED ? 128 : 256;                // output columns of a block
+  const int n0 = col_block * COLS;
+  const size_t w_rows = GATED ? 2 * (size_t)n_out : (size_t)n_out;
+  unsigned xoff[T::XL], woff[T::WL];
+#pragma unroll
+  for (int i = 0; i < T::XL; ++i) {
+    const int row = T::x_row(wave, lane, i), slot = slot0 + (row < rows ? row : rows - 1);
+    xoff[i] = 2u * ((unsigned)(row_index ? row_index[slot] : slot) * (unsigned)ldx + T::k_of(row, lane));
+  }
+#pragma unroll
+  for (int i = 0; i < T::WL; ++i) {
+    const int row = T::w_row(wave, lane, i);
+    int n = n0 + row % COLS;
+    if (n >= n_out) n = n_out - 1;
+    woff[i] = 2u * ((unsigned)((GATED && row >= COLS ? n_out : 0) + n) * (unsigned)K + T::k_of(row, lane));
+  }
+  tile_f32x4 acc[T::TN][T::TM];
+  T::run(tile_stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w + (size_t)e * w_rows * K), woff,
+         K >> 6, wave, lane, 128, acc);
+  // lane (r, g): row r of each 16-row group, four consecutive columns at 4g
+  const int wm = wave >> 1, wn = wave & 1;
+#pragma unroll
+  for (int m = 0; m < T::TM; ++m) {
+    const int row = 64 * wm + 16 * m + r;
+    if (row >= rows) continue;
+#pragma unroll
+    for (int n = 0; n < (GATED ? 4 : 8); ++n) {
+      const int c = n0 + 64 * wn + 16 * (n & 3) + 4 * g + (n < 4 ? 0 : 128);
+      const size_t at = (size_t)(slot0 + row) * ldo + c;
+      if (GATED) {
+        bf16_t* o = reinterpret_cast<bf16_t*>(out_) + at;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n][m][i], acc[n + 4][m][i], limit, alpha);
+        if (c + 3 < n_out && (ldo & 3) == 0) {
+          *reinterpret_cast<uint2*>(o) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (c + i < n_out) o[i] = f32_to_bf16_bits(v[i]);
+        }
+      } else {
+        float* o = reinterpret_cast<float*>(out_) + at;
+        if (c + 3 < n_out && (ldo & 3) == 0) {
+          *reinterpret_cast<float4*>(o) = make_float4(acc[n][m][0], acc[n][m][1], acc[n][m][2], acc[n][m][3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (c + i < n_out) o[i] = acc[n][m][i];
+        }
+      }
+    }
+  }
+}
+
 // Rows of a tile the matrix-core kernels take for a launch made with `tile_rows` rows a tile.
 extern "C" int ullm_moe_mfma_supports(int K, int ldx, int tile_rows) {
-  return K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64 || tile_rows == 128);
+  return K >= 8 && K % 8 == 0 && ldx % 8 == 0 && (tile_rows == 16 || tile_rows == 32 || tile_rows == 64 || tile_rows == 128 ||
+                                                  (tile_rows == 256 && K % 64 == 0));
 }
 
 template <int MT, bool GATED, typename... Args>
@@ -685,6 +765,15 @@ static void launch_tiles(dim3 grid, hipStream_t stream, Args... args) {
   hipLaunchKernelGGL((moe_tiles_mfma_kernel<MT, GATED>), grid, dim3(256), bytes, stream, args...);
 }
 
+template <int WMW, int STAGES, bool GATED, typename... Args>
+static void launch_products(dim3 grid, hipStream_t stream, Args... args) {
+  constexpr int bytes = ProductTiles<WMW, STAGES>::BYTES;
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)moe_products_kernel<WMW, STAGES, GATED>,
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  (void)allowed;
+  hipLaunchKernelGGL((moe_products_kernel<WMW, STAGES, GATED>), grid, dim3(128 * WMW), bytes, stream, args...);
+}
+
 // out[slot] = glu(x[row_index[slot]] Wg^T, x Wu^T) (gated: out in x's dtype, w [experts, 2 n_out, K]) or
 // x[slot] W^T (not gated: out float32, w [experts, n_out, K]) over the tiles' rows.  row_index may be null.
 extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const void* w, const int* tiles,
@@ -693,6 +782,22 @@ extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const
   if (max_tiles <= 0) return 0;
   if (n_out < 1 || K < 1 || ldx < K || ldo < n_out || tile_rows < 1) return ULLM_ERR_SHAPE;
   if (dtype == ULLM_BF16 && ullm_moe_mfma_supports(K, ldx, tile_rows) && !((uintptr_t)x & 15) && !((uintptr_t)w & 15)) {
+    // the loop's loads count bytes from x and from the expert's matrix in 32 bits (a row of x is a token or a slot: never past
+    // the slots of all tiles)
+    const bool near = (long long)max_tiles * tile_rows * ldx < (1LL << 31) && (gated ? 2LL : 1LL) * n_out * K < (1LL << 31);
+    if (tile_rows >= 128 && K % 64 == 0 && near) {
+      const int per_block = gated ? 128 : 256, col_blocks = (n_out + per_block - 1) / per_block;
+      const long long total = (long long)max_tiles * col_blocks;
+      if (total > 0x3fffffffLL) return ULLM_ERR_SHAPE;
+      dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+#define TILES(W, ST, G) launch_products<W, ST, G>(grid, stream, (const bf16_t*)x, ldx, row_index, (const bf16_t*)w, tiles, max_tiles, \
+    col_blocks, out, ldo, n_out, K, limit, alpha)
+      if (tile_rows == 256) { if (gated) TILES(4, 2, true); else TILES(4, 2, false); }
+      else { if (gated) TILES(2, 3, true); else TILES(2, 3, false); }
+#undef TILES
+      ULLM_LAUNCH_CHECK();
+    }
+    if (tile_rows == 256) return ULLM_ERR_SHAPE;
     if (tile_rows >= 64) {
       const int col_blocks = (n_out + (gated ? 63 : 127)) / (gated ? 64 : 128);
       const long long total = (long long)max_tiles * col_blocks;
