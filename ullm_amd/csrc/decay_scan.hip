@@ -14,25 +14,13 @@
 // Everything is 32-bit.  A state element goes through the same operations in the same order wherever a prompt is
 // cut, and a token's output sums its partial sums in a fixed order.
 #include "common.h"
+#include "decay_inputs.h"
 
-enum { DECAY_PER_HEAD = 0, DECAY_SIGMOID_ROOT = 1, DECAY_EXP_EXP = 2, DECAY_READY = 3 };   // READY: z holds the decays themselves
 typedef __attribute__((ext_vector_type(4))) float scan_f32x4;
 enum { GATE_SILU = 0, GATE_SIGMOID = 1 };
 
 #define SCAN_THREADS 256
 #define SCAN_CHUNK 16
-
-__device__ __forceinline__ float exact_silu(float z) { return z / (1.f + expf(-z)); }
-
-// The decay of a raw value.  sigmoid(z)^(1/tau) = exp(-softplus(-z) / tau), with softplus(x) = max(x, 0) + log1p(e^-|x|).
-__device__ __forceinline__ float decay_of(float z, int kind, float inv_tau) {
-  if (kind == DECAY_SIGMOID_ROOT) {
-    const float x = -z;
-    const float sp = fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
-    return expf(-sp * inv_tau);
-  }
-  return expf(-expf(z));
-}
 
 // A barrier for shared memory alone: loads and stores of global memory stay in flight.
 __device__ __forceinline__ void shared_memory_barrier() {

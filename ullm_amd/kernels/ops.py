@@ -727,6 +727,68 @@ def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.T
     return out
 
 
+DECAY_CHUNK = 16             # tokens a chunk of :func:`decay_chunks`
+DECAY_CHUNKS_FROM, DECAY_CHUNKS_MANY = 512, 1024
+
+
+def decay_in_chunks(longest: int, tokens: int) -> bool:
+    """Whether the recurrence of a step of ``tokens`` tokens, its longest portion of ``longest``, is worked in chunks
+    (:func:`decay_chunks`) or token by token (:func:`decay_scan`, what it prepares included).  Token by token costs a step of
+    the chain per token of the longest portion, in chunks an eighth of that and three passes over everything.  16 heads of
+    128 x 128, decays per head / per channel: one portion of 128, 256, 512, 2048 tokens 28 / 44, 51 / 82, 81 / 82, 295 / 308
+    us token by token and 49 / 54, 72 / 75, 77 / 80, 100 / 109 in chunks; eight of 128 69 / 63 and 56 / 60; four of 750
+    214 / 209 and 134 / 149.  32 heads of 64 x 64: 512 tokens 55 / 54 and 43 / 45, eight of 128 52 / 48 and 41 / 45, four
+    of 750 130 / 122 and 114 / 126."""
+    return longest >= DECAY_CHUNKS_FROM or (longest >= 128 and tokens >= DECAY_CHUNKS_MANY)
+
+
+def decay_chunks_supports(key_dim: int, value_dim: int) -> bool:
+    return bool(build.load("decay_chunks").ullm_decay_chunks_supports(_c_int(key_dim), _c_int(value_dim)))
+
+
+def decay_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, decay_kind: int, state: torch.Tensor,
+                 state_off: int, entry_slot: torch.Tensor, n_entries: int, heads: int, key_dim: int, value_dim: int, plan,
+                 tau: float = 1.0, bonus: Optional[torch.Tensor] = None, silu_inputs: bool = False, q_scale: float = 1.0,
+                 write_state: bool = True) -> torch.Tensor:
+    """:func:`decay_scan` for steps with long portions of prompts: every entry's tokens in chunks of ``DECAY_CHUNK``, runs of
+    chunks side by side (``plan``: the step plan of ``parts.decay.plan_decay_chunks``).  The sums are formed in another
+    order than the walk token by token; all 32-bit."""
+    T = q.shape[0]
+    _f32_rows(q, "q", T, heads * key_dim)
+    _f32_rows(k, "k", T, heads * key_dim)
+    _f32_rows(v, "v", T, heads * value_dim)
+    if decay_kind == DECAY_PER_HEAD:
+        _need(decay.dtype == torch.float32 and decay.numel() == heads and decay.is_contiguous(), "decay must be float32 [heads]")
+        z_ld = 0
+    else:
+        _need(decay_kind in (DECAY_SIGMOID_ROOT, DECAY_EXP_EXP, DECAY_READY), "unknown kind of decay")
+        _f32_rows(decay, "decay", T, heads * key_dim)
+        z_ld = decay.stride(0)
+    if bonus is not None:
+        _need(bonus.dtype == torch.float32 and bonus.numel() == heads * key_dim and bonus.is_contiguous(), "bonus must be float32 [heads, key_dim]")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1 and state_off >= 0
+          and state_off + heads * key_dim * value_dim <= state.shape[1], "state must be float32 [slots, row] holding the heads' states")
+    items, segments, entry_segment = plan.arrays["items"], plan.arrays["segments"], plan.arrays["entry_segment"]
+    n_chunks, n_segments = plan.facts["num_chunks"], plan.facts["num_segments"]
+    _i32(entry_slot, "entry_slot", n_entries)
+    _i32(items, "items", 2 * n_chunks)
+    _i32(segments, "segments", 5 * n_segments)
+    _i32(entry_segment, "entry_segment", n_entries)
+    f32 = dict(dtype=torch.float32, device=q.device)
+    chunks = torch.empty(n_chunks * heads * (33 * key_dim + 256), **f32)
+    several = plan.facts["several"]
+    carried = torch.empty(n_segments * heads * (key_dim * value_dim + key_dim), **f32) if several else None
+    out = torch.empty((T, heads * value_dim), **f32)
+    ll = ctypes.c_longlong
+    _check(build.load("decay_chunks").ullm_decay_chunks(
+        _p(q), _c_int(q.stride(0)), _p(k), _c_int(k.stride(0)), _p(v), _c_int(v.stride(0)), _p(decay), _c_int(z_ld),
+        _c_int(decay_kind), _c_float(tau), _p(bonus), _c_int(1 if silu_inputs else 0), _c_float(q_scale), _p(state),
+        ll(state.stride(0)), ll(state_off), _p(entry_slot), _p(items), _c_int(n_chunks), _p(segments), _c_int(n_segments),
+        _p(entry_segment), _c_int(1 if several else 0), _p(chunks), _p(carried), _p(out), _c_int(n_entries), _c_int(heads),
+        _c_int(key_dim), _c_int(value_dim), _c_int(1 if write_state else 0), _stream()), "decay_chunks")
+    return out
+
+
 DECAY_PREPARE_FROM = 16      # from this many tokens a step on, a pass of its own applies the inputs' functions
 
 

@@ -15,22 +15,55 @@ They differ in where q, k, v and the decays d come from and in what stands behin
 
 What a request keeps between steps is one float32 row per slot: the heads' states (for ``time_mix`` the last input
 row ahead of them).  The projections leave float32 rows also where the model computes in bfloat16, so everything
-that enters the recurrence is 32-bit; the recurrence walks an entry's tokens in order whatever the batch holds.
+that enters the recurrence is 32-bit; the recurrence walks an entry's tokens in order whatever the batch holds, in steps
+with long portions of prompts in chunks (``ops.decay_chunks``).
 """
 from __future__ import annotations
 
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from ..kernels import ops
-from .base import LayerCache, Mixer, PartEnv, StateNeed, StepContext, WeightDecl, register_part
+from .base import LayerCache, Mixer, PartEnv, StateNeed, StepContext, StepPlan, StepShape, WeightDecl, register_part
 from .linear import linear, linear_into_stream
+
+
+def chunk_plan(lens: Sequence[int]) -> StepPlan:
+    """Chunks (first token, tokens) of every entry's tokens, an entry's side by side; segments of them (entry, first chunk,
+    chunks, number in the entry, segments of the entry); every entry's first segment.  A segment has eight chunks, or what
+    makes sixteen of the step's where that is more: enough blocks for the chip, as few states between segments as can be."""
+    items: List[int] = []
+    segments: List[int] = []
+    entry_segment: List[int] = []
+    C = ops.DECAY_CHUNK
+    per_segment = max(8, -(-sum(-(-n // C) for n in lens) // 16))
+    t0 = 0
+    for b, n in enumerate(lens):
+        first, chunks = len(items) // 2, -(-n // C)
+        for i in range(chunks):
+            items += (t0 + C * i, min(C, n - C * i))
+        of = -(-chunks // per_segment)
+        entry_segment.append(len(segments) // 5)
+        for i in range(of):
+            segments += (b, first + per_segment * i, min(per_segment, chunks - per_segment * i), i, of)
+        t0 += n
+    i32 = lambda a: np.asarray(a, dtype=np.int32)       # noqa: E731
+    return StepPlan(arrays={"items": i32(items), "segments": i32(segments), "entry_segment": i32(entry_segment)},
+                    facts={"num_chunks": len(items) // 2, "num_segments": len(segments) // 5,
+                           "several": any(-(-n // C) > per_segment for n in lens)})
+
+
+def plan_decay_chunks(shape: StepShape) -> StepPlan:
+    """The chunks of a step whose recurrence is worked in chunks; none for any other step."""
+    return chunk_plan(shape.lens if ops.decay_in_chunks(max(shape.lens, default=0), sum(shape.lens)) else ())
 
 
 class _DecayMixer(Mixer):
     """What the three have in common: sizes, the state row, names."""
     DEFAULT_NAMES: Dict[str, str] = {}
+    step_planners = {"decay chunks": plan_decay_chunks}
 
     def __init__(self, hidden_size: int, heads: int, key_dim: int, value_dim: int, norm_eps: float, prefix: str,
                  names: Optional[Dict[str, str]] = None):
@@ -53,6 +86,14 @@ class _DecayMixer(Mixer):
     @staticmethod
     def _rows(cache: LayerCache) -> torch.Tensor:
         return cache.state.view(cache.state.shape[0], -1)
+
+    def kernel_families(self, dtype):
+        return ("decay_scan", "decay_chunks")
+
+    def _in_chunks(self, ctx: StepContext):
+        """The step's plan if the recurrence is worked in chunks: steps with long portions, sizes the chunks take."""
+        plan = ctx.plans["decay chunks"]
+        return plan if plan.facts["num_chunks"] and ops.decay_chunks_supports(self.key_dim, self.value_dim) else None
 
     @staticmethod
     def _ahead(x: torch.Tensor, ctx: StepContext) -> bool:
@@ -100,14 +141,20 @@ class GatedLinearAttention(_DecayMixer):
         z = linear(linear(x, self.w_a1, out_dtype=torch.float32), self.w_a2, self.b_a2, out_dtype=torch.float32)
         qk, inner = self.qk, self.inner
         kind = ops.DECAY_SIGMOID_ROOT
-        if self._ahead(x, ctx):
-            # many tokens: the decays' function is applied once per value ahead of the recurrence, not by each of its blocks
-            ops.decay_prepare(None, z, kind, self.tau)
-            kind = ops.DECAY_READY
-        o = ops.decay_scan(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], z, kind,
-                           self._rows(cache), 0, ctx.q_start, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim,
-                           self.value_dim, tau=self.tau, q_scale=self.key_dim ** -0.5, write_state=cache.owner,
-                           max_len=ctx.max_q_len)
+        plan = self._in_chunks(ctx)
+        if plan is not None:
+            o = ops.decay_chunks(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], z, kind, self._rows(cache), 0,
+                                 ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim, self.value_dim, plan, tau=self.tau,
+                                 q_scale=self.key_dim ** -0.5, write_state=cache.owner)
+        else:
+            if self._ahead(x, ctx):
+                # many tokens: the decays' function is applied once per value ahead of the recurrence, not by each of its blocks
+                ops.decay_prepare(None, z, kind, self.tau)
+                kind = ops.DECAY_READY
+            o = ops.decay_scan(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], z, kind,
+                               self._rows(cache), 0, ctx.q_start, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim,
+                               self.value_dim, tau=self.tau, q_scale=self.key_dim ** -0.5, write_state=cache.owner,
+                               max_len=ctx.max_q_len)
         y = ops.gated_unit_norm(o, proj[:, 2 * qk + inner:], self.gain, self.norm_eps, self.heads, ops.GATE_SILU, ctx.dtype)
         return linear_into_stream(y, self.w_o, ctx)
 
@@ -142,12 +189,18 @@ class LightningAttention(_DecayMixer):
     def forward(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         proj = linear(x, self.w_in, out_dtype=torch.float32)                        # q | k | v | g
         qk, inner = self.qk, self.inner
-        ahead = self._ahead(x, ctx)
-        if ahead:
-            ops.decay_prepare(proj[:, :2 * qk + inner])              # silu of q | k | v once per value
-        o = ops.decay_scan(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], self.decay, ops.DECAY_PER_HEAD,
-                           self._rows(cache), 0, ctx.q_start, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim,
-                           self.value_dim, silu_inputs=not ahead, write_state=cache.owner, max_len=ctx.max_q_len)
+        plan = self._in_chunks(ctx)
+        if plan is not None:
+            o = ops.decay_chunks(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], self.decay, ops.DECAY_PER_HEAD,
+                                 self._rows(cache), 0, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim, self.value_dim,
+                                 plan, silu_inputs=True, write_state=cache.owner)
+        else:
+            ahead = self._ahead(x, ctx)
+            if ahead:
+                ops.decay_prepare(proj[:, :2 * qk + inner])          # silu of q | k | v once per value
+            o = ops.decay_scan(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], self.decay, ops.DECAY_PER_HEAD,
+                               self._rows(cache), 0, ctx.q_start, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim,
+                               self.value_dim, silu_inputs=not ahead, write_state=cache.owner, max_len=ctx.max_q_len)
         y = ops.gated_unit_norm(o, proj[:, 2 * qk + inner:], self.gain, self.norm_eps, 1, ops.GATE_SIGMOID, ctx.dtype)
         return linear_into_stream(y, self.w_o, ctx)
 
@@ -195,12 +248,17 @@ class TimeMix(_DecayMixer):
         g = linear(blends[3], self.w_g, out_dtype=f32)
         z = linear(linear(blends[4], self.w_w1, out_dtype=f32, act=ops.ACT_TANH), self.w_w2, self.w0, out_dtype=f32)
         kind = ops.DECAY_EXP_EXP
-        if self._ahead(x, ctx):
-            ops.decay_prepare(None, z, kind)
-            kind = ops.DECAY_READY
-        o = ops.decay_scan(r, k, v, z, kind, rows, self.carry, ctx.q_start, ctx.entry_slot, ctx.num_entries,
-                           self.heads, self.key_dim, self.value_dim, bonus=self.bonus, write_state=cache.owner,
-                           max_len=ctx.max_q_len)
+        plan = self._in_chunks(ctx)
+        if plan is not None:
+            o = ops.decay_chunks(r, k, v, z, kind, rows, self.carry, ctx.entry_slot, ctx.num_entries, self.heads, self.key_dim,
+                                 self.value_dim, plan, bonus=self.bonus, write_state=cache.owner)
+        else:
+            if self._ahead(x, ctx):
+                ops.decay_prepare(None, z, kind)
+                kind = ops.DECAY_READY
+            o = ops.decay_scan(r, k, v, z, kind, rows, self.carry, ctx.q_start, ctx.entry_slot, ctx.num_entries,
+                               self.heads, self.key_dim, self.value_dim, bonus=self.bonus, write_state=cache.owner,
+                               max_len=ctx.max_q_len)
         y = ops.gated_unit_norm(o, g, self.gain, self.norm_eps, self.heads, ops.GATE_SILU, ctx.dtype)
         return linear_into_stream(y, self.w_o, ctx)
 
