@@ -10,7 +10,10 @@
 // One wave's instructions keep the matrix pipe busy: the operands of one half of a stage (32 values of K) are read into
 // registers between the products of the half before, and the loads of a stage further on are issued between the products of
 // the second half, behind the one barrier of a stage, which stands where the operands of the half that follows it are in
-// registers already.
+// registers already.  With eight waves, two a unit, the reads stand beside the first six of a half's eight groups of products,
+// so that they are back before the barrier, and a wave between its products lets the other go first: 8192 x 4096 x 12288 625 ->
+// 564 us, 8192 x 6144 x 4096 303 -> 292 us; with four waves that order is 1 to 4 % slower.  Also tried at the first of these sizes:
+// waves of 128 x 128 (one a unit) 725 us, products of 32 x 32 x 16 647 us, stages of 32 values of K, four or five of them, 618 us.
 #pragma once
 #include <type_traits>
 #include "common.h"
@@ -22,6 +25,19 @@ union TilePack {
   tile_bf16x8 v;
   uint4 u4;
 };
+
+// A lane's packed bfloat16 values of two neighbouring 16 x 16 products (columns 4 g .. 4 g + 3 of each, a the left one's) as eight
+// columns of one of them, from pair_column(g) of the left one's first on: whole lines of 64 bytes a row instead of halves.
+__device__ __forceinline__ uint4 pair_columns(const uint2& a, const uint2& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto p = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false);
+  const auto q = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+  return make_uint4(p[0], q[0], p[1], q[1]);
+#else
+  return make_uint4(a.x, a.y, b.x, b.y);
+#endif
+}
+__device__ __forceinline__ int pair_column(int g) { return 16 * (g & 1) + 4 * (g & 2); }
 
 template <int WMW, int STAGES_>
 struct ProductTiles {
@@ -63,9 +79,24 @@ struct ProductTiles {
 #pragma unroll
       for (int m = 0; m < TM; ++m) acc[n][m] = tile_f32x4{0.f, 0.f, 0.f, 0.f};
     TilePack x[2][TM], w[2][TN];
+    // the reads of half s that stand beside its predecessor's n-th group of products
+    auto operands = [&](const unsigned char* st, int s, int n) __attribute__((always_inline)) {
+      if constexpr (WAVES == 8) {
+#pragma unroll
+        for (int q = 2 * n; q < 2 * n + 2; ++q) {
+          if (q < TM) x[s][q].u4 = read_x(st, s, q);
+          else if (q < TM + TN) w[s][q - TM].u4 = read_w(st, s, q - TM);
+        }
+      } else {
+        if (n < TM) x[s][n].u4 = read_x(st, s, n);
+        w[s][n].u4 = read_w(st, s, n);
+      }
+    };
     auto products = [&](int s, int n) __attribute__((always_inline)) {
+      if constexpr (WAVES == 8) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int m = 0; m < TM; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][n].v, x[s][m].v, acc[n][m], 0, 0, 0);
+      if constexpr (WAVES == 8) __builtin_amdgcn_s_setprio(0);
     };
 #pragma unroll
     for (int i = 0; i < STAGES; ++i)
@@ -86,8 +117,7 @@ struct ProductTiles {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
-        if (n < TM) x[1][n].u4 = read_x(st, 1, n);
-        w[1][n].u4 = read_w(st, 1, n);
+        operands(st, 1, n);
         products(0, n);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -100,8 +130,7 @@ struct ProductTiles {
       const unsigned char* const nx = lds + buf * STAGE;
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
-        if (n < TM) x[0][n].u4 = read_x(nx, 0, n);
-        w[0][n].u4 = read_w(nx, 0, n);
+        operands(nx, 0, n);
         if constexpr (decltype(loads)::value) {
 #pragma unroll
           for (int j = n * LOADS / TN; j < (n + 1) * LOADS / TN; ++j) load(j, to);

@@ -677,7 +677,8 @@ moe_tiles_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restri
 // What bounds it: the experts' matrices from memory (268 MB of gate|up: 45 us) and, beside them, the matrix pipe, which the
 // loop keeps busy 57 % of the time where every operand lies in the second-level cache.  32 experts, top 4, width 2048, 1024
 // columns an expert, against the kernel above: gate|up at 2048 / 3000 / 8192 tokens 160 / 217 / 470 -> 117 / 140 / 279 us (590 /
-// 720 / 987 TFLOP/s), down 87 / 120 / 270 -> 73 / 87 / 206 us.  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a
+// 720 / 987 TFLOP/s), down 87 / 120 / 270 -> 73 / 87 / 206 us.  (Replayed back to back the tiles of 256 rows take 108 + 70 us at
+// 3000 and 267 + 192 at 8192 tokens.)  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a
 // stage ahead of its products took 127 to 150 us at 2048 tokens, whatever the number of stages; a wave of its own that asked
 // for the matrix's lines ahead of time made them slower (180 us).
 template <int WMW, int STAGES, bool GATED>
@@ -716,10 +717,28 @@ moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
          K >> 6, wave, lane, 128, acc);
   // lane (r, g): row r of each 16-row group, four consecutive columns at 4g
   const int wm = wave >> 1, wn = wave & 1;
+  const bool whole = ((n_out | ldo) & 7) == 0 && !((uintptr_t)out_ & 15);
 #pragma unroll
   for (int m = 0; m < T::TM; ++m) {
     const int row = 64 * wm + 16 * m + r;
     if (row >= rows) continue;
+    if (GATED && whole) {
+#pragma unroll
+      for (int n = 0; n < 4; n += 2) {
+        uint2 u[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n + h][m][i], acc[n + h + 4][m][i], limit, alpha);
+          u[h] = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        }
+        const uint4 both = pair_columns(u[0], u[1]);
+        const int c = n0 + 64 * wn + 16 * n + pair_column(g);
+        if (c < n_out) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(out_) + (size_t)(slot0 + row) * ldo + c) = both;
+      }
+      continue;
+    }
 #pragma unroll
     for (int n = 0; n < (GATED ? 4 : 8); ++n) {
       const int c = n0 + 64 * wn + 16 * (n & 3) + 4 * g + (n < 4 ? 0 : 128);
