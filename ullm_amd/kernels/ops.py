@@ -1249,6 +1249,61 @@ def gemm_rows(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     return out
 
 
+TILES_STORE, TILES_GATED, TILES_FLOAT = 0, 1, 2
+
+
+def gemm_tiles_rows(M: int, N: int, K: int, gated: bool) -> int:
+    """The 64-row groups a block of :func:`gemm_tiles` should take for x [M, K] times W [N, K] (``gated``: gate and up rows), or
+    0 where the library's product (gated: and the activation kernel behind it) is ahead.
+
+    Ungated the library's best kernels are 5 to 10 % ahead, but from 8192 to 12288 rows it takes others.  Library and this, us:
+    4096 x 4096 8448 / 10 000 / 12 000 rows 319 / 365 / 449 and 260 / 270 / 289, 4096 x 12288 876 / 975 / 1160 and 830 / 892 / 896,
+    6144 x 4096 393 / 355 / 556 and 357 / 366 / 456; 8000 rows 176 and 190 (4096 x 4096), 16 384 rows 354 and 395.
+
+    Gated the activation's pass is saved, worth the more the shorter K is, and what decides is how full the rounds of blocks over
+    256 compute units are, rows and columns of the last tiles included (a round of 128-row tiles takes 0.65 of one of 256 rows).
+    Library and this, 24576 x 4096 at 192 / 256 / 350 / 450 / 700 / 1000 / 1300 / 2048 / 3000 / 6000 / 11 000 rows: 53 / 59 / 73 / 88 / 146 /
+    171 / 226 / 292 / 604 / 886 / 1649 and 58 / 57 / 82 / 82 / 157 / 165 / 256 / 278 / 467 / 882 / 1593 us, shares of 0.43, 0.58, 0.51, 0.66,
+    0.53, 0.75, 0.64, 1, 0.88, 0.98, 0.90; 6144 x 1024 at 350 / 700 / 1300 / 2048 / 2600 / 4000 / 11 000 rows: 19 / 23 / 29 / 36 / 45 / 65 / 177
+    and 19 / 20 / 27 / 28 / 38 / 55 / 129 us, shares of 0.20, 0.39, 0.48, 0.75, 0.73, 0.75, 0.80 (0.48 in two rounds, 45 and 52 us)."""
+    def rounds(groups):
+        return -(-(-(-M // (64 * groups)) * -(-N // 256)) // 256)
+    if not gated:
+        return 4 if 8192 < M < 12288 and 512 <= -(-M // 256) * -(-N // 256) <= 1200 else 0
+    if M < 160 or N < 1:
+        return 0
+    groups, cost = min(((4, rounds(4)), (2, 0.65 * rounds(2))), key=lambda c: c[1])
+    least = (0.62 if rounds(groups) == 1 else 0.84) - 0.27 * min(1.0, 1024 / K)
+    return groups if M * N / (2 ** 24 * cost) >= least else 0
+
+
+def gemm_tiles_supports(x: torch.Tensor, w: torch.Tensor, mode: int = TILES_STORE) -> bool:
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and bool(build.load("gemm_tiles").ullm_gemm_tiles_supports(_c_int(x.shape[0]), _c_int(w.shape[0]), _c_int(x.shape[1]),
+                                                                       _c_int(x.stride(0)), _c_int(w.stride(0)), _c_int(mode))))
+
+
+def gemm_tiles(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, gated: bool = False,
+               out_dtype: torch.dtype = torch.bfloat16, groups: int = 4, limit: float = 0.0,
+               alpha: float = 0.0) -> torch.Tensor:
+    """x [M, K] times w [N, K] transposed, bfloat16 with 32-bit sums, in tiles of 64 ``groups`` (2 or 4) rows by 256 of w:
+    bfloat16 (+ ``bias``) or float32; ``gated``: w holds gate rows, then as many up rows, and the result is silu(gate) * up or
+    with ``limit`` > 0 the clamped unit."""
+    M, K = x.shape
+    N, K2 = w.shape
+    mode = TILES_GATED if gated else TILES_FLOAT if out_dtype == torch.float32 else TILES_STORE
+    _need(K == K2, "inner sizes differ")
+    _need(gemm_tiles_supports(x, w, mode), "operands outside what the kernel takes")
+    _need(bias is None or (mode == TILES_STORE and bias.dtype == torch.float32 and bias.numel() == N and bias.is_contiguous()),
+          "bias must be float32 [N], and joins the bfloat16 result only")
+    out = torch.empty((M, N // 2 if gated else N), dtype=torch.float32 if mode == TILES_FLOAT else torch.bfloat16, device=x.device)
+    _check(build.load("gemm_tiles").ullm_gemm_tiles(
+        _p(x), _c_int(x.stride(0)), _p(w), _c_int(w.stride(0)), _p(bias), _p(out), _c_int(out.shape[1]), _c_int(M), _c_int(N), _c_int(K),
+        _c_int(mode), _c_int(groups), _c_float(limit), _c_float(alpha), _stream()), "gemm_tiles")
+    return out
+
+
 # torch.mm(..., out_dtype=float32) stores the 32-bit accumulator of a bfloat16 product; older torch lacks it
 _MM_TAKES_OUT_DTYPE = "out_dtype" in (torch.mm.__doc__ or "")
 
@@ -1257,7 +1312,8 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
               out_dtype: Optional[torch.dtype] = None, act: Optional[int] = None) -> torch.Tensor:
     """bfloat16 operands, 32-bit accumulation.  Few rows go to the weight-streaming kernels (up to how many
     for this matrix: :func:`dispatch.limits`), some more, where that was measured to be ahead, to the partial-sums
-    kernel and a kernel that adds its stacks; many rows go through the library product (as the reference's
+    kernel and a kernel that adds its stacks; very many rows, where their tiles fill the chip, go to the large product
+    (:func:`gemm_tiles_rows`); the rest go through the library product (as the reference's
     linears do, ullm/layers/linear.py:165), which for 32-bit output (logits) stores the accumulator unrounded.
     ``act`` (ACT_RELU2, ACT_GELU_TANH): that activation of the result, on store in the few-rows and rows kernels, by
     the activation kernel behind the others."""
@@ -1281,6 +1337,13 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     if (out_dtype == torch.bfloat16 and 0 < lim.sums_from <= M <= lim.sums_to and w.shape[0] % 4 == 0
             and gemm_partial_sums_supports(a, w)):
         return sum_stacks(gemm_partial_sums(a, w), bias)
+    if library and out_dtype in (torch.bfloat16, torch.float32):
+        groups = gemm_tiles_rows(M, w.shape[0], w.shape[1], False)
+        if groups and gemm_tiles_supports(a, w):
+            if out_dtype == torch.bfloat16:
+                return gemm_tiles(a, w, bias, groups=groups)
+            y = gemm_tiles(a, w, out_dtype=torch.float32, groups=groups)
+            return y if bias is None else add_bias(y, bias)
     if library and out_dtype == torch.float32 and a.stride(1) == 1 and w.is_contiguous() and _MM_TAKES_OUT_DTYPE:
         y = torch.mm(a, w.t(), out_dtype=torch.float32)
         return y if bias is None else add_bias(y, bias)
