@@ -51,3 +51,36 @@ def test_experts_with_rows_at_every_edge(ops, tile_rows, K, n_out, limit):
     slot2, token2, tiles2, _ = ops.moe_sort(ids, experts, other)
     again = ops.moe_rows(x[token2.long()].contiguous(), None, w, tiles2, other, T, gated=False)
     assert torch.equal(again[slot2.long()], plain[slot.long()])
+
+
+@pytest.mark.parametrize("tile_rows", [16, 32])
+@pytest.mark.parametrize("K,n_out", [(256, 40), (320, 16), (448, 129), (704, 34), (1024, 4), (200, 48)])
+@pytest.mark.parametrize("limit", [0.0, 1.5])
+def test_few_rows_an_expert(ops, tile_rows, K, n_out, limit):
+    """Each wave's share of K one to several stages long, rows on both sides of a tile's edge, columns past the last block's."""
+    g = torch.Generator().manual_seed(K + n_out + tile_rows)
+    counts = [1, 0, 15, 16, 17, 31, 32, 33]
+    experts, T = len(counts), sum(counts)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=g)].int()[:, None].contiguous().to(DEV)
+    x = torch.randn(T, K + 8, generator=g).bfloat16().to(DEV)[:, :K]
+    w_gu = (torch.randn(experts, 2 * n_out, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    w = (torch.randn(experts, n_out, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    slot, token, tiles, offsets = ops.moe_sort(ids, experts, tile_rows)
+    gated = ops.moe_rows(x, token, w_gu, tiles, tile_rows, T, gated=True, limit=limit, alpha=1.3)
+    by_slot = x[token.long()].contiguous()
+    plain = ops.moe_rows(by_slot, None, w, tiles, tile_rows, T, gated=False)
+    at = offsets.cpu().tolist()
+    for e, n in enumerate(counts):
+        rows = slice(at[e], at[e] + n)
+        h = by_slot[rows].double()
+        size = h.abs() @ w[e].double().abs().T
+        assert ((plain[rows].double() - h @ w[e].double().T).abs() <= (K + 1) * 2.0 ** -24 * size).all()    # K 32-bit sums
+        gu = h @ w_gu[e].double().T
+        a, u = gu[:, :n_out], gu[:, n_out:]
+        if limit:
+            a, u = a.clamp(max=limit), u.clamp(-limit, limit)
+            want = a * torch.sigmoid(1.3 * a) * (u + 1)
+        else:
+            want = a * torch.sigmoid(a) * u
+        off = (K + 8) * 2.0 ** -24 * (h.abs() @ w_gu[e].double().abs().T).max() * (4 + u.abs() + a.abs()) if n else 0.0
+        assert ((gated[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + off).all()

@@ -43,6 +43,12 @@ __device__ __forceinline__ void loads_left() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 #endif
 }
+// This wave's reads of shared memory have returned.
+__device__ __forceinline__ void reads_done() {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+#endif
+}
 // Every wave of the block has read what it read of shared memory before this and may write it from here on; loads on
 // their way stay on their way.
 __device__ __forceinline__ void bare_barrier() {

@@ -398,6 +398,40 @@ moe_rows_simple_kernel(const T* __restrict__ x, int ldx, const int* __restrict__
   }
 }
 
+// Lane (r, g): row r of each 16-row group, columns c .. c + 3.
+template <int MT, bool GATED>
+__device__ __forceinline__ void moe_store_rows(const f32x4_t (&acc_g)[MT], const f32x4_t (&acc_u)[MT], void* out_, int ldo, int slot0,
+                                               int rows, int c, int r, int n_out, float limit, float alpha) {
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int row = 16 * t + r;
+    if (row >= rows) continue;
+    const size_t at = (size_t)(slot0 + row) * ldo + c;
+    if (GATED) {
+      bf16_t* o = reinterpret_cast<bf16_t*>(out_) + at;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc_g[t][i], acc_u[t][i], limit, alpha);
+      if (c + 3 < n_out && (ldo & 3) == 0) {
+        *reinterpret_cast<uint2*>(o) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (c + i < n_out) o[i] = f32_to_bf16_bits(v[i]);
+      }
+    } else {
+      float* o = reinterpret_cast<float*>(out_) + at;
+      if (c + 3 < n_out && (ldo & 3) == 0) {
+        *reinterpret_cast<float4*>(o) = make_float4(acc_g[t][0], acc_g[t][1], acc_g[t][2], acc_g[t][3]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (c + i < n_out) o[i] = acc_g[t][i];
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------- products on the matrix cores
 // Few rows a tile (single tokens of a step): grid (tiles, groups of 16 output columns); tile = up to 16 * MT grouped
 // rows of one expert.  The block's four waves share the 16 columns (GATED: the 16 gate rows and the 16 up rows of
@@ -479,36 +513,111 @@ moe_rows_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restric
         acc_g[t][i] += part[v][(GATED ? 8 : 4) * t + i][lane];
         if (GATED) acc_u[t][i] += part[v][8 * t + 4 + i][lane];
       }
-  // lane (r, g): row r of each 16-row group, columns n0 + 4g .. + 4
-  const int c = n0 + 4 * g;
+  moe_store_rows<MT, GATED>(acc_g, acc_u, out_, ldo, slot0, rows, n0 + 4 * g, r, n_out, limit, alpha);
+}
+
+// The same where K is a multiple of 64 and at least 256: a wave takes a run of K of its own (a quarter), so that it reads each
+// of the block's rows of the matrix in one piece, and its stages of 64 values (16 or, gated, 32 rows of the matrix and the tile's
+// rows of x, whole lines of 128 bytes) go straight to shared memory of its own, two taking turns (lds_load.h): no barrier, and
+// nothing but addresses in registers while 8 to 16 KB a wave are on their way.  What bounds it is the experts' matrices from
+// memory (gate|up of 32 experts, width 2048, 1024 columns: 268 MB, 43 us).  The kernel above asks for 64 bytes of a row at a time
+// and holds them in registers; gate|up + down at 8 / 48 / 100 / 190 / 300 tokens, 4 experts each, 52 + 23 / 61 + 33 / 81 + 45 / 134 + 78 / 154 +
+// 91 us there, 40 + 19 / 51 + 30 / 55 + 33 / 81 + 49 / 84 + 59 us here (three stages, and a block less on each compute unit:
+// 40 + 21 / 52 + 30 / 55 + 34 / 82 + 49 / 106 + 66).
+template <int MT, bool GATED>
+__global__ void __launch_bounds__(256)
+moe_rows_dma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
+                    const bf16_t* __restrict__ w, const int* __restrict__ tiles, void* __restrict__ out_, int ldo,
+                    int n_out, int K, float limit, float alpha) {
+  constexpr int VALS = (GATED ? 8 : 4) * MT, WR = GATED ? 32 : 16, ROWS = WR + 16 * MT, LOADS = ROWS / 8, STAGE = ROWS * 128;
+  extern __shared__ __attribute__((aligned(16))) unsigned char row_stages[];
+  const int tile = blockIdx.x, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = tiles[3 * tile], slot0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  if (rows <= 0) return;
+  const int n0 = blockIdx.y * 16;
+  const size_t w_rows = GATED ? 2 * (size_t)n_out : (size_t)n_out;
+  const int stages = K >> 6, s0 = stages * wave / 4, s1 = stages * (wave + 1) / 4;
+  // an instruction of 64 lanes fills 8 rows of a stage; piece c of row r lies at piece c ^ ((r >> 1) & 7)
+  const bf16_t* src[LOADS];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int row = 16 * t + r;
-    if (row >= rows) continue;
-    const size_t at = (size_t)(slot0 + row) * ldo + c;
-    if (GATED) {
-      bf16_t* o = reinterpret_cast<bf16_t*>(out_) + at;
-      float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc_g[t][i], acc_u[t][i], limit, alpha);
-      if (c + 3 < n_out && (ldo & 3) == 0) {
-        *reinterpret_cast<uint2*>(o) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (c + i < n_out) o[i] = f32_to_bf16_bits(v[i]);
-      }
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = 8 * i + (lane >> 3), piece = 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    if (i < WR / 8) {
+      const int n = n0 + (row & 15) < n_out ? n0 + (row & 15) : n_out - 1;
+      src[i] = w + ((size_t)e * w_rows + (row >= 16 ? n_out : 0) + n) * K + 64 * s0 + piece;
     } else {
-      float* o = reinterpret_cast<float*>(out_) + at;
-      if (c + 3 < n_out && (ldo & 3) == 0) {
-        *reinterpret_cast<float4*>(o) = make_float4(acc_g[t][0], acc_g[t][1], acc_g[t][2], acc_g[t][3]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (c + i < n_out) o[i] = acc_g[t][i];
-      }
+      const int m = row - WR < rows ? row - WR : rows - 1;
+      src[i] = x + (size_t)(row_index ? row_index[slot0 + m] : slot0 + m) * ldx + 64 * s0 + piece;
     }
   }
+  unsigned char* const mine = row_stages + 2 * STAGE * wave;
+  auto fetch = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      load16_to_lds(src[i], mine + buf * STAGE + i * 1024);
+      src[i] += 64;
+    }
+  };
+  f32x4_t acc_g[MT], acc_u[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    acc_g[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    acc_u[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  const int n_stages = s1 - s0;                          // at least one
+  for (int i = 0; i < 2 && i < n_stages; ++i) fetch(i);
+  int buf = 0;
+  for (int k = 0; k < n_stages; ++k) {
+    if (k + 1 < n_stages) loads_left<LOADS>();           // those of the stage behind this one
+    else loads_left<0>();
+    const unsigned char* const st = mine + buf * STAGE;
+    Pack8 a_g[2], a_u[2], b[2][MT];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int at = r * 128 + (((4 * s + g) ^ ((r >> 1) & 7)) << 4);
+      a_g[s].u4 = ld16(st + at);
+      if (GATED) a_u[s].u4 = ld16(st + 2048 + at);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) b[s][t].u4 = ld16(st + WR * 128 + t * 2048 + at);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        acc_g[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_g[s].v, b[s][t].v, acc_g[t], 0, 0, 0);
+        if (GATED) acc_u[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_u[s].v, b[s][t].v, acc_u[t], 0, 0, 0);
+      }
+    if (k + 2 < n_stages) {
+      reads_done();
+      fetch(buf);
+    }
+    buf ^= 1;
+  }
+  // the waves' sums, added in wave order (no wave reads a stage any more)
+  __syncthreads();
+  float (*const part)[VALS][64] = reinterpret_cast<float (*)[VALS][64]>(row_stages);
+  if (wave > 0) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        part[wave - 1][(GATED ? 8 : 4) * t + i][lane] = acc_g[t][i];
+        if (GATED) part[wave - 1][8 * t + 4 + i][lane] = acc_u[t][i];
+      }
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int v = 0; v < 3; ++v)
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc_g[t][i] += part[v][(GATED ? 8 : 4) * t + i][lane];
+        if (GATED) acc_u[t][i] += part[v][8 * t + 4 + i][lane];
+      }
+  moe_store_rows<MT, GATED>(acc_g, acc_u, out_, ldo, slot0, rows, n0 + 4 * g, r, n_out, limit, alpha);
 }
 
 // Many rows a tile (prompt portions): a block per (tile, 128 rows of the expert's matrix); tile = up to 16 MT = 64 or 128
@@ -784,6 +893,12 @@ static void launch_tiles(dim3 grid, hipStream_t stream, Args... args) {
   hipLaunchKernelGGL((moe_tiles_mfma_kernel<MT, GATED>), grid, dim3(256), bytes, stream, args...);
 }
 
+template <int MT, bool GATED, typename... Args>
+static void launch_rows_dma(dim3 grid, hipStream_t stream, Args... args) {
+  constexpr int bytes = 4 * 2 * ((GATED ? 32 : 16) + 16 * MT) * 128;          // 32, 48 or 64 KB
+  hipLaunchKernelGGL((moe_rows_dma_kernel<MT, GATED>), grid, dim3(256), bytes, stream, args...);
+}
+
 template <int WMW, int STAGES, bool GATED, typename... Args>
 static void launch_products(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int bytes = ProductTiles<WMW, STAGES>::BYTES;
@@ -831,6 +946,13 @@ extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const
     }
     dim3 grid(max_tiles, (n_out + 15) / 16), block(256);
     if (grid.y > 65535) return ULLM_ERR_SHAPE;
+    if (K % 64 == 0 && K >= 256) {
+#define GO(MT, G) launch_rows_dma<MT, G>(grid, stream, (const bf16_t*)x, ldx, row_index, (const bf16_t*)w, tiles, out, ldo, n_out, K, limit, alpha)
+      if (tile_rows == 16) { if (gated) GO(1, true); else GO(1, false); }
+      else { if (gated) GO(2, true); else GO(2, false); }
+#undef GO
+      ULLM_LAUNCH_CHECK();
+    }
 #define GO(MT, G) hipLaunchKernelGGL((moe_rows_mfma_kernel<MT, G>), grid, block, 0, stream, (const bf16_t*)x, ldx, row_index, \
     (const bf16_t*)w, tiles, out, ldo, n_out, K, limit, alpha)
     if (tile_rows == 16) { if (gated) GO(1, true); else GO(1, false); }
