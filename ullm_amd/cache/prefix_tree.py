@@ -38,9 +38,14 @@ class PrefixTree:
         self.num_nodes = 0
 
     def _keys(self, tokens: Sequence[int], limit: int):
+        """The whole pages of ``tokens[:limit]`` as tuples of Python integers, sixteen pages looked at a time."""
         P = self.page_size
-        for i in range(limit // P):
-            yield tuple(int(t) for t in tokens[i * P:(i + 1) * P])
+        for start in range(0, limit // P * P, 16 * P):
+            run = tokens[start:min(start + 16 * P, limit // P * P)]
+            if type(run) is not list or set(map(type, run)) != {int}:      # the engine's lists need no conversion
+                run = [int(t) for t in run]
+            for i in range(0, len(run), P):
+                yield tuple(run[i:i + P])
 
     def match(self, tokens: Sequence[int], limit: int) -> List[List[int]]:
         """Pages of the longest cached prefix of ``tokens[:limit]`` made of whole pages:

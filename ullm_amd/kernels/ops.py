@@ -5,6 +5,7 @@ A non-zero return of a launcher raises ``KernelError``; nothing falls back to an
 from __future__ import annotations
 
 import ctypes
+import functools
 import logging
 from typing import Optional
 
@@ -13,6 +14,7 @@ import torch
 from . import build, dispatch
 
 F32, BF16 = 0, 1
+_raw_stream, _device = torch._C._cuda_getCurrentRawStream, torch.cuda.current_device
 logger = logging.getLogger("ullm_amd")
 
 
@@ -39,11 +41,12 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """torch's current stream of the current device (asked for without building a Stream object)."""
+    return _c_ptr(_raw_stream(_device()))
 
 
-def _p(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _p(t: Optional[torch.Tensor]) -> Optional[ctypes.c_void_p]:
+    return None if t is None else _c_ptr(t.data_ptr())
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -52,22 +55,24 @@ def _need(cond: bool, msg: str) -> None:
 
 
 def _i32(t: torch.Tensor, name: str, n: Optional[int] = None) -> None:
-    _need(t.dtype == torch.int32 and t.is_contiguous(), f"{name} must be contiguous int32")
-    if n is not None:
-        _need(t.numel() >= n, f"{name} holds {t.numel()} entries, {n} needed")
+    # the messages are formed only where they are needed: these checks stand in front of every launch
+    if t.dtype != torch.int32 or not t.is_contiguous():
+        raise KernelError(f"{name} must be contiguous int32")
+    if n is not None and t.numel() < n:
+        raise KernelError(f"{name} holds {t.numel()} entries, {n} needed")
 
 
-_c_int, _c_float = ctypes.c_int, ctypes.c_float
+# a Python int is passed to a C function as a C int as it is, None as a null pointer
+_c_int, _c_float, _c_ptr = int, ctypes.c_float, ctypes.c_void_p
 
 
 def _check_pools(k_pool, v_pool, nkv: int, page_size: int, hd: int, dtype) -> None:
     """Keys are [pages, nkv, page_size, hd]; values are kept transposed inside a page: [pages, nkv, hd, page_size]."""
-    _need(k_pool is not None and k_pool.dim() == 4 and tuple(k_pool.shape[1:]) == (nkv, page_size, hd)
-          and k_pool.is_contiguous() and k_pool.dtype == dtype,
-          f"k_pool must be contiguous [pages, {nkv}, {page_size}, {hd}] of {dtype}")
-    _need(v_pool is not None and v_pool.dim() == 4 and tuple(v_pool.shape[1:]) == (nkv, hd, page_size)
-          and v_pool.is_contiguous() and v_pool.dtype == dtype and v_pool.shape[0] == k_pool.shape[0],
-          f"v_pool must be contiguous [pages, {nkv}, {hd}, {page_size}] of {dtype}")
+    if not (k_pool is not None and k_pool.shape[1:] == (nkv, page_size, hd) and k_pool.dtype == dtype and k_pool.is_contiguous()):
+        raise KernelError(f"k_pool must be contiguous [pages, {nkv}, {page_size}, {hd}] of {dtype}")
+    if not (v_pool is not None and v_pool.shape[1:] == (nkv, hd, page_size) and v_pool.dtype == dtype and v_pool.is_contiguous()
+            and v_pool.shape[0] == k_pool.shape[0]):
+        raise KernelError(f"v_pool must be contiguous [pages, {nkv}, {hd}, {page_size}] of {dtype}")
 
 
 # ---------------------------------------------------------------------------------- elementwise
@@ -1355,6 +1360,7 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     return gemm_simple(a, w, bias, out_dtype=out_dtype)
 
 
+@functools.lru_cache(maxsize=256)          # of sizes alone, and asked for by every layer of every step
 def attention_mfma_supports(dtype: torch.dtype, hd: int, page_size: int, nq: int, nkv: int) -> bool:
     """True if the matrix-core attention kernels take this shape (bfloat16, head_dim in
     {32, 64, 96, 128, 256}, page size a multiple of 16)."""
@@ -1460,6 +1466,7 @@ def attention_decode_mfma(q, out, k_pool, v_pool, token_list: Optional[torch.Ten
         _c_int(splits), _c_int(waves), _p(ws), _stream()), "attention_decode")
 
 
+@functools.lru_cache(maxsize=256)
 def attention_decode_fused_supports(dtype: torch.dtype, hd: int, page_size: int, nq: int, nkv: int,
                                     rotary_dim: int, style: int) -> bool:
     """Whether the decode kernel can also do the step's per-head norm, rotation and cache write."""
