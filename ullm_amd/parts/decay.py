@@ -57,7 +57,8 @@ def chunk_plan(lens: Sequence[int]) -> StepPlan:
 
 def plan_decay_chunks(shape: StepShape) -> StepPlan:
     """The chunks of a step whose recurrence is worked in chunks; none for any other step."""
-    return chunk_plan(shape.lens if ops.decay_in_chunks(max(shape.lens, default=0), sum(shape.lens)) else ())
+    chunks = min(shape.lens, default=0) > 0 and ops.decay_in_chunks(max(shape.lens), sum(shape.lens))      # an entry has a segment or more
+    return chunk_plan(shape.lens if chunks else ())
 
 
 class _DecayMixer(Mixer):

@@ -38,14 +38,25 @@ DEFAULT_NAMES = {"router": "router", "correction": "correction", "expert": "e{in
 
 def tile_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int = 0) -> int:
     """Grouped rows a block of the expert products takes, from the rows an expert gets on average: a function of
-    the step's size alone.  Tiles of 256 rows, for inner sizes that are multiples of 64 (and rows that 32-bit offsets reach),
-    where few experts spill into a tile more than their mean fills: with a mean of 256 half of them do, and tiles of 128 are
-    ahead (gate|up and down at 150 / 256 / 375 rows an expert, tiles of 256 against 128: 78 + 48 / 124 + 78 / 140 + 87 us against
-    81 + 60 / 117 + 73 / 155 + 96 us; at 100 rows 78 + 46 against 72 + 35)."""
+    the step's and the matrices' sizes alone.
+
+    Inner sizes that are multiples of 64 (and rows that 32-bit offsets reach), enough experts and columns for 256 blocks of 64:
+    tiles of 64 rows read a matrix once from 13 rows an expert on, where tiles of 16 read it again for every further 16 rows, and
+    128 rows from 52 on; gate|up + down at 12 / 24 / 48 / 56 rows an expert, tiles of 16, 32, 64 and 128: 32 experts, width 2048,
+    1024 columns 88, 91, 91, 97 / 126, 104, 92, 99 / 207, 147, 94, 104 / 230, 157, 111, 104 us; 128 experts, 768 columns 252, 244,
+    227, 233 / 371, 301, 232, 244 / 689, 477, 254, 260 / 819, 531, 270, 263 us; 16 experts, width 4096, 1536 columns 129, 120, 128, 122 /
+    186, 145, 131, 125 / 315, 196, 139, 129 us (at 8 rows 82, 88, 91, 96 and 115, 117, 126, 122).  8 experts of 512 columns, width 1024,
+    make 64 such blocks, and more blocks of fewer rows are ahead: at 24 / 48 / 96 rows 16, 13, 20, 26 / 21, 19, 20, 29 / 31, 25, 21, 31 us.
+
+    Tiles of 256 rows where few experts spill into a tile more than their mean fills: with a mean of 256 half of them do, and
+    tiles of 128 are ahead (gate|up and down at 150 / 256 / 375 rows an expert, tiles of 256 against 128: 59 + 34 / 104 + 60 /
+    108 + 70 us against 66 + 43 / 94 + 57 / 121 + 76 us; at 100 rows 75 + 36 against 71 + 33)."""
     mean = tokens * top / max(1, experts)
+    wide = (hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
+            and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31)
+    if wide and experts * (ff // 64) >= 256 and 13 <= mean < 96:
+        return 128 if mean >= 52 else 64
     if mean >= 96:
-        wide = (hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
-                and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31)
         return 256 if wide and (128 <= mean < 208 or mean >= 320) else 128
     if mean >= 48:
         return 64
@@ -146,7 +157,8 @@ class RoutedExperts(FeedForward):
         T = x.shape[0]
         ids, weights = self.route(x)
         y = None
-        tile_rows = tile_rows_for(T, self.top, self.experts, self.hidden_size, self.ff)
+        # in 32-bit a row is worked after the other whatever the tile: the fewer a tile, the more of them side by side
+        tile_rows = tile_rows_for(T, self.top, self.experts, *((self.hidden_size, self.ff) if x.dtype == torch.bfloat16 else (0, 0)))
         slot_of_pair = ids.view(-1)               # read for experts with weights only
         if self.experts:
             slot_of_pair, token_of_slot, tiles, _ = ops.moe_sort(ids, self.experts, tile_rows)
