@@ -20,6 +20,14 @@ __device__ __forceinline__ void load16_to_lds(const void* src, unsigned char* ld
   __builtin_amdgcn_global_load_lds(src, lds_base, 16, 0, 0);
 #endif
 }
+// The same for what is read once and need not stay in the caches.
+__device__ __forceinline__ void load16_to_lds_once(const void* src, unsigned char* lds_base) {
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
+  const unsigned at = (unsigned)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(lds_byte_t*)lds_base);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(src), "s"(at) : "memory", "m0");
+#endif
+}
 // The same from base + off bytes (base the same in the whole wave), to the place `at` of shared memory (lds_place).
 __device__ __forceinline__ void load16_to_lds_from(const void* base, unsigned off, unsigned at) {
 #ifdef __HIP_DEVICE_COMPILE__

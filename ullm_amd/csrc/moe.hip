@@ -521,9 +521,10 @@ moe_rows_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restric
 // rows of x, whole lines of 128 bytes) go straight to shared memory of its own, two taking turns (lds_load.h): no barrier, and
 // nothing but addresses in registers while 8 to 16 KB a wave are on their way.  What bounds it is the experts' matrices from
 // memory (gate|up of 32 experts, width 2048, 1024 columns: 268 MB, 43 us).  The kernel above asks for 64 bytes of a row at a time
-// and holds them in registers; gate|up + down at 8 / 48 / 100 / 190 / 300 tokens, 4 experts each, 52 + 23 / 61 + 33 / 81 + 45 / 134 + 78 / 154 +
-// 91 us there, 40 + 19 / 51 + 30 / 55 + 33 / 81 + 49 / 84 + 59 us here (three stages, and a block less on each compute unit:
-// 40 + 21 / 52 + 30 / 55 + 34 / 82 + 49 / 106 + 66).
+// and holds them in registers; gate|up + down at 8 / 48 / 100 tokens, 4 experts each, 41 + 19 / 61 + 33 / 80 + 44 us
+// there, 28 + 15 / 41 + 22 / 50 + 30 us here.  The matrices' loads do not stay in the caches: without that 32 + 14 / 50 + 29 / 54 + 33,
+// and the kernels around this one found their smaller matrices and rows gone (the router 12.5 against 10.2 us at one token).
+// Three stages, and a block less on each compute unit, were 1 to 4 % slower, and a third with tiles of 32 rows.
 template <int MT, bool GATED>
 __global__ void __launch_bounds__(256)
 moe_rows_dma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
@@ -555,7 +556,8 @@ moe_rows_dma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
   auto fetch = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      load16_to_lds(src[i], mine + buf * STAGE + i * 1024);
+      if (i < WR / 8) load16_to_lds_once(src[i], mine + buf * STAGE + i * 1024);
+      else load16_to_lds(src[i], mine + buf * STAGE + i * 1024);
       src[i] += 64;
     }
   };
