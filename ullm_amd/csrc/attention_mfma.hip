@@ -474,8 +474,7 @@ struct RawQueries {
 #pragma unroll
         for (int ch = 0; ch < m; ++ch) part[ch] += part[ch + m];
       float ss = part[0];
-      ss += __shfl_xor(ss, 32, 64);
-      ss += __shfl_xor(ss, 16, 64);
+      ss = sum_with_lane_xor16(sum_with_lane_xor32(ss));
       const float rs = rsqrtf(ss / (float)HD + fuse.eps);
 #pragma unroll
       for (int ch = 0; ch < NQK; ++ch)
@@ -599,8 +598,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   float& m = ms[0];
   float& l = ls[0];
   if (wave != 0) return;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = sum_with_lane_xor32(sum_with_lane_xor16(l));
   if (!col_ok) return;
   if (num_splits == 1) {
     if constexpr (EXTRA) l += sink_of(extras, head, m);
@@ -903,8 +901,7 @@ __device__ __forceinline__ void prompt_tile_softmax(f32x4_t (&s)[NG][2], int key
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
       float col_max = lane_max[q];
-      col_max = fmaxf(col_max, __shfl_xor(col_max, 16, 64));
-      col_max = fmaxf(col_max, __shfl_xor(col_max, 32, 64));
+      col_max = max_with_lane_xor32(max_with_lane_xor16(col_max));
       const bool had = m[q] > 0.5f * NEG_BIG;
       const bool moves = col_max > 0.5f * NEG_BIG && (!had || col_max > RESCALE_STEP);
       if (moves) {
@@ -1183,8 +1180,7 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __r
 #pragma unroll
   for (int qg = 0; qg < NG; ++qg) {
     float lt = l[qg];
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    lt = sum_with_lane_xor32(sum_with_lane_xor16(lt));
     if (chi[qg] < 0) continue;
     if constexpr (EXTRA) lt += sink_of(extras, head, m[qg]);
     float inv = lt > 0.f ? 1.f / lt : 0.f;
@@ -1521,8 +1517,7 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
 #pragma unroll
   for (int qg = 0; qg < NG; ++qg) {
     float lt = l[qg];
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    lt = sum_with_lane_xor32(sum_with_lane_xor16(lt));
     if (chi[qg] < 0) continue;
     if constexpr (EXTRA) lt += sink_of(extras, head, m[qg]);
     float inv = lt > 0.f ? 1.f / lt : 0.f;

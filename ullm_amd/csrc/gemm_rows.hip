@@ -199,8 +199,7 @@ gemm_rows_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict
       const float4 v = *reinterpret_cast<const float4*>(sq_row + 4 * j);
       q += (v.x + v.y) + (v.z + v.w);
     }
-    q += __shfl_xor(q, 16);
-    q += __shfl_xor(q, 32);
+    q = sum_with_lane_xor32(sum_with_lane_xor16(q));
     if (g == 0) sqs[wn][r] = q;             // read after the barriers of the stages
   }
   int s = 0;

@@ -150,8 +150,7 @@ __device__ __forceinline__ void skinny_finish(f32x4_t (&acc)[NT][MT], RedT& red,
           }
         }
       }
-      q += __shfl_xor(q, 16);
-      q += __shfl_xor(q, 32);
+      q = sum_with_lane_xor32(sum_with_lane_xor16(q));
       if (g == 0 && m < M) {
         ahead.sq[(size_t)m * ahead.ld_sq + blockIdx.x] = q;
         if (blockIdx.x == gridDim.x - 1)
@@ -373,8 +372,7 @@ gemm_skinny_kernel(const void* __restrict__ Xv, int ldx, const bf16_t* __restric
       q += (v.x + v.y) + (v.z + v.w);
     }
     if (SQ_LANES == 8) q += __shfl_xor(q, 8);
-    q += __shfl_xor(q, 16);
-    q += __shfl_xor(q, 32);
+    q = sum_with_lane_xor32(sum_with_lane_xor16(q));
     if (lane < 16) sq[wave][lane] = lane < 64 / SQ_LANES ? q : 0.f;
   }
   // DEPTH stages in flight: registers st[d] hold the stages s = d (mod DEPTH).  Whole rounds whose fetches all lie

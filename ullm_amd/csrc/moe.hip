@@ -113,15 +113,8 @@ __device__ __forceinline__ void route_from_logits(float* z, float* s_choice, flo
         at = e;
       }
     }
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-      const float ob = __shfl_xor(best, m, 64);
-      const int oa = __shfl_xor(at, m, 64);
-      if (ob > best || (ob == best && oa < at)) {
-        best = ob;
-        at = oa;
-      }
-    }
+    const float most = wave_max(best);
+    at = wave_min(best == most ? at : 0x7fffffff);      // ties: the lower index
     if (at >= n_router) at = k < n_router ? k : 0;       // every value a NaN: any expert
     const float s = z[at];
     total += s;
@@ -274,41 +267,78 @@ extern "C" int ullm_moe_router(const void* x, int ldx, const float* w, const flo
 }
 
 // ------------------------------------------------------------------------------- grouping by expert
-// One block.  offsets [experts + 1]; slot_of_pair [pairs] (-1: the pair's expert has no weights); token_of_slot [pairs];
+// One block, bound by its trips to memory and shared memory: the pairs are read once and counted with the addition that gives a
+// pair its place, the running sums over the experts are one wave's (2048 tokens of 4 choices among 32 experts 7.6 -> 6.0 us, 3000
+// 9.8 -> 7.5).  offsets [experts + 1]; slot_of_pair [pairs] (-1: the pair's expert has no weights); token_of_slot [pairs];
 // tiles [max_tiles + 1][3] = (expert, first slot, rows), rows 0 for the tiles no expert filled; the entry behind the
 // list holds the number of tiles in use.
 __global__ void __launch_bounds__(1024)
 moe_sort_kernel(const int* __restrict__ ids, int n_pairs, int top, int n_experts, int tile_rows,
                 int* __restrict__ offsets, int* __restrict__ slot_of_pair, int* __restrict__ token_of_slot,
                 int* __restrict__ tiles, int max_tiles) {
-  __shared__ int count[MOE_MAX_ROUTER], start[MOE_MAX_ROUTER + 1], cursor[MOE_MAX_ROUTER], tile_base[MOE_MAX_ROUTER + 1];
+  constexpr int HELD = 16;
+  __shared__ int count[MOE_MAX_ROUTER], start[MOE_MAX_ROUTER + 1], tile_base[MOE_MAX_ROUTER + 1];
   const int tid = threadIdx.x;
   for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;
   __syncthreads();
-  for (int p = tid; p < n_pairs; p += blockDim.x) {
+  // a pair's place inside its expert is what the count held before it; the first HELD pairs of a thread keep theirs in registers
+  int held_e[HELD], held_at[HELD];
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
+    const int p = tid + i * (int)blockDim.x;
+    held_e[i] = p < n_pairs ? ids[p] : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
+    if (held_e[i] >= n_experts) held_e[i] = -1;
+    held_at[i] = held_e[i] >= 0 ? atomicAdd(&count[held_e[i]], 1) : 0;
+  }
+  for (int p = tid + HELD * (int)blockDim.x; p < n_pairs; p += blockDim.x) {
     const int e = ids[p];
-    if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+    if (e >= 0 && e < n_experts) slot_of_pair[p] = atomicAdd(&count[e], 1);
   }
   __syncthreads();
-  if (tid == 0) {
+  if (tid < 64) {                                         // one wave: running sums over the experts, 64 at a time
     int off = 0, tb = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      start[e] = off;
-      cursor[e] = off;
-      tile_base[e] = tb;
-      off += count[e];
-      tb += (count[e] + tile_rows - 1) / tile_rows;
+    for (int e0 = 0; e0 < n_experts; e0 += 64) {
+      const int e = e0 + tid, n = e < n_experts ? count[e] : 0;
+      int a = n, b = (n + tile_rows - 1) / tile_rows;
+      const int own_tiles = b;
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) {
+        const int pa = __shfl_up(a, m, 64), pb = __shfl_up(b, m, 64);
+        if (tid >= m) {
+          a += pa;
+          b += pb;
+        }
+      }
+      if (e < n_experts) {
+        start[e] = off + a - n;
+        tile_base[e] = tb + b - own_tiles;
+      }
+      off += __shfl(a, 63, 64);
+      tb += __shfl(b, 63, 64);
     }
-    start[n_experts] = off;
-    tile_base[n_experts] = tb;
+    if (tid == 0) {
+      start[n_experts] = off;
+      tile_base[n_experts] = tb;
+    }
   }
   __syncthreads();
   for (int e = tid; e <= n_experts; e += blockDim.x) offsets[e] = start[e];
-  for (int p = tid; p < n_pairs; p += blockDim.x) {
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
+    const int p = tid + i * (int)blockDim.x;
+    if (p >= n_pairs) break;
+    const int slot = held_e[i] >= 0 ? start[held_e[i]] + held_at[i] : -1;
+    if (slot >= 0) token_of_slot[slot] = p / top;
+    slot_of_pair[p] = slot;
+  }
+  for (int p = tid + HELD * (int)blockDim.x; p < n_pairs; p += blockDim.x) {
     const int e = ids[p];
     int slot = -1;
     if (e >= 0 && e < n_experts) {
-      slot = atomicAdd(&cursor[e], 1);
+      slot = start[e] + slot_of_pair[p];                  // this thread's own store above
       token_of_slot[slot] = p / top;
     }
     slot_of_pair[p] = slot;
