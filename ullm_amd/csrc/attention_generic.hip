@@ -15,6 +15,7 @@
 // and the pools lie at addresses of that alignment, the tiled one
 // on the 32-bit matrix instructions; else one block per (token, head).  Which one is a matter of the model's sizes alone,
 // never of the batch.
+#include "lds_load.h"
 #include "mfma_f32.h"
 
 #define ATT_THREADS 128
@@ -123,15 +124,42 @@ paged_attention_generic_kernel(const T* __restrict__ q, int q_stride, T* __restr
 // and a value is not finite is added key by key by ordinary arithmetic (zero times infinity must not reach a row that does
 // not see the key).
 // What bounds it: 16 x 128 x hd products of 32-bit twice a tile (1.7 us of the matrix pipe for a block's tile at hd = 128, shared by
-// the waves of the other blocks) and two barriers; the keys of the next half tile are on their way while this one's values are
-// worked.  500 tokens, 16 heads of 128 over 8 kv heads, 32-bit: 63 us; the kernel above, which reads every
-// key once per query head with the lanes of a wave hd values apart, took 637.
+// the waves of the other blocks), the ordinary arithmetic beside them and two barriers; the keys and values of a tile are on their
+// way while the tile before is worked.  500 tokens, 16 heads of 128 over 8 kv heads, 32-bit: 53 us, 1000 tokens 138 (with the values
+// asked for when their products were next, and pages found by a division under a condition, 62 and 177; in blocks of eight
+// waves, which take a unit each, 62 and 149); the kernel above, which reads every key once per query head with the lanes of
+// a wave hd values apart, took 637.
 __device__ __forceinline__ bool finite4(const float4& v) {
   return isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
 }
 
-template <typename T, int KC>                     // hd = 16 KC
-__global__ void __launch_bounds__(256)
+// Four neighbouring values as they lie in memory, and what becomes of them when they are used.
+template <typename T>
+struct RawFour {
+  typedef float4 type;
+  static __device__ __forceinline__ type load(const float* p) { return *reinterpret_cast<const float4*>(p); }
+  static __device__ __forceinline__ float4 values(const type& v) { return v; }
+  // the first n of them, the others zero
+  static __device__ __forceinline__ type first(const type& v, int n) {
+    return make_float4(n > 0 ? v.x : 0.f, n > 1 ? v.y : 0.f, n > 2 ? v.z : 0.f, n > 3 ? v.w : 0.f);
+  }
+};
+template <>
+struct RawFour<bf16_t> {
+  typedef uint2 type;
+  static __device__ __forceinline__ type load(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
+  static __device__ __forceinline__ float4 values(const type& v) {
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                       __uint_as_float(v.y & 0xffff0000u));
+  }
+  static __device__ __forceinline__ type first(const type& v, int n) {
+    return make_uint2(n > 1 ? v.x : n > 0 ? v.x & 0xffffu : 0u, n > 3 ? v.y : n > 2 ? v.y & 0xffffu : 0u);
+  }
+};
+
+// hd = 16 KC.  POW2: pages of 2^page_shift keys (a division under a run-time condition would put every load in a block of its own)
+template <typename T, int KC, bool POW2>
+__global__ void __launch_bounds__(256, KC <= 8 ? 2 : 1)      // two blocks share a unit where the registers allow it
 paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride,
                              const T* __restrict__ k_pool, const T* __restrict__ v_pool,
                              const int* __restrict__ positions, const int* __restrict__ token_entry,
@@ -162,77 +190,88 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  auto page_index = [&](int j) { return page_shift >= 0 ? j >> page_shift : j / page_size; };
+  auto page_index = [&](int j) { return POW2 ? j >> page_shift : j / page_size; };
 
+  // lane i < n_tok: the block's i-th token
+  const int own_entry = token_entry[t0 + (lane < n_tok ? lane : n_tok - 1)], own_pos = positions[t0 + (lane < n_tok ? lane : n_tok - 1)];
+  using Raw = RawFour<T>;
   for (int first = 0; first < n_tok;) {
     // the tokens of one request; their last position is the largest, their first one's window starts lowest
-    const int seg_entry = token_entry[t0 + first];
-    int end = first, hi = -1, low = 0x7fffffff;
-    while (end < n_tok && token_entry[t0 + end] == seg_entry) {
-      const int p = positions[t0 + end], f = first_seen_key(p, window);
-      hi = p > hi ? p : hi;
-      low = f < low ? f : low;
-      ++end;
-    }
+    const int seg_entry = __builtin_amdgcn_readlane(own_entry, first);
+    const unsigned long long same = __ballot(lane < n_tok && own_entry == seg_entry) >> first;
+    const int end = first + __builtin_ctzll(~same);      // n_tok <= 16: some bit above is clear
+    const bool inside = lane >= first && lane < end;
+    const int hi = -wave_min(inside ? -own_pos : 0x7fffffff), low = wave_min(inside ? first_seen_key(own_pos, window) : 0x7fffffff);
     const bool alone = first == 0 && end == n_tok;       // no row of the block belongs to another request
     first = end;
     const bool active = valid && entry == seg_entry;
     const int* bt = block_table + (size_t)seg_entry * bt_stride;
-    // the page of key j, -1 past the last key
-    auto page_of = [&](int j) __attribute__((always_inline)) {
-      const int page = bt[page_index(j <= hi ? j : hi)];
-      return j <= hi ? page : -1;
+    // Keys and values of both halves of a tile; up to hd = 128 registers hold them together, and the halves' products alternate.
+    // They are loaded a tile ahead, and the entries of the block table they lie by a tile before that; nothing touches a loaded
+    // value or entry until it is used (a select on it would wait for everything on its way).  An entry counts as -1 for
+    // keys past the last.
+    constexpr int SETS = KC <= 8 ? 2 : 1;
+    typename Raw::type kf[SETS][KC], vf[SETS][NT][4];
+    int kpage[2], knext[2], vhave[2], vnext[2][4];
+    // (relaxed loads, or the compiler moves them down to their use a tile later and waits for all the others there)
+    auto entry_of = [&](int j) __attribute__((always_inline)) {
+      return __hip_atomic_load(bt + page_index(j <= hi ? j : hi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     };
-    // keys of both halves of a tile; up to hd = 128 registers hold them together, and the halves' products alternate
-    constexpr int KEY_SETS = KC <= 8 ? 2 : 1;
-    float4 kf[KEY_SETS][KC];
-    auto fetch_keys = [&](int set, int at, int page) __attribute__((always_inline)) {
-      const int j = at + 16 * wave + r;
+    auto key_entry = [&](int half, int at) __attribute__((always_inline)) { knext[half] = entry_of(at + 64 * half + 16 * wave + r); };
+    auto value_entries = [&](int half, int at) __attribute__((always_inline)) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) vnext[half][c] = entry_of(at + 64 * half + 16 * c + 4 * g);
+    };
+    // the keys of half `half` of the tile at `at`, by knext; its page stays in kpage for the tile's tests
+    auto fetch_keys = [&](int half, int at) __attribute__((always_inline)) {
+      const int j = at + 64 * half + 16 * wave + r, page = j <= hi ? knext[half] : -1;
+      kpage[half] = page;
       const T* src = k_pool + (((size_t)(page < 0 ? 0 : page) * nkv + kvh) * page_size + (page < 0 ? 0 : j - page_index(j) * page_size)) * HD + 4 * g;
 #pragma unroll
-      for (int c = 0; c < KC; ++c) kf[set][c] = ld4_f32(src + 16 * c);
+      for (int c = 0; c < KC; ++c) kf[SETS == 2 ? half : 0][c] = Raw::load(src + 16 * c);
     };
-    // half a tile's values for this wave's dims, keys past the end and keys without a page zeroed
-    float4 vf[NT][4];
-    int vpage[4];
-    auto fetch_values = [&](int at) __attribute__((always_inline)) {
+    // half a tile's values for this wave's dims, by vnext; a bit of vhave per chunk: whether the lane's keys of it have a page
+    auto fetch_values = [&](int half, int at) __attribute__((always_inline)) {
+      vhave[half] = 0;
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const int dim = 16 * (wave + 4 * n) + r;
+      for (int c = 0; c < 4; ++c) {
+        const int jv = at + 64 * half + 16 * c + 4 * g, page = vnext[half][c];
+        const bool have = jv <= hi && page >= 0;
+        vhave[half] |= (have ? 1 : 0) << c;
+        const T* src = v_pool + ((size_t)(have ? page : 0) * nkv + kvh) * HD * page_size + (have ? jv - page_index(jv) * page_size : 0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int jv = at + 16 * c + 4 * g;
-          const bool have = vpage[c] >= 0;
-          const size_t row = ((size_t)(have ? vpage[c] : 0) * nkv + kvh) * HD + (dim < HD ? dim : 0);
-          vf[n][c] = ld4_f32(v_pool + row * page_size + (have ? jv - page_index(jv) * page_size : 0));
-          if (!have) vf[n][c].x = 0.f;
-          if (!have || jv + 1 > hi) vf[n][c].y = 0.f;
-          if (!have || jv + 2 > hi) vf[n][c].z = 0.f;
-          if (!have || jv + 3 > hi) vf[n][c].w = 0.f;
+        for (int n = 0; n < NT; ++n) {
+          const int dim = 16 * (wave + 4 * n) + r;
+          vf[SETS == 2 ? half : 0][n][c] = Raw::load(src + (size_t)(dim < HD ? dim : 0) * page_size);
         }
       }
     };
-    auto value_pages = [&](int at) __attribute__((always_inline)) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) vpage[c] = page_of(at + 16 * c + 4 * g);
-    };
     int base = low & ~127;
-    int kpage[2];
 #pragma unroll
-    for (int half = 0; half < KEY_SETS; ++half) {
-      kpage[half] = page_of(base + 64 * half + 16 * wave + r);
-      fetch_keys(half, base + 64 * half, kpage[half]);
+    for (int half = 0; half < 2; ++half) {
+      key_entry(half, base);
+      value_entries(half, base);
+    }
+#pragma unroll
+    for (int half = 0; half < SETS; ++half) fetch_keys(half, base);
+#pragma unroll
+    for (int half = 0; half < SETS; ++half) fetch_values(half, base);
+    // from here on: entries of the half that is fetched next (SETS 1: the tile's second half is, before the next tile's first)
+#pragma unroll
+    for (int half = 0; half < SETS; ++half) {
+      key_entry(half, base + 128);
+      value_entries(half, base + 128);
     }
     for (; base <= hi; base += 128) {
       f32x4_t s[2];
       unsigned long long there[2];                       // bit r: key 16 wave + r of the half has a page
       bool ok[2][4];
       float tile_max = -INFINITY;
-      if constexpr (KEY_SETS == 2) {
+      if constexpr (SETS == 2) {
         s[0] = s[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
-          const f32x4_t k0 = in_order(kf[0][c]), k1 = in_order(kf[1][c]);
+          const f32x4_t k0 = in_order(Raw::values(kf[0][c])), k1 = in_order(Raw::values(kf[1][c]));
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0[i], qf[c][i], s[0], 0, 0, 0);
@@ -242,33 +281,50 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
       }
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        constexpr bool both = KEY_SETS == 2;
-        const int at = base + 64 * half, set = both ? half : 0, next = both ? at + 128 : at + 64;
-        there[half] = __ballot(kpage[set] >= 0);
+        constexpr bool both = SETS == 2;
+        const int at = base + 64 * half;
         if constexpr (!both) {
           s[half] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int c = 0; c < KC; ++c) {
-            const f32x4_t k = in_order(kf[0][c]);
+            const f32x4_t k = in_order(Raw::values(kf[0][c]));
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], qf[c][i], s[half], 0, 0, 0);
           }
         }
-        kpage[set] = page_of(next + 16 * wave + r);
-        fetch_keys(set, next, kpage[set]);
+        there[half] = __ballot(kpage[half] >= 0);
+        if constexpr (both) {
+          fetch_keys(half, base + 128);
+          key_entry(half, base + 256);
+        } else {
+          const int next = half == 0 ? base : base + 128;            // where the other half's next keys lie
+          fetch_keys(half ^ 1, next);
+          key_entry(half ^ 1, next + 128);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = at + 16 * wave + 4 * g + i;
           ok[half][i] = active && j <= pos && j >= lo && ((there[half] >> (4 * g + i)) & 1);
-          if (bias && ok[half][i]) s[half][i] += bias[(size_t)h * bias_rows + (pos - j < bias_rows ? pos - j : bias_rows - 1)];
           if (ok[half][i]) tile_max = fmaxf(tile_max, s[half][i]);
         }
       }
-      value_pages(base);
+      if (bias) {
+        tile_max = -INFINITY;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = base + 64 * half + 16 * wave + 4 * g + i;
+            if (ok[half][i]) {
+              s[half][i] += bias[(size_t)h * bias_rows + (pos - j < bias_rows ? pos - j : bias_rows - 1)];
+              tile_max = fmaxf(tile_max, s[half][i]);
+            }
+          }
+      }
       tile_max = max_with_lane_xor32(max_with_lane_xor16(tile_max));
       if (g == 0) s_max[wave][r] = tile_max;
-      __syncthreads();
-      fetch_values(base);
+      bare_barrier();                                    // the loads on their way stay on their way
       const float m_new = fmaxf(fmaxf(m, fmaxf(s_max[0][r], s_max[1][r])), fmaxf(s_max[2][r], s_max[3][r]));
       const float alpha = m_new == m ? 1.f : expf(m - m_new);
       // the exponentials lie so that a reader of four neighbouring places has keys g, 4 + g, 8 + g, 12 + g of a chunk
@@ -277,7 +333,7 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           s_p[r][64 * half + 16 * wave + 4 * i + g] = ok[half][i] ? expf(s[half][i] - m_new) : 0.f;
-      __syncthreads();
+      bare_barrier();
       m = m_new;
 #pragma unroll
       for (int n = 0; n < NT; ++n)
@@ -287,16 +343,25 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const int at = base + 64 * half;
+        constexpr bool both = SETS == 2;
+        typename Raw::type (&vh)[NT][4] = vf[both ? half : 0];
         f32x4_t pf[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) pf[c] = *reinterpret_cast<const f32x4_t*>(&s_p[r][64 * half + 16 * c + 4 * g]);
         // the half's sum as a tree over the bits of the key's place, the highest first
         {
           const f32x4_t a = (pf[0] + pf[2]) + (pf[1] + pf[3]);          // [i]: places 4 i + g
-          float sum = (a[0] + a[2]) + (a[1] + a[3]);
-          sum += __shfl_xor(sum, 32, 64);
-          sum += __shfl_xor(sum, 16, 64);
-          tile_sum += sum;
+          const float sum = (a[0] + a[2]) + (a[1] + a[3]);
+          tile_sum += sum_with_lane_xor16(sum_with_lane_xor32(sum));
+        }
+        // keys past the end and keys without a page count as zero
+        if (!__all(vhave[half] == 15 && at + 63 <= hi)) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int left = (vhave[half] >> c) & 1 ? hi - (at + 16 * c + 4 * g) + 1 : 0;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) vh[n][c] = Raw::first(vh[n][c], left);
+          }
         }
         // every row sees every key, or every value is finite
         bool plain = alone && __all(!valid || (at >= lo && at + 63 <= pos));
@@ -305,27 +370,26 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
 #pragma unroll
           for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) fine = fine && finite4(vf[n][c]);
+            for (int c = 0; c < 4; ++c) fine = fine && finite4(Raw::values(vh[n][c]));
           plain = __all(fine);
         }
-        int vhave = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) vhave |= (vpage[c] >= 0 ? 1 : 0) << c;
         if (plain) {
 #pragma unroll
-          for (int n = 0; n < NT; ++n)
+          for (int c = 0; c < 4; ++c) {
+            f32x4_t v[NT];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const f32x4_t v = in_order(vf[n][c]);
+            for (int n = 0; n < NT; ++n) v[n] = in_order(Raw::values(vh[n][c]));
 #pragma unroll
-              for (int i = 0; i < 4; ++i) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], pf[c][i], acc[n], 0, 0, 0);
-            }
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][i], pf[c][i], acc[n], 0, 0, 0);
+          }
         } else {
           // lane (r, g) holds dims 4 g + i of row r; the value of key 16 c + 4 o + j at dim 4 g + i lies in lane (4 g + i, o)
 #pragma unroll
           for (int c = 0; c < 4; ++c)
             for (int o = 0; o < 4; ++o) {
-              const int have = __shfl(vhave, 16 * o, 64);
+              const int have = __shfl(vhave[half], 16 * o, 64);
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
                 const int key = at + 16 * c + 4 * o + j;
@@ -335,17 +399,23 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
                   for (int i = 0; i < 4; ++i) {
-                    const float mine = j == 0 ? vf[n][c].x : j == 1 ? vf[n][c].y : j == 2 ? vf[n][c].z : vf[n][c].w;
+                    const float4 four = Raw::values(vh[n][c]);
+                    const float mine = j == 0 ? four.x : j == 1 ? four.y : j == 2 ? four.z : four.w;
                     const float v = __shfl(mine, 16 * o + 4 * g + i, 64);
                     if (sees) acc[n][i] += w * v;
                   }
               }
             }
         }
-        if (half == 0) {
-          value_pages(at + 64);
-          fetch_values(at + 64);
+        if constexpr (both) {
+          fetch_values(half, base + 128);
+          value_entries(half, base + 256);
+        } else {
+          const int next = half == 0 ? base : base + 128;
+          fetch_values(half ^ 1, next);
+          value_entries(half ^ 1, next + 128);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
       l = l * alpha + tile_sum;
     }
@@ -384,14 +454,16 @@ static bool launch_tiles(const T* q, int q_stride, T* out, int out_stride, const
     if (page_size == 1 << b) shift = b;
   if ((long long)nkv * chunks > 65535) return false;
   dim3 grid((T_ + tp - 1) / tp, nkv * chunks), block(256);
-#define GO(KC) case KC: hipLaunchKernelGGL((paged_attention_tiles_kernel<T, KC>), grid, block, 0, stream, q, q_stride, out, \
+#define AS(KC, POW2) hipLaunchKernelGGL((paged_attention_tiles_kernel<T, KC, POW2>), grid, block, 0, stream, q, q_stride, out, \
     out_stride, k_pool, v_pool, positions, token_entry, block_table, bt_stride, page_size, shift, T_, tp, nq, nkv, scale, \
-    window, bias, bias_rows, sink); return true
+    window, bias, bias_rows, sink)
+#define GO(KC) case KC: if (shift >= 0) AS(KC, true); else AS(KC, false); return true
   switch (hd / 16) {
     GO(1); GO(2); GO(3); GO(4); GO(5); GO(6); GO(7); GO(8); GO(10); GO(12); GO(14); GO(16);
     default: return false;
   }
 #undef GO
+#undef AS
 }
 
 extern "C" int ullm_paged_attention_generic(

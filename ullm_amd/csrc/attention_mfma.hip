@@ -567,7 +567,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   f32x4_t accs[1][2 * NQK];
   float ms[1], ls[1];
   {
-    const int* const bt = block_table + (size_t)token_entry[t] * bt_stride;
+    const int* const bt = block_table + (size_t)(token_entry ? token_entry[t] : t) * bt_stride;
     const int clo[1] = {lo}, chi[1] = {col_ok ? pos : -1};
     if constexpr (FUSE) {
       const bool has_own = fuse.k_pool && begin < end && end == pos + 1;

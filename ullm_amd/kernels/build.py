@@ -31,7 +31,7 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 HEADERS = ["common.h"]
-FAMILY_HEADERS = {"gemm_simple": ["mfma_f32.h"], "attention_generic": ["mfma_f32.h"],
+FAMILY_HEADERS = {"gemm_simple": ["mfma_f32.h"], "attention_generic": ["lds_load.h", "mfma_f32.h"],
                   "attention_mfma": ["no_alloc.h", "lds_load.h"], "moe": ["lds_load.h", "mfma_tiles.h"],
                   "decay_scan": ["decay_inputs.h"], "decay_chunks": ["decay_inputs.h"],
                   "gemm_tiles": ["lds_load.h", "mfma_tiles.h"],

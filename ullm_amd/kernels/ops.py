@@ -1466,10 +1466,13 @@ def attention_decode_fused(qkv, out, q_gain: Optional[torch.Tensor], k_gain: Opt
                            cos_sin: Optional[torch.Tensor], rotary_dim: int, style: int, k_pool, v_pool,
                            token_list: Optional[torch.Tensor], n_items: int, positions, token_entry, block_table,
                            page_size: int, nq: int, nkv: int, hd: int, scale: float, window: int, max_kv: int,
-                           write_kv: bool, splits: int = 0, waves: int = 0) -> None:
+                           write_kv: bool, splits: int = 0, waves: int = 0, entry_is_token: bool = False) -> None:
     """``attention_decode_mfma`` for a step in which every item is its request's newest token, with what
     ``qk_norm_rope_write`` does folded in: ``qkv`` [T, (nq + 2 nkv) * hd] is the fused projection as the
-    matrix product left it; the kernel norms and rotates q and k itself and writes k and v to the cache."""
+    matrix product left it; the kernel norms and rotates q and k itself and writes k and v to the cache.
+    ``entry_is_token``: the step holds nothing but one token of every entry, in the entries' order, and ``token_list``
+    names them all; the kernel then need not look up a token's entry, nor, where its waves leave every other SIMD free, the list,
+    which is there for their order (a trip to memory each, one after the other, at the head of every layer's attention)."""
     _check_pools(k_pool, v_pool, nkv, page_size, hd, torch.bfloat16)
     _need(qkv.dtype == torch.bfloat16 and qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] == (nq + 2 * nkv) * hd,
           "qkv must be bfloat16 [T, (nq + 2 nkv) * hd]")
@@ -1502,6 +1505,11 @@ def attention_decode_fused(qkv, out, q_gain: Optional[torch.Tensor], k_gain: Opt
     ws = None
     if splits > 1:
         ws = torch.empty(n_items * nq * splits * (hd + 4), dtype=torch.float32, device=qkv.device)
+    if entry_is_token:
+        _need(n_items == qkv.shape[0] <= block_table.shape[0], "one token of every entry, nothing else")
+        token_entry = None
+        if n_items * nkv * groups * splits * waves <= 2 * compute_units(qkv.device):
+            token_list = None
     _check(lib.ullm_attention_decode_fused(
         _p(qkv), _c_int(qkv.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(token_list),
         _c_int(n_items), _p(positions), _p(token_entry), _p(block_table), _c_int(block_table.stride(0)),

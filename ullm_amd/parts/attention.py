@@ -210,7 +210,7 @@ class GQAttention(Mixer):
                 qkv, out, self.q_gain, self.k_gain, eps, table, rot, style, cache.k_pool, cache.v_pool,
                 plan.arrays["decode_tokens"], work["num_decode"], ctx.positions, ctx.token_entry, group.block_table,
                 group.page_size, self.nq, self.nkv, self.hd, self.scale, self.reach, work["max_decode_kv"],
-                write_kv=cache.owner)
+                write_kv=cache.owner, entry_is_token=ctx.decode_only and ctx.num_entries == T)
             return out
         q = torch.empty((T, self.nq * self.hd), dtype=x.dtype, device=x.device)
         ops.qk_norm_rope_write(
