@@ -425,9 +425,33 @@ __global__ void add_bias_kernel(T* __restrict__ y, const float* __restrict__ bia
   st_f32(p, ld_f32(p) + bias[n]);
 }
 
+// Four neighbouring values a thread (N and the row length multiples of four, 16-byte aligned): two bytes a lane and a 64-bit
+// division a value were what bounded the other.
+template <typename T>
+__global__ void __launch_bounds__(256)
+add_bias_vec_kernel(T* __restrict__ y, const float* __restrict__ bias, unsigned pieces, long long row_stride, unsigned total) {
+  const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+  if (idx >= total) return;
+  const unsigned t = idx / pieces, n = 4 * (idx - t * pieces);
+  T* p = y + (size_t)t * row_stride + n;
+  const float4 v = ld4_f32(p), b = ld4_f32(bias + n);
+  st4_f32(p, make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w));
+}
+
 extern "C" int ullm_add_bias(void* y, const float* bias, int T_, int N, long long row_stride, int dtype, hipStream_t stream) {
   if (T_ <= 0 || N <= 0) return 0;
   const size_t total = (size_t)T_ * N;
+  if (N % 4 == 0 && row_stride % 4 == 0 && (((uintptr_t)y | (uintptr_t)bias) & 15) == 0 && total / 4 < 0x7fffffffu &&
+      (dtype == ULLM_F32 || dtype == ULLM_BF16)) {
+    const dim3 blocks((unsigned)((total / 4 + 255) / 256));
+    if (dtype == ULLM_F32)
+      hipLaunchKernelGGL(add_bias_vec_kernel<float>, blocks, dim3(256), 0, stream, (float*)y, bias, (unsigned)(N / 4), row_stride,
+                         (unsigned)(total / 4));
+    else
+      hipLaunchKernelGGL(add_bias_vec_kernel<bf16_t>, blocks, dim3(256), 0, stream, (bf16_t*)y, bias, (unsigned)(N / 4), row_stride,
+                         (unsigned)(total / 4));
+    ULLM_LAUNCH_CHECK();
+  }
   dim3 block(256), grid((unsigned)((total + 255) / 256));
   if (dtype == ULLM_F32)
     hipLaunchKernelGGL(add_bias_kernel<float>, grid, block, 0, stream, (float*)y, bias, N, row_stride, total);

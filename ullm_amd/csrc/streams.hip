@@ -152,6 +152,97 @@ streams_step_kernel(float* __restrict__ streams, const TY* __restrict__ ya, cons
   }
 }
 
+// The same for many tokens, two to four streams and rows of up to four pieces of four values a thread: with the number of streams a
+// constant every load of the row goes out before the first is used, and the mix stays in registers.  Sums in the order of the
+// kernel above (which waits for each of its four turns' loads): the same bits.
+// 2048 tokens of 2048 values in two streams, 84 MB: 22.9 -> 16.3 us (5.2 TB/s).
+template <typename TY, typename TO, int S>
+__global__ void __launch_bounds__(1024)
+streams_step_row_kernel(float* __restrict__ streams, const TY* __restrict__ ya, const TY* __restrict__ yb, float a, float b,
+                        const float* __restrict__ mix, const float* __restrict__ out_w, float mult,
+                        const float* __restrict__ in_w, const float* __restrict__ gain, float eps, int kind,
+                        TO* __restrict__ normed, const int* __restrict__ rows, int T, int H, int write_back) {
+  constexpr int NP = 4;
+  __shared__ float scratch[16];
+  const int tid = threadIdx.x, nthreads = blockDim.x;
+  const int t = rows ? rows[blockIdx.x] : blockIdx.x;
+  RowPiece<float, 4> x[NP][S], y[NP], g[NP], y2[NP];
+  int col[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    col[p] = 4 * (tid + p * nthreads);
+    const int at = col[p] < H ? col[p] : H - 4;                       // a piece past the row reads its last and is not used
+#pragma unroll
+    for (int s = 0; s < S; ++s) x[p][s] = load_piece<4>(streams + ((size_t)s * T + t) * H + at);
+    y[p] = load_piece<4>(ya + (size_t)t * H + at);
+    g[p] = load_piece<4>(gain + at);
+  }
+  if (yb != nullptr) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) y2[p] = load_piece<4>(yb + (size_t)t * H + (col[p] < H ? col[p] : H - 4));
+  }
+  float in[S], out[S], m[S][S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    in[s] = in_w[s];
+    out[s] = out_w[s];
+#pragma unroll
+    for (int to = 0; to < S; ++to) m[s][to] = mix[s * S + to];
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    if (col[p] >= H) continue;
+    RowPiece<float, 4> nx[S];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float yj = yb != nullptr ? fmaf(a, y[p].v[j], b * y2[p].v[j]) : a * y[p].v[j];     // rounded as above
+#pragma unroll
+      for (int to = 0; to < S; ++to) {
+        float v = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; ++s) v += m[s][to] * x[p][s].v[j];
+        nx[to].v[j] = v + out[to] * (mult * yj);
+      }
+      float u = 0.f;
+#pragma unroll
+      for (int s = 0; s < S; ++s) u += in[s] * nx[s].v[j];
+      y[p].v[j] = u;
+      sum += kind == NORM_LAYER ? u : u * u;
+    }
+    if (write_back) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) store_piece<4>(streams + ((size_t)s * T + t) * H + col[p], nx[s].v);
+    }
+  }
+  TO* dst = normed + (size_t)blockIdx.x * H;
+  float mean = 0.f, r;
+  if (kind == NORM_LAYER) {
+    mean = block_sum(sum, scratch) / (float)H;
+    float dev = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (col[p] < H) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float d = y[p].v[j] - mean;
+          dev += d * d;
+        }
+      }
+    r = 1.f / sqrtf(block_sum(dev, scratch) / (float)H + eps);
+  } else {
+    r = 1.f / sqrtf(block_sum(sum, scratch) / (float)H + eps);
+  }
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    if (col[p] >= H) continue;
+    float o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (y[p].v[j] - mean) * r * g[p].v[j];
+    store_piece<4>(dst + col[p], o);
+  }
+}
+
 // streams [S, T, H] float32.  ya / yb: branches [T, H] of dtype y_dtype (yb and ya may be null); normed [n, H] of
 // out_dtype (null with gain null).  rows: int32 [n] or null (then n == T and the streams are written back).
 extern "C" int ullm_streams_step(float* streams, const void* ya, const void* yb, float a, float b, int y_dtype,
@@ -186,13 +277,20 @@ extern "C" int ullm_streams_step(float* streams, const void* ya, const void* yb,
                        (const TY*)ya, (const TY*)yb, a, b, mix, out_w, mult, in_w, gain, eps, kind, (TO*)normed,     \
                        rows, T_, H, S, write_back);                                                                  \
   } while (0)
-#define STREAMS_GO(TY, TO) do { if (vec) STREAMS_GO_V(TY, TO, 4); else STREAMS_GO_V(TY, TO, 1); } while (0)
+  // the row in registers: where a thread has all four pieces of it in turn
+  const bool in_row = vec && per_thread == 4 && pieces <= 4 * threads && S >= 2 && S <= 4 && ya != nullptr && gain != nullptr &&
+                      ((uintptr_t)gain & 15) == 0;
+#define STREAMS_ROW(TY, TO, N) hipLaunchKernelGGL((streams_step_row_kernel<TY, TO, N>), dim3(n), dim3(threads), 0, stream, streams,    \
+    (const TY*)ya, (const TY*)yb, a, b, mix, out_w, mult, in_w, gain, eps, kind, (TO*)normed, rows, T_, H, write_back)
+#define STREAMS_GO(TY, TO) do { if (in_row && S == 2) STREAMS_ROW(TY, TO, 2); else if (in_row && S == 3) STREAMS_ROW(TY, TO, 3);      \
+    else if (in_row) STREAMS_ROW(TY, TO, 4); else if (vec) STREAMS_GO_V(TY, TO, 4); else STREAMS_GO_V(TY, TO, 1); } while (0)
   if (y_dtype == ULLM_F32 && out_dtype == ULLM_F32) STREAMS_GO(float, float);
   else if (y_dtype == ULLM_F32 && out_dtype == ULLM_BF16) STREAMS_GO(float, bf16_t);
   else if (y_dtype == ULLM_BF16 && out_dtype == ULLM_F32) STREAMS_GO(bf16_t, float);
   else if (y_dtype == ULLM_BF16 && out_dtype == ULLM_BF16) STREAMS_GO(bf16_t, bf16_t);
   else return ULLM_ERR_DTYPE;
 #undef STREAMS_GO
+#undef STREAMS_ROW
 #undef STREAMS_GO_V
   ULLM_LAUNCH_CHECK();
 }
