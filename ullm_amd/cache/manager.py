@@ -116,10 +116,8 @@ class CacheManager:
         rc = RequestCache(request_id, slot, 0, [[] for _ in self.groups], [0] * len(self.groups))
         if self.prefix_tree is not None and prompt is not None and len(prompt) > 1:
             matched = self.prefix_tree.match(prompt, len(prompt) - 1)
-            for per_group in matched:
-                for g, page in enumerate(per_group):
-                    rc.tables[g].append(page)
             for g in range(len(self.groups)):
+                rc.tables[g].extend([pages[g] for pages in matched])
                 self._put_row(g, slot, 0, rc.tables[g])
             rc.num_computed = len(matched) * self.page_size
         self.requests[request_id] = rc
@@ -211,9 +209,7 @@ class CacheManager:
         if self.prefix_tree is not None and tokens is not None:
             self.prefix_tree.insert(tokens, min(rc.num_computed, len(tokens)), rc.tables)
         for g, table in enumerate(rc.tables):
-            for p in table:
-                if p >= 0:
-                    self.allocators[g].decref(p)
+            self.allocators[g].decref_all(table)
             table.clear()
             self._rows[g][rc.slot] = -1
         rc.released = True
@@ -223,9 +219,7 @@ class CacheManager:
     def rewind(self, rc: RequestCache) -> None:
         """Forget the request's cache but keep its slot (recompute from the first token)."""
         for g, table in enumerate(rc.tables):
-            for p in table:
-                if p >= 0:
-                    self.allocators[g].decref(p)
+            self.allocators[g].decref_all(table)
             table.clear()
             self._rows[g][rc.slot] = -1
             rc.first_live[g] = 0

@@ -8,7 +8,7 @@ error instead of a silent corruption.
 """
 from __future__ import annotations
 
-from typing import List, Optional
+from typing import List, Optional, Sequence
 
 
 class PageError(RuntimeError):
@@ -42,6 +42,25 @@ class PageAllocator:
         if not (0 <= page < self.num_pages) or self._ref[page] <= 0:
             raise PageError(f"incref of page {page} that nobody holds")
         self._ref[page] += 1
+
+    def incref_all(self, pages: Sequence[int]) -> None:
+        """:meth:`incref` of every page, all or none."""
+        ref = self._ref
+        if pages and not (0 <= min(pages) and max(pages) < self.num_pages and all([ref[p] > 0 for p in pages])):
+            raise PageError("incref of a page that nobody holds")
+        for p in pages:
+            ref[p] += 1
+
+    def decref_all(self, pages: Sequence[int]) -> None:
+        """:meth:`decref` of every page, in order; entries below zero stand for no page."""
+        ref, free, n = self._ref, self._free, self.num_pages
+        for p in pages:
+            if p >= 0:
+                if p >= n or ref[p] <= 0:
+                    raise PageError(f"page {p} freed more often than it was held")
+                ref[p] -= 1
+                if ref[p] == 0:
+                    free.append(p)
 
     def decref(self, page: int) -> bool:
         """Drop one holder; returns True if the page went back to the free list."""

@@ -51,17 +51,17 @@ class PrefixTree:
         """Pages of the longest cached prefix of ``tokens[:limit]`` made of whole pages:
         a list (one entry per matched page) of per-group page ids.  Every returned page gets
         one more holder (the caller's block table)."""
-        node = self.root
+        node, clock = self.root, self._clock
         out: List[List[int]] = []
         for key in self._keys(tokens, limit):
-            child = node.children.get(key)
-            if child is None:
+            node = node.children.get(key)
+            if node is None:
                 break
-            child.stamp = next(self._clock)
-            for alloc, page in zip(self.allocators, child.pages):
-                alloc.incref(page)
-            out.append(list(child.pages))
-            node = child
+            node.stamp = next(clock)
+            out.append(node.pages[:])
+        # a long prompt matches hundreds of pages: their holders are counted together
+        for g, alloc in enumerate(self.allocators):
+            alloc.incref_all([pages[g] for pages in out])
         return out
 
     def insert(self, tokens: Sequence[int], num_computed: int, tables: Sequence[Sequence[int]]) -> int:
