@@ -1,5 +1,6 @@
-"""The step of several streams with a row in registers: row lengths at the edges of what its threads hold, rows picked and all, one
-branch and two, both norms; against the same in 64 bits."""
+"""The step of several streams with a row in registers: row lengths at the edges of a block's width and of the longest row its threads
+hold, rows picked and all, one branch and two, both norms; against the same in 64 bits, and bit for bit against the kernel that takes
+the rows it does not."""
 import pytest
 import torch
 
@@ -39,3 +40,29 @@ def test_step_of_many_tokens(S, H, kind, two, picked):
     assert ((got.cpu().double() - expect).abs().amax(-1) <= bound).all()
     if not picked:
         assert ((dev["x"].cpu().double() - new).abs() <= (S + 8) * 2.0 ** -24 * terms).all()
+    else:
+        assert torch.equal(dev["x"].cpu(), x)            # picked rows: nothing is written back
+
+
+@pytest.mark.parametrize("S,H", [(2, 4), (2, 252), (2, 1028), (2, 2048), (3, 1024), (3, 2052), (4, 1020), (4, 2048), (2, 16384), (4, 16384),
+                                 (2, 16388)])
+@pytest.mark.parametrize("kind", ["rms", "layer"])
+@pytest.mark.parametrize("two,picked", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("y_type,out_type", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
+def test_bits_of_the_kernel_without_the_row(S, H, kind, two, picked, y_type, out_type):
+    """Gains at an address that is no multiple of 16 are all that keeps the row out of registers: threads and pieces stay the same."""
+    g = torch.Generator(device="cuda").manual_seed(S * H)
+    T = 300
+    normal = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    x, ya, yb = normal(S, T, H), normal(T, H).to(y_type), normal(T, H).to(y_type)
+    mix, out_w, in_w, gain = normal(S, S), normal(S), normal(S), normal(H)
+    aside = torch.empty(H + 1, device="cuda")[1:].copy_(gain)
+    assert gain.data_ptr() % 16 == 0 and aside.data_ptr() % 16 == 4
+    rows = torch.arange(T, device="cuda").flip(0)[:260].int() if picked else None
+    got = []
+    for weight in (gain, aside):
+        streams = x.clone()
+        normed = ops.streams_step(streams, ya, mix, out_w, 0.5, in_w, weight, 1e-5, ops.NORM_RMS if kind == "rms" else ops.NORM_LAYER,
+                                  out_type, rows, yb if two else None, 0.5, 0.75)
+        got.append((streams, normed))
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][0], got[1][0])
