@@ -124,11 +124,13 @@ paged_attention_generic_kernel(const T* __restrict__ q, int q_stride, T* __restr
 // and a value is not finite is added key by key by ordinary arithmetic (zero times infinity must not reach a row that does
 // not see the key).
 // What bounds it: 16 x 128 x hd products of 32-bit twice a tile (1.7 us of the matrix pipe for a block's tile at hd = 128, shared by
-// the waves of the other blocks), the ordinary arithmetic beside them and two barriers; the keys and values of a tile are on their
-// way while the tile before is worked.  500 tokens, 16 heads of 128 over 8 kv heads, 32-bit: 53 us, 1000 tokens 138 (with the values
-// asked for when their products were next, and pages found by a division under a condition, 62 and 177; in blocks of eight
-// waves, which take a unit each, 62 and 149); the kernel above, which reads every key once per query head with the lanes of
-// a wave hd values apart, took 637.
+// the waves of the other blocks), the ordinary arithmetic beside them and two barriers; keys are on their way while the values before
+// them are worked, values while keys are.  The order of the loads is set by registers: at hd = 128 a unit holds two blocks of at most 256
+// a lane, with a word more in scratch every tile would wait for all that was just asked for.  500 tokens, 16 heads of 128 over 8 kv
+// heads, 32-bit: 46 us, 1000 tokens 122, 8 tokens 12.3 (keys and values of a tile both a tile ahead, 26 words in scratch: 53, 138,
+// 14.2; no load sent past a request's last tile, by a condition, behind which the compiler waits for every load: 47, 129, 11.7, but
+// 133 for 100 at hd = 256; values asked for when their products were next 62, 177, 13.5); the kernel above, which reads every key
+// once per query head with the lanes of a wave hd values apart, took 637.
 __device__ __forceinline__ bool finite4(const float4& v) {
   return isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
 }
@@ -159,7 +161,7 @@ struct RawFour<bf16_t> {
 
 // hd = 16 KC.  POW2: pages of 2^page_shift keys (a division under a run-time condition would put every load in a block of its own)
 template <typename T, int KC, bool POW2>
-__global__ void __launch_bounds__(256, KC <= 8 ? 2 : 1)      // two blocks share a unit where the registers allow it
+__global__ void __launch_bounds__(256, KC <= 8 ? 2 : 1)
 paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride,
                              const T* __restrict__ k_pool, const T* __restrict__ v_pool,
                              const int* __restrict__ positions, const int* __restrict__ token_entry,
@@ -169,7 +171,7 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
   constexpr int HD = 16 * KC, NT = (KC + 3) / 4;
   __shared__ float s_max[4][16];
   __shared__ __attribute__((aligned(16))) float s_p[16][132];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
   const int group = nq / nkv, gh = group < 16 ? group : 16, chunks = (group + 15) / 16;
   const int kvh = blockIdx.y / chunks, h0 = blockIdx.y % chunks * 16;
   const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * tp;          // later tokens see more keys: they start first
@@ -191,6 +193,7 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
   for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   auto page_index = [&](int j) { return POW2 ? j >> page_shift : j / page_size; };
+  auto in_page = [&](int j) { return POW2 ? j & (page_size - 1) : j - j / page_size * page_size; };
 
   // lane i < n_tok: the block's i-th token
   const int own_entry = token_entry[t0 + (lane < n_tok ? lane : n_tok - 1)], own_pos = positions[t0 + (lane < n_tok ? lane : n_tok - 1)];
@@ -201,15 +204,18 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
     const unsigned long long same = __ballot(lane < n_tok && own_entry == seg_entry) >> first;
     const int end = first + __builtin_ctzll(~same);      // n_tok <= 16: some bit above is clear
     const bool inside = lane >= first && lane < end;
-    const int hi = -wave_min(inside ? -own_pos : 0x7fffffff), low = wave_min(inside ? first_seen_key(own_pos, window) : 0x7fffffff);
+    const int hi = -__builtin_amdgcn_readfirstlane(wave_min(inside ? -own_pos : 0x7fffffff));
+    const int low = __builtin_amdgcn_readfirstlane(wave_min(inside ? first_seen_key(own_pos, window) : 0x7fffffff));
     const bool alone = first == 0 && end == n_tok;       // no row of the block belongs to another request
     first = end;
     const bool active = valid && entry == seg_entry;
     const int* bt = block_table + (size_t)seg_entry * bt_stride;
-    // Keys and values of both halves of a tile; up to hd = 128 registers hold them together, and the halves' products alternate.
-    // They are loaded a tile ahead, and the entries of the block table they lie by a tile before that; nothing touches a loaded
-    // value or entry until it is used (a select on it would wait for everything on its way).  An entry counts as -1 for
-    // keys past the last.
+    // Keys and values of both halves of a tile.  Up to hd = 128 registers hold three of the four at a time, and the halves' products
+    // with the queries alternate: a tile's first keys are asked for before the exponentials of the tile before, its second keys
+    // behind the first half of that tile's values, its first values behind the second, its second values when its keys are used up.
+    // The entries of the block table they lie by are loaded a tile before them; nothing touches a loaded value or entry until it
+    // is used (a select on it would wait for everything on its way).  An entry counts as -1 for keys past the last, and page 0
+    // stands in for what has none.
     constexpr int SETS = KC <= 8 ? 2 : 1;
     typename Raw::type kf[SETS][KC], vf[SETS][NT][4];
     int kpage[2], knext[2], vhave[2], vnext[2][4];
@@ -224,25 +230,27 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
     };
     // the keys of half `half` of the tile at `at`, by knext; its page stays in kpage for the tile's tests
     auto fetch_keys = [&](int half, int at) __attribute__((always_inline)) {
+      typename Raw::type (&k)[KC] = kf[SETS == 2 ? half : 0];
       const int j = at + 64 * half + 16 * wave + r, page = j <= hi ? knext[half] : -1;
       kpage[half] = page;
-      const T* src = k_pool + (((size_t)(page < 0 ? 0 : page) * nkv + kvh) * page_size + (page < 0 ? 0 : j - page_index(j) * page_size)) * HD + 4 * g;
+      const T* src = k_pool + (((size_t)(page < 0 ? 0 : page) * nkv + kvh) * page_size + (page < 0 ? 0 : in_page(j))) * HD + 4 * g;
 #pragma unroll
-      for (int c = 0; c < KC; ++c) kf[SETS == 2 ? half : 0][c] = Raw::load(src + 16 * c);
+      for (int c = 0; c < KC; ++c) k[c] = Raw::load(src + 16 * c);
     };
     // half a tile's values for this wave's dims, by vnext; a bit of vhave per chunk: whether the lane's keys of it have a page
     auto fetch_values = [&](int half, int at) __attribute__((always_inline)) {
+      typename Raw::type (&v)[NT][4] = vf[SETS == 2 ? half : 0];
       vhave[half] = 0;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const int jv = at + 64 * half + 16 * c + 4 * g, page = vnext[half][c];
         const bool have = jv <= hi && page >= 0;
         vhave[half] |= (have ? 1 : 0) << c;
-        const T* src = v_pool + ((size_t)(have ? page : 0) * nkv + kvh) * HD * page_size + (have ? jv - page_index(jv) * page_size : 0);
+        const T* src = v_pool + ((size_t)(have ? page : 0) * nkv + kvh) * HD * page_size + (have ? in_page(jv) : 0);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const int dim = 16 * (wave + 4 * n) + r;
-          vf[SETS == 2 ? half : 0][n][c] = Raw::load(src + (size_t)(dim < HD ? dim : 0) * page_size);
+          v[n][c] = Raw::load(src + (size_t)(dim < HD ? dim : 0) * page_size);
         }
       }
     };
@@ -254,14 +262,11 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
     }
 #pragma unroll
     for (int half = 0; half < SETS; ++half) fetch_keys(half, base);
+    fetch_values(0, base);
+    // from here on: entries of the half that is fetched next
 #pragma unroll
-    for (int half = 0; half < SETS; ++half) fetch_values(half, base);
-    // from here on: entries of the half that is fetched next (SETS 1: the tile's second half is, before the next tile's first)
-#pragma unroll
-    for (int half = 0; half < SETS; ++half) {
-      key_entry(half, base + 128);
-      value_entries(half, base + 128);
-    }
+    for (int half = 0; half < SETS; ++half) key_entry(half, base + 128);
+    value_entries(0, base + 128);
     for (; base <= hi; base += 128) {
       f32x4_t s[2];
       unsigned long long there[2];                       // bit r: key 16 wave + r of the half has a page
@@ -294,8 +299,12 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
         }
         there[half] = __ballot(kpage[half] >= 0);
         if constexpr (both) {
-          fetch_keys(half, base + 128);
-          key_entry(half, base + 256);
+          if (half == 0) {
+            fetch_values(1, base);
+            value_entries(1, base + 128);
+            fetch_keys(0, base + 128);
+            key_entry(0, base + 256);
+          }
         } else {
           const int next = half == 0 ? base : base + 128;            // where the other half's next keys lie
           fetch_keys(half ^ 1, next);
@@ -389,6 +398,7 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
 #pragma unroll
           for (int c = 0; c < 4; ++c)
             for (int o = 0; o < 4; ++o) {
+              __builtin_amdgcn_sched_barrier(0);         // four keys' values at a time, or this rare path sets the kernel's registers
               const int have = __shfl(vhave[half], 16 * o, 64);
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
@@ -408,8 +418,13 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
             }
         }
         if constexpr (both) {
-          fetch_values(half, base + 128);
-          value_entries(half, base + 256);
+          if (half == 0) {
+            fetch_keys(1, base + 128);
+            key_entry(1, base + 256);
+          } else {
+            fetch_values(0, base + 128);
+            value_entries(0, base + 256);
+          }
         } else {
           const int next = half == 0 ? base : base + 128;
           fetch_values(half ^ 1, next);
