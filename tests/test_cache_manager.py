@@ -28,6 +28,26 @@ def test_allocator_all_or_nothing_and_double_free():
     assert a.alloc(1) == [pages[0]]
 
 
+def test_counting_many_pages_at_once():
+    a = PageAllocator(6)
+    held = a.alloc(4)
+    a.incref_all([])
+    a.incref_all(held[:3])
+    assert [a.refcount(p) for p in held] == [2, 2, 2, 1]
+    for bad in ([held[0], 5], [held[0], 6], [-1, held[0]]):       # nobody holds it, no such page, no page: nothing is counted
+        with pytest.raises(PageError):
+            a.incref_all(bad)
+    assert [a.refcount(p) for p in held] == [2, 2, 2, 1] and a.num_free == 2
+    a.decref_all([held[3], -1, held[0], held[0]])                 # -1 stands for no page
+    assert [a.refcount(p) for p in held] == [0, 2, 2, 0] and a.num_free == 4
+    a.check()
+    assert a.alloc(2) == [held[0], held[3]]                       # freed in order: the last one freed is the first handed out
+    for bad in (5, 6):
+        with pytest.raises(PageError):
+            a.decref_all([bad])
+    a.check()
+
+
 def test_reserve_commit_release_and_table_growth():
     m = CacheManager([FULL], [6], page_size=4, max_requests=2)
     rc = m.admit("a")

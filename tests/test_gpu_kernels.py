@@ -730,6 +730,40 @@ def test_decode_attention_with_norm_rotation_and_cache_write_folded_in(ops, case
     assert (out[:len(lens)].float().cpu() - want).abs().max() <= tol(dtype, want)
 
 
+# with few waves the list of tokens is not read either, with many its order stays; requests of one key and a padding entry among them
+@pytest.mark.parametrize("requests,nkv,splits,waves,list_read", [(1, 2, 0, 0, False), (5, 2, 3, 4, False), (31, 8, 2, 1, False),
+                                                                 (32, 8, 2, 1, True), (90, 8, 0, 0, True), (40, 8, 3, 4, True)])
+def test_one_token_of_every_entry_needs_no_look_up(ops, requests, nkv, splits, waves, list_read):
+    """A step that holds one token of every entry, said to be one: the bits of the call that looks the entries up, in the output and
+    in the cache."""
+    g = torch.Generator().manual_seed(requests)
+    nq, hd, P, dtype = 2 * nkv, 128, 16, torch.bfloat16
+    lens = [1 + (37 * b) % 200 if b else 640 for b in range(requests)]
+    ks, vs = ([torch.randn(S, nkv, hd, generator=g).to(dtype).float() for S in lens] for _ in range(2))
+    k_pool, v_pool, tables = paged_cache(ks, vs, P, dtype, DEV)
+    B = requests + 1
+    positions = torch.tensor([S - 1 for S in lens] + [0], dtype=torch.int32, device=DEV)
+    entry, bt = torch.arange(B, dtype=torch.int32, device=DEV), table_tensor(tables + [[]], DEV)
+    order = sorted(range(requests), key=lambda b: -lens[b]) + [requests]
+    assert requests < 3 or order != list(range(B))
+    dec = torch.tensor(order, dtype=torch.int32, device=DEV)
+    qkv = torch.randn(B, (nq + 2 * nkv) * hd, generator=g).to(DEV, dtype)
+    used_waves, used_splits = ops.decode_split(B, nkv, 1, max(lens), hd, 0, ops.compute_units(DEV))
+    launched = B * nkv * (splits or used_splits) * (waves or used_waves)
+    assert (launched > 2 * ops.compute_units(DEV)) == list_read
+    got = []
+    for known in (False, True):
+        k_one, v_one, out = k_pool.clone(), v_pool.clone(), torch.full((B, nq * hd), float("nan"), dtype=dtype, device=DEV)
+        ops.attention_decode_fused(qkv, out, None, None, 1e-5, None, 0, 0, k_one, v_one, dec, B, positions, entry, bt, P, nq, nkv, hd,
+                                   hd ** -0.5, 0, max(lens), write_kv=True, splits=splits, waves=waves, entry_is_token=known)
+        got.append((out[:requests], k_one, v_one))
+    assert not torch.isnan(got[0][0]).any() and not torch.equal(got[0][1].view(torch.int16), k_pool.view(torch.int16))
+    assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(*got))      # pool rows without a key hold NaN
+    with pytest.raises(ops.KernelError):                   # not every token is an item
+        ops.attention_decode_fused(qkv, out, None, None, 1e-5, None, 0, 0, k_one, v_one, dec[:B - 1], B - 1, positions, entry, bt, P, nq,
+                                   nkv, hd, hd ** -0.5, 0, max(lens), write_kv=True, entry_is_token=True)
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 def test_two_large_scores_half_a_unit_apart_weigh_the_same_in_prompt_and_decode_steps(ops, hd):
     """Two keys whose scores are near 50 in the units of the exponent and half a unit apart, with opposite

@@ -1650,7 +1650,8 @@ extern "C" int ullm_attention_decode_fused_supports(int hd, int page_size, int n
 // `qkv` [tokens, (nq + 2 nkv) * hd] is the fused projection as it leaves the matrix product.  q_gain /
 // k_gain float32 [hd] or null (no norm); cos_sin float32 [table_rows, rot] or null; write_kv = 0 for a
 // layer that reads a cache another layer writes (then k and v of the projection are not used).
-// Every item must be the last token of its request so far (its position is the newest key).
+// Every item must be the last token of its request so far (its position is the newest key).  token_list null: item i is token i;
+// token_entry null: token t is entry t's.
 extern "C" int ullm_attention_decode_fused(
     const void* qkv, int qkv_stride, void* out, int out_stride, void* k_pool, void* v_pool,
     const int* token_list, int n_items, const int* positions, const int* token_entry,
