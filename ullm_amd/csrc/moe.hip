@@ -267,9 +267,10 @@ extern "C" int ullm_moe_router(const void* x, int ldx, const float* w, const flo
 }
 
 // ------------------------------------------------------------------------------- grouping by expert
-// One block, bound by its trips to memory and shared memory: the pairs are read once and counted with the addition that gives a
-// pair its place, the running sums over the experts are one wave's (2048 tokens of 4 choices among 32 experts 7.6 -> 6.0 us, 3000
-// 9.8 -> 7.5).  offsets [experts + 1]; slot_of_pair [pairs] (-1: the pair's expert has no weights); token_of_slot [pairs];
+// One block, bound by its trips to memory and shared memory: the first 16384 pairs are read once and counted with the addition that
+// gives a pair its place, the running sums over the experts are one wave's (2048 tokens of 4 choices among 32 experts 7.6 -> 6.0 us,
+// 3000 9.8 -> 7.5).  Pairs behind those are read twice, to be counted and to take their places (96000 pairs among 128 experts 68 us;
+// with their places kept in slot_of_pair from the count on 79, as it took them all before 75).  offsets [experts + 1]; slot_of_pair [pairs] (-1: the pair's expert has no weights); token_of_slot [pairs];
 // tiles [max_tiles + 1][3] = (expert, first slot, rows), rows 0 for the tiles no expert filled; the entry behind the
 // list holds the number of tiles in use.
 __global__ void __launch_bounds__(1024)
@@ -277,7 +278,7 @@ moe_sort_kernel(const int* __restrict__ ids, int n_pairs, int top, int n_experts
                 int* __restrict__ offsets, int* __restrict__ slot_of_pair, int* __restrict__ token_of_slot,
                 int* __restrict__ tiles, int max_tiles) {
   constexpr int HELD = 16;
-  __shared__ int count[MOE_MAX_ROUTER], start[MOE_MAX_ROUTER + 1], tile_base[MOE_MAX_ROUTER + 1];
+  __shared__ int count[MOE_MAX_ROUTER], start[MOE_MAX_ROUTER + 1], tile_base[MOE_MAX_ROUTER + 1], taken[MOE_MAX_ROUTER];
   const int tid = threadIdx.x;
   for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;
   __syncthreads();
@@ -293,9 +294,15 @@ moe_sort_kernel(const int* __restrict__ ids, int n_pairs, int top, int n_experts
     if (held_e[i] >= n_experts) held_e[i] = -1;
     held_at[i] = held_e[i] >= 0 ? atomicAdd(&count[held_e[i]], 1) : 0;
   }
-  for (int p = tid + HELD * (int)blockDim.x; p < n_pairs; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < n_experts) slot_of_pair[p] = atomicAdd(&count[e], 1);
+  // the pairs behind those come after them: counted here, given their places below
+  if (n_pairs > HELD * (int)blockDim.x) {
+    __syncthreads();
+    for (int e = tid; e < n_experts; e += blockDim.x) taken[e] = count[e];
+    __syncthreads();
+    for (int p = tid + HELD * (int)blockDim.x; p < n_pairs; p += blockDim.x) {
+      const int e = ids[p];
+      if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+    }
   }
   __syncthreads();
   if (tid < 64) {                                         // one wave: running sums over the experts, 64 at a time
@@ -338,7 +345,7 @@ moe_sort_kernel(const int* __restrict__ ids, int n_pairs, int top, int n_experts
     const int e = ids[p];
     int slot = -1;
     if (e >= 0 && e < n_experts) {
-      slot = start[e] + slot_of_pair[p];                  // this thread's own store above
+      slot = start[e] + atomicAdd(&taken[e], 1);
       token_of_slot[slot] = p / top;
     }
     slot_of_pair[p] = slot;
