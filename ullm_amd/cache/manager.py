@@ -116,9 +116,10 @@ class CacheManager:
         rc = RequestCache(request_id, slot, 0, [[] for _ in self.groups], [0] * len(self.groups))
         if self.prefix_tree is not None and prompt is not None and len(prompt) > 1:
             matched = self.prefix_tree.match(prompt, len(prompt) - 1)
-            for g in range(len(self.groups)):
-                rc.tables[g].extend([pages[g] for pages in matched])
-                self._put_row(g, slot, 0, rc.tables[g])
+            if matched:
+                for g in range(len(self.groups)):
+                    rc.tables[g].extend([pages[g] for pages in matched])
+                    self._put_row(g, slot, 0, rc.tables[g])
             rc.num_computed = len(matched) * self.page_size
         self.requests[request_id] = rc
         return rc

@@ -59,9 +59,9 @@ class PrefixTree:
                 break
             node.stamp = next(clock)
             out.append(node.pages[:])
-        # a long prompt matches hundreds of pages: their holders are counted together
-        for g, alloc in enumerate(self.allocators):
-            alloc.incref_all([pages[g] for pages in out])
+        if out:                     # a long prompt matches hundreds of pages: their holders are counted together
+            for g, alloc in enumerate(self.allocators):
+                alloc.incref_all([pages[g] for pages in out])
         return out
 
     def insert(self, tokens: Sequence[int], num_computed: int, tables: Sequence[Sequence[int]]) -> int:
