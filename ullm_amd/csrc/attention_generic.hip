@@ -394,24 +394,35 @@ paged_attention_tiles_kernel(const T* __restrict__ q, int q_stride, T* __restric
               for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[n][i], pf[c][i], acc[n], 0, 0, 0);
           }
         } else {
-          // lane (r, g) holds dims 4 g + i of row r; the value of key 16 c + 4 o + j at dim 4 g + i lies in lane (4 g + i, o)
+          // lane (r, g) holds dims 4 g + i of row r; the value of key 16 c + 4 o + j at dim 4 g + i lies in lane (4 g + i, o).
+          // This rare path must not set the kernel's registers: four keys' values at a time.  For pages that are no power of two it is a
+          // loop (written out for every kernel it was half of the family's code, 69 s to compile, now 50), a key at a time, and nothing
+          // ahead for all keys: `none` is a zero that the compiler does not see through.
 #pragma unroll
           for (int c = 0; c < 4; ++c)
+#pragma unroll (POW2 ? 4 : 1)
             for (int o = 0; o < 4; ++o) {
-              __builtin_amdgcn_sched_barrier(0);         // four keys' values at a time, or this rare path sets the kernel's registers
+              if constexpr (POW2) __builtin_amdgcn_sched_barrier(0);
               const int have = __shfl(vhave[half], 16 * o, 64);
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
+                int none = 0;
+                if constexpr (!POW2) {
+                  __builtin_amdgcn_sched_barrier(0);
+#ifdef __HIP_DEVICE_COMPILE__
+                  asm volatile("" : "+s"(none));
+#endif
+                }
                 const int key = at + 16 * c + 4 * o + j;
                 const bool sees = active && key <= pos && key >= lo && ((have >> c) & 1);
-                const float w = s_p[r][64 * half + 16 * c + 4 * j + o];
+                const float w = s_p[r][64 * half + 16 * c + 4 * j + o + none];
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
                   for (int i = 0; i < 4; ++i) {
                     const float4 four = Raw::values(vh[n][c]);
                     const float mine = j == 0 ? four.x : j == 1 ? four.y : j == 2 ? four.z : four.w;
-                    const float v = __shfl(mine, 16 * o + 4 * g + i, 64);
+                    const float v = __shfl(mine, 16 * o + 4 * g + i + none, 64);
                     if (sees) acc[n][i] += w * v;
                   }
               }
