@@ -1,0 +1,116 @@
+"""The panels kernel's shapes at the edges of their tiles: rows and columns past the last tile's, K that no number of parts divides, one
+stage a part, against 64-bit results; and the rule by which calls come to it."""
+import pytest
+import torch
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from ullm_amd.kernels import ops
+    return ops
+
+
+def _operands(M, N, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K + 8, generator=g, device=DEV).bfloat16()[:, :K]            # rows further apart than they are long
+    return x, (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).bfloat16(), torch.randn(N, generator=g, device=DEV)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 256), (31, 48, 320), (33, 176, 256), (97, 208, 576), (129, 272, 1024), (161, 144, 704), (255, 400, 832),
+                                   (258, 1040, 1088)])
+def test_every_shape_at_tile_edges(ops, M, N, K):
+    from ullm_amd.kernels import build, dispatch
+    lib = build.load("gemm_panels")
+    x, w, bias = _operands(M, N, K, M + N)
+    want = x.double() @ w.double().T
+    off = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)             # K products added in 32-bit
+    ref, half = want + bias.double(), N // 2
+    taken = 0
+    for shape in range(lib.ullm_gemm_panels_shapes()):
+        takes = lambda mode, slices: lib.ullm_gemm_panels_supports(M, N, K, K + 8, K, mode, shape, slices)      # noqa: B023, E731
+        for slices in (1, 2, 3, 8):
+            if not takes(dispatch.PANELS_FLOAT, slices):
+                continue
+            taken += 1
+            sums = ops.gemm_panels(x, w, shape | slices << 8, dispatch.PANELS_FLOAT)
+            assert sums.shape == (slices, M, N) and ((sums.double().sum(0) - want).abs() <= off).all(), (shape, slices)
+            assert torch.equal(ops.gemm_panels(x, w, shape | slices << 8, dispatch.PANELS_FLOAT), sums)          # by no timing
+        one = shape | 1 << 8
+        if not takes(dispatch.PANELS_STORE, 1):
+            continue
+        full = ops.gemm_panels(x, w, one, dispatch.PANELS_FLOAT)[0]
+        assert torch.equal(ops.gemm_panels(x, w, one, dispatch.PANELS_STORE), full.bfloat16()), shape
+        got = ops.gemm_panels(x, w, one, dispatch.PANELS_STORE, bias)
+        assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + off + 2.0 ** -23 * ref.abs()).all(), shape
+        act = ops.gemm_panels(x, w, one, dispatch.PANELS_STORE, bias, act=ops.ACT_RELU2)
+        assert ((act.double() - ref.clamp(min=0) ** 2).abs() <= 2.0 ** -8 * ref ** 2 + 4 * off * (ref.abs() + off)).all(), shape
+        if not takes(dispatch.PANELS_GATED, 1):
+            continue
+        for limit, alpha in ((0.0, 0.0), (1.0, 1.7)):
+            unit = ops.gemm_panels(x, w, one, dispatch.PANELS_GATED, limit=limit, alpha=alpha)
+            g, u = want[:, :half], want[:, half:]
+            if limit:
+                g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+                expect = g * torch.sigmoid(alpha * g) * (u + 1)
+            else:
+                expect = g * torch.sigmoid(g) * u
+            slack = 4 * off.amax(-1, keepdim=True) * (2 + g.abs() + u.abs()) + 2.0 ** -21 * expect.abs()        # sums, and the unit's own ulps
+            assert ((unit.double() - expect).abs() <= 2.0 ** -8 * expect.abs() + slack).all(), (shape, limit)
+    assert taken >= (24 if K >= 1024 else 8)
+
+
+@pytest.mark.gpu
+def test_what_it_refuses(ops):
+    from ullm_amd.kernels import dispatch
+    x, w, bias = _operands(40, 64, 256, 1)
+    with pytest.raises(ops.KernelError):
+        ops.gemm_panels(x, w, 99 | 1 << 8, dispatch.PANELS_STORE)                    # no such shape
+    with pytest.raises(ops.KernelError):
+        ops.gemm_panels(x, w, 0 | 2 << 8, dispatch.PANELS_STORE)                     # slices of a rounded result
+    with pytest.raises(ops.KernelError):
+        ops.gemm_panels(x, w, 1 << 8, dispatch.PANELS_GATED, bias)
+    assert not ops.gemm_panels_supports(x[:, 4:], w[:, 4:]) and not ops.gemm_panels_supports(x[:, :128], w)
+
+
+def test_when_it_is_taken():
+    """CPU: sizes on both sides of every line of the rule; every plan is one that the kernel takes, in one round of blocks."""
+    from ullm_amd.kernels import build, dispatch
+    lib = build.load("gemm_panels")
+    P = dispatch.panels
+    assert [P(r, 24576, 4096, "gated")[0] >= 0 for r in (16, 17, 256, 257, 3000)] == [False, True, True, False, False]
+    assert [P(r, 1024, 3072, "stream")[0] >= 0 for r in (16, 17, 1024, 1025)] == [False, True, True, False]
+    assert [P(r, 4096, 12288, "stream")[0] >= 0 for r in (17, 2048, 2049)] == [True, True, False]
+    assert P(64, 1000, 1024, "store")[0] < 0 and P(64, 1024, 1024, "store")[0] >= 0            # a smaller matrix than measured
+    assert P(64, 2052, 1024, "store")[0] < 0 and P(64, 2048, 1000, "store")[0] < 0 and P(64, 8200, 1024, "gated")[0] < 0
+    for rows in list(range(17, 2200, 61)) + [2048]:
+        for N, K in ((1024, 1024), (4096, 1024), (6144, 4096), (1024, 3072), (4096, 12288), (24576, 4096), (2048, 2048), (51200, 5120)):
+            for role, keep in (("store", False), ("gated", False), ("stream", False), ("stream", True)):
+                plan, mode = P(rows, N, K, role, keep)
+                if plan < 0:
+                    continue
+                assert lib.ullm_gemm_panels_supports(rows, N, K, K, K, mode, plan & 255, plan >> 8)
+                assert mode == dispatch.PANELS_FLOAT or (not keep and (mode == dispatch.PANELS_GATED) == (role == "gated"))
+
+
+@pytest.mark.gpu
+def test_parts_take_it_where_the_rule_says(ops, monkeypatch):
+    from types import SimpleNamespace
+    from ullm_amd.kernels import dispatch
+    from ullm_amd.parts.linear import gate_up, linear, linear_into_stream
+    calls, real = [], ops.gemm_panels
+    monkeypatch.setattr(ops, "gemm_panels", lambda *a, **k: calls.append(a[3]) or real(*a, **k))
+    ctx = SimpleNamespace(stacked_branches=True)
+    for rows in (16, 17, 130):
+        x, w, bias = _operands(rows, 1024, 2048, rows)
+        want = x.double() @ w.double().T
+        close = lambda y, ref: float((y.double() - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())      # noqa: E731
+        assert close(linear(x, w, bias), want + bias.double())
+        g, u = want[:, :512], want[:, 512:]
+        assert close(gate_up(x, w), g * torch.sigmoid(g) * u)
+        y = linear_into_stream(x, w, ctx)
+        assert close(y if y.dim() == 2 else y.sum(0), want)
+        assert (len(calls) == 3) == (rows > 16) and (rows == 16 or set(calls) >= {dispatch.PANELS_GATED, dispatch.PANELS_FLOAT})
+        del calls[:]

@@ -34,6 +34,12 @@ __device__ __forceinline__ void load16_to_lds_from(const void* base, unsigned of
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(at) : "memory", "m0");
 #endif
 }
+// The same for what is read once and need not stay in the caches.
+__device__ __forceinline__ void load16_to_lds_from_once(const void* base, unsigned off, unsigned at) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(off), "s"(base), "s"(at) : "memory", "m0");
+#endif
+}
 #pragma clang diagnostic pop
 __device__ __forceinline__ unsigned lds_place(unsigned char* p) {
 #ifdef __HIP_DEVICE_COMPILE__

@@ -13,10 +13,13 @@ entry costs time, never a result.
 """
 from __future__ import annotations
 
+import functools
 import json
 import os
 from dataclasses import asdict, dataclass, fields
 from typing import Dict, Optional, Tuple
+
+from . import build
 
 TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned_gfx950.json")
 
@@ -132,6 +135,50 @@ def write_entry(columns: int, inner: int, fields_measured: Dict[str, object]) ->
         json.dump(raw, f, indent=1, sort_keys=True)
         f.write("\n")
     _table = None
+
+
+PANELS_STORE, PANELS_GATED, PANELS_FLOAT = 0, 1, 2
+PANELS_MIN_ROWS = 17          # up to 16 rows the few-rows kernel, which folds what stands around the product into itself
+PANELS_MIN_WEIGHT = 1 << 20   # values of the smallest matrix it was measured on
+PANELS_MAX_SLICES = 8
+SUM_US = 4.0                  # the kernel that adds slices: its launch and the trip to memory
+
+
+@functools.lru_cache(maxsize=8192)           # of sizes alone, and asked for by every layer of every step
+def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int) -> Tuple[int, float]:
+    """The panels kernel's plan and its estimated us; a plan of -1 where it does not take the product or its blocks need more
+    than one round."""
+    plan = int(build.load("gemm_panels").ullm_gemm_panels_plan(rows, columns, inner, mode, max_slices))
+    if plan < 0 or plan >> 16 & 1:
+        return -1, 0.0
+    return plan & 0xffff, (plan >> 17) / 8
+
+
+@functools.lru_cache(maxsize=8192)
+def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False) -> Tuple[int, int]:
+    """The plan by which the panels kernel (``ops.gemm_panels``) takes x [rows, inner] times W [columns, inner], and its mode; a plan of -1
+    where another product is ahead.  Roles: ``store`` (a bfloat16 result; in float mode the slices are added by a kernel),
+    ``gated`` (W is gate | up) and ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
+    ``keep_sums`` always the sums).
+
+    It is taken from 17 rows on while its blocks fit one round of the chip: there its tiles fill it (us, what took the calls
+    before and this: gate|up 24576 x 4096 at 17 / 64 / 256 rows 36 / 43 / 64 and 32 / 36 / 58; 6144 x 1024 at 40 / 256 / 800 7.9 / 15.1 / 17.3 and
+    5.8 / 9.6 / 15.0; 4096 x 12288 into the stream at 130 / 512 / 1024 30.6 / 83 / 118 and 26.4 / 51 / 94; 6144 x 4096 at 64 / 256 / 1024 17.8 / 31 / 53
+    and 16.8 / 25.7 / 53.3).  In two rounds the library's tiles are ahead (6144 x 4096 at 1300 rows 65 and 83, gate|up 24576 x 4096 at 320
+    79 and 87), and from 1025 rows on also in one where a matrix has few columns (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 /
+    24.1; 4096 x 1024 at 1300 20.1 and 16.0, 4096 x 12288 at 1300 / 2048 146 / 191 and 133 / 174)."""
+    if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and columns < 2048):
+        return -1, 0
+    if role == "gated":
+        return _panels_plan(rows, columns, inner, PANELS_GATED, 1)[0], PANELS_GATED
+    sums, sums_us = _panels_plan(rows, columns, inner, PANELS_FLOAT, PANELS_MAX_SLICES)
+    if role == "stream" and keep_sums:
+        return sums, PANELS_FLOAT
+    whole, whole_us = _panels_plan(rows, columns, inner, PANELS_STORE, 1)
+    whole_us += rows * columns * 2 / 5e6 if role == "stream" else 0.0
+    if sums >= 0 and sums_us + (SUM_US if role == "store" else 0.0) < whole_us or whole < 0:
+        return sums, PANELS_FLOAT
+    return whole, PANELS_STORE
 
 
 def gated_tile_groups(rows: int, columns: int, inner: int) -> int:

@@ -215,7 +215,7 @@ def derive_limits(times: dict, roles, columns: int, inner: int) -> dict:
         changes["fold_norm"] = _ahead_up_to(rows, get("skinny+norm"), [unfolded])
         # above the rows the weight-streaming kernels take: partial sums and the kernel that adds them, against the library
         taken = max(changes["skinny"], changes["rows"])
-        upto = _ahead_up_to(rows, get("partial sums>sum"), [get("library")], start=taken)
+        upto = _ahead_up_to(rows, get("partial sums>sum"), [get("library"), get("panels")], start=taken)
         changes["sums_from"], changes["sums_to"] = (taken + 1, upto) if upto > taken else (0, 0)
     if "silu" in roles:
         changes["silu_skinny"] = _ahead_up_to(rows, get("skinny+silu"), [get("rows+silu"), get("library+silu")])
@@ -295,6 +295,9 @@ def tune(args) -> None:
                 timed("skinny+norm", M, lambda v: (lambda: ops.gemm_skinny_normed(stream, gain, 1e-6, ws[v])))
             if M <= ops.ROWS_MAX_ROWS and ops.gemm_rows_supports(x, ws[0]):
                 timed("rows", M, lambda v: (lambda: ops.gemm_rows(x, ws[v])))
+            plan, mode = dispatch.panels(M, N, K, "store")
+            if plan >= 0 and ops.gemm_panels_supports(x, ws[0]):
+                timed("panels", M, lambda v: (lambda: ops.gemm_bf16(x, ws[v])))
             if M > 16 and N % 4 == 0 and ops.gemm_partial_sums_supports(x, ws[0]):
                 timed("partial sums>sum", M, lambda v: (lambda: ops.sum_stacks(ops.gemm_partial_sums(x, ws[v]))))
         if "silu" in roles:

@@ -1268,6 +1268,33 @@ def gemm_rows(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
 TILES_STORE, TILES_GATED, TILES_FLOAT = 0, 1, 2
 
 
+def gemm_panels_supports(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the operands lie as the panels kernel wants them (whether it takes their sizes: ``dispatch.panels``)."""
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
+            and x.shape[1] == w.shape[1] and (x.data_ptr() | w.data_ptr()) % 16 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+            and x.shape[0] * x.stride(0) < 2 ** 31 and w.shape[0] * w.stride(0) < 2 ** 31)
+
+
+def gemm_panels(x: torch.Tensor, w: torch.Tensor, plan: int, mode: int, bias: Optional[torch.Tensor] = None, limit: float = 0.0,
+                alpha: float = 0.0, act: Optional[int] = None) -> torch.Tensor:
+    """x [M, K] times W [N, K] transposed by the panels kernel in the shape that ``plan`` names (``dispatch.panels``): bfloat16
+    [M, N], of gate|up weights [M, N / 2], or the slices' sums, float32 [slices, M, N]."""
+    M, K = x.shape
+    N = w.shape[0]
+    _need(plan >= 0 and gemm_panels_supports(x, w), "operands outside what the kernel takes")
+    if bias is not None:
+        _need(bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == N, "bias must be contiguous float32 [N]")
+    if mode == dispatch.PANELS_FLOAT:
+        out = torch.empty((plan >> 8, M, N), dtype=torch.float32, device=x.device)
+    else:
+        out = torch.empty((M, N // 2 if mode == dispatch.PANELS_GATED else N), dtype=torch.bfloat16, device=x.device)
+    _check(build.load("gemm_panels").ullm_gemm_panels(
+        _p(x), _c_int(x.stride(0)), _p(w), _c_int(w.stride(0)), _p(bias), _p(out), _c_int(out.shape[-1]), _c_int(M), _c_int(N), _c_int(K),
+        _c_int(mode), _c_int(plan & 0xff), _c_int(plan >> 8), _c_float(limit), _c_float(alpha), _c_int(0 if act is None else act + 1),
+        _stream()), "gemm_panels")
+    return out
+
+
 def gemm_tiles_supports(x: torch.Tensor, w: torch.Tensor, mode: int = TILES_STORE) -> bool:
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
             and (x.data_ptr() | w.data_ptr()) % 16 == 0
@@ -1301,8 +1328,9 @@ _MM_TAKES_OUT_DTYPE = "out_dtype" in (torch.mm.__doc__ or "")
 
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
               out_dtype: Optional[torch.dtype] = None, act: Optional[int] = None) -> torch.Tensor:
-    """bfloat16 operands, 32-bit accumulation.  Few rows go to the weight-streaming kernels (up to how many
-    for this matrix: :func:`dispatch.limits`), some more, where that was measured to be ahead, to the partial-sums
+    """bfloat16 operands, 32-bit accumulation.  Up to 16 rows go to the weight-streaming kernels, up to one or two thousand, as
+    the matrix has it, to the panels kernel (:func:`dispatch.panels`; not where a matrix's limits name rows for the partial-sums kernel).  What it does not take goes, up to how many rows
+    for this matrix :func:`dispatch.limits` says, to the weight-streaming kernels, some more, where that was measured to be ahead, to the partial-sums
     kernel and a kernel that adds its stacks; thousands of rows, where the library's choice for them was measured to
     fall off, go to the large product (:func:`gemm_tiles`); the rest go through the library product (as the reference's
     linears do, ullm/layers/linear.py:165), which for 32-bit output (logits) stores the accumulator unrounded.
@@ -1310,6 +1338,14 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     the activation kernel behind the others."""
     out_dtype = out_dtype or a.dtype
     M = a.shape[0]
+    if (out_dtype == torch.bfloat16 and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w)
+            and not dispatch.limits(w.shape[0], w.shape[1]).sums_from):
+        plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "store")
+        if plan >= 0 and mode == dispatch.PANELS_STORE:
+            return gemm_panels(a, w, plan, mode, bias, act=act)
+        if plan >= 0:
+            y = sum_stacks(gemm_panels(a, w, plan, mode), bias)
+            return y if act is None else activation(y, act, out=y)
     if act is not None:
         lim = dispatch.limits(w.shape[0], w.shape[1])
         if M <= (lim.f32_skinny if out_dtype == torch.float32 else lim.skinny) and gemm_skinny_supports(a, w):

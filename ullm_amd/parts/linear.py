@@ -84,7 +84,8 @@ def add_into_stream(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tenso
 
 
 def gate_up(x: torch.Tensor, weight: torch.Tensor, limit: float = 0.0, alpha: float = 0.0) -> torch.Tensor:
-    """silu(x g^T) * (x u^T) for the stacked weights g | u [2 I, K]: by the few-rows kernel or the kernel for up
+    """silu(x g^T) * (x u^T) for the stacked weights g | u [2 I, K]: from 17 rows on by the panels kernel while its blocks
+    fit one round (``dispatch.panels``), else by the few-rows kernel or the kernel for up
     to 128 rows with the activation on store, up to the row counts the matrix's limits name; beyond, by the large product with the
     activation on store where its tiles fill the chip (``dispatch.gated_tile_groups``); else by the
     library product and the activation kernel (float32 always: the 32-bit product, then the kernel).  With
@@ -93,6 +94,10 @@ def gate_up(x: torch.Tensor, weight: torch.Tensor, limit: float = 0.0, alpha: fl
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
         lim = dispatch.limits(weight.shape[0], weight.shape[1])
         unit = dict(limit=limit, alpha=alpha) if limit > 0 else {}
+        if rows >= dispatch.PANELS_MIN_ROWS and ops.gemm_panels_supports(x, weight):
+            plan, mode = dispatch.panels(rows, weight.shape[0], weight.shape[1], "gated")
+            if plan >= 0:
+                return ops.gemm_panels(x, weight, plan, mode, **unit)
         if rows <= lim.silu_skinny and ops.gemm_skinny_supports(x, weight):
             return ops.gemm_skinny_silu(x, weight, **unit)
         if rows <= min(lim.silu_rows, ops.ROWS_MAX_ROWS) and ops.gemm_rows_supports(x, weight, silu=True):
@@ -120,12 +125,17 @@ def can_fuse(residual: torch.Tensor, dtype: torch.dtype, *weights: torch.Tensor)
 
 def linear_into_stream(x: torch.Tensor, weight: torch.Tensor, ctx) -> torch.Tensor:
     """The last projection of a mixer or feed-forward, whose result the next norm adds to the residual
-    stream.  For a range of row counts that depends on the matrix (17 to 256 for all but small ones), in
-    bfloat16 and where the model's norms add stacks, it is a stack of float32 partial sums over slices of
-    the inner dimension (the slices fill the chip, the norm adds them in order); otherwise the plain
-    product.  For few long rows the library's choice of kernel is two to five times off the memory
-    roofline at these row counts."""
+    stream.  In bfloat16 and where the model's norms add stacks it is, from 17 rows on, a stack of float32 partial sums over slices of
+    the inner dimension (the slices fill the chip, the norm adds them in order), by the panels kernel while its blocks fit
+    one round of the chip (``dispatch.panels``; where one slice is ahead, beyond the rows that always were 32-bit sums, a
+    bfloat16 result) or for the matrices' rows that :func:`dispatch.limits` names by the partial-sums kernel (inner sizes that are no whole stages
+    of 64); otherwise the plain product."""
     lim = dispatch.limits(weight.shape[0], weight.shape[1])
+    rows = x.shape[0]
+    if ctx.stacked_branches and rows >= dispatch.PANELS_MIN_ROWS and ops.gemm_panels_supports(x, weight):
+        plan, mode = dispatch.panels(rows, weight.shape[0], weight.shape[1], "stream", lim.stacked_from <= rows <= lim.stacked_to)
+        if plan >= 0:
+            return ops.gemm_panels(x, weight, plan, mode)
     if (ctx.stacked_branches and x.dtype == torch.bfloat16 and lim.stacked_from > 0
             and lim.stacked_from <= x.shape[0] <= lim.stacked_to and ops.gemm_partial_sums_supports(x, weight)):
         return ops.gemm_partial_sums(x, weight)
