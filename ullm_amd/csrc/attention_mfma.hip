@@ -18,6 +18,7 @@
 // Semantics as in the general kernel: causal with the queries at the end of the keys, optional
 // window or chunk (a negative `window`: see first_seen_key), query head h reads kv head h / (nq / nkv) (ullm/layers/attention.py:76-104,271,298-309).
 #include "common.h"
+#include "launchers.h"
 #include <type_traits>
 #include "lds_load.h"
 #include "no_alloc.h"

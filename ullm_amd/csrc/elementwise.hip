@@ -7,6 +7,7 @@
 // (ullm/layers/activation.py:16-18), cache write of k after norm+rotation and raw v
 // (ullm/layers/attention.py:288-296).
 #include "common.h"
+#include "launchers.h"
 
 __device__ __forceinline__ float4 ld4_f32(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 ld4_f32(const bf16_t* p) {

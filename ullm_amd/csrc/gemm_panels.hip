@@ -29,6 +29,7 @@
 // unit of them, 16 TB/s in all, and the larger a tile the more products it makes of that; around it a launch, the first loads' way
 // and the store, 2 to 7 us.
 #include "mfma_tiles.h"
+#include "launchers.h"
 
 enum { PANELS_STORE = 0, PANELS_GATED = 1, PANELS_FLOAT = 2 };
 

@@ -11,6 +11,7 @@
 // form writes half the columns and spares the activation kernel's pass (604 -> 467 us at 3000 x 24576 x 4096).  Two neighbouring
 // 16 x 16 results leave as lines of 64 bytes a row: 8192 x 6144 x 4096 302 -> 293 us against lines of 32.
 #include "mfma_tiles.h"
+#include "launchers.h"
 
 enum { TILES_STORE = 0, TILES_GATED = 1, TILES_FLOAT = 2 };
 

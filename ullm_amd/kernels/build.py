@@ -32,9 +32,11 @@ HIPCC_FLAGS = [
 ]
 HEADERS = ["common.h"]
 FAMILY_HEADERS = {"gemm_simple": ["mfma_f32.h"], "attention_generic": ["lds_load.h", "mfma_f32.h"],
-                  "attention_mfma": ["no_alloc.h", "lds_load.h"], "moe": ["lds_load.h", "mfma_tiles.h"],
+                  "attention_mfma": ["no_alloc.h", "lds_load.h", "launchers.h"], "moe": ["lds_load.h", "mfma_tiles.h"],
                   "decay_scan": ["decay_inputs.h"], "decay_chunks": ["decay_inputs.h"],
-                  "gemm_tiles": ["lds_load.h", "mfma_tiles.h"], "gemm_panels": ["lds_load.h", "mfma_tiles.h"],
+                  "gemm_tiles": ["lds_load.h", "mfma_tiles.h", "launchers.h"],
+                  "gemm_panels": ["lds_load.h", "mfma_tiles.h", "launchers.h"],
+                  "elementwise": ["launchers.h"], "dense_layers": ["launchers.h"],
                   "short_conv": ["short_conv.h"], "pooled": ["short_conv.h"], "matrix_memory": ["short_conv.h"]}     # headers only this family includes
 
 _lock = threading.Lock()

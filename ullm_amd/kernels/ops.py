@@ -1266,6 +1266,7 @@ def gemm_rows(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
 
 
 TILES_STORE, TILES_GATED, TILES_FLOAT = 0, 1, 2
+TILES_GROUPS = 4                         # 64-row groups a block of the large product takes where nobody says
 
 
 def gemm_panels_supports(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -1303,7 +1304,7 @@ def gemm_tiles_supports(x: torch.Tensor, w: torch.Tensor, mode: int = TILES_STOR
 
 
 def gemm_tiles(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, gated: bool = False,
-               out_dtype: torch.dtype = torch.bfloat16, groups: int = 4, limit: float = 0.0,
+               out_dtype: torch.dtype = torch.bfloat16, groups: int = TILES_GROUPS, limit: float = 0.0,
                alpha: float = 0.0) -> torch.Tensor:
     """x [M, K] times w [N, K] transposed, bfloat16 with 32-bit sums, in tiles of 64 ``groups`` (2 or 4) rows by 256 of w:
     bfloat16 (+ ``bias``) or float32; ``gated``: w holds gate rows, then as many up rows, and the result is silu(gate) * up or

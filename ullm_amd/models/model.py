@@ -17,6 +17,7 @@ from ..kernels import ops
 from ..parts import (Block, KVNeed, LayerCache, Norm, Part, PartEnv, StateNeed, StepContext, WeightDecl,
                      build_part, cache_needs_of, walk)
 from ..parts.block import join_streams
+from ..parts.dense import alike_layers, run_layers
 from ..parts.linear import linear
 
 
@@ -89,6 +90,8 @@ class Model:
                     or self.cache_owner[source] >= self.cache_owner[reader]):
                 raise ValueError(f"cache {reader} reads the keys of cache {source}: no layer with keys of its own that runs before it")
         self._keeps_embedding = any(b.needs_embedding for b in self.blocks)
+        # how many of the first layers run are alike, so that their launches can go out from one native call
+        self._alike = alike_layers([self.blocks[layer] for layer, _ in self.run_order]) if plan.streams == 0 else 0
         self.embedding: Optional[torch.Tensor] = None
         self.head: Optional[torch.Tensor] = None
         self.head_bias: Optional[torch.Tensor] = None
@@ -186,6 +189,14 @@ class Model:
         return len(cache_needs_of(self.blocks[self.run_order[self.cache_owner[cache_id]][0]]))
 
     # ------------------------------------------------------------------ forward
+    def _cache_of(self, idx: int, caches: Dict[int, LayerCache]) -> LayerCache:
+        """What the idx-th layer run sees of the cache."""
+        cache_id = self.run_order[idx][1]
+        cache = caches.get(cache_id)
+        if cache is None:
+            return LayerCache()
+        return cache if self.cache_owner[cache_id] == idx else cache.reader()
+
     def forward(self, ctx: StepContext, caches: Dict[int, LayerCache], logit_rows: Optional[torch.Tensor]):
         """Runs the batch through every layer of the run order and returns float32 logits
         [len(logit_rows), vocab] (None if no row is wanted)."""
@@ -198,12 +209,15 @@ class Model:
             residual = ops.streams_spread(residual, self.plan.streams)
         if self._keeps_embedding:
             ctx.embedded = residual.clone()      # the stream's rows are written in place from here on
-        for idx, (layer, cache_id) in enumerate(self.run_order):
-            cache = caches.get(cache_id)
-            if cache is None:
-                cache = LayerCache()
-            elif self.cache_owner[cache_id] != idx:
-                cache = cache.reader()
+        first = 0
+        if self._alike > 1 and not ctx.decode_only:
+            run = range(self._alike)
+            pending = run_layers([self.blocks[self.run_order[i][0]] for i in run], [self._cache_of(i, caches) for i in run],
+                                 residual, ctx)
+            first = 0 if pending is None else self._alike
+        for idx in range(first, len(self.run_order)):
+            layer = self.run_order[idx][0]
+            cache = self._cache_of(idx, caches)
             block = self.blocks[layer]
             if block.hands_norm_ahead and idx + 1 < len(self.run_order):
                 # a block whose last kernel can prepare the norm that follows is told which norm that is
