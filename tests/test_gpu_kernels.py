@@ -1387,3 +1387,29 @@ def test_gemm_rows(ops, shape):
             assert torch.equal(again, got[3:20])
     with pytest.raises(ops.KernelError):
         ops.gemm_rows(torch.randn(129, K, device=DEV).bfloat16(), w[:N])
+
+
+@pytest.mark.parametrize("requests,longest", [(24, 500), (32, 700), (40, 520), (64, 700), (80, 640), (100, 900), (64, 1500), (33, 40)])
+def test_decode_launches_by_pairs_and_keys(ops, requests, longest):
+    """Every way the keys of many requests are cut (waves of a block, blocks, both), requests of one key to the longest among them, with
+    the new key made by the kernel and found in the cache: against softmax in 64 bits."""
+    g = torch.Generator().manual_seed(requests)
+    nkv, hd, P, dtype = 8, 64, 16, torch.bfloat16
+    nq = 2 * nkv
+    lens = [1 + (longest - 1) * ((11 * b) % 16) // 15 for b in range(requests)]
+    ks, vs = ([torch.randn(S, nkv, hd, generator=g).to(dtype).float() for S in lens] for _ in range(2))
+    k_pool, v_pool, tables = paged_cache(ks, vs, P, dtype, DEV)
+    positions = torch.tensor([S - 1 for S in lens], dtype=torch.int32, device=DEV)
+    entry, bt = torch.arange(requests, dtype=torch.int32, device=DEV), table_tensor(tables, DEV)
+    dec = torch.tensor(sorted(range(requests), key=lambda b: -lens[b]), dtype=torch.int32, device=DEV)
+    q = torch.randn(requests, nq * hd, generator=g).to(dtype)
+    want = torch.stack([torch.cat([torch.softmax(ks[b][:, h // 2].double() @ q[b, h * hd:(h + 1) * hd].double() * hd ** -0.5, 0)
+                                   @ vs[b][:, h // 2].double() for h in range(nq)]) for b in range(requests)]).float()
+    out = torch.full((requests, nq * hd), float("nan"), dtype=dtype, device=DEV)
+    ops.attention_decode_mfma(q.to(DEV), out, k_pool, v_pool, dec, requests, positions, entry, bt, P, nq, nkv, hd, hd ** -0.5, 0, longest)
+    assert (out.float().cpu() - want).abs().max() <= tol(dtype, want), ops.decode_split(requests, nkv, 1, longest, hd)
+    qkv = torch.cat([q] + [torch.stack([t[b][-1].reshape(-1) for b in range(requests)]).to(dtype) for t in (ks, vs)], 1).to(DEV)
+    fused = torch.full_like(out, float("nan"))
+    ops.attention_decode_fused(qkv, fused, None, None, 1e-5, None, 0, 0, k_pool, v_pool, dec, requests, positions, entry, bt, P, nq, nkv, hd,
+                               hd ** -0.5, 0, longest, write_kv=True, entry_is_token=True)
+    assert (fused.float().cpu() - want).abs().max() <= tol(dtype, want)

@@ -1566,7 +1566,7 @@ static int decode_launch(
   if (extras && fuse) return ULLM_ERR_UNSUPPORTED;
   if (extras && extras->bias && extras->bias_rows <= 0) return ULLM_ERR_SHAPE;
   if (!ullm_attention_mfma_supports(hd, page_size, nq, nkv)) return ULLM_ERR_UNSUPPORTED;
-  if (waves != 1 && waves != 4 && waves != 8) return ULLM_ERR_UNSUPPORTED;
+  if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return ULLM_ERR_UNSUPPORTED;
   if (hd == 256 && waves == 8) waves = 4;                // shared memory of the merge
   if (num_splits < 1 || num_splits > 65535) return ULLM_ERR_SHAPE;
   if (num_splits > 1 && !workspace) return ULLM_ERR_SHAPE;
@@ -1581,11 +1581,13 @@ static int decode_launch(
 #define CALL_AS(N, F) do {                                                                                     \
     if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, F>), grid, block, 0, stream, ARGS);      \
     else if (waves == 4) hipLaunchKernelGGL((attention_decode_kernel<N, 4, F>), grid, block, 0, stream, ARGS); \
+    else if (waves == 2) hipLaunchKernelGGL((attention_decode_kernel<N, 2, F>), grid, block, 0, stream, ARGS); \
     else hipLaunchKernelGGL((attention_decode_kernel<N, 1, F>), grid, block, 0, stream, ARGS);                 \
   } while (0)
 #define CALL_EXTRA(N) do {                                                                                               \
     if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, false, true>), grid, block, 0, stream, ARGS);      \
     else if (waves == 4) hipLaunchKernelGGL((attention_decode_kernel<N, 4, false, true>), grid, block, 0, stream, ARGS); \
+    else if (waves == 2) hipLaunchKernelGGL((attention_decode_kernel<N, 2, false, true>), grid, block, 0, stream, ARGS); \
     else hipLaunchKernelGGL((attention_decode_kernel<N, 1, false, true>), grid, block, 0, stream, ARGS);                 \
   } while (0)
   if (extras) {

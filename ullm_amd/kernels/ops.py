@@ -1409,25 +1409,44 @@ def decode_split(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128
     the other, each a round trip to memory, so few (token, kv head) pairs with many keys are cut over
     several blocks, up to one block per compute unit (more would run in a second round), and a second
     small kernel adds the blocks' partial results; that kernel costs about as much as walking eight more
-    tiles, so short contexts are not cut.  Mostly a block is a single wave (several are resident on a
-    SIMD, they start and end independently and one's start overlaps the others' streaming, and their number
-    need not be a multiple of the compute units); four waves a block where few pairs have very many keys.
+    tiles, so short contexts are not cut.  A pair of half the compute units' number and more is cut into as many waves as make one
+    a SIMD, two with long contexts; they share a block, which adds their results itself, where there are two or four of them
+    (their number need not be a multiple of the compute units; four waves a block where few pairs have very many keys).
     With a window or a chunk (``window`` < 0) a token reads at most its keys (and up to 31 before them, to the tile's edge),
     however long its context is.  ``units``: the device's compute units, four SIMDs each."""
     pairs = max(1, n_items * nkv * groups)
     simds = 4 * units
-    if pairs >= simds:
+    if pairs > simds:
         return 1, 1
     if window != 0:
         max_kv = min(max_kv, abs(window) + 31)
     tiles = -(-max_kv // 32)
-    if pairs > units:
-        # single waves, two to four to a SIMD, so that the launch has no rounds of whole blocks (four-wave blocks,
-        # one to a compute unit, take 49 us at 264 pairs against 30 us at 256); up to 2.25 pairs a unit cut in three
-        # where that still gives at most one wave per SIMD and compute unit, else in two
-        return 1, (max(2, min(3, simds // pairs)) if pairs <= units * 9 // 4 and tiles > 16 else 1)
-    if pairs == units:
-        return (4 if tiles > 16 else 1), 1
+    if tiles >= (96 if pairs == units else 64 if 8 * pairs <= 13 * units else 36) and pairs >= units:
+        # two waves a SIMD, also where that takes blocks whose results a second kernel adds: us of 384 / 512 pairs with 8192 keys 232 -> 202 /
+        # 292 -> 264, of 640 421 -> 329, of 800 529 -> 423, of 256 with 4096 82 -> 74
+        n = 2 * simds // pairs
+        return {2: (1, 2), 3: (1, 3), 4: (4, 1)}.get(n) or ((2, 3) if n in (6, 7) else (2, 4))
+    if pairs > 2 * units:
+        # more than half a wave a SIMD already: three single waves a pair that two a SIMD hold, a second wave in the block only of longer
+        # contexts (576 pairs with 512 keys 31.9 -> 28.8, 640 with 1024 58.3 -> 52.0, 896 with 768 55.6 -> 54.5; 720 with 512 34.2, in
+        # two waves 35.6)
+        if pairs * 3 <= 2 * simds:
+            return (1, 3) if tiles >= 16 else (1, 1)
+        return (2, 1) if tiles >= 24 and pairs * 4 >= 3 * simds else (1, 1)
+    if pairs >= units:
+        # a wave a SIMD, the waves of a pair in one block where they are two or four (64 requests of an 8B model, 512 pairs, with 768 keys 35.6 ->
+        # 32.5 and no second kernel, 384 with 512 26.7 -> 22.3, 256 with 512 23.0 -> 15.2); three make blocks of their own
+        # (288 with 512 23.8 -> 19.1), short contexts two (256 keys 14.3 -> 12.3)
+        n = simds // pairs
+        if n == 2 and tiles >= 30 and 8 * pairs <= 13 * units:
+            return 1, 2                                    # 384 with 1400 keys 48.1, in one block 50.7
+        return (1, 1) if tiles <= 2 else (4, 1) if n == 4 else (1, 3) if n == 3 and tiles > 8 else (2, 1)
+    if 2 * pairs > units and 2 < tiles <= 16:
+        # short contexts: no second kernel (192 pairs with 256 keys 12.7 -> 9.9, 248 with 512 18.0 -> 15.3; 192 with 512 18.4 -> 14.2)
+        if tiles <= 8 or 8 * pairs >= 7 * units:
+            return 4, 1
+        if 4 * pairs >= 3 * units:
+            return 1, 4
     # up to 16 blocks a pair; up to 32 where very few pairs have very many keys (one request at 4 096 keys and
     # more: 134 MB of cache at 32 768 keys in 34 us against 49 us with 16; three or four requests at 32 000 keys:
     # 70 and 89 us against 89 and 93 us; two requests are better off with 16 blocks of four waves)
