@@ -1211,14 +1211,18 @@ attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __r
 // shared memory depends on, would otherwise wait for all of them before every read.  The waits for them
 // stand in the code, by count (a wave's loads complete in order), and the loop holds no load of the
 // compiler's own whose wait could be off by the ones it does not see: the page ids lie in shared memory.
-#define DMA_TILES 4                       // tiles of shared memory that take turns
+// Who does what in a block: TEAM waves take a part of the keys (KS parts), TILES tiles of shared memory a part take turns.
+//   HEADS 4   one query head a wave, 32 tokens (head groups of three and more; with fewer heads waves would only load)
+//   HEADS 2   groups of at most two heads.  KS 1 and 2: two heads by two tiles of 32 tokens that follow one another, so that every
+//             wave has work (8000 tokens of 16 heads over 8 502 TFLOP/s with waves idle); KS 4: two heads, the keys in four parts by teams of
+//             two waves, where tiles are few
 #define DMA_TABLE_TILES 128               // tiles whose page ids shared memory holds at a time (and 4 more, for the loads ahead)
 
-template <int NQK>
+template <int NQK, int TEAM_ = PREFILL_WAVES>
 struct DmaTile {
-  static constexpr int HD = 32 * NQK;
+  static constexpr int HD = 32 * NQK, TEAM = TEAM_;
   static constexpr int PR = HD / 8;       // 16-byte pieces of a key row
-  static constexpr int ROUNDS = NQK / 2;  // load instructions per wave for a tile's keys, and as many for its values
+  static constexpr int ROUNDS = 2 * NQK / TEAM;  // load instructions per wave for a tile's keys, and as many for its values
   static constexpr int KBYTES = 32 * 2 * HD, VBYTES = HD * 64;
   static constexpr int BYTES = KBYTES + VBYTES;
   static_assert(NQK == 4, "head size 128 (with 64 the staged kernel is the faster one)");
@@ -1228,23 +1232,22 @@ struct DmaTile {
 };
 
 // What a lane's loads need that does not change from tile to tile.
-template <int NQK>
+template <class T>
 struct DmaLanes {
-  unsigned k_off[DmaTile<NQK>::ROUNDS];   // bytes from the first key row of the instruction's 16-key sub-block
-  int k_sub[DmaTile<NQK>::ROUNDS];        // which of the tile's two sub-blocks (the same in the whole wave)
-  unsigned v_off[DmaTile<NQK>::ROUNDS];   // bytes from the sub-block's first key in dim 0
-  int v_sub[DmaTile<NQK>::ROUNDS];        // which sub-block this lane's piece lies in
-  int dest[DmaTile<NQK>::ROUNDS];         // where the instruction's 1024 bytes go inside the tile's keys (and values)
+  unsigned k_off[T::ROUNDS];   // bytes from the first key row of the instruction's 16-key sub-block
+  int k_sub[T::ROUNDS];        // which of the tile's two sub-blocks (the same in the whole wave)
+  unsigned v_off[T::ROUNDS];   // bytes from the sub-block's first key in dim 0
+  int v_sub[T::ROUNDS];        // which sub-block this lane's piece lies in
+  int dest[T::ROUNDS];         // where the instruction's 1024 bytes go inside the tile's keys (and values)
 };
 
-template <int NQK>
-__device__ __forceinline__ DmaLanes<NQK> dma_lanes(int page_size) {
-  using T = DmaTile<NQK>;
-  DmaLanes<NQK> d;
-  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % PREFILL_WAVES;
+template <class T>
+__device__ __forceinline__ DmaLanes<T> dma_lanes(int page_size) {
+  DmaLanes<T> d;
+  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % T::TEAM;
 #pragma unroll
   for (int rd = 0; rd < T::ROUNDS; ++rd) {
-    const int ins = wave + PREFILL_WAVES * rd;
+    const int ins = wave + T::TEAM * rd;
     const int at = 64 * ins + lane;                       // the lane's place among the tile's pieces, as they lie in LDS
     const int key = at / T::PR, kpiece = (at % T::PR) ^ T::key_swizzle(key);
     d.k_sub[rd] = __builtin_amdgcn_readfirstlane(key >> 4);
@@ -1260,11 +1263,10 @@ __device__ __forceinline__ DmaLanes<NQK> dma_lanes(int page_size) {
 // Start the loads of the tile at key0 into the tile of shared memory at `tile` (keys, then values); page0 / page1
 // are the page ids of its two 16-key sub-blocks.  A sub-block without a page reads page 0: its keys are
 // never seen, and its values count as zero in the products.
-template <int NQK>
+template <class T>
 __device__ __forceinline__ void dma_tile_load(unsigned char* tile, int key0, int page0, int page1, int page_size,
-                                              const DmaLanes<NQK>& dl, const bf16_t* __restrict__ k_head,
+                                              const DmaLanes<T>& dl, const bf16_t* __restrict__ k_head,
                                               const bf16_t* __restrict__ v_head, unsigned page_elems) {
-  using T = DmaTile<NQK>;
   const unsigned off0 = (unsigned)(key0 % page_size), off1 = (unsigned)((key0 + 16) % page_size);
   const size_t base0 = (size_t)(unsigned)(page0 < 0 ? 0 : page0) * page_elems;
   const size_t base1 = (size_t)(unsigned)(page1 < 0 ? 0 : page1) * page_elems;
@@ -1329,31 +1331,34 @@ __device__ __forceinline__ void dma_tile_products(const unsigned char* __restric
   }
 }
 
-// EXTRA: a bias by distance (never null here; the block's four heads' rows are copied to dynamic shared memory
+// EXTRA: a bias by distance (never null here; the waves' heads' rows are copied to dynamic shared memory
 // first, [PREFILL_WAVES][bias_rows] floats) and the gate per head, as in attention_prefill_kernel.
-template <int NQK, int KS, bool EXTRA = false>
-__global__ void __launch_bounds__(64 * PREFILL_WAVES * KS, 2 / KS)
+template <int NQK, int HEADS, int KS, bool EXTRA = false>
+__global__ void __launch_bounds__(KS == 4 ? 512 : 64 * PREFILL_WAVES * KS, KS == 1 ? 2 : 1)
 attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
                              const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
                              const int* __restrict__ tiles, const int* __restrict__ positions,
                              const int* __restrict__ token_entry, const int* __restrict__ block_table,
                              int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
                              int n_tiles, ScoreExtras extras) {
-  using T = DmaTile<NQK>;
+  static_assert(HEADS == 4 || HEADS == 2, "heads a block takes");
+  static_assert(KS == 1 || KS == 2 || (KS == 4 && HEADS == 2), "parts of the keys");
+  constexpr int TEAM = KS == 4 ? HEADS : PREFILL_WAVES, SUBS = TEAM / HEADS, TILES = KS == 4 ? 2 : 4;
+  using T = DmaTile<NQK, TEAM>;
   constexpr int HD = 32 * NQK;
   constexpr int NG = PREFILL_GROUPS;
   constexpr int PER_LANE = NG * (8 * NQK + 2);            // floats a lane hands over in the merge
   constexpr int PER = 2 * T::ROUNDS;                      // load instructions of a wave per tile
   constexpr int TABLE = 2 * (DMA_TABLE_TILES + 4);        // page ids in shared memory, one per 16-key sub-block
-  static_assert(KS == 1 || PREFILL_WAVES * PER_LANE * 64 * 4 <= KS * DMA_TILES * T::BYTES, "the merge reuses the tiles' memory");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[KS * DMA_TILES * T::BYTES];   // [half][tile][keys | values]
+  static_assert((KS - 1) * TEAM * PER_LANE * 64 * 4 <= KS * TILES * T::BYTES, "the merge reuses the tiles' memory");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[KS * TILES * T::BYTES];   // [part][tile][keys | values]
   __shared__ int page_ids[KS][TABLE];
   const int wave_id = (int)(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, wave = wave_id % PREFILL_WAVES, half = wave_id / PREFILL_WAVES;
+  const int lane = threadIdx.x & 63, wave = wave_id % TEAM, part = wave_id / TEAM;
   const int g = lane >> 4, c = lane & 15;
-  unsigned char* const tile_lds = lds + half * DMA_TILES * T::BYTES;
-  int* const pages = page_ids[half];
-  const int G = nq / nkv, chunks = (G + PREFILL_WAVES - 1) / PREFILL_WAVES, per_kv = n_tiles * chunks;
+  unsigned char* const tile_lds = lds + part * TILES * T::BYTES;
+  int* const pages = page_ids[part];
+  const int G = nq / nkv, chunks = (G + HEADS - 1) / HEADS, per_kv = n_tiles * chunks;
   int kvh, rest;
   if (nkv % 8 == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -1364,7 +1369,7 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
     rest = blockIdx.x % per_kv;
   }
   const int tile_idx = n_tiles - 1 - rest / chunks;
-  const int head_in_group = (rest % chunks) * PREFILL_WAVES + wave;
+  const int head_in_group = (rest % chunks) * HEADS + wave % HEADS;
   const bool head_ok = head_in_group < G;                 // a wave without a head still helps to load
   const int head = kvh * G + (head_ok ? head_in_group : G - 1);
   extern __shared__ float dma_bias_stage[];
@@ -1374,18 +1379,21 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
   if constexpr (EXTRA) {
     if (extras.bias) {                                    // extras without a bias (a gate, a sink) stage nothing
       const float* const bias_global = extras.bias + (size_t)head * extras.bias_rows;
-      for (int i = lane + 64 * half; i <= bias_last; i += 64 * KS) dma_bias_stage[wave * extras.bias_rows + i] = bias_global[i];
+      for (int i = lane + 64 * part; i <= bias_last; i += 64 * KS) dma_bias_stage[wave * extras.bias_rows + i] = bias_global[i];
       bias_row = (lds_bias_ptr)dma_bias_stage + wave * extras.bias_rows;
     }
   }
   const int first = tiles[2 * tile_idx], count = tiles[2 * tile_idx + 1];
+  // this wave's 32 tokens of the tile; a wave behind its end still helps to load
+  const int skip = SUBS == 1 ? 0 : 16 * NG * (wave / HEADS);
+  const int my_first = skip < count ? first + skip : first, my_count = count - skip < 16 * NG ? count - skip : 16 * NG;
   int clo[NG], chi[NG], tok[NG];
   Pack8 qreg[NG][NQK];
   const ScoreScale score_scale = split_scale(scale_log2e);
 #pragma unroll
   for (int qg = 0; qg < NG; ++qg) {
-    const bool ok = head_ok && 16 * qg + c < count;
-    tok[qg] = first + (16 * qg + c < count ? 16 * qg + c : 0);
+    const bool ok = head_ok && 16 * qg + c < my_count;
+    tok[qg] = my_first + (16 * qg + c < my_count ? 16 * qg + c : 0);
     const int pos = positions[tok[qg]];
     clo[qg] = first_seen_key(pos, window);
     chi[qg] = ok ? pos : -1;
@@ -1404,12 +1412,12 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
     }
   }
   const int last_pos = positions[first + count - 1];
-  const int first_pos = positions[first];
+  const int first_pos = positions[my_first];                // of this wave's tokens: what they see is open up to here
   const int open_lo = first_seen_key(last_pos, window);
-  const int key_begin = first_seen_key(first_pos, window) & ~31;
+  const int key_begin = first_seen_key(SUBS == 1 ? first_pos : positions[first], window) & ~31;
   const int key_end = last_pos + 1;
-  const int steps = ((key_end - key_begin + 31) / 32 + KS - 1) / KS;    // this half's share of the 32-key tiles
-  const int my_begin = key_begin + half * steps * 32;
+  const int steps = ((key_end - key_begin + 31) / 32 + KS - 1) / KS;    // this part's share of the 32-key tiles
+  const int my_begin = key_begin + part * steps * 32;
   const int* bt = block_table + (size_t)token_entry[first] * bt_stride;
   f32x4_t acc[NG][2 * NQK];
   float m[NG], l[NG];
@@ -1432,36 +1440,36 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
       k_at[sb][ch] = key * 2 * HD + 16 * ((4 * ch + g) ^ T::key_swizzle(key));
     }
   const int v_at = c * 64 + 16 * (g ^ (c >> 2));
-  const DmaLanes<NQK> dl = dma_lanes<NQK>(page_size);
+  const DmaLanes<T> dl = dma_lanes<T>(page_size);
   const unsigned page_elems = (unsigned)(nkv * page_size * HD);
   const bf16_t* const k_head = k_pool + (size_t)kvh * page_size * HD;
   const bf16_t* const v_head = v_pool + (size_t)kvh * page_size * HD;
-  // Tile i of this half is loaded with the page ids pages[2 (i - t0)], pages[2 (i - t0) + 1].
-#define TILE_LOAD(I, T0) dma_tile_load<NQK>(tile_lds + ((I) % DMA_TILES) * T::BYTES, my_begin + 32 * (I), pages[2 * ((I) - (T0))], \
+  // Tile i of this part is loaded with the page ids pages[2 (i - t0)], pages[2 (i - t0) + 1].
+#define TILE_LOAD(I, T0) dma_tile_load<T>(tile_lds + ((I) % TILES) * T::BYTES, my_begin + 32 * (I), pages[2 * ((I) - (T0))], \
                                             pages[2 * ((I) - (T0)) + 1], page_size, dl, k_head, v_head, page_elems)
-  // Tiles 0, 1 and 2 go on their way; in step i tile i + 3 follows, into the place of tile i - 1, which every wave
-  // has left behind when it passes the step's barrier.  Loads are started for the tiles of this half's steps only,
+  // All tiles but one go on their way; in step i tile i + TILES - 1 follows, into the place of tile i - 1, which every wave
+  // has left behind when it passes the step's barrier.  Loads are started for the tiles of this part's steps only,
   // so the last steps wait for fewer loads to be left.
   for (int t0 = 0; t0 < steps; t0 += DMA_TABLE_TILES) {
     // page ids of the tiles t0 .. t0 + DMA_TABLE_TILES + 3 (the loads run up to three tiles ahead of the steps)
     __syncthreads();
-    for (int e = threadIdx.x & (64 * PREFILL_WAVES - 1); e < TABLE; e += 64 * PREFILL_WAVES) {
+    for (int e = threadIdx.x & (64 * TEAM - 1); e < TABLE; e += 64 * TEAM) {
       const int kb = my_begin + 32 * t0 + 16 * e;
       pages[e] = kb < key_end ? bt[kb / page_size] : -1;
     }
     __syncthreads();
     if (t0 == 0) {
       if (steps > 0) TILE_LOAD(0, 0);
-      if (steps > 1) TILE_LOAD(1, 0);
-      if (steps > 2) TILE_LOAD(2, 0);
+      if (TILES > 2 && steps > 1) TILE_LOAD(1, 0);
+      if (TILES > 2 && steps > 2) TILE_LOAD(2, 0);
     }
     const int t1 = t0 + DMA_TABLE_TILES < steps ? t0 + DMA_TABLE_TILES : steps;
     for (int i = t0; i < t1; ++i) {
       const int K0 = my_begin + 32 * i;
-      unsigned char* const tile = tile_lds + (i % DMA_TILES) * T::BYTES;
+      unsigned char* const tile = tile_lds + (i % TILES) * T::BYTES;
       // this wave's part of tile i has landed once only the loads of the tiles after it are left
-      if (i + 2 < steps) loads_left<2 * PER>();
-      else if (i + 1 < steps) loads_left<PER>();
+      if (TILES > 2 && i + 2 < steps) loads_left<2 * PER>();
+      else if (TILES > 2 && i + 1 < steps) loads_left<PER>();
       else loads_left<0>();
       // The bare barrier: with the fence of __syncthreads the compiler would wait here for every load it
       // knows of.  No access to memory may move across it: the next loads overwrite what other waves read
@@ -1469,7 +1477,7 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (i + 3 < steps) TILE_LOAD(i + 3, t0);
+      if (i + TILES - 1 < steps) TILE_LOAD(i + TILES - 1, t0);
       if (K0 + 31 > first_pos || K0 < open_lo) {
         const bool ok0 = pages[2 * (i - t0)] >= 0, ok1 = pages[2 * (i - t0) + 1] >= 0;
         dma_tile_products<NQK, NG, true, EXTRA, BiasPtr>(tile, K0, qreg, clo, chi, acc, m, negm, l, k_at, v_at, last_pos, ok0, ok1,
@@ -1484,36 +1492,41 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
   // nothing is on its way any more, and every wave is done with the tiles: their memory serves the merge
   loads_left<0>();
   __syncthreads();
-  if (KS == 2) {
-    float* w = reinterpret_cast<float*>(lds) + (size_t)wave * PER_LANE * 64 + lane;
-    if (half == 1) {
+  if (KS > 1) {
+    // the parts behind the first hand (reference value, sum, output) over, which the first adds in their order
+    float* const w = reinterpret_cast<float*>(lds) + (size_t)wave * PER_LANE * 64 + lane;
+    constexpr int PART = TEAM * PER_LANE * 64;
+    if (part > 0) {
+      float* const mine = w + (part - 1) * PART;
 #pragma unroll
       for (int qg = 0; qg < NG; ++qg) {
 #pragma unroll
         for (int n = 0; n < 2 * NQK; ++n)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) w[(qg * (8 * NQK + 2) + 4 * n + e) * 64] = acc[qg][n][e];
-        w[(qg * (8 * NQK + 2) + 8 * NQK) * 64] = m[qg];
-        w[(qg * (8 * NQK + 2) + 8 * NQK + 1) * 64] = l[qg];
+          for (int e = 0; e < 4; ++e) mine[(qg * (8 * NQK + 2) + 4 * n + e) * 64] = acc[qg][n][e];
+        mine[(qg * (8 * NQK + 2) + 8 * NQK) * 64] = m[qg];
+        mine[(qg * (8 * NQK + 2) + 8 * NQK + 1) * 64] = l[qg];
       }
     }
     __syncthreads();
-    if (half == 0) {
+    if (part > 0) return;
+#pragma unroll 1
+    for (int other = 0; other < KS - 1; ++other) {
+      const float* const its = w + other * PART;
 #pragma unroll
       for (int qg = 0; qg < NG; ++qg) {
-        const float m_b = w[(qg * (8 * NQK + 2) + 8 * NQK) * 64], l_b = w[(qg * (8 * NQK + 2) + 8 * NQK + 1) * 64];
+        const float m_b = its[(qg * (8 * NQK + 2) + 8 * NQK) * 64], l_b = its[(qg * (8 * NQK + 2) + 8 * NQK + 1) * 64];
         const float M = fmaxf(m[qg], m_b);
         const float fa = fast_exp2(m[qg] - M), fb = fast_exp2(m_b - M);
 #pragma unroll
         for (int n = 0; n < 2 * NQK; ++n)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            acc[qg][n][e] = acc[qg][n][e] * fa + w[(qg * (8 * NQK + 2) + 4 * n + e) * 64] * fb;
+            acc[qg][n][e] = acc[qg][n][e] * fa + its[(qg * (8 * NQK + 2) + 4 * n + e) * 64] * fb;
         l[qg] = l[qg] * fa + l_b * fb;
         m[qg] = M;
       }
     }
-    if (half == 1) return;
   }
 #pragma unroll
   for (int qg = 0; qg < NG; ++qg) {
@@ -1726,23 +1739,27 @@ extern "C" int ullm_attention_decode_static(
 // `bias_bytes` > 0: the bias rows of a block's heads fit shared memory beside the tiles and are looked up there.
 #define BIAS_STAGE_ROWS 2048
 #define BIAS_STAGE_MAX (PREFILL_WAVES * BIAS_STAGE_ROWS * (int)sizeof(float))
+// Ways of a prompt launch beside one and two halves (`halves` of prefill_any), for groups of at most two heads of size 128
+enum { PREFILL_QUARTERS = 3, PREFILL_WIDE = 4, PREFILL_WIDE_HALVES = 5 };
 #define DMA_BIAS_ROWS 1792                // what fits beside four tiles a half and the page ids, for both halves
 template <int N, typename... Args>
 static void prefill_launch_extras(int halves, size_t bias_bytes, bool no_bias, unsigned blocks, hipStream_t stream, Args... args) {
   if constexpr (N == 4) {                 // tiles straight to shared memory, as without extras
     if (no_bias || (bias_bytes && bias_bytes <= (size_t)PREFILL_WAVES * DMA_BIAS_ROWS * sizeof(float))) {
-      if (halves == 2) {
-        static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_prefill_dma_kernel<N, 2, true>,
-            hipFuncAttributeMaxDynamicSharedMemorySize, PREFILL_WAVES * DMA_BIAS_ROWS * (int)sizeof(float));
-        (void)allowed;
-        hipLaunchKernelGGL((attention_prefill_dma_kernel<N, 2, true>), dim3(blocks), dim3(64 * PREFILL_WAVES * 2), bias_bytes, stream, args...);
-      } else {
-        static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_prefill_dma_kernel<N, 1, true>,
-            hipFuncAttributeMaxDynamicSharedMemorySize, PREFILL_WAVES * DMA_BIAS_ROWS * (int)sizeof(float));
-        (void)allowed;
-        hipLaunchKernelGGL((attention_prefill_dma_kernel<N, 1, true>), dim3(blocks), dim3(64 * PREFILL_WAVES), bias_bytes, stream, args...);
-      }
-      return;
+#define GO(HEADS, KS, WAVES, ROWS) do {                                                                                        \
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)attention_prefill_dma_kernel<N, HEADS, KS, true>,      \
+        hipFuncAttributeMaxDynamicSharedMemorySize, ROWS * DMA_BIAS_ROWS * (int)sizeof(float));                               \
+    (void)allowed;                                                                                                            \
+    hipLaunchKernelGGL((attention_prefill_dma_kernel<N, HEADS, KS, true>), dim3(blocks), dim3(64 * WAVES),                    \
+                       bias_bytes / PREFILL_WAVES * ROWS, stream, args...);                                                   \
+    return;                                                                                                                   \
+  } while (0)
+      if (halves == PREFILL_QUARTERS) GO(2, 4, 8, 2);
+      if (halves == PREFILL_WIDE) GO(2, 1, 4, 4);
+      if (halves == PREFILL_WIDE_HALVES) GO(2, 2, 8, 4);
+      if (halves == 2) GO(4, 2, 8, 4);
+      GO(4, 1, 4, 4);
+#undef GO
     }
   }
   if constexpr (N <= 4) {
@@ -1773,10 +1790,14 @@ static void prefill_launch(int halves, bool staged, unsigned blocks, hipStream_t
   const ScoreExtras none{nullptr, 0, nullptr, 0};
   if constexpr (N == 4) {
     if (!staged) {                                        // tiles straight to shared memory
-      if (halves == 2)
-        hipLaunchKernelGGL((attention_prefill_dma_kernel<N, 2>), dim3(blocks), dim3(64 * PREFILL_WAVES * 2), 0, stream, args..., none);
-      else
-        hipLaunchKernelGGL((attention_prefill_dma_kernel<N, 1>), dim3(blocks), dim3(64 * PREFILL_WAVES), 0, stream, args..., none);
+#define GO(HEADS, KS, WAVES) \
+    hipLaunchKernelGGL((attention_prefill_dma_kernel<N, HEADS, KS>), dim3(blocks), dim3(64 * WAVES), 0, stream, args..., none)
+      if (halves == PREFILL_QUARTERS) GO(2, 4, 8);
+      else if (halves == PREFILL_WIDE) GO(2, 1, 4);
+      else if (halves == PREFILL_WIDE_HALVES) GO(2, 2, 8);
+      else if (halves == 2) GO(4, 2, 8);
+      else GO(4, 1, 4);
+#undef GO
       return;
     }
   }
@@ -1809,44 +1830,56 @@ static int compute_units() {
 // keep every unit busy to the end); 0 = choose.  The choice compares the work per unit,
 // `keys_total` (sum over the tiles of the keys each sees) spread over two blocks per unit, with the
 // longest tile `keys_max`; without these figures (0) it goes by the number of blocks.
+//
+// Groups of at most two heads of size 128 leave half of a block's waves without a head there.  They go two heads by 64 tokens a block
+// (`wide_tiles`: up to twice as many tokens a tile, listed alike) where such blocks fill the chip, 4: all of their
+// keys, 5: two halves of them; else (3) by 32 tokens, the keys in four parts.  16 heads over 8, us before (1 or 2) and in the ways 3 / 5 / 4:
+// 700 tokens behind 2100 57 and 40 / 59 / 87, 2048 53 and 43 / 47 / 66, 3000 92 and 83 / 63 / 93, 4000 156 and 126 / 95 / 120, 8000 523 and
+// 402 / 321 / 304, 11 000 980 and 711 / 589 / 536 (925 TFLOP/s).
 static int prefill_any(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
     const int* tiles, int n_tiles, const int* positions, const int* token_entry, const int* block_table,
     int bt_stride, int page_size, int nq, int nkv, int hd, float scale, int window, int halves,
-    long long keys_total, int keys_max, hipStream_t stream, const ScoreExtras* extras) {
+    long long keys_total, int keys_max, const int* wide_tiles, int n_wide, long long wide_total, int wide_max, hipStream_t stream,
+    const ScoreExtras* extras) {
   if (n_tiles <= 0) return 0;
   if (extras && extras->bias && extras->bias_rows <= 0) return ULLM_ERR_SHAPE;
   if (!ullm_attention_mfma_supports(hd, page_size, nq, nkv)) return ULLM_ERR_UNSUPPORTED;
   const bool staged = halves >= 10;                       // 10, 11, 12: as 0, 1, 2 with the kernel that stages tiles in registers
   if (staged) halves -= 10;
-  if (halves < 0 || halves > 2) return ULLM_ERR_SHAPE;
+  // rows of up to 2048 distances go to shared memory (four heads a block: 32 KiB at most beside the tiles)
+  const size_t bias_bytes = extras && extras->bias && extras->bias_rows <= BIAS_STAGE_ROWS
+                                ? (size_t)PREFILL_WAVES * extras->bias_rows * sizeof(float) : 0;
+  const bool two_heads = hd == 128 && nq / nkv <= 2 && !staged &&
+                         (!extras || !extras->bias || (bias_bytes && extras->bias_rows <= DMA_BIAS_ROWS));
+  const bool wide = two_heads && wide_tiles && n_wide > 0;
+  if (halves < 0 || halves > (wide ? PREFILL_WIDE_HALVES : two_heads ? PREFILL_QUARTERS : 2)) return ULLM_ERR_SHAPE;
   const int chunks = (nq / nkv + PREFILL_WAVES - 1) / PREFILL_WAVES;
+  const long long units = compute_units();
+  const int reach = window == 0 ? 0x7fffffff : (window > 0 ? window : -window) + 32;      // keys a tile may see
+  // is there work for two blocks a unit to the end: `total` keys over the tiles, `most` of one
+  auto enough = [&](long long count, long long total, int most) {
+    if (total <= 0 || most <= 0) return count * nkv * chunks >= 3 * units;
+    if (most > reach) most = reach;
+    if (total > count * reach) total = count * reach;
+    return (double)total * nkv * chunks / (2.0 * units) >= 0.6 * most && count * nkv * chunks >= 2 * units;
+  };
+  // few keys are walked sooner than parts of them are added (130 tokens 8.7 us in one part, 10.3 in two, 300 13.4 and 13.5)
+  if (halves == 0 && hd == 128 && keys_max > 0 && (keys_max < reach ? keys_max : reach) <= 320) halves = 1;
+  if (halves == 0 && two_heads)
+    halves = wide && enough(n_wide, wide_total, wide_max)  ? PREFILL_WIDE
+             : wide && (long long)n_wide * nkv > units ? PREFILL_WIDE_HALVES
+                                                           : PREFILL_QUARTERS;
+  if (hd > 128) halves = 1;                              // shared memory holds one half's tiles only
+  if (halves == 0) halves = enough(n_tiles, keys_total, keys_max) ? 1 : 2;
+  if (halves >= PREFILL_WIDE) tiles = wide_tiles, n_tiles = n_wide;
   const long long blocks = (long long)n_tiles * nkv * chunks;
   if (blocks > 0x7fffffffLL) return ULLM_ERR_SHAPE;
   if ((long long)nkv * page_size * hd > 0x7fffffffLL) return ULLM_ERR_SHAPE;   // 32-bit distance between pages
-  if (hd > 128) halves = 1;                              // shared memory holds one half's tiles only
-  if (halves == 0) {
-    const long long units = compute_units();
-    bool enough;
-    if (keys_total > 0 && keys_max > 0) {
-      if (window != 0) {
-        const int reach = (window > 0 ? window : -window) + 32;
-        if (keys_max > reach) keys_max = reach;
-        if (keys_total > (long long)n_tiles * reach) keys_total = (long long)n_tiles * reach;
-      }
-      enough = (double)keys_total * nkv * chunks / (2.0 * units) >= 0.6 * keys_max;
-    } else {
-      enough = blocks >= 3 * units;
-    }
-    halves = (enough && blocks >= 2 * units) ? 1 : 2;
-  }
   const float sl = scale * 1.4426950408889634f;
 #define CALL(N) prefill_launch<N>(halves, staged, (unsigned)blocks, stream, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, \
     (const bf16_t*)k_pool, (const bf16_t*)v_pool, tiles, positions, token_entry, block_table, bt_stride, page_size,    \
     nq, nkv, sl, window, n_tiles)
-  // rows of up to 2048 distances go to shared memory (four heads a block: 32 KiB at most beside the tiles)
-  const size_t bias_bytes = extras && extras->bias && extras->bias_rows <= BIAS_STAGE_ROWS
-                                ? (size_t)PREFILL_WAVES * extras->bias_rows * sizeof(float) : 0;
 #define CALL_EXTRA(N) prefill_launch_extras<N>(halves, bias_bytes, extras->bias == nullptr, (unsigned)blocks, stream, (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, \
     (const bf16_t*)k_pool, (const bf16_t*)v_pool, tiles, positions, token_entry, block_table, bt_stride, page_size,    \
     nq, nkv, sl, window, n_tiles, *extras)
@@ -1864,9 +1897,10 @@ extern "C" int ullm_attention_prefill(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
     const int* tiles, int n_tiles, const int* positions, const int* token_entry, const int* block_table,
     int bt_stride, int page_size, int nq, int nkv, int hd, float scale, int window, int halves,
-    long long keys_total, int keys_max, hipStream_t stream) {
+    long long keys_total, int keys_max, const int* wide_tiles, int n_wide, long long wide_total, int wide_max, hipStream_t stream) {
   return prefill_any(q, q_stride, out, out_stride, k_pool, v_pool, tiles, n_tiles, positions, token_entry, block_table,
-                     bt_stride, page_size, nq, nkv, hd, scale, window, halves, keys_total, keys_max, stream, nullptr);
+                     bt_stride, page_size, nq, nkv, hd, scale, window, halves, keys_total, keys_max, wide_tiles, n_wide, wide_total,
+                     wide_max, stream, nullptr);
 }
 
 // ullm_attention_prefill with a bias by distance on the scores and a gate per head on the outputs (as
@@ -1875,9 +1909,10 @@ extern "C" int ullm_attention_prefill_extras(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
     const int* tiles, int n_tiles, const int* positions, const int* token_entry, const int* block_table,
     int bt_stride, int page_size, int nq, int nkv, int hd, float scale, int window, int halves,
-    long long keys_total, int keys_max, const float* bias, int bias_rows, const void* gate, int gate_stride,
+    long long keys_total, int keys_max, const int* wide_tiles, int n_wide, long long wide_total, int wide_max, const float* bias, int bias_rows, const void* gate, int gate_stride,
     const float* sink, hipStream_t stream) {
   const ScoreExtras x{bias, bias_rows, (const bf16_t*)gate, gate_stride, sink};
   return prefill_any(q, q_stride, out, out_stride, k_pool, v_pool, tiles, n_tiles, positions, token_entry, block_table,
-                     bt_stride, page_size, nq, nkv, hd, scale, window, halves % 10, keys_total, keys_max, stream, &x);
+                     bt_stride, page_size, nq, nkv, hd, scale, window, halves % 10, keys_total, keys_max, wide_tiles, n_wide, wide_total,
+                     wide_max, stream, &x);
 }

@@ -35,11 +35,11 @@ struct DenseStep {
   void *normed, *qkv, *q, *attended, *act;
   float *sums, *decode_parts;
   void *mixed, *fed;
-  const int *positions, *token_entry, *decode_tokens, *prompt_tiles;
-  long long tile_keys_total;
+  const int *positions, *token_entry, *decode_tokens, *prompt_tiles, *wide_tiles;
+  long long tile_keys_total, wide_keys_total;
   DenseProduct into, out, gate_up, down;
   int tokens, width, heads, kv_heads, head_dim, inner, table_rows, rot, style, page_size, window;
-  int num_decode, decode_splits, decode_waves, num_tiles, tile_keys_max;
+  int num_decode, decode_splits, decode_waves, num_tiles, tile_keys_max, num_wide, wide_keys_max;
   float eps1, eps2, qk_eps, scale;
 };
 
@@ -95,7 +95,7 @@ extern "C" int ullm_dense_layers(const DenseStep* step, const DenseLayer* layers
     if (s.num_tiles > 0)
       STEP(s.prefill(s.q, q_width, s.attended, q_width, l.k_pool, l.v_pool, s.prompt_tiles, s.num_tiles, s.positions, s.token_entry,
                      l.block_table, (int)l.bt_stride, s.page_size, s.heads, s.kv_heads, s.head_dim, s.scale, s.window, 0,
-                     s.tile_keys_total, s.tile_keys_max, stream));
+                     s.tile_keys_total, s.tile_keys_max, s.wide_tiles, s.num_wide, s.wide_keys_total, s.wide_keys_max, stream));
     STEP(dense_product(s, s.out, s.attended, q_width, l.w_o, nullptr, s.mixed, H, 0, stream));
     leave(s.out, s.mixed);
     STEP(norm(l.norm2, s.eps2));

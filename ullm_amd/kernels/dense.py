@@ -25,12 +25,12 @@ class Product(ctypes.Structure):
 class Step(ctypes.Structure):
     _fields_ = ([(name, _ptr) for _, name in LAUNCHERS]
                 + [(name, _ptr) for name in ("residual", "normed", "qkv", "q", "attended", "act", "sums", "decode_parts", "mixed", "fed",
-                                             "positions", "token_entry", "decode_tokens", "prompt_tiles")]
-                + [("tile_keys_total", _long)]
+                                             "positions", "token_entry", "decode_tokens", "prompt_tiles", "wide_tiles")]
+                + [("tile_keys_total", _long), ("wide_keys_total", _long)]
                 + [(name, Product) for name in ("into", "out", "gate_up", "down")]
                 + [(name, _int) for name in ("tokens", "width", "heads", "kv_heads", "head_dim", "inner",
                                              "table_rows", "rot", "style", "page_size", "window", "num_decode", "decode_splits",
-                                             "decode_waves", "num_tiles", "tile_keys_max")]
+                                             "decode_waves", "num_tiles", "tile_keys_max", "num_wide", "wide_keys_max")]
                 + [(name, _float) for name in ("eps1", "eps2", "qk_eps", "scale")])
 
 

@@ -1582,16 +1582,21 @@ def attention_prefill_mfma(q, out, k_pool, v_pool, tiles: torch.Tensor, n_tiles:
                            block_table, page_size: int, nq: int, nkv: int, hd: int, scale: float,
                            window: int, halves: int = 0, keys_total: int = 0, keys_max: int = 0,
                            bias_log2: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                           sink_log2: Optional[torch.Tensor] = None) -> None:
+                           sink_log2: Optional[torch.Tensor] = None, wide_tiles: Optional[torch.Tensor] = None, n_wide: int = 0,
+                           wide_keys_total: int = 0, wide_keys_max: int = 0) -> None:
     """Tiles (first token, count <= PREFILL_TILE) of consecutive tokens of one request each, every
     token against the keys up to its own position.  ``halves``: 2 = two halves of a block share a
     tile's keys, 1 = one block takes them all, 0 = chosen from ``keys_total`` (the sum over the tiles of
     the keys each sees) and ``keys_max`` (the most any tile sees), or from the number of tiles if
-    these are 0.  Every choice computes the same function."""
+    these are 0.  ``wide_tiles``: the same tokens in tiles of up to twice as many (``n_wide``, ``wide_keys_total``, ``wide_keys_max`` of them),
+    for groups of at most two heads of size 128, whose launches have ways of their own (``halves`` 3: the keys of a tile in four parts,
+    4 and 5: wide tiles, whole or in two halves).  Every choice computes the same function."""
     _check_pools(k_pool, v_pool, nkv, page_size, hd, torch.bfloat16)
     _need(q.dtype == torch.bfloat16 and q.stride(1) == 1 and q.shape[1] == nq * hd, "q must be bfloat16 [T, nq*hd]")
     _need(out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.shape == q.shape, "bad attention output")
     _need(tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.numel() >= 2 * n_tiles, "tiles must be int32 [n, 2]")
+    _need(wide_tiles is None or (wide_tiles.dtype == torch.int32 and wide_tiles.is_contiguous() and wide_tiles.numel() >= 2 * n_wide),
+          "wide tiles must be int32 [n, 2]")
     _i32(positions, "positions")
     _i32(token_entry, "token_entry")
     _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1,
@@ -1604,7 +1609,8 @@ def attention_prefill_mfma(q, out, k_pool, v_pool, tiles: torch.Tensor, n_tiles:
             _p(q), _c_int(q.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(tiles),
             _c_int(n_tiles), _p(positions), _p(token_entry), _p(block_table), _c_int(block_table.stride(0)),
             _c_int(page_size), _c_int(nq), _c_int(nkv), _c_int(hd), _c_float(scale), _c_int(window),
-            _c_int(halves), ctypes.c_longlong(int(keys_total)), _c_int(keys_max), _p(bias_log2),
+            _c_int(halves), ctypes.c_longlong(int(keys_total)), _c_int(keys_max), _p(wide_tiles), _c_int(n_wide),
+            ctypes.c_longlong(int(wide_keys_total)), _c_int(wide_keys_max), _p(bias_log2),
             _c_int(_check_distance_bias(bias_log2, nq)), _p(gate), _c_int(gate.stride(0) if gate is not None else 0),
             _p(sink_log2), _stream()), "attention_prefill_extras")
         return
@@ -1612,8 +1618,8 @@ def attention_prefill_mfma(q, out, k_pool, v_pool, tiles: torch.Tensor, n_tiles:
         _p(q), _c_int(q.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(tiles),
         _c_int(n_tiles), _p(positions), _p(token_entry), _p(block_table), _c_int(block_table.stride(0)),
         _c_int(page_size), _c_int(nq), _c_int(nkv), _c_int(hd), _c_float(scale), _c_int(window),
-        _c_int(halves), ctypes.c_longlong(int(keys_total)), _c_int(keys_max), _stream()),
-        "attention_prefill")
+        _c_int(halves), ctypes.c_longlong(int(keys_total)), _c_int(keys_max), _p(wide_tiles), _c_int(n_wide),
+        ctypes.c_longlong(int(wide_keys_total)), _c_int(wide_keys_max), _stream()), "attention_prefill")
 
 
 _warned_general_attention = set()
@@ -1670,7 +1676,8 @@ def paged_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     if n["num_tiles"]:
         attention_prefill_mfma(q, out, k_pool, v_pool, plan.arrays["tiles"], n["num_tiles"], ctx.positions,
                                ctx.token_entry, group.block_table, group.page_size, nq, nkv, hd, scale, window,
-                               keys_total=n["tile_keys_total"], keys_max=n["tile_keys_max"],
+                               keys_total=n["tile_keys_total"], keys_max=n["tile_keys_max"], wide_tiles=plan.arrays.get("wide_tiles"),
+                               n_wide=n.get("num_wide", 0), wide_keys_total=n.get("wide_keys_total", 0), wide_keys_max=n.get("wide_keys_max", 0),
                                bias_log2=bias_log2 if bias is not None else None, gate=gate,
                                sink_log2=sink_log2 if sink is not None else None)
     return out

@@ -61,28 +61,32 @@ def padded_head_size(*sizes: int) -> int:
 def plan_attention_step(shape: StepShape) -> StepPlan:
     """How the attention kernels split a batch: the tokens of one-token entries (``decode_tokens``, longest
     context first: the short ones fill the tail of the launch), and tiles of up to ``ops.PREFILL_TILE``
-    consecutive tokens (first token, count) of the longer entries by rising number of keys (``tiles``), with
-    the numbers the launches are shaped by.  Padding entries of a captured batch are one-token entries."""
-    dec, tiles, max_decode_kv, t0 = [], [], 0, 0
+    consecutive tokens (first token, count) of the longer entries by rising number of keys (``tiles``), and the same of twice as
+    many tokens (``wide_tiles``, for blocks that take two tiles of one request), with the numbers the launches are shaped by.  Padding entries of a captured batch are one-token entries."""
+    dec, tiles, wide, max_decode_kv, t0 = [], [], [], 0, 0
     for n, start in zip(shape.lens, shape.starts):
         if n == 1:
             dec.append((-start, t0))
             max_decode_kv = max(max_decode_kv, start + 1)
         else:
-            for first in range(0, n, ops.PREFILL_TILE):
-                count = min(ops.PREFILL_TILE, n - first)
-                tiles.append((start + first + count, t0 + first, count))
+            for size, into in ((ops.PREFILL_TILE, tiles), (2 * ops.PREFILL_TILE, wide)):
+                for first in range(0, n, size):
+                    count = min(size, n - first)
+                    into.append((start + first + count, t0 + first, count))
         t0 += n
     tiles.sort()
+    wide.sort()
     dec.sort()
     decode_tokens = [t for _, t in dec] + list(range(t0, t0 + shape.pad_entries))
     if shape.kv_bucket is not None:
         max_decode_kv = shape.kv_bucket                   # a captured launch: the split of the keys is fixed
     return StepPlan(
         arrays={"decode_tokens": np.asarray(decode_tokens, dtype=np.int32),
-                "tiles": np.asarray([x for _, first, count in tiles for x in (first, count)], dtype=np.int32)},
+                "tiles": np.asarray([x for _, first, count in tiles for x in (first, count)], dtype=np.int32),
+                "wide_tiles": np.asarray([x for _, first, count in wide for x in (first, count)], dtype=np.int32)},
         facts={"num_decode": len(decode_tokens), "max_decode_kv": max_decode_kv, "num_tiles": len(tiles),
-               "tile_keys_total": sum(k for k, _, _ in tiles), "tile_keys_max": tiles[-1][0] if tiles else 0})
+               "tile_keys_total": sum(k for k, _, _ in tiles), "tile_keys_max": tiles[-1][0] if tiles else 0,
+               "num_wide": len(wide), "wide_keys_total": sum(k for k, _, _ in wide), "wide_keys_max": wide[-1][0] if wide else 0})
 
 
 @register_part("mixer", "gqa_attention")

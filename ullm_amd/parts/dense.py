@@ -128,7 +128,8 @@ def run_layers(blocks: List[Block], caches: List[LayerCache], residual: torch.Te
             return None
         table_rows = angles.shape[0]
     bt, plan = group.block_table, ctx.plans["attention"].arrays
-    for t, n in ((ctx.positions, T), (ctx.token_entry, T), (plan["decode_tokens"], work["num_decode"]), (plan["tiles"], 2 * work["num_tiles"])):
+    for t, n in ((ctx.positions, T), (ctx.token_entry, T), (plan["decode_tokens"], work["num_decode"]), (plan["tiles"], 2 * work["num_tiles"]),
+                 (plan["wide_tiles"], 2 * work["num_wide"])):
         if t.dtype != torch.int32 or not t.is_contiguous() or t.numel() < n:
             return None
     if bt.dtype != torch.int32 or bt.dim() != 2 or bt.stride(1) != 1 or -(-work["max_decode_kv"] // group.page_size) > bt.shape[1]:
@@ -159,10 +160,12 @@ def run_layers(blocks: List[Block], caches: List[LayerCache], residual: torch.Te
         residual=residual.data_ptr(), normed=normed.data_ptr(), qkv=qkv.data_ptr(), q=q.data_ptr(), attended=attended.data_ptr(),
         act=act.data_ptr(), sums=address(sums), decode_parts=address(parts), mixed=mixed.data_ptr(), fed=fed.data_ptr(),
         positions=ctx.positions.data_ptr(), token_entry=ctx.token_entry.data_ptr(), decode_tokens=plan["decode_tokens"].data_ptr(),
-        prompt_tiles=plan["tiles"].data_ptr(), tile_keys_total=int(work["tile_keys_total"]), into=into, out=out, gate_up=gate_up, down=down, tokens=T, width=H,
+        prompt_tiles=plan["tiles"].data_ptr(), wide_tiles=plan["wide_tiles"].data_ptr(), tile_keys_total=int(work["tile_keys_total"]),
+        wide_keys_total=int(work["wide_keys_total"]), into=into, out=out, gate_up=gate_up, down=down, tokens=T, width=H,
         heads=m.nq, kv_heads=m.nkv, head_dim=m.hd, inner=I, table_rows=table_rows, rot=rot, style=style, page_size=group.page_size,
         window=m.reach, num_decode=work["num_decode"], decode_splits=splits, decode_waves=4 if m.hd == 256 and waves == 8 else waves,
-        num_tiles=work["num_tiles"], tile_keys_max=work["tile_keys_max"], eps1=first.mixer_norm.eps, eps2=first.ffn_norm.eps,
+        num_tiles=work["num_tiles"], tile_keys_max=work["tile_keys_max"], num_wide=work["num_wide"], wide_keys_max=work["wide_keys_max"],
+        eps1=first.mixer_norm.eps, eps2=first.ffn_norm.eps,
         qk_eps=m.qk_norm_eps if m.qk_norm_eps is not None else 0.0, scale=m.scale)
     dense.dense_layers(step, layers)
     return fed
