@@ -82,6 +82,7 @@ def test_when_it_is_taken():
     P = dispatch.panels
     assert [P(r, 24576, 4096, "gated")[0] >= 0 for r in (16, 17, 256, 257, 3000)] == [False, True, True, False, False]
     assert [P(r, 1024, 3072, "stream")[0] >= 0 for r in (16, 17, 1024, 1025)] == [False, True, True, False]
+    assert [P(r, 1024, 3072, "stream", False, True)[0] >= 0 for r in (16, 1025, 1800, 20000)] == [False, True, True, False]
     assert [P(r, 4096, 12288, "stream")[0] >= 0 for r in (17, 2048, 2049)] == [True, True, False]
     assert P(64, 1000, 1024, "store")[0] < 0 and P(64, 1024, 1024, "store")[0] >= 0            # a smaller matrix than measured
     assert P(64, 2052, 1024, "store")[0] < 0 and P(64, 2048, 1000, "store")[0] < 0 and P(64, 8200, 1024, "gated")[0] < 0

@@ -155,7 +155,7 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
 
 
 @functools.lru_cache(maxsize=8192)
-def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False) -> Tuple[int, int]:
+def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False) -> Tuple[int, int]:
     """The plan by which the panels kernel (``ops.gemm_panels``) takes x [rows, inner] times W [columns, inner], and its mode; a plan of -1
     where another product is ahead.  Roles: ``store`` (a bfloat16 result; in float mode the slices are added by a kernel),
     ``gated`` (W is gate | up) and ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
@@ -166,8 +166,9 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     5.8 / 9.6 / 15.0; 4096 x 12288 into the stream at 130 / 512 / 1024 30.6 / 83 / 118 and 26.4 / 51 / 94; 6144 x 4096 at 64 / 256 / 1024 17.8 / 31 / 53
     and 16.8 / 25.7 / 53.3).  In two rounds the library's tiles are ahead (6144 x 4096 at 1300 rows 65 and 83, gate|up 24576 x 4096 at 320
     79 and 87), and from 1025 rows on also in one where a matrix has few columns (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 /
-    24.1; 4096 x 1024 at 1300 20.1 and 16.0, 4096 x 12288 at 1300 / 2048 146 / 191 and 133 / 174)."""
-    if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and columns < 2048):
+    24.1, 2048 x 2048 at 2048 / 3000 21.0 / 26.5 and 23.0 / 27.6; 4096 x 1024 at 1300 20.1 and 16.0, 4096 x 12288 at 1300 / 2048 146 / 191
+    and 133 / 174), where ``host_bound`` does not say that launches are what takes the time."""
+    if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and columns < 4096 and not host_bound):
         return -1, 0
     if role == "gated":
         return _panels_plan(rows, columns, inner, PANELS_GATED, 1)[0], PANELS_GATED

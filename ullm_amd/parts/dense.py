@@ -3,7 +3,7 @@
 A step of few tokens is bound by the host: a layer's ten launches cost the interpreter more than its kernels take (0.6B: 160 us,
 and 60 us of kernels at 300 tokens).  What a part's ``forward`` decides from sizes alone is decided here once for all layers, and the
 launches go out from one call (``kernels/dense.py``).  The kernels, their order and so the results are those of the blocks'
-own ``forward``, which takes whatever this does not: float32, steps of single tokens (captured graphs, mostly), up to 16 rows
+own ``forward`` (but for products that are not worth the library's launch here), which takes whatever this does not: float32, steps of single tokens (captured graphs, mostly), up to 16 rows
 (the folded kernels), products that the library is ahead for (their kernels then take longer than the host) and parts of
 any other kind.
 """
@@ -41,12 +41,17 @@ def alike_layers(blocks: Sequence[Block]) -> int:
     return n
 
 
-def _product(rows: int, columns: int, inner: int, role: str) -> Optional[dense.Product]:
+# Up to this many multiplications and additions a layer's kernels take less time than the interpreter's launches (0.6B at 1200 tokens: 130
+# us, 140): own products are then worth it also where the library's are a few us ahead.
+HOST_BOUND = 19_000_000_000
+
+
+def _product(rows: int, columns: int, inner: int, role: str, host_bound: bool) -> Optional[dense.Product]:
     """The framework's own product that the parts' ``linear``, ``gate_up`` and ``linear_into_stream`` would take, if it is one for
-    many rows."""
+    many rows; with ``host_bound`` also one that the library's is ahead of."""
     lim = dispatch.limits(columns, inner)
     if not (role == "store" and lim.sums_from):
-        plan, mode = dispatch.panels(rows, columns, inner, role, role == "stream" and lim.stacked_from <= rows <= lim.stacked_to)
+        plan, mode = dispatch.panels(rows, columns, inner, role, role == "stream" and lim.stacked_from <= rows <= lim.stacked_to, host_bound)
         if plan >= 0:
             return dense.Product(0, mode, plan & 0xff, plan >> 8)
     if role == "gated":
@@ -117,8 +122,9 @@ def run_layers(blocks: List[Block], caches: List[LayerCache], residual: torch.Te
     q_width, qkv_width = m.nq * m.hd, (m.nq + 2 * m.nkv) * m.hd
     if max(T, 2 * I, qkv_width) * max(H, I, q_width) >= 2 ** 31:
         return None
-    into, out = _product(T, qkv_width, H, "store"), _product(T, H, q_width, "stream")
-    gate_up, down = _product(T, 2 * I, H, "gated"), _product(T, H, I, "stream")
+    host_bound = T * (H * (qkv_width + q_width) + 3 * I * H) <= HOST_BOUND
+    into, out, gate_up, down = (_product(T, *product, host_bound) for product in (
+        (qkv_width, H, "store"), (H, q_width, "stream"), (2 * I, H, "gated"), (H, I, "stream")))
     if into is None or out is None or gate_up is None or down is None:
         return None
     angles, rot, style = m.position.kernel_args() if m.position is not None else (None, 0, 0)
