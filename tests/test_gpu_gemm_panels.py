@@ -84,6 +84,8 @@ def test_when_it_is_taken():
     assert [P(r, 1024, 3072, "stream")[0] >= 0 for r in (16, 17, 1024, 1025)] == [False, True, True, False]
     assert [P(r, 1024, 3072, "stream", False, True)[0] >= 0 for r in (16, 1025, 1800, 20000)] == [False, True, True, False]
     assert [P(r, 4096, 12288, "stream")[0] >= 0 for r in (17, 2048, 2049)] == [True, True, False]
+    assert [P(r, 151936, 1024, "float")[0] >= 0 for r in (16, 17, 256, 257)] == [False, True, True, False]      # in more than one round
+    assert [P(r, 2048, 2048, "float")[0] >= 0 for r in (17, 512, 513)] == [True, True, False] and P(600, 4096, 2048, "float")[0] >= 0
     assert P(64, 1000, 1024, "store")[0] < 0 and P(64, 1024, 1024, "store")[0] >= 0            # a smaller matrix than measured
     assert P(64, 2052, 1024, "store")[0] < 0 and P(64, 2048, 1000, "store")[0] < 0 and P(64, 8200, 1024, "gated")[0] < 0
     for rows in list(range(17, 2200, 61)) + [2048]:
@@ -109,9 +111,11 @@ def test_parts_take_it_where_the_rule_says(ops, monkeypatch):
         want = x.double() @ w.double().T
         close = lambda y, ref: float((y.double() - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())      # noqa: E731
         assert close(linear(x, w, bias), want + bias.double())
+        full = linear(x, w, bias, out_dtype=torch.float32)
+        assert full.dtype == torch.float32 and float((full.double() - want - bias.double()).abs().max()) <= 1e-5 * float(want.abs().max())
         g, u = want[:, :512], want[:, 512:]
         assert close(gate_up(x, w), g * torch.sigmoid(g) * u)
         y = linear_into_stream(x, w, ctx)
         assert close(y if y.dim() == 2 else y.sum(0), want)
-        assert (len(calls) == 3) == (rows > 16) and (rows == 16 or set(calls) >= {dispatch.PANELS_GATED, dispatch.PANELS_FLOAT})
+        assert (len(calls) == 4) == (rows > 16) and (rows == 16 or set(calls) >= {dispatch.PANELS_GATED, dispatch.PANELS_FLOAT})
         del calls[:]

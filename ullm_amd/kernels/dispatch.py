@@ -145,11 +145,11 @@ SUM_US = 4.0                  # the kernel that adds slices: its launch and the 
 
 
 @functools.lru_cache(maxsize=8192)           # of sizes alone, and asked for by every layer of every step
-def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int) -> Tuple[int, float]:
-    """The panels kernel's plan and its estimated us; a plan of -1 where it does not take the product or its blocks need more
-    than one round."""
+def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int, rounds: bool = False) -> Tuple[int, float]:
+    """The panels kernel's plan and its estimated us; a plan of -1 where it does not take the product or (unless ``rounds``) its
+    blocks need more than one round."""
     plan = int(build.load("gemm_panels").ullm_gemm_panels_plan(rows, columns, inner, mode, max_slices))
-    if plan < 0 or plan >> 16 & 1:
+    if plan < 0 or (plan >> 16 & 1 and not rounds):
         return -1, 0.0
     return plan & 0xffff, (plan >> 17) / 8
 
@@ -158,8 +158,8 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
 def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False) -> Tuple[int, int]:
     """The plan by which the panels kernel (``ops.gemm_panels``) takes x [rows, inner] times W [columns, inner], and its mode; a plan of -1
     where another product is ahead.  Roles: ``store`` (a bfloat16 result; in float mode the slices are added by a kernel),
-    ``gated`` (W is gate | up) and ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
-    ``keep_sums`` always the sums).
+    ``gated`` (W is gate | up), ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
+    ``keep_sums`` always the sums) and ``float`` (the 32-bit sums as they are, one slice: logits, branches).
 
     It is taken from 17 rows on while its blocks fit one round of the chip: there its tiles fill it (us, what took the calls
     before and this: gate|up 24576 x 4096 at 17 / 64 / 256 rows 36 / 43 / 64 and 32 / 36 / 58; 6144 x 1024 at 40 / 256 / 800 7.9 / 15.1 / 17.3 and
@@ -169,6 +169,14 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     24.1, 2048 x 2048 at 2048 / 3000 21.0 / 26.5 and 23.0 / 27.6; 4096 x 1024 at 1300 20.1 and 16.0, 4096 x 12288 at 1300 / 2048 146 / 191
     and 133 / 174), where ``host_bound`` does not say that launches are what takes the time."""
     if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and columns < 4096 and not host_bound):
+        return -1, 0
+    if role == "float":
+        # logits heads are read once at these rows, in however many rounds (library and this: 151936 x 4096 at 17 / 64 / 128 rows 266 / 270 /
+        # 290 and 192 / 223 / 268, 151936 x 1024 at 101 91 and 81, 32768 x 2048 at 48 / 256 37 / 46 and 25 / 41); smaller matrices go to the
+        # library sooner than where the result is rounded (2048 x 2048 at 300 / 600 / 1024 rows 10.8 / 13.1 / 15.4 and 10.3 / 13.2 / 17.2, 4096 x 2048
+        # at 600 / 1024 23 / 26 and 18 / 23)
+        if rows <= (256 if columns >= 16384 else 1024 if columns >= 4096 else 512):
+            return _panels_plan(rows, columns, inner, PANELS_FLOAT, 1, columns >= 16384)[0], PANELS_FLOAT
         return -1, 0
     if role == "gated":
         return _panels_plan(rows, columns, inner, PANELS_GATED, 1)[0], PANELS_GATED

@@ -1347,6 +1347,11 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
         if plan >= 0:
             y = sum_stacks(gemm_panels(a, w, plan, mode), bias)
             return y if act is None else activation(y, act, out=y)
+    if out_dtype == torch.float32 and act is None and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w):
+        plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "float")
+        if plan >= 0:
+            y = gemm_panels(a, w, plan, mode)[0]
+            return y if bias is None else add_bias(y, bias)
     if act is not None:
         lim = dispatch.limits(w.shape[0], w.shape[1])
         if M <= (lim.f32_skinny if out_dtype == torch.float32 else lim.skinny) and gemm_skinny_supports(a, w):
