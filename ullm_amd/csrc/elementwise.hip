@@ -795,19 +795,19 @@ __device__ __forceinline__ void value_runs_block(
     *reinterpret_cast<uint4*>(tile + tok * hd + part * PER16) = *reinterpret_cast<const uint4*>(
         qkv + (size_t)(tok0 + tok) * qkv_stride + (size_t)(v_head0 + kvh) * hd + part * PER16);
   }
-  if ((int)threadIdx.x < n) {
-    // a token leads a run if it is the block's first or does not continue its predecessor's group of 8
-    const int i = threadIdx.x, t = tok0 + i;
+  if (threadIdx.x < WAVE) {
+    // a token leads a run if it is the block's first or does not continue its predecessor's group of 8; the run ends where the next
+    // token leads, or the block does (asked of the lanes that hold the tokens: every step of a walk over them would be a trip to memory)
+    const int i = threadIdx.x, t = tok0 + (i < n ? i : n - 1);
     const int pos = positions[t], ent = token_entry[t];
-    s_page[i] = block_table[(size_t)ent * bt_stride + pos / page_size];
-    s_off[i] = pos % page_size;
-    const bool leads = i == 0 || token_entry[t - 1] != ent || positions[t - 1] != pos - 1 || (pos & 7) == 0;
-    int run = 0;
-    if (leads) {
-      run = 1;
-      while (i + run < n && token_entry[t + run] == ent && positions[t + run] == pos + run && ((pos + run) & 7) != 0) ++run;
+    const int pos_before = __shfl_up(pos, 1, WAVE), ent_before = __shfl_up(ent, 1, WAVE);
+    const bool leads = i == 0 || i >= n || ent_before != ent || pos_before != pos - 1 || (pos & 7) == 0;
+    const unsigned long long leaders = __ballot(leads) >> 1 >> i;          // of the tokens behind this one
+    if (i < n) {
+      s_page[i] = block_table[(size_t)ent * bt_stride + pos / page_size];
+      s_off[i] = pos % page_size;
+      s_run[i] = leads ? __ffsll(leaders) : 0;
     }
-    s_run[i] = run;
   }
   __syncthreads();
   // item = (dim, half of the block's tokens)
@@ -835,11 +835,53 @@ __device__ __forceinline__ void value_runs_block(
   }
 }
 
+// Eight consecutive values of a row that is read once, on their way and in 32 bits.
+template <typename T> struct EightValues;
+template <> struct EightValues<bf16_t> {
+  uint4 u;
+  __device__ __forceinline__ void fetch(const bf16_t* p) { u = ld_stream16(p); }
+  __device__ __forceinline__ void values(float (&x)[8]) const {
+    const unsigned w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[2 * i] = __uint_as_float(w[i] << 16), x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, const float (&x)[8]) {
+    st16(p, make_uint4(pack2_bf16(x[0], x[1]), pack2_bf16(x[2], x[3]), pack2_bf16(x[4], x[5]), pack2_bf16(x[6], x[7])));
+  }
+};
+template <> struct EightValues<float> {
+  float4 lo, hi;
+  __device__ __forceinline__ void fetch(const float* p) { lo = ld4_f32_stream(p), hi = ld4_f32_stream(p + 4); }
+  __device__ __forceinline__ void values(float (&x)[8]) const {
+    x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w, x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
+  }
+  static __device__ __forceinline__ void store(float* p, const float (&x)[8]) {
+    st4_f32(p, make_float4(x[0], x[1], x[2], x[3]));
+    st4_f32(p + 4, make_float4(x[4], x[5], x[6], x[7]));
+  }
+};
+
+// v of the lane N further back in its row of 16 lanes, the first behind the last
+template <int N>
+__device__ __forceinline__ float row_rotated(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
+#else
+  return v;
+#endif
+}
+
 // The same for head sizes of 8 * (a power of two): a head is held by head_dim / 8 neighbouring lanes
 // with 8 consecutive dims each (16-byte loads and stores for bfloat16), a block of 256 threads takes
-// 2048 / head_dim heads of one token at a time, heads_per_thread times in turn.  For half-split pairs the partner dims come from the lane
-// rot / 16 further on (or back) by shuffles, which needs rot to be a multiple of 16.
-template <typename T>
+// 2048 / head_dim heads of one token at a time, PASSES times.  For half-split pairs the partner dims come from the lane
+// rot / 16 further on (or back) by shuffles, which needs rot to be a multiple of 16; heads of 128 lie in a row of 16 lanes, whose
+// rotations do the sums and, where all of the head turns, the partners without a trip to shared memory.
+//
+// What bounds it is, over few tokens, the chain of trips to memory (the token's position, its cosines and its page), over many the
+// projection's bytes: so the heads of all passes are asked for before anything else, the page once, and value heads that blocks of
+// their own write are not read here.  32 heads over 8 of 128, us with a head's values and page asked for in its pass, eight bytes at a
+// time: 130 tokens 4.9 -> 3.5, 800 10.2 -> 7.1, 2048 18.6 -> 13.3, 12 000 83.6 -> 58.0 (5.0 TB/s).
+template <typename T, int PASSES>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_write_vec_kernel(
     const T* __restrict__ qkv, int qkv_stride, T* __restrict__ q_out, int q_out_stride,
@@ -847,7 +889,7 @@ qk_norm_rope_write_vec_kernel(
     const float* __restrict__ cos_sin, int table_rows, int rot, int style,
     const int* __restrict__ positions, const int* __restrict__ token_entry,
     const int* __restrict__ block_table, int bt_stride, T* __restrict__ k_pool, T* __restrict__ v_pool,
-    int page_size, int nq, int nkv, int hd, int write_kv, int n_tokens, int blocks_per_token, int heads_per_thread,
+    int page_size, int nq, int nkv, int hd, int write_kv, int n_tokens, int blocks_per_token,
     int v_head0, int norm_dim) {
   if (blockIdx.x >= (unsigned)(n_tokens * blocks_per_token)) {
     value_runs_block<T>(qkv, qkv_stride, positions, token_entry, block_table, bt_stride, v_pool, page_size, v_head0, nkv,
@@ -857,12 +899,24 @@ qk_norm_rope_write_vec_kernel(
   const int lph = hd >> 3;                                  // lanes per head
   const int t = blockIdx.x / blocks_per_token;
   const int part = threadIdx.x % lph, d0 = 8 * part;
+  const int head0 = (blockIdx.x % blocks_per_token) * PASSES * (256 / lph) + threadIdx.x / lph;
+  const int heads = write_kv & 2 ? nq + 2 * nkv : nq + nkv;     // those that this kernel reads
+  const T* const row = qkv + (size_t)t * qkv_stride;
+  EightValues<T> held[PASSES];
+#pragma unroll
+  for (int pass = 0; pass < PASSES; ++pass) {
+    int head = head0 + pass * (256 / lph);
+    if (head >= heads) head = 0;                            // no load under a condition; not used
+    held[pass].fetch(row + (size_t)(head < nq + nkv ? head : v_head0 + head - nq - nkv) * hd + d0);
+  }
   const int pos = positions[t];
+  const int entry = token_entry[t];
   const int off = pos % page_size;
   // what depends on the token and the lane's dims alone is fetched once for all the heads the thread takes
   const bool rotates = style != 0 && rot > 0;
   const int half = rot / 2;
   const bool first = d0 < half, in = d0 < rot;              // rot and half are multiples of 8: a lane is on one side
+  const int page = write_kv ? block_table[(size_t)entry * bt_stride + pos / page_size] : -1;
   float c[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sn[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const float* cs = nullptr;
   if (rotates) {
@@ -876,19 +930,13 @@ qk_norm_rope_write_vec_kernel(
       sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
     }
   }
-  for (int pass = 0; pass < heads_per_thread; ++pass) {
-    const int head = ((blockIdx.x % blocks_per_token) * heads_per_thread + pass) * (256 / lph) + threadIdx.x / lph;
-    const bool live = head < nq + 2 * nkv;
+#pragma unroll
+  for (int pass = 0; pass < PASSES; ++pass) {
+    const int head = head0 + pass * (256 / lph);
+    const bool live = head < heads;
     const bool is_q = head < nq, is_k = !is_q && head < nq + nkv;
-    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (live) {
-      const T* src = qkv + (size_t)t * qkv_stride + (size_t)(is_q || is_k ? head : v_head0 + head - nq - nkv) * hd + d0;
-      const float4 lo = ld4_f32_stream(src), hi = ld4_f32_stream(src + 4);     // the projection row is read once
-      x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w; x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
-    }
-    int page = -1;
-    if (live && !is_q && (write_kv & (is_k ? 1 : 2)))
-      page = block_table[(size_t)token_entry[t] * bt_stride + pos / page_size];
+    float x[8];
+    held[pass].values(x);
     if (live && !is_q && !is_k) {                             // v: transposed copy, no arithmetic
       if (page >= 0) {
         const int kvh = head - nq - nkv;
@@ -897,18 +945,25 @@ qk_norm_rope_write_vec_kernel(
         for (int j = 0; j < 8; ++j) st_f32(vdst + (size_t)j * page_size, x[j]);
       }
     }
-    // every lane takes part in the shuffles below; lanes of value heads and dead lanes carry zeros
+    // every lane takes part in the exchanges below; what lanes of value heads and lanes without a head make of it goes nowhere
     const float* gain = is_q ? q_gain : k_gain;
     const bool arith = live && (is_q || is_k);
-    if (gain) {
+    if (q_gain || k_gain) {
       float ss = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
       // pairwise, the most distant lanes of a head first: the decode attention kernel, which does this
       // norm itself for single new tokens, adds in the same order (multiply-adds spelled out in both)
-      for (int m = lph >> 1; m > 0; m >>= 1) ss += __shfl_xor(ss, m, WAVE);
+      if (lph == 16) {
+        ss += row_rotated<8>(ss);
+        ss += row_rotated<4>(ss);
+        ss += row_rotated<2>(ss);
+        ss += row_rotated<1>(ss);
+      } else {
+        for (int m = lph >> 1; m > 0; m >>= 1) ss += __shfl_xor(ss, m, WAVE);
+      }
       const float rs = rsqrtf(ss / (float)norm_dim + eps);
-      if (arith) {
+      if (arith && gain) {
         const float4 g0 = *reinterpret_cast<const float4*>(gain + d0), g1 = *reinterpret_cast<const float4*>(gain + d0 + 4);
         const float gg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
@@ -917,10 +972,15 @@ qk_norm_rope_write_vec_kernel(
     }
     if (rotates) {
       if (style == 1) {
-        const int src_lane = (int)(threadIdx.x & (WAVE - 1)) + (first ? half / 8 : -(half / 8));
         float y[8];
+        if (lph == 16 && half == 64) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] = __shfl(x[j], in ? src_lane : (int)(threadIdx.x & (WAVE - 1)), WAVE);
+          for (int j = 0; j < 8; ++j) y[j] = row_rotated<8>(x[j]);
+        } else {
+          const int src_lane = (int)(threadIdx.x & (WAVE - 1)) + (first ? half / 8 : -(half / 8));
+#pragma unroll
+          for (int j = 0; j < 8; ++j) y[j] = __shfl(x[j], in ? src_lane : (int)(threadIdx.x & (WAVE - 1)), WAVE);
+        }
         if (in && arith) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) x[j] = first ? fmaf(x[j], c[j], -(y[j] * sn[j])) : fmaf(x[j], c[j], y[j] * sn[j]);
@@ -938,15 +998,8 @@ qk_norm_rope_write_vec_kernel(
       }
     }
     if (!arith) continue;
-    T* dst;
-    if (is_q) {
-      dst = q_out + (size_t)t * q_out_stride + (size_t)head * hd + d0;
-    } else {
-      if (page < 0) continue;
-      dst = k_pool + (((size_t)page * nkv + (head - nq)) * page_size + off) * hd + d0;
-    }
-    st4_f32(dst, make_float4(x[0], x[1], x[2], x[3]));
-    st4_f32(dst + 4, make_float4(x[4], x[5], x[6], x[7]));
+    if (is_q) EightValues<T>::store(q_out + (size_t)t * q_out_stride + (size_t)head * hd + d0, x);
+    else if (page >= 0) EightValues<T>::store(k_pool + (((size_t)page * nkv + (head - nq)) * page_size + off) * hd + d0, x);
   }
 }
 
@@ -970,30 +1023,33 @@ extern "C" int ullm_qk_norm_rope_write(
                    (!k_gain || ((uintptr_t)k_gain & 15) == 0) && rot % 8 == 0;
   if (vec) {
     // with few tokens a thread takes one head, so that many blocks are under way; with many it takes up to four
-    // in turn, for which it fetches its cosines and sines once
-    const int heads_per_block = 256 / lph;
-    int blocks_per_token = (nq + 2 * nkv + heads_per_block - 1) / heads_per_block;
-    int heads_per_thread = 1;
-    if (T_ >= 1024) {
-      heads_per_thread = blocks_per_token < 4 ? blocks_per_token : 4;
-      blocks_per_token = (blocks_per_token + heads_per_thread - 1) / heads_per_thread;
-    }
+    // in turn, for which it fetches its cosines and sines once (40 heads of 128: 300 tokens 4.9 us, in passes 5.1; 800 8.0 and 7.1)
     // with many tokens the values go through blocks of their own that write runs of eight at once
     const bool runs = write_kv && T_ >= 128 && page_size % 8 == 0 && hd <= VALUE_RUN_MAX_HD &&
                       ((uintptr_t)v_pool & 15) == 0;
+    const int heads_per_block = 256 / lph, read_heads = write_kv && !runs ? nq + 2 * nkv : nq + nkv;
+    int blocks_per_token = (read_heads + heads_per_block - 1) / heads_per_block;
+    int heads_per_thread = 1;
+    if (T_ >= 512) {
+      heads_per_thread = blocks_per_token < 4 ? blocks_per_token : 4;
+      blocks_per_token = (blocks_per_token + heads_per_thread - 1) / heads_per_thread;
+    }
     const long long value_blocks = runs ? (long long)((T_ + VALUE_RUN_TOKENS - 1) / VALUE_RUN_TOKENS) * nkv : 0;
     const long long all_blocks = (long long)T_ * blocks_per_token + value_blocks;
     if (all_blocks > 0x7fffffffLL) return ULLM_ERR_SHAPE;
     const int kv_flags = !write_kv ? 0 : (runs ? 1 : 3);   // bit 0: keys, bit 1: values token by token
     dim3 vgrid((unsigned)all_blocks), vblock(256);
-#define GOV(TT) hipLaunchKernelGGL(qk_norm_rope_write_vec_kernel<TT>, vgrid, vblock, 0, stream, \
+#define GO(TT, PASSES) hipLaunchKernelGGL((qk_norm_rope_write_vec_kernel<TT, PASSES>), vgrid, vblock, 0, stream, \
     (const TT*)qkv, qkv_stride, (TT*)q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, \
     rot, style, positions, token_entry, block_table, bt_stride, (TT*)k_pool, (TT*)v_pool, page_size, \
-    nq, nkv, hd, kv_flags, T_, blocks_per_token, heads_per_thread, v_head0, norm_dim)
+    nq, nkv, hd, kv_flags, T_, blocks_per_token, v_head0, norm_dim)
+#define GOV(TT) do { if (heads_per_thread == 1) GO(TT, 1); else if (heads_per_thread == 2) GO(TT, 2); \
+    else if (heads_per_thread == 3) GO(TT, 3); else GO(TT, 4); } while (0)
     if (dtype == ULLM_F32) GOV(float);
     else if (dtype == ULLM_BF16) GOV(bf16_t);
     else return ULLM_ERR_DTYPE;
 #undef GOV
+#undef GO
     ULLM_LAUNCH_CHECK();
   }
   dim3 grid(T_, nq + 2 * nkv), block(WAVE);
