@@ -2,7 +2,7 @@
 stages and float32 among them; and that every size gets a tile the kernels know."""
 import pytest
 
-from ullm_amd.parts.moe import tile_rows_for
+from ullm_amd.parts.moe import product_rows_for, tile_rows_for
 
 # microseconds of gate|up and down in tiles of 16, 32, 64, 128 and 256 rows, by the mean of rows an expert
 MEASURED = {
@@ -41,3 +41,16 @@ def test_every_size_gets_a_tile_the_kernels_know(experts, top, hidden, ff):
         assert rows in (16, 32, 64, 128, 256)
         if rows == 256:                                # what that kernel's 32-bit offsets reach
             assert hidden % 64 == ff % 64 == 0 and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31
+
+
+@pytest.mark.parametrize("sizes,mean,rows", [
+    ((32, 4, 2048, 1024), 15, 16), ((32, 4, 2048, 1024), 20, 256), ((32, 4, 2048, 1024), 84, 128), ((32, 4, 2048, 1024), 256, 256), ((64, 8, 2048, 768), 48, 256),
+    ((16, 4, 5120, 1536), 16, 256), ((128, 8, 1024, 512), 40, 256), ((8, 2, 4096, 1536), 128, 64), ((8, 2, 1024, 512), 96, 64),
+    ((32, 4, 2048, 1000), 96, 128), ((32, 4, 2056, 1024), 96, 128)])
+def test_tiles_by_their_rows_where_experts_fill_a_round(sizes, mean, rows):
+    experts, top, hidden, ff = sizes
+    if rows != 256:
+        rows = tile_rows_for(mean * experts // top, top, experts, hidden, ff)
+        assert rows != 256
+    assert product_rows_for(mean * experts // top, top, experts, hidden, ff) == rows
+    assert product_rows_for(2 ** 31 // (top * hidden), top, experts, hidden, ff) <= 128          # past what 32-bit offsets reach

@@ -84,3 +84,27 @@ def test_few_rows_an_expert(ops, tile_rows, K, n_out, limit):
             want = a * torch.sigmoid(a) * u
         off = (K + 8) * 2.0 ** -24 * (h.abs() @ w_gu[e].double().abs().T).max() * (4 + u.abs() + a.abs()) if n else 0.0
         assert ((gated[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + off).all()
+
+
+@pytest.mark.parametrize("K,n_out,experts", [(64, 1040, 24), (192, 1096, 24), (128, 520, 300)])
+def test_tiles_of_every_height_in_more_than_a_round(ops, K, n_out, experts):
+    """Lists of more blocks than a round, the last of them begun, whose long tiles go before the others, and one of more tiles than
+    that order takes: the same sums as in tiles of 128, whose blocks go by the list."""
+    g = torch.Generator().manual_seed(K + n_out)
+    cycle = [300, 1, 64, 65, 0, 128, 129, 256, 257, 520, 20, 192]
+    counts = [cycle[e % len(cycle)] if experts < 256 else 3 + e % 5 for e in range(experts)]
+    T = sum(counts)
+    if experts < 256:
+        blocks = -(-n_out // 128)
+        used, short = sum(-(-n // 256) for n in counts) * blocks, sum(0 < n % 256 <= 128 for n in counts) * blocks
+        assert used > 256 and 0 < used % 256 <= 204 and 0 < short <= 160
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=g)].int()[:, None].contiguous().to(DEV)
+    x = torch.randn(T, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(experts, 2 * n_out, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    results = []
+    for tile_rows in (128, 256):
+        slot, token, tiles, _ = ops.moe_sort(ids, experts, tile_rows)
+        at = slot.long()
+        results.append((ops.moe_rows(x, token, w, tiles, tile_rows, T, gated=True)[at],
+                        ops.moe_rows(x[token.long()].contiguous(), None, w, tiles, tile_rows, T, gated=False)[at]))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])

@@ -48,7 +48,7 @@ gemm_tiles_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restric
     woff[i] = 2u * ((unsigned)((GATED && row >= COLS ? n_out : 0) + n) * (unsigned)ldw + T::k_of(row, lane));
   }
   tile_f32x4 acc[T::TN][T::TM];
-  T::run(tile_stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w), woff, K >> 6, wave, lane, 128, acc);
+  T::run(tile_stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w), woff, K >> 6, 0, wave, lane, 128, acc);
   const int wm = wave >> 1, wn = wave & 1;
   const bool whole = ((n_out | ldo) & 7) == 0;
 #pragma unroll

@@ -1,11 +1,11 @@
-// The inner loop of large bfloat16 products out = x W^T: a block of 2 WMW waves takes 64 WMW rows of x against 256 rows of W,
+// The inner loop of large bfloat16 products out = x W^T: a block of WMW x WN waves takes 64 WMW rows of x against 256 rows of W,
 // 64 values of K a stage.
 //
 // Stages go straight to shared memory (lds_load.h), STAGES of them taking turns: rows of 128 bytes, the 64 WMW rows of x and
 // then the 256 of W, whose 16-byte piece c of row r lies at piece c ^ ((r >> 1) & 7) (the 16 lanes that shared memory serves
 // together then read 16 different bank groups).  A load instruction fills 8 rows.  Wave (wm, wn) makes rows 64 wm .. of x
-// against two strips of 64 rows of W: 12 reads of 1 KB per 32 products of v_mfma_f32_16x16x32_bf16, 96 of shared memory's
-// 128 bytes a cycle at the matrix pipe's full rate.
+// against two strips of 128 / WN rows of W: with WN = 2 that is 12 reads of 1 KB per 32 products of v_mfma_f32_16x16x32_bf16, 96 of
+// shared memory's 128 bytes a cycle at the matrix pipe's full rate.  WN = 8 is for eight waves over 64 rows of x.
 //
 // One wave's instructions keep the matrix pipe busy: the operands of one half of a stage (32 values of K) are read into
 // registers between the products of the half before, and the loads of a stage further on are issued between the products of
@@ -39,11 +39,11 @@ __device__ __forceinline__ uint4 pair_columns(const uint2& a, const uint2& b) {
 }
 __device__ __forceinline__ int pair_column(int g) { return 16 * (g & 1) + 4 * (g & 2); }
 
-template <int WMW, int STAGES_>
+template <int WMW, int STAGES_, int WN = 2>
 struct ProductTiles {
-  static_assert(WMW == 2 || WMW == 4, "whole pieces of W a wave");
-  static constexpr int WAVES = 2 * WMW, BM = 64 * WMW, BN = 256, STAGES = STAGES_, STAGE = (BM + BN) * 128;
-  static constexpr int XL = 4, WL = 32 / WAVES, LOADS = XL + WL, TM = 4, TN = 8;
+  static constexpr int WAVES = WN * WMW, BM = 64 * WMW, BN = 256, STAGES = STAGES_, STAGE = (BM + BN) * 128;
+  static_assert(WAVES == 4 || WAVES == 8, "whole pieces of x and of W a wave");
+  static constexpr int XL = 8 / WN, WL = 32 / WAVES, LOADS = XL + WL, TM = 4, TN = 16 / WN, STRIP = TN / 2;
   static constexpr int BYTES = STAGES * STAGE;
 
   // row of x (of W) that this lane's i-th load brings, and the value of K in it
@@ -51,13 +51,22 @@ struct ProductTiles {
   static __device__ __forceinline__ int w_row(int wave, int lane, int i) { return 8 * (WL * wave + i) + (lane >> 3); }
   static __device__ __forceinline__ int k_of(int row, int lane) { return 8 * ((lane & 7) ^ ((row >> 1) & 7)); }
 
-  // xb, wb: addresses of K = 0 that the byte offsets xoff, woff count from; steps = K / 64 >= 1; strip: rows between the two
-  // strips of W that a wave takes (strip 0 begins at 64 wn of them).  acc[n][m]: lane (r, g) holds row 64 wm + 16 m + r of x,
-  // rows 4 g .. 4 g + 3 of the n-th 16 rows of the wave's strips (n < 4: the first).
+  // xb, wb: addresses of K = 0 that the byte offsets xoff, woff count from; steps = K / 64 >= 1, of which the start-th is the first
+  // and the one before it the last; strip: rows between the two
+  // strips of W that a wave takes (strip 0 begins at 16 STRIP wn of them).  acc[n][m]: lane (r, g) holds row 64 wm + 16 m + r of x,
+  // rows 4 g .. 4 g + 3 of the n-th 16 rows of the wave's strips (n < STRIP: the first).
   static __device__ __forceinline__ void run(unsigned char* lds, const char* xb, const unsigned (&xoff)[XL], const char* wb,
-                                             const unsigned (&woff)[WL], int steps, int wave, int lane, int strip,
+                                             const unsigned (&woff)[WL], int steps, int start, int wave, int lane, int strip,
                                              tile_f32x4 (&acc)[TN][TM]) {
-    const int r = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
+    xb += start * 128, wb += start * 128;
+    int until_end = steps - start;
+    auto advance = [&]() __attribute__((always_inline)) {
+      const bool wrap = --until_end == 0;
+      const int by = wrap ? 128 - 128 * steps : 128;
+      xb += by, wb += by;
+      if (wrap) until_end = steps;
+    };
+    const int r = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
     const unsigned place = lds_place(lds);
     const unsigned xdest = place + XL * wave * 1024, wdest = place + BM * 128 + WL * wave * 1024;
     auto load = [&](int i, unsigned to) __attribute__((always_inline)) {
@@ -67,12 +76,12 @@ struct ProductTiles {
     int at[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) at[s] = ((4 * s + g) ^ ((r >> 1) & 7)) << 4;
-    const int xat = (64 * wm + r) * 128, wat = (BM + 64 * wn + r) * 128, next = strip * 128;
+    const int xat = (64 * wm + r) * 128, wat = (BM + 16 * STRIP * wn + r) * 128, next = strip * 128;
     auto read_x = [&](const unsigned char* st, int s, int m) __attribute__((always_inline)) {
       return ld16(st + xat + at[s] + m * 2048);
     };
     auto read_w = [&](const unsigned char* st, int s, int n) __attribute__((always_inline)) {
-      return ld16(st + wat + at[s] + (n & 3) * 2048 + (n < 4 ? 0 : next));
+      return ld16(st + wat + at[s] + n % STRIP * 2048 + (n < STRIP ? 0 : next));
     };
 #pragma unroll
     for (int n = 0; n < TN; ++n)
@@ -82,8 +91,9 @@ struct ProductTiles {
     // the reads of half s that stand beside its predecessor's n-th group of products
     auto operands = [&](const unsigned char* st, int s, int n) __attribute__((always_inline)) {
       if constexpr (WAVES == 8) {
+        constexpr int EACH = (TM + TN + TN - 1) / TN;
 #pragma unroll
-        for (int q = 2 * n; q < 2 * n + 2; ++q) {
+        for (int q = EACH * n; q < EACH * (n + 1); ++q) {
           if (q < TM) x[s][q].u4 = read_x(st, s, q);
           else if (q < TM + TN) w[s][q - TM].u4 = read_w(st, s, q - TM);
         }
@@ -103,7 +113,7 @@ struct ProductTiles {
       if (i < steps) {
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) load(j, i * STAGE);
-        xb += 128, wb += 128;
+        advance();
       }
     if (steps >= STAGES) loads_left<(STAGES - 1) * LOADS>();
     else loads_left<0>();
@@ -138,7 +148,7 @@ struct ProductTiles {
         products(1, n);
         __builtin_amdgcn_sched_barrier(0);
       }
-      xb += 128, wb += 128;
+      if constexpr (decltype(loads)::value) advance();
     };
     int k = 0;
 #pragma unroll 1

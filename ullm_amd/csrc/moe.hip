@@ -820,32 +820,28 @@ moe_tiles_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restri
   }
 }
 
-// The same products where K is a multiple of 64, by the loop of mfma_tiles.h: a block takes a tile of up to 64 WMW rows against
-// 256 rows of the expert's matrix (GATED: the gate rows and the up rows of 128 output columns, a wave the same 64 of each).
+// The same products where K is a multiple of 64, by the loop of mfma_tiles.h: a block takes a tile of rows against 256 rows of the
+// expert's matrix (GATED: the gate rows and the up rows of 128 output columns, a wave the same number of each).  Tiles of up to 128
+// rows have four waves, tiles of up to 256 eight, which take 64 or 256 rows by 256, whichever holds the tile: an expert's
+// short last tile is paid by its rows.  (128 rows by waves of their own, 64 by 64 each: 800 tokens gate|up + down 72 -> 70 us alone, but more reads of
+// shared memory a product, and prompts of 3000 tokens in 4.29 ms instead of 4.27.)
 // What bounds it: the experts' matrices from memory (268 MB of gate|up: 45 us) and, beside them, the matrix pipe, which the
-// loop keeps busy 57 % of the time where every operand lies in the second-level cache.  32 experts, top 4, width 2048, 1024
-// columns an expert, against the kernel above: gate|up at 2048 / 3000 / 8192 tokens 160 / 217 / 470 -> 117 / 140 / 279 us (590 /
-// 720 / 987 TFLOP/s), down 87 / 120 / 270 -> 73 / 87 / 206 us.  (Replayed back to back the tiles of 256 rows take 108 + 70 us at
-// 3000 and 267 + 192 at 8192 tokens.)  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a
-// stage ahead of its products took 127 to 150 us at 2048 tokens, whatever the number of stages; a wave of its own that asked
-// for the matrix's lines ahead of time made them slower (180 us).
-template <int WMW, int STAGES, bool GATED>
-__global__ void __launch_bounds__(128 * WMW)
-moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
-                    const bf16_t* __restrict__ w, const int* __restrict__ tiles, int n_tiles, int n_col_blocks,
-                    void* __restrict__ out_, int ldo, int n_out, int K, float limit, float alpha) {
-  using T = ProductTiles<WMW, STAGES>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char tile_stages[];
-  const int used = tiles[3 * n_tiles];                   // dies and tiles as above
-  const int total = used * n_col_blocks, per_die = (total + 7) / 8;
-  const int item = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_die || item >= total) return;
-  const int tile = item / n_col_blocks, col_block = item % n_col_blocks;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
-  const int e = tiles[3 * tile], slot0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-  if (rows <= 0) return;
+// loop keeps busy 57 % of the time where every operand lies in the second-level cache.  Rows of the matrices lie a power of two apart, and
+// blocks in step ask the same memory channels: so a block's K begins at the stage of its expert's number (32 experts, width 2048, 1024
+// columns, gate|up + down at 400 / 800 tokens, top 4, 71 + 26 / 73 + 35 -> 50 + 27 / 52 + 40 us; the stage by the columns too, 51 + 27 / 54 + 38,
+// leaves less to share between the blocks of a tile: 1500 tokens 69 + 49 and 67 + 45).
+// All of it together, us before and now of what takes the call: 400 / 800 / 1100 / 1500 / 2048 / 2500 / 3000 / 4000 / 8000 tokens 98 / 107 / 119 / 125 /
+// 173 / 187 / 192 / 270 / 450 -> 75 / 93 / 114 / 115 / 143 / 181 / 192 / 236 / 420.  Before that loop, by the kernel above, gate|up took
+// 160 us at 2048 tokens and 470 at 8192.  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a stage ahead of its products
+// took 127 to 150 us at 2048 tokens, whatever the number of stages; a wave of its own that asked for the matrix's lines ahead
+// of time made them slower (180 us).
+template <class T, bool GATED>
+__device__ __forceinline__ void moe_products_tile(unsigned char* stages, const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
+                                                  const bf16_t* __restrict__ w, int e, int slot0, int rows, int n0,
+                                                  void* __restrict__ out_, int ldo, int n_out, int K, float limit, float alpha) {
   constexpr int COLS = GATED ? 128 : 256;                // output columns of a block
-  const int n0 = col_block * COLS;
+  constexpr int H = T::STRIP, WN = 8 / H;                // 16-row pieces of a wave's strip of W, waves beside each other
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const size_t w_rows = GATED ? 2 * (size_t)n_out : (size_t)n_out;
   unsigned xoff[T::XL], woff[T::WL];
 #pragma unroll
@@ -861,41 +857,51 @@ moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
     woff[i] = 2u * ((unsigned)((GATED && row >= COLS ? n_out : 0) + n) * (unsigned)K + T::k_of(row, lane));
   }
   tile_f32x4 acc[T::TN][T::TM];
-  T::run(tile_stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w + (size_t)e * w_rows * K), woff,
-         K >> 6, wave, lane, 128, acc);
+  T::run(stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w + (size_t)e * w_rows * K), woff,
+         K >> 6, (int)((unsigned)e % (unsigned)(K >> 6)), wave, lane, 128, acc);
   // lane (r, g): row r of each 16-row group, four consecutive columns at 4g
-  const int wm = wave >> 1, wn = wave & 1;
-  const bool whole = ((n_out | ldo) & 7) == 0 && !((uintptr_t)out_ & 15);
+  const int wm = wave / WN, wn = wave % WN;
+  const bool whole = ((n_out | ldo) & (GATED ? 7 : 3)) == 0 && !((uintptr_t)out_ & 15);
 #pragma unroll
   for (int m = 0; m < T::TM; ++m) {
     const int row = 64 * wm + 16 * m + r;
     if (row >= rows) continue;
-    if (GATED && whole) {
+    if (whole) {
+      if constexpr (!GATED) {
+        float* const o = reinterpret_cast<float*>(out_) + (size_t)(slot0 + row) * ldo;
 #pragma unroll
-      for (int n = 0; n < 4; n += 2) {
-        uint2 u[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float v[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n + h][m][i], acc[n + h + 4][m][i], limit, alpha);
-          u[h] = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        for (int n = 0; n < 2 * H; ++n) {
+          const int c = n0 + 16 * H * wn + 16 * (n % H) + 4 * g + (n < H ? 0 : 128);
+          if (c < n_out) *reinterpret_cast<float4*>(o + c) = make_float4(acc[n][m][0], acc[n][m][1], acc[n][m][2], acc[n][m][3]);
         }
-        const uint4 both = pair_columns(u[0], u[1]);
-        const int c = n0 + 64 * wn + 16 * n + pair_column(g);
-        if (c < n_out) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(out_) + (size_t)(slot0 + row) * ldo + c) = both;
+        continue;
+      } else if constexpr (H > 1) {
+#pragma unroll
+        for (int n = 0; n < H; n += 2) {
+          uint2 u[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n + h][m][i], acc[n + h + H][m][i], limit, alpha);
+            u[h] = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+          }
+          const uint4 both = pair_columns(u[0], u[1]);
+          const int c = n0 + 16 * H * wn + 16 * n + pair_column(g);
+          if (c < n_out) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(out_) + (size_t)(slot0 + row) * ldo + c) = both;
+        }
+        continue;
       }
-      continue;
     }
 #pragma unroll
-    for (int n = 0; n < (GATED ? 4 : 8); ++n) {
-      const int c = n0 + 64 * wn + 16 * (n & 3) + 4 * g + (n < 4 ? 0 : 128);
+    for (int n = 0; n < (GATED ? H : 2 * H); ++n) {
+      const int c = n0 + 16 * H * wn + 16 * (n % H) + 4 * g + (n < H ? 0 : 128);
       const size_t at = (size_t)(slot0 + row) * ldo + c;
-      if (GATED) {
-        bf16_t* o = reinterpret_cast<bf16_t*>(out_) + at;
+      if constexpr (GATED) {
+        bf16_t* const o = reinterpret_cast<bf16_t*>(out_) + at;
         float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n][m][i], acc[n + 4][m][i], limit, alpha);
+        for (int i = 0; i < 4; ++i) v[i] = moe_glu<false>(acc[n][m][i], acc[n + H][m][i], limit, alpha);
         if (c + 3 < n_out && (ldo & 3) == 0) {
           *reinterpret_cast<uint2*>(o) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
         } else {
@@ -904,17 +910,88 @@ moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
             if (c + i < n_out) o[i] = f32_to_bf16_bits(v[i]);
         }
       } else {
-        float* o = reinterpret_cast<float*>(out_) + at;
-        if (c + 3 < n_out && (ldo & 3) == 0) {
-          *reinterpret_cast<float4*>(o) = make_float4(acc[n][m][0], acc[n][m][1], acc[n][m][2], acc[n][m][3]);
-        } else {
+        float* const o = reinterpret_cast<float*>(out_) + at;
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (c + i < n_out) o[i] = acc[n][m][i];
-        }
+        for (int i = 0; i < 4; ++i)
+          if (c + i < n_out) o[i] = acc[n][m][i];
       }
     }
   }
+}
+
+// The tile and the block of its columns that this block takes, or a tile of -1: die d (blocks go to the dies round-robin) takes the
+// d-th eighth of the tiles in use, a tile's columns side by side.
+__device__ __forceinline__ int tile_in_turn(const int* __restrict__ tiles, int n_tiles, int n_col_blocks, int* columns) {
+  const int total = tiles[3 * n_tiles] * n_col_blocks, per_die = (total + 7) / 8;
+  const int item = ((int)blockIdx.x & 7) * per_die + ((int)blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_die || item >= total) return -1;
+  *columns = item % n_col_blocks;
+  return item / n_col_blocks;
+}
+// As above where the blocks fill whole rounds of a die's 32 units, or nearly, or where most experts have a tile of 64 rows or less:
+// a tile's neighbours of the same expert then run beside it and share its matrix.  Else every die takes its eighth of the tiles of more than
+// 64 rows, and behind them its eighth of the others, which take about half a round (32 experts of 256 rows by chance, half of them
+// with a few rows more, gate|up 111 us in turn, 92 so; of 500 162 and 141, of 750 210 and 192; of 312, every one with a second tile, 104 in
+// turn, 115 so; of 625 168 and 178).
+__device__ __forceinline__ int tile_by_rows(const int* __restrict__ tiles, int n_tiles, int n_col_blocks, int* columns) {
+  constexpr int HELD = 4;                                // 64 tiles each; a longer list makes many rounds
+  const int lane = threadIdx.x & 63, die = (int)blockIdx.x & 7;
+  int rows[HELD], big = 0;
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) rows[i] = tiles[3 * (64 * i + lane < n_tiles ? 64 * i + lane : 0) + 2];   // beside the list's length
+  const int used = tiles[3 * n_tiles], last = used * n_col_blocks & 255;
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
+    rows[i] = 64 * i + lane < used ? rows[i] : 0;
+    big += __popcll(__ballot(rows[i] > 64));
+  }
+  if (used > 64 * HELD || used * n_col_blocks <= 256 || last == 0 || last > 204 || (used - big) * n_col_blocks > 160)
+    return tile_in_turn(tiles, n_tiles, n_col_blocks, columns);
+  int at = (int)blockIdx.x >> 3;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    unsigned long long of[HELD];
+    int total = 0;
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+      of[i] = __ballot(k == 0 ? rows[i] > 64 : rows[i] > 0 && rows[i] <= 64);
+      total += n_col_blocks * __popcll(of[i]);
+    }
+    const int per_die = (total + 7) / 8, left = total - die * per_die, mine = left < per_die ? left : per_die;
+    if (at < mine) {
+      const int item = die * per_die + at;
+      int nth = item / n_col_blocks;
+      *columns = item % n_col_blocks;
+#pragma unroll
+      for (int i = 0; i < HELD; ++i) {
+        const int here = __popcll(of[i]);
+        if (nth < here) return 64 * i + __ffsll(__ballot((of[i] >> lane & 1) && __popcll(of[i] & ((1ull << lane) - 1)) == nth)) - 1;
+        nth -= here;
+      }
+    }
+    at -= mine > 0 ? mine : 0;
+  }
+  return -1;
+}
+
+template <int WMW, int STAGES, bool GATED>
+__global__ void __launch_bounds__(128 * WMW)
+moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
+                    const bf16_t* __restrict__ w, const int* __restrict__ tiles, int n_tiles, int n_col_blocks,
+                    void* __restrict__ out, int ldo, int n_out, int K, float limit, float alpha) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char tile_stages[];
+  int item;
+  const int tile = WMW == 4 ? tile_by_rows(tiles, n_tiles, n_col_blocks, &item) : tile_in_turn(tiles, n_tiles, n_col_blocks, &item);
+  if (tile < 0) return;
+  const int n0 = item * (GATED ? 128 : 256);
+  const int e = tiles[3 * tile], slot0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+  if (rows <= 0) return;
+#define TILE(...) moe_products_tile<__VA_ARGS__, GATED>(tile_stages, x, ldx, row_index, w, e, slot0, rows, n0, out, ldo, n_out, K, limit, alpha)
+  if constexpr (WMW == 4) {
+    if (rows <= 64) return TILE(ProductTiles<1, 3, 8>);
+  }
+  TILE(ProductTiles<WMW, STAGES>);
+#undef TILE
 }
 
 // Rows of a tile the matrix-core kernels take for a launch made with `tile_rows` rows a tile.
@@ -941,6 +1018,7 @@ static void launch_rows_dma(dim3 grid, hipStream_t stream, Args... args) {
 template <int WMW, int STAGES, bool GATED, typename... Args>
 static void launch_products(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int bytes = ProductTiles<WMW, STAGES>::BYTES;
+  static_assert(WMW != 4 || bytes >= ProductTiles<1, 3, 8>::BYTES, "the largest of a launch's");
   static const hipError_t allowed = hipFuncSetAttribute((const void*)moe_products_kernel<WMW, STAGES, GATED>,
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   (void)allowed;
@@ -962,7 +1040,7 @@ extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const
       const int per_block = gated ? 128 : 256, col_blocks = (n_out + per_block - 1) / per_block;
       const long long total = (long long)max_tiles * col_blocks;
       if (total > 0x3fffffffLL) return ULLM_ERR_SHAPE;
-      dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+      dim3 grid((unsigned)(8 * ((total + 7) / 8 + (tile_rows == 256 ? 1 : 0))));   // two eighths, each rounded up
 #define TILES(W, ST, G) launch_products<W, ST, G>(grid, stream, (const bf16_t*)x, ldx, row_index, (const bf16_t*)w, tiles, max_tiles, \
     col_blocks, out, ldo, n_out, K, limit, alpha)
       if (tile_rows == 256) { if (gated) TILES(4, 2, true); else TILES(4, 2, false); }

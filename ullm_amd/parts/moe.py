@@ -91,7 +91,8 @@ def tile_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int 
     - / - / 110 / 103 / 112, - / - / 119 / 126 / 119, - / - / 141 / 133 / 120; 8 experts, width 1024, 512 columns at 36, 96, 160, 320, 1024
     19 / 17 / 19 / 26 / 35, 38 / 30 / 20 / 29 / 39, - / - / 21 / 30 / 41, - / - / 29 / 32 / 45, - / - / 56 / 61 / 51; 8 experts, width 4096, 1536
     columns at 24, 36, 128, 320 106 / 68 / 71 / 87 / 125, 146 / 110 / 71 / 90 / 127, - / - / 116 / 102 / 133, - / - / 231 / 168 / 150.
-    A prompt of 440 tokens of a stack with six such layer runs took 2.42 ms in tiles of 64, 2.37 in tiles of 128."""
+    A prompt of 440 tokens of a stack with six such layer runs took 2.42 ms in tiles of 64, 2.37 in tiles of 128.  (Tiles of 128 and 256
+    have become faster since, where the experts' matrices come from memory by up to a quarter: :func:`product_rows_for`.)"""
     mean = tokens * top / max(1, experts)
     if (mean > 0 and experts > 0 and hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
             and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31):
@@ -101,6 +102,26 @@ def tile_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int 
     if mean >= 48:
         return 64
     return 32 if mean >= 24 else 16
+
+
+def product_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int = 0) -> int:
+    """Grouped rows a block of the expert products takes: up to 256, a tile of 64 rows or less at its own cost, where the experts'
+    first tiles alone make about a round of blocks over 256 compute units and most experts' last tiles are short or long, else what
+    :func:`tile_rows_for` says.
+
+    That kernel reads the matrices at 5.5 TB/s whatever the rows, so it is ahead from few rows on (us of gate|up + down,
+    the best of the tiles of 16 to 128 rows and this: 32 experts, width 2048, 1024 columns at means of 12, 18, 36, 50, 100, 137, 187, 256 and
+    500 73 / 70, 81 / 71, 77 / 73, 84 / 75, 93 / 105, 123 / 114, 132 / 115, 173 / 143, 287 / 236; 64 experts of 768 columns at 12, 18, 48, 512 107 / 113,
+    118 / 114, 130 / 123, 432 / 393; 16 experts, width 5120, 1536 columns at 12, 18, 512 137 / 144, 148 / 144, 544 / 443; 128 experts,
+    width 1024, 512 columns at 24, 48, 512 79 / 81, 91 / 91, 325 / 293).  With fewer blocks a tile of 256 rows leaves
+    most units idle (8 experts, width 4096, 1536 columns at 128 / 288 97 / 131, 158 / 150)."""
+    rows = tile_rows_for(tokens, top, experts, hidden, ff)
+    mean = tokens * top / max(1, experts)
+    if (mean >= max(16, 40 * 1024 / max(1, hidden)) and not 56 <= mean <= 104 and hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
+            and experts * (-(-ff // 128) - (-hidden // 256)) >= 460
+            and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31):
+        return 256
+    return rows
 
 
 @register_part("ffn", "routed_experts")
@@ -198,7 +219,7 @@ class RoutedExperts(FeedForward):
         ids, weights = self.route(x)
         y = None
         # in 32-bit a row is worked after the other whatever the tile: the fewer a tile, the more of them side by side
-        tile_rows = tile_rows_for(T, self.top, self.experts, *((self.hidden_size, self.ff) if x.dtype == torch.bfloat16 else (0, 0)))
+        tile_rows = product_rows_for(T, self.top, self.experts, *((self.hidden_size, self.ff) if x.dtype == torch.bfloat16 else (0, 0)))
         slot_of_pair = ids.view(-1)               # read for experts with weights only
         if self.experts:
             slot_of_pair, token_of_slot, tiles, _ = ops.moe_sort(ids, self.experts, tile_rows)
