@@ -83,7 +83,7 @@ def test_when_it_is_taken():
     assert [P(r, 24576, 4096, "gated")[0] >= 0 for r in (16, 17, 256, 257, 3000)] == [False, True, True, False, False]
     assert [P(r, 1024, 3072, "stream")[0] >= 0 for r in (16, 17, 1024, 1025)] == [False, True, True, False]
     assert [P(r, 1024, 3072, "stream", False, True)[0] >= 0 for r in (16, 1025, 1800, 20000)] == [False, True, True, False]
-    assert [P(r, 4096, 12288, "stream")[0] >= 0 for r in (17, 2048, 2049)] == [True, True, False]
+    assert [P(r, 4096, 12288, "stream")[0] >= 0 for r in (17, 1024, 1025)] == [True, True, False]
     assert [P(r, 151936, 1024, "float")[0] >= 0 for r in (16, 17, 256, 257)] == [False, True, True, False]      # in more than one round
     assert [P(r, 2048, 2048, "float")[0] >= 0 for r in (17, 512, 513)] == [True, True, False] and P(600, 4096, 2048, "float")[0] >= 0
     assert P(64, 1000, 1024, "store")[0] < 0 and P(64, 1024, 1024, "store")[0] >= 0            # a smaller matrix than measured

@@ -165,10 +165,10 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     before and this: gate|up 24576 x 4096 at 17 / 64 / 256 rows 36 / 43 / 64 and 32 / 36 / 58; 6144 x 1024 at 40 / 256 / 800 7.9 / 15.1 / 17.3 and
     5.8 / 9.6 / 15.0; 4096 x 12288 into the stream at 130 / 512 / 1024 30.6 / 83 / 118 and 26.4 / 51 / 94; 6144 x 4096 at 64 / 256 / 1024 17.8 / 31 / 53
     and 16.8 / 25.7 / 53.3).  In two rounds the library's tiles are ahead (6144 x 4096 at 1300 rows 65 and 83, gate|up 24576 x 4096 at 320
-    79 and 87), and from 1025 rows on also in one where a matrix has few columns (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 /
-    24.1, 2048 x 2048 at 2048 / 3000 21.0 / 26.5 and 23.0 / 27.6; 4096 x 1024 at 1300 20.1 and 16.0, 4096 x 12288 at 1300 / 2048 146 / 191
-    and 133 / 174), where ``host_bound`` does not say that launches are what takes the time."""
-    if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and columns < 4096 and not host_bound):
+    79 and 87), and from 1025 rows on also in one (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 / 24.1, 2048 x 2048 at 2048 / 3000
+    21.0 / 26.5 and 23.0 / 27.6; inside a prompt of 1064 rows 6144 x 4096 59 and 63, 4096 x 4096 and 4096 x 12288 183 and 189 together,
+    the prompt 17.9 and 18.4 ms; level at 2048), where ``host_bound`` does not say that launches are what takes the time."""
+    if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and not host_bound):
         return -1, 0
     if role == "float":
         # logits heads are read once at these rows, in however many rounds (library and this: 151936 x 4096 at 17 / 64 / 128 rows 266 / 270 /
