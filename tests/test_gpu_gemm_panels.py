@@ -119,3 +119,20 @@ def test_parts_take_it_where_the_rule_says(ops, monkeypatch):
         assert close(y if y.dim() == 2 else y.sum(0), want)
         assert (len(calls) == 4) == (rows > 16) and (rows == 16 or set(calls) >= {dispatch.PANELS_GATED, dispatch.PANELS_FLOAT})
         del calls[:]
+
+
+# products whose fastest plan without an activation is slices that a kernel adds (at 17 rows; one that fits no round in one slice), and
+# one whose plan is whole
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rows", [(10240, 2560, (17, 32, 40, 64)), (12288, 3072, (17, 24)), (5120, 5120, (17, 64, 130, 400)), (4096, 1024, (17, 100))])
+def test_an_activation_sees_the_32_bit_sums(ops, N, K, rows):
+    from ullm_amd.kernels import dispatch
+    from ullm_amd.parts.linear import linear
+    assert any(dispatch.panels(r, N, K, "store")[1] == dispatch.PANELS_FLOAT for r in rows) == (N != 4096)
+    for M in rows:
+        x, w, bias = _operands(M, N, K, M)
+        off = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + bias.double().abs())
+        y = x.double() @ w.double().T + bias.double()
+        ref = y.clamp(min=0) ** 2
+        # one rounding to bfloat16 behind the square: the sums' own rounding would be doubled by it and come on top
+        assert ((linear(x, w, bias, act=ops.ACT_RELU2).double() - ref).abs() <= 2.0 ** -8 * ref + 4 * off * (y.abs() + off)).all(), M

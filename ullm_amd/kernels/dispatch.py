@@ -158,7 +158,7 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
 def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False) -> Tuple[int, int]:
     """The plan by which the panels kernel (``ops.gemm_panels``) takes x [rows, inner] times W [columns, inner], and its mode; a plan of -1
     where another product is ahead.  Roles: ``store`` (a bfloat16 result; in float mode the slices are added by a kernel),
-    ``gated`` (W is gate | up), ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
+    ``activated`` (the same with an activation on store), ``gated`` (W is gate | up), ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
     ``keep_sums`` always the sums) and ``float`` (the 32-bit sums as they are, one slice: logits, branches).
 
     It is taken from 17 rows on while its blocks fit one round of the chip: there its tiles fill it (us, what took the calls
@@ -180,6 +180,8 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
         return -1, 0
     if role == "gated":
         return _panels_plan(rows, columns, inner, PANELS_GATED, 1)[0], PANELS_GATED
+    if role == "activated":                          # the 32-bit sums are one block's: an activation of added slices would see them rounded
+        return _panels_plan(rows, columns, inner, PANELS_STORE, 1)[0], PANELS_STORE
     sums, sums_us = _panels_plan(rows, columns, inner, PANELS_FLOAT, PANELS_MAX_SLICES)
     if role == "stream" and keep_sums:
         return sums, PANELS_FLOAT

@@ -1335,18 +1335,17 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     kernel and a kernel that adds its stacks; thousands of rows, where the library's choice for them was measured to
     fall off, go to the large product (:func:`gemm_tiles`); the rest go through the library product (as the reference's
     linears do, ullm/layers/linear.py:165), which for 32-bit output (logits) stores the accumulator unrounded.
-    ``act`` (ACT_RELU2, ACT_GELU_TANH): that activation of the result, on store in the few-rows and rows kernels, by
-    the activation kernel behind the others."""
+    ``act`` (ACT_RELU2, ACT_GELU_TANH): that activation of the result, of the 32-bit sums on store in the few-rows, rows and panels
+    kernels (then without slices), by the activation kernel behind the others."""
     out_dtype = out_dtype or a.dtype
     M = a.shape[0]
     if (out_dtype == torch.bfloat16 and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w)
             and not dispatch.limits(w.shape[0], w.shape[1]).sums_from):
-        plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "store")
+        plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "store" if act is None else "activated")
         if plan >= 0 and mode == dispatch.PANELS_STORE:
             return gemm_panels(a, w, plan, mode, bias, act=act)
         if plan >= 0:
-            y = sum_stacks(gemm_panels(a, w, plan, mode), bias)
-            return y if act is None else activation(y, act, out=y)
+            return sum_stacks(gemm_panels(a, w, plan, mode), bias)
     if out_dtype == torch.float32 and act is None and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w):
         plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "float")
         if plan >= 0:
