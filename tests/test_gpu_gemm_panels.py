@@ -136,3 +136,24 @@ def test_an_activation_sees_the_32_bit_sums(ops, N, K, rows):
         ref = y.clamp(min=0) ** 2
         # one rounding to bfloat16 behind the square: the sums' own rounding would be doubled by it and come on top
         assert ((linear(x, w, bias, act=ops.ACT_RELU2).double() - ref).abs() <= 2.0 ** -8 * ref + 4 * off * (y.abs() + off)).all(), M
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [130, 400])
+def test_rows_that_overlap_go_where_they_went(ops, rows):
+    """An expanded row, and windows of one buffer, as x and as W: refused by the kernel, so the other products take them."""
+    from types import SimpleNamespace
+    from ullm_amd.parts.linear import gate_up, linear, linear_into_stream
+    x, w, bias = _operands(rows, 2048, 1024, rows)
+    x = x.contiguous()
+    row, windows = x[:1].expand(rows, 1024), x.flatten()[:1024 + 1016 * (rows - 1)].as_strided((rows, 1024), (1016, 1))
+    w_row, ctx = w[:1].expand(2048, 1024), SimpleNamespace(stacked_branches=True)
+    for a, b in ((row, w), (windows, w), (x, w_row)):
+        assert not ops.gemm_panels_supports(a, b)
+        want = a.double() @ b.double().T
+        close = lambda y, ref: float((y.double() - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())      # noqa: E731
+        y = linear_into_stream(a, b, ctx)
+        assert close(y if y.dim() == 2 else y.sum(0), want) and close(linear(a, b, bias), want + bias.double())
+        assert b is w_row or close(linear(a, b, out_dtype=torch.float32), want)          # 32-bit results of such a W always were refused
+        g, u = want[:, :1024], want[:, 1024:]
+        assert close(gate_up(a, b), g * torch.sigmoid(g) * u)
