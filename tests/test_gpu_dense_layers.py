@@ -30,6 +30,8 @@ def test_which_layers_are_alike():
     assert alike_layers(blocks) == 2
     blocks[1].ffn.__class__ = type("Other", (type(blocks[1].ffn),), {})
     assert layer_form(blocks[1]) is None and alike_layers(blocks) == 1
+    blocks[0].mixer_norm.add_norm = blocks[0].mixer_norm.add_norm              # a method of the part's own
+    assert alike_layers(blocks) == 0
 
 
 def _runner(size, seed):
@@ -122,3 +124,47 @@ def test_what_is_left_to_the_blocks(monkeypatch):
     assert calls == [40, 40] and (a - b).abs().max() <= 3e-2 * b.abs().max()
     for rc in rcs:
         cache.release(rc)
+
+
+def _scaled(model):
+    model.blocks[1].mixer.scale *= 2.0
+
+
+def _narrowed(model):
+    model.blocks[2].mixer.reach = 24
+
+
+def _other_eps(model):
+    model.blocks[1].ffn_norm.eps = 1.0
+
+
+def _wrapped(model):
+    part = model.blocks[1].ffn
+    real = part.forward
+    part.forward = lambda x, ctx: real(x * 2, ctx)
+
+
+def _shorter(model):
+    model.run_order = model.run_order[:2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", [_scaled, _narrowed, _other_eps, _wrapped, _shorter])
+def test_layers_changed_after_the_model_was_built(change, monkeypatch):
+    """A run takes the layers as they are when the step comes: what was exchanged in one of them is not run with the first one's numbers."""
+    from ullm_amd.engine.runner import StepEntry
+    from ullm_amd.models import model as models
+
+    def logits():
+        runner = _runner("plain", 4)
+        rc, out = runner.cache.admit("r"), []
+        for k in range(2):
+            assert runner.cache.reserve(rc, 60)
+            out.append(runner.step([StepEntry(rc, [(11 * i + k) % 512 for i in range(60)], [59])]).clone())
+            if k == 0:
+                change(runner.model)
+        return out
+    got = logits()
+    monkeypatch.setattr(models, "run_layers", lambda *a: None)
+    want = logits()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

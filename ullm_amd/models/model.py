@@ -90,7 +90,7 @@ class Model:
                     or self.cache_owner[source] >= self.cache_owner[reader]):
                 raise ValueError(f"cache {reader} reads the keys of cache {source}: no layer with keys of its own that runs before it")
         self._keeps_embedding = any(b.needs_embedding for b in self.blocks)
-        # how many of the first layers run are alike, so that their launches can go out from one native call
+        # how many of the first layers run are alike, so that their launches can go out from one native call (which looks again)
         self._alike = alike_layers([self.blocks[layer] for layer, _ in self.run_order]) if plan.streams == 0 else 0
         self.embedding: Optional[torch.Tensor] = None
         self.head: Optional[torch.Tensor] = None
@@ -211,10 +211,10 @@ class Model:
             ctx.embedded = residual.clone()      # the stream's rows are written in place from here on
         first = 0
         if self._alike > 1 and not ctx.decode_only:
-            run = range(self._alike)
+            run = range(min(self._alike, len(self.run_order)))
             pending = run_layers([self.blocks[self.run_order[i][0]] for i in run], [self._cache_of(i, caches) for i in run],
                                  residual, ctx)
-            first = 0 if pending is None else self._alike
+            first = 0 if pending is None else len(run)
         for idx in range(first, len(self.run_order)):
             layer = self.run_order[idx][0]
             cache = self._cache_of(idx, caches)
