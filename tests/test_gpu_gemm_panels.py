@@ -157,3 +157,30 @@ def test_rows_that_overlap_go_where_they_went(ops, rows):
         assert b is w_row or close(linear(a, b, out_dtype=torch.float32), want)          # 32-bit results of such a W always were refused
         g, u = want[:, :1024], want[:, 1024:]
         assert close(gate_up(a, b), g * torch.sigmoid(g) * u)
+
+
+def test_operands_that_are_the_librarys(ops):
+    """CPU, with stand-ins for device tensors: a matrix on another device than x is never handed to the kernel (the library refuses it),
+    nor is a single vector, which the library takes."""
+    from types import SimpleNamespace
+
+    def tensor(device, *shape):
+        strides = (shape[-1], 1)[-len(shape):]
+        return SimpleNamespace(dtype=torch.bfloat16, device=torch.device(device), is_cuda=device != "cpu", shape=shape, data_ptr=lambda: 0,
+                               dim=lambda: len(shape), stride=lambda i: strides[i])
+    takes = lambda x, w: ops.gemm_panels_supports(x, w)        # noqa: E731
+    x = tensor("cuda:0", 130, 1024)
+    assert takes(x, tensor("cuda:0", 2048, 1024))
+    assert not takes(x, tensor("cpu", 2048, 1024)) and not takes(x, tensor("cuda:1", 2048, 1024))
+    assert not takes(tensor("cpu", 130, 1024), tensor("cpu", 2048, 1024))
+    assert not takes(tensor("cuda:0", 1024), tensor("cuda:0", 2048, 1024))
+
+
+@pytest.mark.gpu
+def test_a_vector_and_operands_of_two_devices(ops):
+    x, w, _ = _operands(200, 2048, 1024, 3)
+    want = x[0].double() @ w.double().T
+    assert (ops.gemm_bf16(x[0].contiguous(), w).double() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+    for M in (130, 200):
+        with pytest.raises(RuntimeError):
+            ops.gemm_bf16(x[:M], w.cpu())

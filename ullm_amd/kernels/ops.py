@@ -1271,9 +1271,11 @@ TILES_GROUPS = 4                         # 64-row groups a block of the large pr
 
 def gemm_panels_supports(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the operands lie as the panels kernel wants them (whether it takes their sizes: ``dispatch.panels``): rows that overlap, as
-    an expanded row's or windows of one buffer, are the library's."""
-    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1
-            and x.shape[1] == w.shape[1] and x.stride(0) >= x.shape[1] and w.stride(0) >= w.shape[1] and (x.data_ptr() | w.data_ptr()) % 16 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
+    an expanded row's or windows of one buffer, and a single vector are the library's, which also refuses operands of two devices."""
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and w.device == x.device and x.dim() == 2
+            and x.stride(1) == 1 and w.stride(1) == 1
+            and x.shape[1] == w.shape[1] and x.stride(0) >= x.shape[1] and w.stride(0) >= w.shape[1]
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
             and x.shape[0] * x.stride(0) < 2 ** 31 and w.shape[0] * w.stride(0) < 2 ** 31)
 
 
