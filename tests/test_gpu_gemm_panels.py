@@ -184,3 +184,36 @@ def test_a_vector_and_operands_of_two_devices(ops):
     for M in (130, 200):
         with pytest.raises(RuntimeError):
             ops.gemm_bf16(x[:M], w.cpu())
+
+
+# one slice is ahead of four and the kernel that adds them; slices are ahead
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rows,sums", [(2048, 2048, (17, 48, 200, 1000), 0), (1024, 2048, (48,), 0), (5120, 17408, (17, 130), 1)])
+def test_blocks_that_want_a_branch_whole(ops, monkeypatch, N, K, rows, sums):
+    """Where no norm adds slices, a branch is made in one piece unless slices and the kernel that adds them are ahead."""
+    from types import SimpleNamespace
+    from ullm_amd.parts import LayerCache
+    from ullm_amd.parts.block import ParallelBlock, SandwichBlock
+    from ullm_amd.parts.decay import SideBySide
+    from ullm_amd.parts.linear import linear_into_stream
+    launched, real = [], ops.branch_sum
+    monkeypatch.setattr(ops, "branch_sum", lambda a, b=None: launched.append(b is None) or real(a, b))
+    for M in rows:
+        x, w, _ = _operands(M, N, K, M)
+        ctx = SimpleNamespace(stacked_branches=True, whole_branch=False, dtype=torch.bfloat16)
+        want = x.double() @ w.double().T
+        product = SimpleNamespace(forward=lambda h, c, cache=None: linear_into_stream(h, w, c), cache_need=lambda: None,
+                                  step_planners={})
+        norm = SimpleNamespace(add_norm=lambda branch, residual, rows=None, out_dtype=None: x, kernel_form=lambda: (None, 0.0, 0))
+        onto = SimpleNamespace(forward_onto=lambda h, c, base: base)
+        branches = [SandwichBlock(norm, product, norm).forward(None, None, ctx, None)[1].branch,
+                    SandwichBlock(norm, product, norm, 1.0, norm, product, norm).forward(None, None, ctx, None)[1].branch,
+                    ParallelBlock(norm, product, None).forward(None, None, ctx, None)[1].branch,
+                    ParallelBlock(norm, product, onto).forward(None, None, ctx, None)[1].branch,
+                    *SideBySide(product, product).forward_pair(x, ctx, LayerCache())[::2]]
+        assert len(launched) == 7 * sums and not ctx.whole_branch
+        for y in branches:
+            assert y.dim() == 2 and (y.double() - want).abs().max() <= 2.0 ** -8 * want.abs().max()
+        del launched[:]
+        stack = linear_into_stream(x, w, ctx)                # a norm adds slices as before
+        assert (stack if stack.dim() == 2 else stack.sum(0)).shape == (M, N)

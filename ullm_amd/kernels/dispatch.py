@@ -155,11 +155,13 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
 
 
 @functools.lru_cache(maxsize=8192)
-def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False) -> Tuple[int, int]:
+def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False,
+           whole: bool = False) -> Tuple[int, int]:
     """The plan by which the panels kernel (``ops.gemm_panels``) takes x [rows, inner] times W [columns, inner], and its mode; a plan of -1
     where another product is ahead.  Roles: ``store`` (a bfloat16 result; in float mode the slices are added by a kernel),
     ``activated`` (the same with an activation on store), ``gated`` (W is gate | up), ``stream`` (a result that the next norm adds: bfloat16, or slices' 32-bit sums; with
-    ``keep_sums`` always the sums) and ``float`` (the 32-bit sums as they are, one slice: logits, branches).
+    ``keep_sums`` always the sums; where what follows wants it ``whole``, slices only if they make up for the kernel that adds them: 48 x
+    2048 x 2048 in one slice 5.0 us, in four 4.4 and 4.8 to add them) and ``float`` (the 32-bit sums as they are, one slice: logits, branches).
 
     It is taken from 17 rows on while its blocks fit one round of the chip: there its tiles fill it (us, what took the calls
     before and this: gate|up 24576 x 4096 at 17 / 64 / 256 rows 36 / 43 / 64 and 32 / 36 / 58; 6144 x 1024 at 40 / 256 / 800 7.9 / 15.1 / 17.3 and
@@ -183,13 +185,15 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     if role == "activated":                          # the 32-bit sums are one block's: an activation of added slices would see them rounded
         return _panels_plan(rows, columns, inner, PANELS_STORE, 1)[0], PANELS_STORE
     sums, sums_us = _panels_plan(rows, columns, inner, PANELS_FLOAT, PANELS_MAX_SLICES)
+    one, one_us = _panels_plan(rows, columns, inner, PANELS_FLOAT, 1) if whole else (-1, 0.0)
+    added = one if 0 <= one and one_us <= sums_us + SUM_US else sums          # as 32-bit sums
     if role == "stream" and keep_sums:
-        return sums, PANELS_FLOAT
-    whole, whole_us = _panels_plan(rows, columns, inner, PANELS_STORE, 1)
-    whole_us += rows * columns * 2 / 5e6 if role == "stream" else 0.0
-    if sums >= 0 and sums_us + (SUM_US if role == "store" else 0.0) < whole_us or whole < 0:
-        return sums, PANELS_FLOAT
-    return whole, PANELS_STORE
+        return added, PANELS_FLOAT
+    stored, stored_us = _panels_plan(rows, columns, inner, PANELS_STORE, 1)
+    stored_us += rows * columns * 2 / 5e6 if role == "stream" else 0.0
+    if sums >= 0 and sums_us + (SUM_US if role == "store" else 0.0) < stored_us or stored < 0:
+        return added, PANELS_FLOAT
+    return stored, PANELS_STORE
 
 
 def gated_tile_groups(rows: int, columns: int, inner: int) -> int:

@@ -205,6 +205,9 @@ class StepContext:
     # every norm of the model takes a stack [S, T, hidden] of float32 partial sums as its branch and
     # adds them up (Norm.adds_stacks): a mixer or feed-forward may then return such a stack
     stacked_branches: bool = False
+    # what runs now is followed by something that wants its branch as one tensor [T, hidden] (``whole_branch``): slices would be added by a
+    # kernel of their own
+    whole_branch: bool = False
     # the embedding output (float32 [T, hidden], never written again), kept by the model where one of its blocks
     # says ``needs_embedding``; None otherwise
     embedded: Optional[torch.Tensor] = None
@@ -337,10 +340,26 @@ class NormedBranch:
     def joined(self) -> torch.Tensor:
         """The branch as one tensor [T, hidden]."""
         from ..kernels import ops
-        one = lambda y: ops.branch_sum(y) if y.dim() == 3 else y        # noqa: E731
         if self.second is None:
-            return one(self.branch)
-        return ops.weighted_sum(one(self.branch), one(self.second), self.a, self.b)
+            return one_branch(self.branch)
+        return ops.weighted_sum(one_branch(self.branch), one_branch(self.second), self.a, self.b)
+
+
+def one_branch(y: torch.Tensor) -> torch.Tensor:
+    """A branch as one tensor [T, hidden]: a stack [S, T, hidden] of partial sums is added up."""
+    from ..kernels import ops
+    if y.dim() == 2:
+        return y
+    return y[0] if y.shape[0] == 1 and y.dtype == torch.float32 else ops.branch_sum(y)
+
+
+def whole_branch(part: Callable[..., torch.Tensor], ctx: StepContext, *args) -> torch.Tensor:
+    """The branch that ``part(*args)`` returns in this step, as one tensor [T, hidden], for a caller that cannot add slices."""
+    before, ctx.whole_branch = ctx.whole_branch, True
+    try:
+        return one_branch(part(*args))
+    finally:
+        ctx.whole_branch = before
 
 
 @dataclass

@@ -13,7 +13,7 @@ import torch
 
 from ..kernels import ops
 from .base import (Block, FeedForward, LayerCache, Mixer, Norm, NormedBranch, PartEnv, PendingNorm, StateNeed, StepContext, StreamsBranch,
-                   WeightDecl, register_part)
+                   WeightDecl, one_branch, register_part, whole_branch)
 
 
 @register_part("block", "prenorm")
@@ -101,16 +101,11 @@ class SandwichBlock(Block):
         if isinstance(pending, PendingNorm):
             pending = None                               # the stream is complete; this block norms it itself
         x = self.mixer_norm.add_norm(pending, residual, out_dtype=ctx.dtype)
-        pending = NormedBranch(_one_branch(self.mixer.forward(x, ctx, cache)), self.mixer_post, self.mult)
+        pending = NormedBranch(whole_branch(self.mixer.forward, ctx, x, ctx, cache), self.mixer_post, self.mult)
         if self.ffn is None:
             return residual, pending
         x = self.ffn_norm.add_norm(pending, residual, out_dtype=ctx.dtype)
-        return residual, NormedBranch(_one_branch(self.ffn.forward(x, ctx)), self.ffn_post, self.mult)
-
-
-def _one_branch(y):
-    """A stack of partial sums [S, T, hidden] added up: a norm behind the branch needs the whole rows."""
-    return ops.branch_sum(y) if y.dim() == 3 else y
+        return residual, NormedBranch(whole_branch(self.ffn.forward, ctx, x, ctx), self.ffn_post, self.mult)
 
 
 @register_part("block", "parallel")
@@ -137,12 +132,13 @@ class ParallelBlock(Block):
         if isinstance(pending, PendingNorm):
             pending = None                               # the stream is complete; this block norms it itself
         h = self.norm.add_norm(pending, residual, out_dtype=ctx.dtype)
-        mixed = self.mixer.forward(h, ctx, cache)
         if self.ffn is None:
-            return residual, NormedBranch(_one_branch(mixed), None, self.mult)
+            return residual, NormedBranch(whole_branch(self.mixer.forward, ctx, h, ctx, cache), None, self.mult)
         if hasattr(self.ffn, "forward_onto"):
-            return residual, NormedBranch(self.ffn.forward_onto(h, ctx, _one_branch(mixed)), None, self.mult)
+            mixed = whole_branch(self.mixer.forward, ctx, h, ctx, cache)
+            return residual, NormedBranch(self.ffn.forward_onto(h, ctx, mixed), None, self.mult)
         # one kernel adds the two branches, whichever of them are stacks of partial sums
+        mixed = self.mixer.forward(h, ctx, cache)
         return residual, NormedBranch(ops.branch_sum(mixed, self.ffn.forward(h, ctx)), None, self.mult)
 
 
@@ -263,9 +259,9 @@ class MixInEmbedding(Block):
                                      post_gain=pending.post.kernel_form()[0], post_eps=pending.post.kernel_form()[1],
                                      post_kind=pending.post.kernel_form()[2], mult=pending.mult)
             else:
-                branch, mult = _one_branch(pending.branch), pending.mult
+                branch, mult = one_branch(pending.branch), pending.mult
         elif pending is not None and not isinstance(pending, PendingNorm):
-            branch = _one_branch(pending)
+            branch = one_branch(pending)
         both = ops.stream_pair(branch, mult, residual, ctx.embedded, ctx.dtype)
         return linear(both, self.w, out_dtype=torch.float32), None
 
@@ -341,7 +337,7 @@ class HyperPreNormBlock(Block):
             if first.dtype == second.dtype:
                 return StreamsBranch(first, mix, out_w, self.mult, second, a, b)
             y = ops.weighted_sum(first, second, a, b)
-        return StreamsBranch(_one_branch(y), mix, out_w, self.mult)
+        return StreamsBranch(one_branch(y), mix, out_w, self.mult)
 
     def forward(self, residual, pending, ctx: StepContext, cache: LayerCache):
         if residual.dim() != 3 or residual.shape[0] != self.streams:
@@ -350,12 +346,12 @@ class HyperPreNormBlock(Block):
         if hasattr(self.mixer, "forward_pair"):
             y = self.mixer.forward_pair(x, ctx, cache)
         else:
-            y = self.mixer.forward(x, ctx, cache)
+            y = whole_branch(self.mixer.forward, ctx, x, ctx, cache)
         pending = self._branch(y, self.coeffs[0])
         if self.ffn is None:
             return residual, pending
         x = self._read(residual, pending, self.ffn_norm, self.coeffs[1][0], ctx)
-        return residual, self._branch(self.ffn.forward(x, ctx), self.coeffs[1])
+        return residual, self._branch(whole_branch(self.ffn.forward, ctx, x, ctx), self.coeffs[1])
 
 
 def join_streams(streams, pending, norm: Norm, rows, out_dtype):

@@ -28,7 +28,7 @@ import numpy as np
 import torch
 
 from ..kernels import ops
-from .base import LayerCache, Mixer, PartEnv, StateNeed, StepContext, StepPlan, StepShape, WeightDecl, register_part
+from .base import LayerCache, Mixer, PartEnv, StateNeed, StepContext, StepPlan, StepShape, WeightDecl, register_part, whole_branch
 from .linear import linear, linear_into_stream
 
 
@@ -328,16 +328,12 @@ class SideBySide(Mixer):
     def forward_pair(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache, stacks: bool = False):
         """(left, left_scale, right, right_scale): the two branches, not yet added.  ``stacks``: the caller also takes a
         branch that is a stack of partial sums."""
-        one = (lambda y: y) if stacks else _plain
         left_cache, right_cache = self._views(cache)
-        return (one(self.left.forward(x, ctx, left_cache)), self.left_scale,
-                one(self.right.forward(x, ctx, right_cache)), self.right_scale)
+        if stacks:
+            return self.left.forward(x, ctx, left_cache), self.left_scale, self.right.forward(x, ctx, right_cache), self.right_scale
+        return (whole_branch(self.left.forward, ctx, x, ctx, left_cache), self.left_scale,
+                whole_branch(self.right.forward, ctx, x, ctx, right_cache), self.right_scale)
 
     def forward(self, x: torch.Tensor, ctx: StepContext, cache: LayerCache) -> torch.Tensor:
         left, a, right, b = self.forward_pair(x, ctx, cache)
         return ops.weighted_sum(left, right, a, b)
-
-
-def _plain(y: torch.Tensor) -> torch.Tensor:
-    """A stack of partial sums added up."""
-    return ops.branch_sum(y) if y.dim() == 3 else y

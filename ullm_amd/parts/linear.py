@@ -125,7 +125,8 @@ def can_fuse(residual: torch.Tensor, dtype: torch.dtype, *weights: torch.Tensor)
 
 def linear_into_stream(x: torch.Tensor, weight: torch.Tensor, ctx) -> torch.Tensor:
     """The last projection of a mixer or feed-forward, whose result the next norm adds to the residual
-    stream.  In bfloat16 and where the model's norms add stacks it is, from 17 rows on, a stack of float32 partial sums over slices of
+    stream (or, where ``ctx.whole_branch`` says so, something that wants it whole: slices then have to make up for the kernel that adds them, or
+    are left alone).  In bfloat16 and where the model's norms add stacks it is, from 17 rows on, a stack of float32 partial sums over slices of
     the inner dimension (the slices fill the chip, the norm adds them in order), by the panels kernel while its blocks fit
     one round of the chip (``dispatch.panels``; where one slice is ahead, beyond the rows that always were 32-bit sums, a
     bfloat16 result) or for the matrices' rows that :func:`dispatch.limits` names by the partial-sums kernel (inner sizes that are no whole stages
@@ -133,7 +134,8 @@ def linear_into_stream(x: torch.Tensor, weight: torch.Tensor, ctx) -> torch.Tens
     lim = dispatch.limits(weight.shape[0], weight.shape[1])
     rows = x.shape[0]
     if ctx.stacked_branches and rows >= dispatch.PANELS_MIN_ROWS and ops.gemm_panels_supports(x, weight):
-        plan, mode = dispatch.panels(rows, weight.shape[0], weight.shape[1], "stream", lim.stacked_from <= rows <= lim.stacked_to)
+        plan, mode = dispatch.panels(rows, weight.shape[0], weight.shape[1], "stream", lim.stacked_from <= rows <= lim.stacked_to,
+                                     whole=getattr(ctx, "whole_branch", False))
         if plan >= 0:
             return ops.gemm_panels(x, weight, plan, mode)
     if (ctx.stacked_branches and x.dtype == torch.bfloat16 and lim.stacked_from > 0
