@@ -415,6 +415,13 @@ static long long panels_blocks(const PanelsShape& s, int M, int N, int mode, int
   return (long long)((M + s.rows - 1) / s.rows) * ((n_out + cols - 1) / cols) * slices;
 }
 
+// Blocks of a product by a shape (and slices) that takes it.
+extern "C" int ullm_gemm_panels_blocks(int M, int N, int mode, int shape, int slices) {
+  if (shape < 0 || shape >= panels_shape_count) return 0;
+  const long long blocks = panels_blocks(panels_shapes[shape], M, N, mode, slices);
+  return blocks < (1LL << 24) ? (int)blocks : 1 << 24;
+}
+
 // Whether a shape and a number of slices take the product: K in whole stages, one at least for every part of it; rows whose ends
 // 32-bit byte offsets reach.
 extern "C" int ullm_gemm_panels_supports(int M, int N, int K, int ldx, int ldw, int mode, int shape, int slices) {

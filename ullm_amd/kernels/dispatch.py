@@ -26,7 +26,9 @@ TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned_gfx
 
 @dataclass(frozen=True)
 class Limits:
-    """Row limits of one weight matrix [columns, inner] (for gate|up: columns = 2 x intermediate)."""
+    """Row limits of one weight matrix [columns, inner] (for gate|up: columns = 2 x intermediate).  From 17 rows on they say which kernel
+    takes a product that the panels kernel (:func:`panels`) does not: inner sizes that are no whole stages of 64, small matrices, the rows
+    of the ``kept`` fields and more blocks than fit a round."""
     # y = x W^T in bfloat16: the few-rows kernel up to ``skinny`` rows, then the rows kernel up to ``rows``
     # (0: never), then the library
     skinny: int = 16
@@ -49,6 +51,11 @@ class Limits:
     # y = x W^T over thousands of rows: the framework's large product (``ops.gemm_tiles``) in these ranges of rows, (first,
     # last) each, where the library's choices fall off (only measured matrices have any)
     tiles: Tuple[Tuple[int, int], ...] = ()
+    # ranges of rows, (first, last) each, that the kernels named above keep because they were measured to be ahead of the panels kernel
+    # there, for the three kinds of product; None: not measured (:func:`_rows_kernel_ahead` answers for the first two)
+    store_kept: Optional[Tuple[Tuple[int, int], ...]] = None
+    silu_kept: Optional[Tuple[Tuple[int, int], ...]] = None
+    stream_kept: Optional[Tuple[Tuple[int, int], ...]] = None
     # 32-bit results (the logits head): the few-rows kernel up to here, then the library
     f32_skinny: int = 16
 
@@ -77,6 +84,7 @@ def _ranges(text: str) -> Tuple[Tuple[int, int], ...]:
     return tuple((int(a), int(b)) for a, b in (r.split("-") for r in text.split()))
 
 
+RANGES = ("tiles", "store_kept", "silu_kept", "stream_kept")          # written as text in the table
 _table: Optional[dict] = None
 
 
@@ -94,7 +102,7 @@ def _load() -> dict:
                 except ValueError:
                     raise ValueError(f"{TABLE_PATH}: key {key!r} is not COLUMNSxINNER") from None
                 base = asdict(default_limits(columns, inner))
-                base.update({k: _ranges(v) if k == "tiles" else int(v) for k, v in entry.items() if k in names})
+                base.update({k: _ranges(v) if k in RANGES else int(v) for k, v in entry.items() if k in names})
                 table[key] = Limits(**base)
         _table = table
     return _table
@@ -130,11 +138,12 @@ def write_entry(columns: int, inner: int, fields_measured: Dict[str, object]) ->
         with open(TABLE_PATH, "r", encoding="utf-8") as f:
             raw = json.load(f)
     entry = raw.setdefault("matrices", {}).setdefault(f"{columns}x{inner}", {})
-    entry.update({k: " ".join(f"{a}-{b}" for a, b in v) if k == "tiles" else int(v) for k, v in fields_measured.items()})
+    entry.update({k: " ".join(f"{a}-{b}" for a, b in v) if k in RANGES else int(v) for k, v in fields_measured.items()})
     with open(TABLE_PATH, "w", encoding="utf-8") as f:
         json.dump(raw, f, indent=1, sort_keys=True)
         f.write("\n")
     _table = None
+    panels.cache_clear()
 
 
 PANELS_STORE, PANELS_GATED, PANELS_FLOAT = 0, 1, 2
@@ -154,6 +163,23 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
     return plan & 0xffff, (plan >> 17) / 8
 
 
+ROWS_AHEAD_ROWS, ROWS_AHEAD_WEIGHTS, ROWS_AHEAD_BLOCKS = 48, (24_000_000, 64_000_000), 230
+
+
+def _rows_kernel_ahead(rows: int, columns: int, inner: int, plan: int, mode: int) -> bool:
+    """Whether the rows kernel, where it is what takes the call, is ahead of the panels kernel's plan in one slice, for matrices that were
+    not measured: those of 24 to 64 M values at up to 48 rows whose plan leaves a tenth of the compute units and more without a block.
+    Such a product is a read of W by the units that have one, while the rows kernel gives every unit as many columns (us, the
+    rows kernel and this: 5120 x 5120 at 17 / 32 / 48 rows 14.2 / 14.9 / 19.2 and 15.8 / 17.7 / 20.8, with an activation 10240 x 2560 at 36 / 48
+    14.5 / 15.6 and 16.5 / 17.3, 11008 x 4096 21.5 / 21.4 and 24.4 / 23.4, 12288 x 3072 18.3 / 18.0 and 19.5 / 19.6; gate|up 19456 x 2560 20.5 /
+    21.2 and 22.4 / 23.2).  Smaller matrices are read in time by fewer units (4096 x 4096 at 40 rows 14.6 and 11.5), larger ones bound by memory
+    either way (gate|up 22016 x 4096 at 48 rows 10 % behind, 16384 x 4096 9 %)."""
+    lim, weight = limits(columns, inner), columns * inner
+    few, most = (lim.silu_skinny, lim.silu_rows) if mode == PANELS_GATED else (lim.skinny, lim.rows)
+    return (few < rows <= min(most, ROWS_AHEAD_ROWS) and ROWS_AHEAD_WEIGHTS[0] <= weight < ROWS_AHEAD_WEIGHTS[1] and plan >> 8 == 1
+            and build.load("gemm_panels").ullm_gemm_panels_blocks(rows, columns, mode, plan & 0xff, 1) < ROWS_AHEAD_BLOCKS)
+
+
 @functools.lru_cache(maxsize=8192)
 def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = False, host_bound: bool = False,
            whole: bool = False) -> Tuple[int, int]:
@@ -169,9 +195,24 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     and 16.8 / 25.7 / 53.3).  In two rounds the library's tiles are ahead (6144 x 4096 at 1300 rows 65 and 83, gate|up 24576 x 4096 at 320
     79 and 87), and from 1025 rows on also in one (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 / 24.1, 2048 x 2048 at 2048 / 3000
     21.0 / 26.5 and 23.0 / 27.6; inside a prompt of 1064 rows 6144 x 4096 59 and 63, 4096 x 4096 and 4096 x 12288 183 and 189 together,
-    the prompt 17.9 and 18.4 ms; level at 2048), where ``host_bound`` does not say that launches are what takes the time."""
+    the prompt 17.9 and 18.4 ms; level at 2048).  Rows for which the kernels that took the calls before were measured to be ahead, or
+    for matrices that were not measured are expected to be (:func:`_rows_kernel_ahead`), are left to them.  Neither holds where ``host_bound``
+    says that launches are what takes the time."""
     if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and not host_bound):
         return -1, 0
+    plan, mode = _panels_of_role(rows, columns, inner, role, keep_sums, whole)
+    if plan < 0 or host_bound or role == "float":
+        return plan, mode
+    kept = getattr(limits(columns, inner), {"gated": "silu_kept", "stream": "stream_kept"}.get(role, "store_kept"))
+    if any(first <= rows <= last for first, last in kept or ()):
+        return -1, 0
+    if kept is None and role != "stream" and mode != PANELS_FLOAT and _rows_kernel_ahead(rows, columns, inner, plan, mode):
+        return -1, 0
+    return plan, mode
+
+
+def _panels_of_role(rows: int, columns: int, inner: int, role: str, keep_sums: bool, whole: bool) -> Tuple[int, int]:
+    """The panels kernel's fastest plan for a role, and its mode."""
     if role == "float":
         # logits heads are read once at these rows, in however many rounds (library and this: 151936 x 4096 at 17 / 64 / 128 rows 266 / 270 /
         # 290 and 192 / 223 / 268, 151936 x 1024 at 101 91 and 81, 32768 x 2048 at 48 / 256 37 / 46 and 25 / 41); smaller matrices go to the

@@ -159,7 +159,8 @@ def projection(args) -> None:
 
 
 LARGE_ROWS = list(range(4096, 16385, 64))
-TUNE_ROWS = [1, 4, 8, 9, 12, 16, 17, 24, 32, 33, 48, 64, 65, 96, 128, 192, 256]
+TUNE_ROWS = [1, 4, 8, 9, 12, 16, 17, 24, 32, 33, 40, 48, 56, 64, 65, 80, 96, 112, 128, 160, 192, 224, 256]
+KEPT_ROWS = list(range(288, 513, 32)) + list(range(576, 1025, 64))          # above them the panels kernel against the library alone
 
 
 def _ahead_up_to(rows, mine, others, start=0):
@@ -183,11 +184,11 @@ def _ahead_up_to(rows, mine, others, start=0):
 
 
 def _ahead_ranges(rows, mine, other):
-    """The ranges of rows, (first, last) each, over which ``mine`` was at least 3 % ahead of ``other`` at two or more measured row
-    counts in a row.  A library's choices change from one row count to the next and back: what it loses here says nothing of
+    """The ranges of rows, (first, last) each, over which ``mine`` was at least 3 % ahead of ``other`` at two or more row counts in a
+    row that have a time of ``other``.  A library's choices change from one row count to the next and back: what it loses here says nothing of
     what it loses there.  Between two measured counts it does what it does at the larger (kernels round rows up to tiles)."""
     ranges, before, run = [], 0, 0
-    for r in sorted(rows):
+    for r in sorted(r for r in rows if r in other):
         run = run + 1 if r in mine and mine[r] <= 0.97 * other.get(r, 0.0) else 0
         if run == 1:
             first = before + 1 if before else r
@@ -197,6 +198,13 @@ def _ahead_ranges(rows, mine, other):
             ranges[-1][1] = r
         before = r
     return ranges
+
+
+def _kept_ranges(rows, panels, few, few_to, beyond):
+    """The ranges over which the kernels that take a product without the panels kernel were ahead of it: ``few`` up to ``few_to`` rows,
+    then the fastest of ``beyond``."""
+    before = {r: few[r] if r <= few_to and r in few else min((t[r] for t in beyond if r in t), default=float("inf")) for r in rows}
+    return _ahead_ranges(rows, before, panels)
 
 
 def derive_limits(times: dict, roles, columns: int, inner: int) -> dict:
@@ -215,13 +223,20 @@ def derive_limits(times: dict, roles, columns: int, inner: int) -> dict:
         changes["fold_norm"] = _ahead_up_to(rows, get("skinny+norm"), [unfolded])
         # above the rows the weight-streaming kernels take: partial sums and the kernel that adds them, against the library
         taken = max(changes["skinny"], changes["rows"])
-        upto = _ahead_up_to(rows, get("partial sums>sum"), [get("library"), get("panels")], start=taken)
+        upto = _ahead_up_to(rows, get("partial sums>sum"), [get("library")], start=taken)
         changes["sums_from"], changes["sums_to"] = (taken + 1, upto) if upto > taken else (0, 0)
+        if get("panels"):
+            sums = {r: t for r, t in get("partial sums>sum").items() if taken < r <= upto}
+            changes["store_kept"] = _kept_ranges(rows, get("panels"), get("rows"), changes["rows"], [sums] if sums else [get("library")])
     if "silu" in roles:
         changes["silu_skinny"] = _ahead_up_to(rows, get("skinny+silu"), [get("rows+silu"), get("library+silu")])
         changes["silu_rows"] = _ahead_up_to(rows, get("rows+silu"), [get("library+silu")], start=changes["silu_skinny"])
         if changes["silu_rows"] == changes["silu_skinny"]:
             changes["silu_rows"] = 0
+        if get("panels+silu"):
+            few = {r: get("skinny+silu" if r <= changes["silu_skinny"] else "rows+silu").get(r, float("inf")) for r in rows}
+            changes["silu_kept"] = _kept_ranges(rows, get("panels+silu"), few, max(changes["silu_skinny"], changes["silu_rows"]),
+                                                [get("library+silu")])
         best = {r: min(t[r] for t in (get("skinny+silu"), get("rows+silu"), get("library+silu")) if r in t) for r in rows}
         unfolded = {r: best[r] + get("norm")[r] for r in rows if r in get("norm")}
         changes["fold_norm"] = _ahead_up_to(rows, get("skinny+norm+silu"), [unfolded])
@@ -229,6 +244,8 @@ def derive_limits(times: dict, roles, columns: int, inner: int) -> dict:
         # up to 16 rows the few-rows kernel adds into the stream itself; the stacks serve the rows after that
         upto = _ahead_up_to(rows, get("partial sums>norm"), [get("library>norm")], start=16)
         changes["stacked_from"], changes["stacked_to"] = (17, upto) if upto > 16 else (0, 0)
+        if get("panels>norm"):
+            changes["stream_kept"] = _kept_ranges(rows, get("panels>norm"), get("partial sums>norm"), upto, [get("library>norm")])
     if "large" in roles:
         changes["tiles"] = _ahead_ranges(rows, get("tiles"), get("library many"))
     if "logits" in roles:
@@ -280,7 +297,13 @@ def tune(args) -> None:
         times.setdefault("library many", {})[M], times.setdefault("tiles", {})[M] = round(lib, 2), round(own, 2)
         print(f"rows {M}: library {lib:.1f}  tiles {own:.1f}  ({own / lib:.3f})", flush=True)
     roles = {"large" if r == "large-f32" else r for r in roles}
-    for M in TUNE_ROWS if roles - {"large"} else []:
+    def panels(name, role, x, make, **more):
+        """The panels kernel by its own plan, whatever the table says so far."""
+        plan, mode = dispatch.panels(x.shape[0], N, K, role, host_bound=True, **more) if x.shape[0] <= 1024 else (-1, 0)
+        if plan >= 0 and ops.gemm_panels_supports(x, ws[0]):
+            timed(name, x.shape[0], lambda v: make(lambda: ops.gemm_panels(x, ws[v], plan, mode), mode))
+
+    for M in TUNE_ROWS + (KEPT_ROWS if roles & {"store", "silu", "stream"} else []) if roles - {"large"} else []:
         x = torch.randn(M, K, device=DEV).bfloat16()
         stream = torch.randn(M, K, device=DEV)
         skinny_ok = ops.gemm_skinny_supports(x, ws[0])
@@ -295,9 +318,7 @@ def tune(args) -> None:
                 timed("skinny+norm", M, lambda v: (lambda: ops.gemm_skinny_normed(stream, gain, 1e-6, ws[v])))
             if M <= ops.ROWS_MAX_ROWS and ops.gemm_rows_supports(x, ws[0]):
                 timed("rows", M, lambda v: (lambda: ops.gemm_rows(x, ws[v])))
-            plan, mode = dispatch.panels(M, N, K, "store")
-            if plan >= 0 and ops.gemm_panels_supports(x, ws[0]):
-                timed("panels", M, lambda v: (lambda: ops.gemm_bf16(x, ws[v])))
+            panels("panels", "store", x, lambda f, mode: (lambda: ops.sum_stacks(f())) if mode == dispatch.PANELS_FLOAT else f)
             if M > 16 and N % 4 == 0 and ops.gemm_partial_sums_supports(x, ws[0]):
                 timed("partial sums>sum", M, lambda v: (lambda: ops.sum_stacks(ops.gemm_partial_sums(x, ws[v]))))
         if "silu" in roles:
@@ -308,6 +329,7 @@ def tune(args) -> None:
                 timed("skinny+norm+silu", M, lambda v: (lambda: ops.gemm_skinny_normed(stream, gain, 1e-6, ws[v], silu=True)))
             if M <= ops.ROWS_MAX_ROWS and ops.gemm_rows_supports(x, ws[0], silu=True):
                 timed("rows+silu", M, lambda v: (lambda: ops.gemm_rows(x, ws[v], silu=True)))
+            panels("panels+silu", "gated", x, lambda f, mode: f)
         if "stream" in roles:
             resid = torch.zeros(M, N, device=DEV)
             gain_n = torch.ones(N, device=DEV)
@@ -317,6 +339,9 @@ def tune(args) -> None:
             if ops.gemm_partial_sums_supports(x, ws[0]):
                 timed("partial sums>norm", M, lambda v: (lambda: ops.add_rmsnorm(ops.gemm_partial_sums(x, ws[v]), resid, gain_n, 1e-6,
                                                                                  torch.bfloat16)))
+            lim = dispatch.limits(N, K)
+            panels("panels>norm", "stream", x, lambda f, mode: (lambda: ops.add_rmsnorm(f(), resid, gain_n, 1e-6, torch.bfloat16)),
+                   keep_sums=lim.stacked_from <= M <= lim.stacked_to)
         if "logits" in roles:
             timed("library f32", M, lambda v: (lambda: torch.mm(x, ws[v].t(), out_dtype=torch.float32)))
             if skinny_ok and M <= 64:

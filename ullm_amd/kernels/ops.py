@@ -1332,8 +1332,8 @@ _MM_TAKES_OUT_DTYPE = "out_dtype" in (torch.mm.__doc__ or "")
 
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
               out_dtype: Optional[torch.dtype] = None, act: Optional[int] = None) -> torch.Tensor:
-    """bfloat16 operands, 32-bit accumulation.  Up to 16 rows go to the weight-streaming kernels, up to one or two thousand, as
-    the matrix has it, to the panels kernel (:func:`dispatch.panels`; not where a matrix's limits name rows for the partial-sums kernel).  What it does not take goes, up to how many rows
+    """bfloat16 operands, 32-bit accumulation.  Up to 16 rows go to the weight-streaming kernels, up to 1024, as
+    the matrix has it, to the panels kernel (:func:`dispatch.panels`).  What it does not take goes, up to how many rows
     for this matrix :func:`dispatch.limits` says, to the weight-streaming kernels, some more, where that was measured to be ahead, to the partial-sums
     kernel and a kernel that adds its stacks; thousands of rows, where the library's choice for them was measured to
     fall off, go to the large product (:func:`gemm_tiles`); the rest go through the library product (as the reference's
@@ -1342,8 +1342,7 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = N
     kernels (then without slices), by the activation kernel behind the others."""
     out_dtype = out_dtype or a.dtype
     M = a.shape[0]
-    if (out_dtype == torch.bfloat16 and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w)
-            and not dispatch.limits(w.shape[0], w.shape[1]).sums_from):
+    if out_dtype == torch.bfloat16 and M >= dispatch.PANELS_MIN_ROWS and gemm_panels_supports(a, w):
         plan, mode = dispatch.panels(M, w.shape[0], w.shape[1], "store" if act is None else "activated")
         if plan >= 0 and mode == dispatch.PANELS_STORE:
             return gemm_panels(a, w, plan, mode, bias, act=act)

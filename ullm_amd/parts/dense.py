@@ -3,7 +3,7 @@
 A step of few tokens is bound by the host: a layer's ten launches cost the interpreter more than its kernels take (0.6B: 160 us,
 and 60 us of kernels at 300 tokens).  What a part's ``forward`` decides from sizes alone is decided here once for all layers, and the
 launches go out from one call (``kernels/dense.py``).  The kernels, their order and so the results are those of the blocks'
-own ``forward`` (but for products that are not worth the library's launch here), which takes whatever this does not: float32, steps of single tokens (captured graphs, mostly), up to 16 rows
+own ``forward`` (but for products that are not worth the library's launch, or a kernel for few rows, here), which takes whatever this does not: float32, steps of single tokens (captured graphs, mostly), up to 16 rows
 (the folded kernels), products that the library is ahead for (their kernels then take longer than the host) and parts of
 any other kind.
 """
@@ -61,12 +61,11 @@ HOST_BOUND = 19_000_000_000
 
 def _product(rows: int, columns: int, inner: int, role: str, host_bound: bool) -> Optional[dense.Product]:
     """The framework's own product that the parts' ``linear``, ``gate_up`` and ``linear_into_stream`` would take, if it is one for
-    many rows; with ``host_bound`` also one that the library's is ahead of."""
+    many rows; with ``host_bound`` also one that another kernel is ahead of."""
     lim = dispatch.limits(columns, inner)
-    if not (role == "store" and lim.sums_from):
-        plan, mode = dispatch.panels(rows, columns, inner, role, role == "stream" and lim.stacked_from <= rows <= lim.stacked_to, host_bound)
-        if plan >= 0:
-            return dense.Product(0, mode, plan & 0xff, plan >> 8)
+    plan, mode = dispatch.panels(rows, columns, inner, role, role == "stream" and lim.stacked_from <= rows <= lim.stacked_to, host_bound)
+    if plan >= 0:
+        return dense.Product(0, mode, plan & 0xff, plan >> 8)
     if role == "gated":
         groups = dispatch.gated_tile_groups(rows, columns, inner)
         return dense.Product(1, ops.TILES_GATED, groups, 1) if groups and rows > max(lim.silu_skinny, lim.silu_rows) else None
