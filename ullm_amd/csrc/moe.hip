@@ -988,9 +988,9 @@ moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
   if (rows <= 0) return;
 #define TILE(...) moe_products_tile<__VA_ARGS__, GATED>(tile_stages, x, ldx, row_index, w, e, slot0, rows, n0, out, ldo, n_out, K, limit, alpha)
   if constexpr (WMW == 4) {
-    if (rows <= 64) return TILE(ProductTiles<1, 3, 8>);
+    if (rows <= 64) return TILE(ProductTiles<1, 3, 8, true>);
   }
-  TILE(ProductTiles<WMW, STAGES>);
+  TILE(ProductTiles<WMW, STAGES, 2, true>);
 #undef TILE
 }
 
