@@ -8,6 +8,7 @@ import torch
 DEV = "cuda:0"
 # width, heads, kv heads, head size, inner size, bias, window
 SIZES = {"plain": (1024, 8, 4, 128, 1024, False, 0), "wide": (1024, 16, 8, 128, 3072, True, 0), "window": (2048, 8, 8, 64, 1024, True, 40)}
+LARGE = (4096, 32, 8, 128, 12288, True, 0)
 
 
 def test_the_structures_agree():
@@ -39,7 +40,7 @@ def _runner(size, seed):
     from ullm_amd.engine.runner import ModelRunner
     from ullm_amd.models import build_model
     from ullm_amd.weights.random_init import bind_random_weights
-    H, nq, nkv, hd, inner, bias, window = SIZES[size]
+    H, nq, nkv, hd, inner, bias, window = LARGE if size == "large" else SIZES[size]
     cfg = dict(architectures=["Qwen3ForCausalLM"], hidden_size=H, num_hidden_layers=3, num_attention_heads=nq, num_key_value_heads=nkv,
                head_dim=hd, intermediate_size=inner, vocab_size=512, rope_theta=10000.0, rms_norm_eps=1e-6, max_position_embeddings=4096,
                tie_word_embeddings=False, attention_bias=bias, use_sliding_window=window > 0, sliding_window=window or None,
@@ -93,16 +94,64 @@ def test_the_blocks_bits(size, monkeypatch):
         assert torch.equal(a, b)
 
 
+def _logits(runner, *steps):
+    """The last tokens' logits of steps of as many tokens for one request each."""
+    from ullm_amd.engine.runner import StepEntry
+    cache, out, entries = runner.cache, [], []
+    for counts in steps:
+        entries = [StepEntry(cache.admit(f"r{i}"), [(13 * j + i) % 512 for j in range(n)], [n - 1]) for i, n in enumerate(counts)]
+        assert all(cache.reserve(e.cache, len(e.tokens)) for e in entries)
+        out.append(runner.step(entries).clone())
+        for e in entries:
+            cache.release(e.cache)
+    return out
+
+
+@pytest.mark.gpu
+def test_the_blocks_bits_by_every_way_of_the_products(monkeypatch):
+    """A width of 4096 with biases: q|k|v in slices that a kernel adds with the bias, gate|up by the large tiles beside panels, all four
+    products by the large tiles."""
+    from ullm_amd.kernels import dense
+    from ullm_amd.models import model as models
+    ways, real = [], dense.dense_layers
+    monkeypatch.setattr(dense, "dense_layers", lambda step, layers: ways.append([(p.tiles, p.mode) for p in (
+        step.into, step.out, step.gate_up, step.down)]) or real(step, layers))
+    steps = ([90, 40], [512], [2040] * 4 + [200])
+    got = _logits(_runner("large", 6), *steps)
+    store, gated, sums = ((0, mode) for mode in range(3))
+    assert ways == [[sums, sums, gated, sums], [store, sums, (1, 1), sums], [(1, 0), (1, 0), (1, 1), (1, 0)]]
+    monkeypatch.setattr(models, "run_layers", lambda *a: None)
+    for a, b in zip(got, _logits(_runner("large", 6), *steps)):
+        assert torch.isfinite(b).all() and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_launches_that_take_longer_than_the_products(monkeypatch):
+    """Steps of 1025 to about 1200 rows of a small width take panels that the blocks leave to the library: not its bits, so against the
+    blocks' with the roundings of three layers of bfloat16 between them (2^-9 each of q|k|v, heads, activation, branch: a dozen of 2^-9
+    at most add up to 2.4 %, by chance 0.7 %)."""
+    from ullm_amd.kernels import dense
+    from ullm_amd.models import model as models
+    rows, real = [], dense.dense_layers
+    monkeypatch.setattr(dense, "dense_layers", lambda step, layers: rows.append((step.tokens, step.into.tiles)) or real(step, layers))
+    steps = ([1025], [700, 500])
+    got = _logits(_runner("wide", 7), *steps)
+    assert rows == [(1025, 0), (1200, 0)]
+    monkeypatch.setattr(models, "run_layers", lambda *a: None)
+    for a, b in zip(got, _logits(_runner("wide", 7), *steps)):
+        assert (a - b).norm() <= 2.4e-2 * b.norm()
+
+
 @pytest.mark.gpu
 def test_what_is_left_to_the_blocks(monkeypatch):
-    """16 rows, single tokens, float32 sums not wanted, a matrix that lies off 16 bytes: the blocks' own forward passes."""
+    """16 rows, single tokens, a step whose branches are not to come as sums, a matrix that lies off 16 bytes: the blocks' own forward passes."""
     from ullm_amd.engine.runner import StepEntry
     from ullm_amd.kernels import dense
     calls, real = [], dense.dense_layers
     monkeypatch.setattr(dense, "dense_layers", lambda step, layers: calls.append(step.tokens) or real(step, layers))
     runner = _runner("plain", 3)
     cache = runner.cache
-    rcs = [cache.admit(f"r{i}") for i in range(4)]
+    rcs = [cache.admit(f"r{i}") for i in range(5)]
 
     def step(*counts):
         entries = [StepEntry(rc, [7] * n, [n - 1]) for rc, n in zip(rcs, counts) if n]
@@ -111,6 +160,10 @@ def test_what_is_left_to_the_blocks(monkeypatch):
     step(16)
     step(1, 0, 0, 0)
     assert not calls
+    runner._stacked_branches = False
+    step(0, 0, 0, 0, 40)
+    assert not calls
+    runner._stacked_branches = True
     step(0, 40)
     assert calls == [40]
     mixer = runner.model.blocks[1].mixer

@@ -78,6 +78,39 @@ def test_every_way_of_the_launch(ops, entries, nq, nkv, window, extras):
         assert torch.isnan(out.float().cpu()[~rows]).all()
 
 
+@pytest.mark.parametrize("window,gated", [(0, False), (0, True), (16700, False)])
+def test_more_keys_than_the_page_ids_in_shared_memory(ops, window, gated):
+    """Every part of the keys has the page ids of 128 tiles (4096 keys) at hand and refills them on the way: with 17 001 keys all of the
+    ways do, the quarters with their two tiles in turn from the 129th of their 132 or 133 steps on.  Every query looks at one key beside
+    a part's first or a refill's (its score there is about 128 / 2, elsewhere 60 / 2 at most)."""
+    S, n, nq, nkv, hd, P, scale = 17001, 94, 2, 1, 128, 16, 0.5
+    g = torch.Generator().manual_seed(7 + window)
+    k, v = (torch.randn(S, nkv, hd, generator=g).bfloat16().float() for _ in range(2))
+    begin = max(0, S - n - window + 1) // 32 * 32 if window else 0           # of the first tile's keys
+    seams = set()
+    for parts in (1, 2, 4):
+        share = -(-(-(-(S - begin) // 32)) // parts) * 32
+        for first in range(begin, S, share):
+            seams |= {first + at + by for at in range(0, share, 4096) for by in (-1, 0, 31, 32)}
+    seams = sorted(t for t in seams if (S - window if window else 0) <= t <= S - n)       # those that every query sees
+    assert 40 < len(seams) <= n * nq // 3
+    at = torch.tensor((seams * 5)[:n * nq])                                  # each by queries of three waves at least
+    q = k[at, 0].view(n, nq, hd).bfloat16()
+    k_pool, v_pool, tables = paged_cache([k], [v], P, torch.bfloat16, DEV)
+    tiles, wide = (torch.tensor([x for f in range(0, n, size) for x in (f, min(size, n - f))], dtype=torch.int32, device=DEV)
+                   for size in (ops.PREFILL_TILE, 2 * ops.PREFILL_TILE))
+    want = _attention(q, k, v, window, scale)
+    gate = torch.randn(n, nq, generator=g).bfloat16()
+    if gated:
+        want = (want.view(n, nq, hd) * torch.sigmoid(gate.double())[:, :, None]).view(n, -1)
+    for way in (0, 1, 2, 3, 4, 5):
+        out = torch.full((n, nq * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.attention_prefill_mfma(q.view(n, -1).to(DEV), out, k_pool, v_pool, tiles, len(tiles) // 2, torch.arange(S - n, S).int().to(DEV),
+                                   torch.zeros(n, dtype=torch.int32, device=DEV), table_tensor(tables, DEV), P, nq, nkv, hd, scale, window, halves=way,
+                                   wide_tiles=wide, n_wide=len(wide) // 2, gate=gate.to(DEV) if gated else None)
+        assert (out.float().cpu() - want.float()).abs().max() <= tol(torch.bfloat16, want), way
+
+
 def test_ways_that_other_groups_do_not_have(ops):
     """Wide tiles and quarters are for groups of at most two heads of size 128."""
     nq, nkv, hd, P = 8, 2, 128, 16
