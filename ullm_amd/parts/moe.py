@@ -92,7 +92,7 @@ def tile_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int 
     19 / 17 / 19 / 26 / 35, 38 / 30 / 20 / 29 / 39, - / - / 21 / 30 / 41, - / - / 29 / 32 / 45, - / - / 56 / 61 / 51; 8 experts, width 4096, 1536
     columns at 24, 36, 128, 320 106 / 68 / 71 / 87 / 125, 146 / 110 / 71 / 90 / 127, - / - / 116 / 102 / 133, - / - / 231 / 168 / 150.
     A prompt of 440 tokens of a stack with six such layer runs took 2.42 ms in tiles of 64, 2.37 in tiles of 128.  (Tiles of 128 and 256
-    have become faster since, where the experts' matrices come from memory by up to a quarter: :func:`product_rows_for`.)"""
+    have become faster since, where the experts' matrices come from memory, by up to a quarter: :func:`product_rows_for`.)"""
     mean = tokens * top / max(1, experts)
     if (mean > 0 and experts > 0 and hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
             and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31):
@@ -105,21 +105,34 @@ def tile_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int 
 
 
 def product_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: int = 0) -> int:
-    """Grouped rows a block of the expert products takes: up to 256, a tile of 64 rows or less at its own cost, where the experts'
-    first tiles alone make about a round of blocks over 256 compute units and most experts' last tiles are short or long, else what
-    :func:`tile_rows_for` says.
+    """Grouped rows a block of the expert products takes: what :func:`tile_rows_for` says, but where its figures for tiles of 128 and
+    256 rows are behind the kernels'.
 
-    That kernel reads the matrices at 5.5 TB/s whatever the rows, so it is ahead from few rows on (us of gate|up + down,
-    the best of the tiles of 16 to 128 rows and this: 32 experts, width 2048, 1024 columns at means of 12, 18, 36, 50, 100, 137, 187, 256 and
-    500 73 / 70, 81 / 71, 77 / 73, 84 / 75, 93 / 105, 123 / 114, 132 / 115, 173 / 143, 287 / 236; 64 experts of 768 columns at 12, 18, 48, 512 107 / 113,
-    118 / 114, 130 / 123, 432 / 393; 16 experts, width 5120, 1536 columns at 12, 18, 512 137 / 144, 148 / 144, 544 / 443; 128 experts,
-    width 1024, 512 columns at 24, 48, 512 79 / 81, 91 / 91, 325 / 293).  With fewer blocks a tile of 256 rows leaves
-    most units idle (8 experts, width 4096, 1536 columns at 128 / 288 97 / 131, 158 / 150)."""
+    From 20 rows an expert on tiles of 128 in place of 32 and 64, where the rows of the matrices are long enough that blocks in step got
+    in each other's way (width 2048 and more) and the gate|up of the experts' first tiles fills every compute unit.  us of gate|up +
+    down, the smaller tiles and 128, for routings by chance / unequal experts / very unequal ones: 32 experts, width 2048, 1024 columns at a mean of
+    36 92 / 97 / 89 and 80 / 85 / 77, at 20 79 / 94 / 92 and 78 / 79 / 63; 64 experts of 768 columns at 20 118 / 142 / 133 and 125 / 124 / 110, at 42
+    140 / 145 / 127 and 134 / 136 / 122.  Not with fewer blocks or shorter rows (24 experts, width 3072, 1024 columns 1.04 of it, 40 of width 1536 1.13).
+
+    From 250 on tiles of 256, whose blocks take a last tile of 64 rows or less at its own cost, where the experts' first tiles make
+    about a round of blocks in each product (256 rows, 128 and 256: 16 experts, width 5120, 1536 columns 322 / 317 / 311 and 274 / 312 / 317; 32
+    experts, width 2048, 1024 columns 176 / 170 / 176 and 158 / 183 / 182; 48 experts, width 1024, 1024 columns 135 / 134 / 131 and 120 / 141 / 121).  With fewer
+    rows they are ahead only while every expert's last tile is short or long, as none is that is not routed to by chance alone: at
+    30 to 55 rows 0.84 to 1.05 of the time of 64 by chance and 0.92 to 1.32 where experts are unequal (16 experts of 1536
+    columns, 36 rows 159 / 161 / 161 and 153 / 198 / 197), at 106 to 120 of 128 1.05 to 1.26.  With fewer blocks they leave most units
+    idle (8 experts, width 4096, 1536 columns 125 / 120 / 124 and 151 / 142 / 148).
+
+    Over sixteen shapes (8 to 256 experts, width 512 to 5120) and 2 to 750 rows an expert 0.995 / 0.991 / 0.988 of the time by
+    :func:`tile_rows_for` alone."""
     rows = tile_rows_for(tokens, top, experts, hidden, ff)
     mean = tokens * top / max(1, experts)
-    if (mean >= max(16, 40 * 1024 / max(1, hidden)) and not 56 <= mean <= 104 and hidden > 0 and hidden % 64 == 0 and ff > 0 and ff % 64 == 0
-            and experts * (-(-ff // 128) - (-hidden // 256)) >= 460
-            and (tokens * top + 256 * experts) * max(hidden, ff) < 2 ** 31 and 2 * hidden * ff < 2 ** 31):
+    if (hidden <= 0 or hidden % 64 or ff <= 0 or ff % 64 or (tokens * top + 256 * experts) * max(hidden, ff) >= 2 ** 31
+            or 2 * hidden * ff >= 2 ** 31):
+        return rows
+    first_up, first_down = experts * -(-ff // 128), experts * -(-hidden // 256)          # blocks of the experts' first tiles
+    if mean >= 20 and rows < 128 and hidden >= 2048 and first_up >= 256:
+        return 128
+    if mean >= 250 and first_up + first_down >= 460:
         return 256
     return rows
 
