@@ -39,8 +39,9 @@ __device__ __forceinline__ uint4 pair_columns(const uint2& a, const uint2& b) {
 }
 __device__ __forceinline__ int pair_column(int g) { return 16 * (g & 1) + 4 * (g & 2); }
 
-template <int WMW, int STAGES_, int WN = 2, bool TURNED = false>
+template <int WMW, int STAGES_, int WN = 2, bool TURNED_ = false>
 struct ProductTiles {
+  static constexpr bool TURNED = TURNED_;
   static constexpr int WAVES = WN * WMW, BM = 64 * WMW, BN = 256, STAGES = STAGES_, STAGE = (BM + BN) * 128;
   static_assert(WAVES == 4 || WAVES == 8, "whole pieces of x and of W a wave");
   static constexpr int XL = 8 / WN, WL = 32 / WAVES, LOADS = XL + WL, TM = 4, TN = 16 / WN, STRIP = TN / 2;

@@ -827,7 +827,7 @@ moe_tiles_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restri
 // shared memory a product, and prompts of 3000 tokens in 4.29 ms instead of 4.27.)
 // What bounds it: the experts' matrices from memory (268 MB of gate|up: 45 us) and, beside them, the matrix pipe, which the
 // loop keeps busy 57 % of the time where every operand lies in the second-level cache.  Rows of the matrices lie a power of two apart, and
-// blocks in step ask the same memory channels: so a block's K begins at the stage of its expert's number (32 experts, width 2048, 1024
+// blocks in step ask the same memory channels: so a block's K begins at the stage of its expert's number (where K is TURNED_K and more; 32 experts, width 2048, 1024
 // columns, gate|up + down at 400 / 800 tokens, top 4, 71 + 26 / 73 + 35 -> 50 + 27 / 52 + 40 us; the stage by the columns too, 51 + 27 / 54 + 38,
 // leaves less to share between the blocks of a tile: 1500 tokens 69 + 49 and 67 + 45).
 // All of it together, us before and now of what takes the call: 400 / 800 / 1100 / 1500 / 2048 / 2500 / 3000 / 4000 / 8000 tokens 98 / 107 / 119 / 125 /
@@ -858,7 +858,7 @@ __device__ __forceinline__ void moe_products_tile(unsigned char* stages, const b
   }
   tile_f32x4 acc[T::TN][T::TM];
   T::run(stages, reinterpret_cast<const char*>(x), xoff, reinterpret_cast<const char*>(w + (size_t)e * w_rows * K), woff,
-         K >> 6, (int)((unsigned)e % (unsigned)(K >> 6)), wave, lane, 128, acc);
+         K >> 6, T::TURNED ? (int)((unsigned)e % (unsigned)(K >> 6)) : 0, wave, lane, 128, acc);
   // lane (r, g): row r of each 16-row group, four consecutive columns at 4g
   const int wm = wave / WN, wn = wave % WN;
   const bool whole = ((n_out | ldo) & (GATED ? 7 : 3)) == 0 && !((uintptr_t)out_ & 15);
@@ -974,7 +974,7 @@ __device__ __forceinline__ int tile_by_rows(const int* __restrict__ tiles, int n
   return -1;
 }
 
-template <int WMW, int STAGES, bool GATED>
+template <int WMW, int STAGES, bool GATED, bool TURNED>
 __global__ void __launch_bounds__(128 * WMW)
 moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict__ row_index,
                     const bf16_t* __restrict__ w, const int* __restrict__ tiles, int n_tiles, int n_col_blocks,
@@ -988,9 +988,9 @@ moe_products_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restrict
   if (rows <= 0) return;
 #define TILE(...) moe_products_tile<__VA_ARGS__, GATED>(tile_stages, x, ldx, row_index, w, e, slot0, rows, n0, out, ldo, n_out, K, limit, alpha)
   if constexpr (WMW == 4) {
-    if (rows <= 64) return TILE(ProductTiles<1, 3, 8, true>);
+    if (rows <= 64) return TILE(ProductTiles<1, 3, 8, TURNED>);
   }
-  TILE(ProductTiles<WMW, STAGES, 2, true>);
+  TILE(ProductTiles<WMW, STAGES, 2, TURNED>);
 #undef TILE
 }
 
@@ -1015,14 +1015,18 @@ static void launch_rows_dma(dim3 grid, hipStream_t stream, Args... args) {
   hipLaunchKernelGGL((moe_rows_dma_kernel<MT, GATED>), grid, dim3(256), bytes, stream, args...);
 }
 
-template <int WMW, int STAGES, bool GATED, typename... Args>
+// Experts begin K at different stages from this K on, whatever the tile (a row's sums do not depend on the rows beside it): us of gate|up + down from one stage and so, 32 experts, width 2048, 1024 columns
+// 24 / 80 / 220 rows an expert 98 / 108 / 143 and 80 / 87 / 134, 16 experts of them 56 / 64 / 71 and 51 / 60 / 67; with both products' rows shorter
+// they were slower so (64 experts, width 1024, 768 columns 71 / 82 / 139 and 75 / 84 / 145, 40 experts, width 1536 93 / 102 / 145 and 96 / 106 / 148).
+#define TURNED_K 2048
+template <int WMW, int STAGES, bool GATED, bool TURNED, typename... Args>
 static void launch_products(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int bytes = ProductTiles<WMW, STAGES>::BYTES;
   static_assert(WMW != 4 || bytes >= ProductTiles<1, 3, 8>::BYTES, "the largest of a launch's");
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)moe_products_kernel<WMW, STAGES, GATED>,
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)moe_products_kernel<WMW, STAGES, GATED, TURNED>,
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   (void)allowed;
-  hipLaunchKernelGGL((moe_products_kernel<WMW, STAGES, GATED>), grid, dim3(128 * WMW), bytes, stream, args...);
+  hipLaunchKernelGGL((moe_products_kernel<WMW, STAGES, GATED, TURNED>), grid, dim3(128 * WMW), bytes, stream, args...);
 }
 
 // out[slot] = glu(x[row_index[slot]] Wg^T, x Wu^T) (gated: out in x's dtype, w [experts, 2 n_out, K]) or
@@ -1041,10 +1045,15 @@ extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const
       const long long total = (long long)max_tiles * col_blocks;
       if (total > 0x3fffffffLL) return ULLM_ERR_SHAPE;
       dim3 grid((unsigned)(8 * ((total + 7) / 8 + (tile_rows == 256 ? 1 : 0))));   // two eighths, each rounded up
-#define TILES(W, ST, G) launch_products<W, ST, G>(grid, stream, (const bf16_t*)x, ldx, row_index, (const bf16_t*)w, tiles, max_tiles, \
+#define TILES(W, ST, G, TURNED) launch_products<W, ST, G, TURNED>(grid, stream, (const bf16_t*)x, ldx, row_index, (const bf16_t*)w, tiles, max_tiles, \
     col_blocks, out, ldo, n_out, K, limit, alpha)
-      if (tile_rows == 256) { if (gated) TILES(4, 2, true); else TILES(4, 2, false); }
-      else { if (gated) TILES(2, 3, true); else TILES(2, 3, false); }
+#define TILES_BY(TURNED) do {                                                                                   \
+        if (tile_rows == 256) { if (gated) TILES(4, 2, true, TURNED); else TILES(4, 2, false, TURNED); }         \
+        else { if (gated) TILES(2, 3, true, TURNED); else TILES(2, 3, false, TURNED); }                          \
+      } while (0)
+      if (K >= TURNED_K) TILES_BY(true);
+      else TILES_BY(false);
+#undef TILES_BY
 #undef TILES
       ULLM_LAUNCH_CHECK();
     }

@@ -108,11 +108,10 @@ def product_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: i
     """Grouped rows a block of the expert products takes: what :func:`tile_rows_for` says, but where its figures for tiles of 128 and
     256 rows are behind the kernels'.
 
-    From 20 rows an expert on tiles of 128 in place of 32 and 64, where the rows of the matrices are long enough that blocks in step got
+    From 24 rows an expert on tiles of 128 in place of 32 and 64, where the rows of the matrices are long enough that blocks in step got
     in each other's way (width 2048 and more) and the gate|up of the experts' first tiles fills every compute unit.  us of gate|up +
-    down, the smaller tiles and 128, for routings by chance / unequal experts / very unequal ones: 32 experts, width 2048, 1024 columns at a mean of
-    36 92 / 97 / 89 and 80 / 85 / 77, at 20 79 / 94 / 92 and 78 / 79 / 63; 64 experts of 768 columns at 20 118 / 142 / 133 and 125 / 124 / 110, at 42
-    140 / 145 / 127 and 134 / 136 / 122.  Not with fewer blocks or shorter rows (24 experts, width 3072, 1024 columns 1.04 of it, 40 of width 1536 1.13).
+    down, tiles of 64 and of 128, for routings by chance / unequal experts / very unequal ones: 32 experts, width 2048, 1024 columns at a mean of
+    36 92 / 97 / 89 and 80 / 85 / 77; 64 experts of 768 columns at 42 140 / 145 / 127 and 134 / 136 / 122.  Not with fewer blocks or shorter rows (24 experts, width 3072, 1024 columns 1.04 of it, 40 of width 1536 1.13).
 
     From 250 on tiles of 256, whose blocks take a last tile of 64 rows or less at its own cost, where the experts' first tiles make
     about a round of blocks in each product (256 rows, 128 and 256: 16 experts, width 5120, 1536 columns 322 / 317 / 311 and 274 / 312 / 317; 32
@@ -122,7 +121,7 @@ def product_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: i
     columns, 36 rows 159 / 161 / 161 and 153 / 198 / 197), at 106 to 120 of 128 1.05 to 1.26.  With fewer blocks they leave most units
     idle (8 experts, width 4096, 1536 columns 125 / 120 / 124 and 151 / 142 / 148).
 
-    Over sixteen shapes (8 to 256 experts, width 512 to 5120) and 2 to 750 rows an expert 0.995 / 0.991 / 0.988 of the time by
+    Over sixteen shapes (8 to 256 experts, width 512 to 5120) and 2 to 750 rows an expert 0.995 / 0.993 / 0.992 of the time by
     :func:`tile_rows_for` alone."""
     rows = tile_rows_for(tokens, top, experts, hidden, ff)
     mean = tokens * top / max(1, experts)
@@ -130,7 +129,7 @@ def product_rows_for(tokens: int, top: int, experts: int, hidden: int = 0, ff: i
             or 2 * hidden * ff >= 2 ** 31):
         return rows
     first_up, first_down = experts * -(-ff // 128), experts * -(-hidden // 256)          # blocks of the experts' first tiles
-    if mean >= 20 and rows < 128 and hidden >= 2048 and first_up >= 256:
+    if mean >= 24 and rows < 128 and hidden >= 2048 and first_up >= 256:
         return 128
     if mean >= 250 and first_up + first_down >= 460:
         return 256
