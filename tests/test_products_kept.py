@@ -39,11 +39,15 @@ def test_measured_ranges(table):
 
 
 def test_rows_for_partial_sums_leave_the_others_to_the_panels_kernel(table):
-    """What a table names for the partial-sums kernel is for calls that the panels kernel does not take: it used to be off at every row count."""
-    table({"4096x1024": {"sums_from": 33, "sums_to": 256}})
+    """Rows that a table names for the partial sums stay with them unless they were compared with the panels kernel; the others do not: it
+    used to be off at every row count."""
+    table({"4096x1024": {"sums_from": 33, "sums_to": 256}, "4096x2048": {"sums_from": 33, "sums_to": 256, "store_kept": "33-40"}})
     from ullm_amd.parts.dense import _product
-    for rows in (17, 40, 300):
+    for rows in (17, 32, 257, 300):
         assert _takes(rows, 4096, 1024) and _product(rows, 4096, 1024, "store", False).tiles == 0
+    for rows in (33, 40, 256):
+        assert not _takes(rows, 4096, 1024) and _takes(rows, 4096, 1024, "activated") and _takes(rows, 4096, 1024, "stream")
+    assert [_takes(rows, 4096, 2048) for rows in (32, 33, 40, 41)] == [True, False, False, True]
 
 
 @pytest.mark.parametrize("columns,inner,role,rows", [(5632, 5120, "store", (17, 32, 48)), (10240, 2560, "activated", (40, 48)),

@@ -52,7 +52,8 @@ class Limits:
     # last) each, where the library's choices fall off (only measured matrices have any)
     tiles: Tuple[Tuple[int, int], ...] = ()
     # ranges of rows, (first, last) each, that the kernels named above keep because they were measured to be ahead of the panels kernel
-    # there, for the three kinds of product; None: not measured (:func:`_rows_kernel_ahead` answers for the first two)
+    # there, for the three kinds of product; None: not measured (the rows of ``sums_from`` .. ``sums_to`` then stay with the partial sums,
+    # :func:`_rows_kernel_ahead` answers for the others of the first two kinds)
     store_kept: Optional[Tuple[Tuple[int, int], ...]] = None
     silu_kept: Optional[Tuple[Tuple[int, int], ...]] = None
     stream_kept: Optional[Tuple[Tuple[int, int], ...]] = None
@@ -203,9 +204,12 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     plan, mode = _panels_of_role(rows, columns, inner, role, keep_sums, whole)
     if plan < 0 or host_bound or role == "float":
         return plan, mode
-    kept = getattr(limits(columns, inner), {"gated": "silu_kept", "stream": "stream_kept"}.get(role, "store_kept"))
+    lim = limits(columns, inner)
+    kept = getattr(lim, {"gated": "silu_kept", "stream": "stream_kept"}.get(role, "store_kept"))
     if any(first <= rows <= last for first, last in kept or ()):
         return -1, 0
+    if kept is None and role == "store" and lim.sums_from > 0 and lim.sums_from <= rows <= lim.sums_to:
+        return -1, 0                                       # named for the partial sums, not compared with this kernel
     if kept is None and role != "stream" and mode != PANELS_FLOAT and _rows_kernel_ahead(rows, columns, inner, plan, mode):
         return -1, 0
     return plan, mode
