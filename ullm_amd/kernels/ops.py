@@ -1415,8 +1415,8 @@ def decode_split(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128
     the other, each a round trip to memory, so few (token, kv head) pairs with many keys are cut over
     several blocks, up to one block per compute unit (more would run in a second round), and a second
     small kernel adds the blocks' partial results; that kernel costs about as much as walking eight more
-    tiles, so short contexts are not cut.  A pair of half the compute units' number and more is cut into as many waves as make one
-    a SIMD, two with long contexts; they share a block, which adds their results itself, where there are two or four of them
+    tiles, so short contexts are not cut.  Where there are half as many pairs as compute units and more, a pair is cut into as many waves as make one
+    a SIMD, two to three with long contexts; they share a block, which adds their results itself, where there are two or four of them
     (their number need not be a multiple of the compute units; four waves a block where few pairs have very many keys).
     With a window or a chunk (``window`` < 0) a token reads at most its keys (and up to 31 before them, to the tile's edge),
     however long its context is.  ``units``: the device's compute units, four SIMDs each."""
@@ -1427,25 +1427,33 @@ def decode_split(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128
     if window != 0:
         max_kv = min(max_kv, abs(window) + 31)
     tiles = -(-max_kv // 32)
-    if tiles >= (96 if pairs == units else 64 if 8 * pairs <= 13 * units else 36) and pairs >= units:
-        # two waves a SIMD, also where that takes blocks whose results a second kernel adds: us of 384 / 512 pairs with 8192 keys 232 -> 202 /
-        # 292 -> 264, of 640 421 -> 329, of 800 529 -> 423, of 256 with 4096 82 -> 74
-        n = 2 * simds // pairs
-        return {2: (1, 2), 3: (1, 3), 4: (4, 1)}.get(n) or ((2, 3) if n in (6, 7) else (2, 4))
+    # What follows compares a wave a pair (or two or three single waves, where fewer pairs leave SIMDs idle) with more of them, us for
+    # contexts that are equal / that spread evenly from a tenth of the longest to it, by which most requests in flight are: their
+    # longest ones are what more waves share, while equal ones fill three or four waves a unit as they are
     if pairs > 2 * units:
-        # more than half a wave a SIMD already: three single waves a pair that two a SIMD hold, a second wave in the block only of longer
-        # contexts (576 pairs with 512 keys 31.9 -> 28.8, 640 with 1024 58.3 -> 52.0, 896 with 768 55.6 -> 54.5; 720 with 512 34.2, in
-        # two waves 35.6)
-        if pairs * 3 <= 2 * simds:
-            return (1, 3) if tiles >= 16 else (1, 1)
-        return (2, 1) if tiles >= 24 and pairs * 4 >= 3 * simds else (1, 1)
+        if 3 * pairs <= 2 * simds:
+            # 640 with 512 keys 33 / 29 and (1, 3) 37 / 26, with 1000 61 / 50 and 63 / 41, 2047 0.98 / 0.68 of it; up to 9/4 units against two
+            # waves, 576 with 1000 keys 0.83 / 0.89
+            return (1, 3) if tiles >= (17 if 4 * pairs <= 9 * units else 30) else (1, 1)
+        if pairs <= 3 * units:
+            # three waves a unit read at 6.1 TB/s where they are equal: 736 with 1152 keys 72 / 58 and in four waves a pair 79 / 51, 1400 88 / 69
+            # and 95 / 59, 2047 123 / 96 and 130 / 73, 8192 471 / 376 and 480 / 275 (two waves 1.2 / 0.75 everywhere)
+            return (4, 1) if tiles >= 44 else (1, 1)
+        # 800 with 512 keys 1.05 / 0.80 of it in two waves, with 1000 1.02 / 0.76, 2047 0.99 / 0.75; 1024 with 1000 85 / 60 and 88 / 51
+        return (2, 1) if tiles >= 24 else (1, 1)
+    if 2 * pairs > 3 * units and tiles >= 36:
+        return 4, 1                                        # 408 with 2047 keys 1.00 / 0.78 of two single waves, 512 with 1400 64 / 48 and 66 / 42
+    if pairs >= units and tiles >= (128 if pairs == units else 64 if 3 * pairs <= simds else 96):
+        # two to three waves a SIMD, in blocks whose results a second kernel adds: 256 with 4096 keys 86 / 71 and (2, 4) 91 / 51, 288 with 2047 58 / 42
+        # and (2, 3) 60 / 34, 384 with 3100 101 / 78 and (2, 4) 108 / 62 (with 2047 70 / 56 and 76 / 49), with 8192 249 / 196 and 255 / 151
+        return (2, 3) if units < pairs and 3 * pairs <= simds else (2, 4)
     if pairs >= units:
         # a wave a SIMD, the waves of a pair in one block where they are two or four (64 requests of an 8B model, 512 pairs, with 768 keys 35.6 ->
         # 32.5 and no second kernel, 384 with 512 26.7 -> 22.3, 256 with 512 23.0 -> 15.2); three make blocks of their own
         # (288 with 512 23.8 -> 19.1), short contexts two (256 keys 14.3 -> 12.3)
         n = simds // pairs
-        if n == 2 and tiles >= 30 and 8 * pairs <= 13 * units:
-            return 1, 2                                    # 384 with 1400 keys 48.1, in one block 50.7
+        if n == 2 and tiles >= 30 and 2 * pairs <= 3 * units:
+            return 1, 2                                    # 384 with 1400 keys 48.1, in one block 50.7; 408 1.00 and 0.93
         return (1, 1) if tiles <= 2 else (4, 1) if n == 4 else (1, 3) if n == 3 and tiles > 8 else (2, 1)
     if 2 * pairs > units and 2 < tiles <= 16:
         # short contexts: no second kernel (192 pairs with 256 keys 12.7 -> 9.9, 248 with 512 18.0 -> 15.3; 192 with 512 18.4 -> 14.2)
