@@ -1864,12 +1864,19 @@ static int prefill_any(
     if (total > count * reach) total = count * reach;
     return (double)total * nkv * chunks / (2.0 * units) >= 0.6 * most && count * nkv * chunks >= 2 * units;
   };
-  // few keys are walked sooner than parts of them are added (130 tokens 8.7 us in one part, 10.3 in two, 300 13.4 and 13.5)
-  if (halves == 0 && hd == 128 && keys_max > 0 && (keys_max < reach ? keys_max : reach) <= 320) halves = 1;
+  // What a tile walks where it is known.  Few keys are walked sooner than parts of them are added, those that a window cuts, whose tiles are
+  // nearly all masked, fewer (us, few tiles of 32 heads over 8, one part and two: 130 keys 8.7 and 10.3; of 16 over 8, one, two and four: 320 keys
+  // 13.7, 12.7 and 13.8, windows of 128 / 200 / 256 keys 12.4, 11.5, 12.5 / 13.3, 12.5, 12.2 / 15.9, 14.3, 13.9; 2048 tokens behind windows of
+  // 256 / 512 17.5 / 28.5 in one, 24.8 / 34.3 in four)
+  const int walk = keys_max <= 0 ? reach : keys_max < reach ? keys_max : reach;
+  const bool cut = walk == reach, few = walk <= 352;
+  if (halves == 0 && hd == 128 && keys_max > 0 && walk <= (cut ? 128 : 224)) halves = 1;
   if (halves == 0 && two_heads)
-    halves = wide && enough(n_wide, wide_total, wide_max)  ? PREFILL_WIDE
-             : wide && (long long)n_wide * nkv > units ? PREFILL_WIDE_HALVES
-                                                           : PREFILL_QUARTERS;
+    halves = wide && enough(n_wide, wide_total, wide_max)              ? PREFILL_WIDE
+             : !few && wide && (long long)n_wide * nkv > units         ? PREFILL_WIDE_HALVES
+             : (few || cut) && enough(n_tiles, keys_total, keys_max)   ? 1
+             : walk <= (cut ? 192 : 352)                               ? 2
+                                                                       : PREFILL_QUARTERS;
   if (hd > 128) halves = 1;                              // shared memory holds one half's tiles only
   if (halves == 0) halves = enough(n_tiles, keys_total, keys_max) ? 1 : 2;
   if (halves >= PREFILL_WIDE) tiles = wide_tiles, n_tiles = n_wide;
