@@ -17,9 +17,10 @@ def ops():
 # heads, kv heads, head size, page size, rotated dims, pairing, q gain, k gain
 @pytest.mark.parametrize("nq,nkv,hd,P,rot,style,q_norm,k_norm", [
     (4, 2, 128, 16, 128, 1, True, True), (16, 8, 128, 16, 128, 1, True, False), (40, 8, 128, 16, 64, 1, True, True),
-    (60, 4, 128, 8, 128, 2, False, True), (24, 4, 64, 16, 64, 1, True, True), (8, 8, 256, 32, 256, 1, False, False)])
+    (60, 4, 128, 8, 128, 2, False, True), (24, 4, 64, 16, 64, 1, True, True), (8, 8, 256, 32, 256, 1, False, False),
+    (64, 8, 128, 16, 128, 1, True, True)])                                # two blocks a token, three heads a thread in both
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("lens", [[127, 1], [128], [511], [300, 1, 7, 204], [9, 3, 700]])
+@pytest.mark.parametrize("lens", [[127, 1], [128], [511], [300, 1, 7, 204], [9, 3, 700], [1024]])
 def test_long_batches_write_what_short_ones_do(ops, nq, nkv, hd, P, rot, style, q_norm, k_norm, dtype, lens):
     g = torch.Generator().manual_seed(nq + len(lens))
     T = sum(lens)

@@ -1023,16 +1023,19 @@ extern "C" int ullm_qk_norm_rope_write(
                    (!k_gain || ((uintptr_t)k_gain & 15) == 0) && rot % 8 == 0;
   if (vec) {
     // with few tokens a thread takes one head, so that many blocks are under way; with many it takes up to four
-    // in turn, for which it fetches its cosines and sines once (40 heads of 128: 300 tokens 4.9 us, in passes 5.1; 800 8.0 and 7.1)
+    // in turn, for which it fetches its cosines and sines once (40 heads of 128: 300 tokens 4.9 us, in passes 5.1; 800 8.0 and 7.1;
+    // in 32 bits, twice the registers, later: 72 heads, 700 tokens 14.7 and 17.3), every block of a token as many (72 heads by 3 and 3 passes:
+    // 1000 tokens in 32 bits 21.7 us, by 4 and 1 24.8)
     // with many tokens the values go through blocks of their own that write runs of eight at once
     const bool runs = write_kv && T_ >= 128 && page_size % 8 == 0 && hd <= VALUE_RUN_MAX_HD &&
                       ((uintptr_t)v_pool & 15) == 0;
     const int heads_per_block = 256 / lph, read_heads = write_kv && !runs ? nq + 2 * nkv : nq + nkv;
     int blocks_per_token = (read_heads + heads_per_block - 1) / heads_per_block;
     int heads_per_thread = 1;
-    if (T_ >= 512) {
-      heads_per_thread = blocks_per_token < 4 ? blocks_per_token : 4;
-      blocks_per_token = (blocks_per_token + heads_per_thread - 1) / heads_per_thread;
+    if (T_ >= (dtype == ULLM_F32 ? 1024 : 512)) {
+      const int few = (blocks_per_token + 3) / 4;          // blocks of up to four passes, as many in each
+      heads_per_thread = (blocks_per_token + few - 1) / few;
+      blocks_per_token = few;
     }
     const long long value_blocks = runs ? (long long)((T_ + VALUE_RUN_TOKENS - 1) / VALUE_RUN_TOKENS) * nkv : 0;
     const long long all_blocks = (long long)T_ * blocks_per_token + value_blocks;
