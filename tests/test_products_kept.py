@@ -50,7 +50,7 @@ def test_rows_for_partial_sums_leave_the_others_to_the_panels_kernel(table):
     assert [_takes(rows, 4096, 2048) for rows in (32, 33, 40, 41)] == [True, False, False, True]
 
 
-@pytest.mark.parametrize("columns,inner,role,rows", [(5632, 5120, "store", (17, 32, 48)), (10240, 2560, "activated", (40, 48)),
+@pytest.mark.parametrize("columns,inner,role,rows", [(5632, 5120, "store", (17, 32, 48)), (5120, 3072, "store", (17, 32)), (10240, 2560, "activated", (40, 48)),
                                                      (19456, 2560, "gated", (40, 48))])
 def test_matrices_that_were_not_measured(columns, inner, role, rows):
     """Of 24 to 64 M values, up to 48 rows, with units left idle by the plan; not where the rows kernel is not what takes the call."""
@@ -60,6 +60,19 @@ def test_matrices_that_were_not_measured(columns, inner, role, rows):
     assert _takes(64, columns, inner, role) and _takes(100, columns, inner, role)
     assert _takes(17, 19456, 2560, "gated")                     # the few-rows kernel's call
     assert _takes(40, 4096, 4608) and _takes(40, 16384, 4096, "activated") and _takes(40, 8192, 3584)      # small, large, no unit idle
+
+
+def test_few_columns_that_were_not_measured(table):
+    """From 513 rows on the library's; not with other sizes, an activation, for a stream that adds slices or where launches count."""
+    table({"1024x3072": {"stacked_from": 17, "stacked_to": 96}, "1024x2048": {"store_kept": "769-1024"}})
+    for columns, inner, last in ((1024, 2560, 512), (1024, 3072, 512), (768, 1536, 512)):
+        for role, more in (("store", {}), ("stream", {"whole": True})):
+            assert [_takes(r, columns, inner, role, **more) for r in (last, last + 1, 1024)] == [True, False, False]
+            assert _takes(900, columns, inner, role, host_bound=True, **more)
+        assert _takes(900, columns, inner, "activated") and _takes(900, columns, inner, "stream")
+    assert [_takes(r, 1024, 2048) for r in (640, 768, 769)] == [True, True, False]                  # measured
+    for columns, inner in ((1024, 1024), (1024, 4096), (1536, 2048), (2048, 2048), (2560, 2560)):
+        assert _takes(640, columns, inner) and _takes(640, columns, inner, "stream", whole=True)
 
 
 def test_ranges_from_times():

@@ -53,7 +53,7 @@ class Limits:
     tiles: Tuple[Tuple[int, int], ...] = ()
     # ranges of rows, (first, last) each, that the kernels named above keep because they were measured to be ahead of the panels kernel
     # there, for the three kinds of product; None: not measured (the rows of ``sums_from`` .. ``sums_to`` then stay with the partial sums,
-    # :func:`_rows_kernel_ahead` answers for the others of the first two kinds)
+    # :func:`_rows_kernel_ahead` and :func:`_library_ahead` answer for the others)
     store_kept: Optional[Tuple[Tuple[int, int], ...]] = None
     silu_kept: Optional[Tuple[Tuple[int, int], ...]] = None
     stream_kept: Optional[Tuple[Tuple[int, int], ...]] = None
@@ -164,21 +164,35 @@ def _panels_plan(rows: int, columns: int, inner: int, mode: int, max_slices: int
     return plan & 0xffff, (plan >> 17) / 8
 
 
-ROWS_AHEAD_ROWS, ROWS_AHEAD_WEIGHTS, ROWS_AHEAD_BLOCKS = 48, (24_000_000, 64_000_000), 230
+ROWS_AHEAD_ROWS, ROWS_AHEAD_WEIGHTS, ROWS_AHEAD_COLUMNS, ROWS_AHEAD_BLOCKS = 48, (13_000_000, 64_000_000), 4096, 230
 
 
 def _rows_kernel_ahead(rows: int, columns: int, inner: int, plan: int, mode: int) -> bool:
     """Whether the rows kernel, where it is what takes the call, is ahead of the panels kernel's plan in one slice, for matrices that were
-    not measured: those of 24 to 64 M values at up to 48 rows whose plan leaves a tenth of the compute units and more without a block.
+    not measured: those of 13 to 64 M values and more than 4096 columns at up to 48 rows whose plan leaves a tenth of the compute units and more
+    without a block.
     Such a product is a read of W by the units that have one, while the rows kernel gives every unit as many columns (us, the
-    rows kernel and this: 5120 x 5120 at 17 / 32 / 48 rows 14.2 / 14.9 / 19.2 and 15.8 / 17.7 / 20.8, with an activation 10240 x 2560 at 36 / 48
+    rows kernel and this: 5120 x 5120 at 17 / 32 / 48 rows 14.2 / 14.9 / 19.2 and 15.8 / 17.7 / 20.8, 5120 x 3072 at 17 / 32 9.8 / 10.0 and 11.4 / 11.0, with
+    an activation 10240 x 2560 at 36 / 48
     14.5 / 15.6 and 16.5 / 17.3, 11008 x 4096 21.5 / 21.4 and 24.4 / 23.4, 12288 x 3072 18.3 / 18.0 and 19.5 / 19.6; gate|up 19456 x 2560 20.5 /
-    21.2 and 22.4 / 23.2).  Smaller matrices are read in time by fewer units (4096 x 4096 at 40 rows 14.6 and 11.5), larger ones bound by memory
+    21.2 and 22.4 / 23.2).  Smaller matrices are read in time by fewer units (4096 x 4096 at 40 rows 14.6 and 11.5, 5120 x 2048 level, 4096 x
+    6144 and 4096 x 8192 at 17 to 48 0.68 to 0.93 of the rows kernel's time), larger ones bound by memory
     either way (gate|up 22016 x 4096 at 48 rows 10 % behind, 16384 x 4096 9 %)."""
     lim, weight = limits(columns, inner), columns * inner
     few, most = (lim.silu_skinny, lim.silu_rows) if mode == PANELS_GATED else (lim.skinny, lim.rows)
-    return (few < rows <= min(most, ROWS_AHEAD_ROWS) and ROWS_AHEAD_WEIGHTS[0] <= weight < ROWS_AHEAD_WEIGHTS[1] and plan >> 8 == 1
+    return (few < rows <= min(most, ROWS_AHEAD_ROWS) and ROWS_AHEAD_WEIGHTS[0] <= weight < ROWS_AHEAD_WEIGHTS[1]
+            and columns > ROWS_AHEAD_COLUMNS and plan >> 8 == 1
             and build.load("gemm_panels").ullm_gemm_panels_blocks(rows, columns, mode, plan & 0xff, 1) < ROWS_AHEAD_BLOCKS)
+
+
+def _library_ahead(rows: int, columns: int, inner: int) -> bool:
+    """Whether the library is ahead of the panels kernel for a matrix of few columns that was not measured: up to 1024 of them and 1536 to 3072
+    values a row, from 513 rows on, where the panels' tiles make one or two hundred blocks that each walk
+    half of K or all of it (time of the panels kernel over the library's at 400 / 640 / 900 rows: 768 x 2560 1.03 / 1.12 / 1.23, 1024 x 2048 0.89 / 1.05 /
+    1.22; 1024 x 1024 0.69 / 0.87 / 0.94, 1024 x 4096 0.86 / 0.99 / 1.03, 2048 x 2048 0.88 / 0.92 / 1.06).  1536 x 2048 (1.10 / 1.17 / 1.07) and
+    sums that the stream adds (1024 x 2048 0.98 / 1.11 / 1.20) are left as they are: alike layers launched together take the panels kernel there,
+    as launches are what takes the time, and have the bits of the layers one by one."""
+    return columns <= 1024 and 1536 <= inner <= 3072 and rows > 512
 
 
 @functools.lru_cache(maxsize=8192)
@@ -197,7 +211,7 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     79 and 87), and from 1025 rows on also in one (1024 x 3072 at 1300 / 2048 rows 17.2 / 20.0 and 20.4 / 24.1, 2048 x 2048 at 2048 / 3000
     21.0 / 26.5 and 23.0 / 27.6; inside a prompt of 1064 rows 6144 x 4096 59 and 63, 4096 x 4096 and 4096 x 12288 183 and 189 together,
     the prompt 17.9 and 18.4 ms; level at 2048).  Rows for which the kernels that took the calls before were measured to be ahead, or
-    for matrices that were not measured are expected to be (:func:`_rows_kernel_ahead`), are left to them.  Neither holds where ``host_bound``
+    for matrices that were not measured are expected to be (:func:`_rows_kernel_ahead`, :func:`_library_ahead`), are left to them.  Neither holds where ``host_bound``
     says that launches are what takes the time."""
     if rows < PANELS_MIN_ROWS or columns * inner < PANELS_MIN_WEIGHT or (rows > 1024 and not host_bound):
         return -1, 0
@@ -211,6 +225,8 @@ def panels(rows: int, columns: int, inner: int, role: str, keep_sums: bool = Fal
     if kept is None and role == "store" and lim.sums_from > 0 and lim.sums_from <= rows <= lim.sums_to:
         return -1, 0                                       # named for the partial sums, not compared with this kernel
     if kept is None and role != "stream" and mode != PANELS_FLOAT and _rows_kernel_ahead(rows, columns, inner, plan, mode):
+        return -1, 0
+    if kept is None and (role == "store" or role == "stream" and whole) and _library_ahead(rows, columns, inner):
         return -1, 0
     return plan, mode
 
