@@ -225,7 +225,7 @@ def test_stacks_of_partial_sums_added_to_one_result(ops, monkeypatch):
                                  dict(nq=5, nkv=1, hd=128, P=16, rot=64, style=2),      # 7 heads: one block, one turn
                                  dict(nq=40, nkv=40, hd=64, P=16, rot=32, style=1)])    # 120 heads: four in turn, a spare turn
 def test_qk_norm_rope_write_of_a_long_prompt(ops, dtype, cfg):
-    """From 1 024 tokens on a thread takes several heads in turn with one fetch of its cosines and sines; what it
+    """From 512 tokens on (1 024 in 32 bits) a thread takes several heads in turn with one fetch of its cosines and sines; what it
     writes is, bit for bit, what the same tokens give in portions below that length (which the test above
     checks against the plain formulas)."""
     torch.manual_seed(41)

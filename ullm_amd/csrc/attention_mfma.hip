@@ -1833,7 +1833,7 @@ static int compute_units() {
 //
 // Groups of at most two heads of size 128 leave half of a block's waves without a head there.  They go two heads by 64 tokens a block
 // (`wide_tiles`: up to twice as many tokens a tile, listed alike) where such blocks fill the chip, 4: all of their
-// keys, 5: two halves of them; else (3) by 32 tokens, the keys in four parts.  16 heads over 8, us before (1 or 2) and in the ways 3 / 5 / 4:
+// keys, 5: two halves of them; else by 32 tokens, the keys in four parts (3), or in one or two where a tile walks few of them.  16 heads over 8, us before (1 or 2) and in the ways 3 / 5 / 4:
 // 700 tokens behind 2100 57 and 40 / 59 / 87, 2048 53 and 43 / 47 / 66, 3000 92 and 83 / 63 / 93, 4000 156 and 126 / 95 / 120, 8000 523 and
 // 402 / 321 / 304, 11 000 980 and 711 / 589 / 536 (925 TFLOP/s).
 static int prefill_any(

@@ -1,4 +1,4 @@
-// out = x W^T in bfloat16 for 17 rows up to what one round of blocks holds (one to two thousand): x [M, K], W [N, K] as the
+// out = x W^T in bfloat16 for 17 to 1024 rows where one round of blocks holds them (beyond 1024 only where launches take the time): x [M, K], W [N, K] as the
 // reference stores its linears' weights (ullm/layers/linear.py:165,268).
 //   store   bfloat16 [M, N], with an optional bias and activation
 //   gated   W holds gate rows, then as many up rows: bfloat16 [M, N / 2] of silu(gate) * up (or the clamped unit)
@@ -21,10 +21,10 @@
 //             shared memory a product, and a quarter as many stages one after the other; the four sums meet in shared memory at
 //             the end.  For tiles of 32 x 16 up to 64 x 96, what small matrices and few rows leave a compute unit
 //
-// Measured against the kernels that took these calls before, us (cold weights): gate|up 24576 x 4096 17 / 32 / 64 / 130 / 256 rows
+// Measured alone (inside a step some 5 % more: gate|up of 130 rows 49) against the kernels that took these calls before, us (cold weights): gate|up 24576 x 4096 17 / 32 / 64 / 130 / 256 rows
 // 36 / 38 / 43 / 62 / 69 -> 32 / 33 / 36 / 46 / 58 (130 on: the library and the activation kernel), 6144 x 1024 40 / 130 / 256 / 512 /
 // 800 rows 7.9 / 11.6 / 15.1 / 16.4 / 17.3 -> 5.8 / 8.4 / 9.6 / 12.7 / 15.0; partial sums of 4096 x 12288 130 / 256 / 512 rows 31 / 42 / 83
-// -> 26 / 36 / 51, of 4096 x 4096 12.9 / 19.4 / 30.0 -> 13.8 / 17 / 24; 1024 x 2048 256 / 512 rows 8.6 / 9.5 -> 6.3 / 7.8.  What bounds them at few
+// -> 26 / 36 / 51, of 4096 x 4096 12.9 / 19.4 / 30.0 -> 13.8 / 17 / 24 (at 130 rows with the norm that adds them 21.8 -> 18.1); 1024 x 2048 256 / 512 rows 8.6 / 9.5 -> 6.3 / 7.8.  What bounds them at few
 // rows is W (201 MB at 64 rows 5.6 TB/s), else what the second-level caches deliver: every shape gets 64 KB a us and compute
 // unit of them, 16 TB/s in all, and the larger a tile the more products it makes of that; around it a launch, the first loads' way
 // and the store, 2 to 7 us.

@@ -830,7 +830,7 @@ moe_tiles_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const int* __restri
 // blocks in step ask the same memory channels: so a block's K begins at the stage of its expert's number (where K is TURNED_K and more; 32 experts, width 2048, 1024
 // columns, gate|up + down at 400 / 800 tokens, top 4, 71 + 26 / 73 + 35 -> 50 + 27 / 52 + 40 us; the stage by the columns too, 51 + 27 / 54 + 38,
 // leaves less to share between the blocks of a tile: 1500 tokens 69 + 49 and 67 + 45).
-// All of it together, us before and now of what takes the call: 400 / 800 / 1100 / 1500 / 2048 / 2500 / 3000 / 4000 / 8000 tokens 98 / 107 / 119 / 125 /
+// All of it together, us before and now of the best tile for routings by chance: 400 / 800 / 1100 / 1500 / 2048 / 2500 / 3000 / 4000 / 8000 tokens 98 / 107 / 119 / 125 /
 // 173 / 187 / 192 / 270 / 450 -> 75 / 93 / 114 / 115 / 143 / 181 / 192 / 236 / 420.  Before that loop, by the kernel above, gate|up took
 // 160 us at 2048 tokens and 470 at 8192.  Blocks of 128 x 128 or 128 x 256 with one barrier and all reads of a stage ahead of its products
 // took 127 to 150 us at 2048 tokens, whatever the number of stages; a wave of its own that asked for the matrix's lines ahead
