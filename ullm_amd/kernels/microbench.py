@@ -69,22 +69,26 @@ def decode_attention(args) -> None:
             tables = torch.randperm(n_pages).int().reshape(nv, B, pages_per).to(DEV)
             q = torch.randn(B, nq * hd, device=DEV).bfloat16()
             out = torch.empty_like(q)
-            pos = torch.full((B,), ctx - 1, dtype=torch.int32, device=DEV)
             ent = torch.arange(B, dtype=torch.int32, device=DEV)
             groups = -(-(nq // nkv) // 16)
             auto = ops.decode_split(B, nkv, groups, ctx, hd)
-            cells = []
-            for splits, waves in [(0, 0)] + [(s, w) for w in (4, 8, 1) for s in (1, 2, 4, 8, 16, 32, 64)]:
-                if splits * B * nkv * groups > 2048 or (hd == 256 and waves == 8):
+            # all contexts equal, and (longest first, as a step lists them) from the longest to a tenth of it
+            for shape, lens in (("equal", [ctx] * B), ("spread", [max(1, round(ctx * (1 - 0.9 * b / max(1, B - 1)))) for b in range(B)])):
+                if shape == "spread" and B == 1:
                     continue
-                calls = [(lambda v=v: ops.attention_decode_mfma(q, out, k_pool, v_pool, None, B, pos, ent, tables[v], P, nq,
-                                                                nkv, hd, hd ** -0.5, 0, ctx, splits=splits, waves=waves))
-                         for v in range(nv)]
-                t = graph_time(calls)
-                name = f"chosen {auto[1]}x{auto[0]}" if splits == 0 else f"{splits}x{waves}"
-                cells.append(f"{name}: {t:.1f}")
-            print(f"decode attention, batch {B}, context {ctx}, {nq}/{nkv} heads of {hd} ({kv_bytes / 1e6:.0f} MB of cache); "
-                  f"us by splits x waves: " + "  ".join(cells), flush=True)
+                pos = torch.tensor(lens, dtype=torch.int32, device=DEV) - 1
+                cells = []
+                for splits, waves in [(0, 0)] + [(s, w) for w in (2, 4, 8, 1) for s in (1, 2, 3, 4, 8, 16, 32, 64)]:
+                    if splits * B * nkv * groups > 2048 or (hd == 256 and waves == 8):
+                        continue
+                    calls = [(lambda v=v: ops.attention_decode_mfma(q, out, k_pool, v_pool, ent, B, pos, ent, tables[v], P, nq,
+                                                                    nkv, hd, hd ** -0.5, 0, ctx, splits=splits, waves=waves))
+                             for v in range(nv)]
+                    t = graph_time(calls)
+                    name = f"chosen {auto[1]}x{auto[0]}" if splits == 0 else f"{splits}x{waves}"
+                    cells.append(f"{name}: {t:.1f}")
+                print(f"decode attention, batch {B}, {shape} contexts of {'' if shape == 'equal' else 'up to '}{ctx}, {nq}/{nkv} heads of {hd} "
+                      f"({sum(lens) * nkv * hd * 4 / 1e6:.0f} MB of cache); us by splits x waves: " + "  ".join(cells), flush=True)
             del k_pool, v_pool
 
 
