@@ -1443,20 +1443,23 @@ def decode_split(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128
         return (2, 1) if tiles >= 24 else (1, 1)
     if 2 * pairs > 3 * units and tiles >= 36:
         return 4, 1                                        # 408 with 2047 keys 1.00 / 0.78 of two single waves, 512 with 1400 64 / 48 and 66 / 42
-    if pairs >= units and tiles >= (128 if pairs == units else 64 if 3 * pairs <= simds else 96):
+    if pairs >= units and hd <= 128 and tiles >= (128 if pairs == units else 64 if 3 * pairs <= simds else 96):
         # two to three waves a SIMD, in blocks whose results a second kernel adds: 256 with 4096 keys 86 / 71 and (2, 4) 91 / 51, 288 with 2047 58 / 42
-        # and (2, 3) 60 / 34, 384 with 3100 101 / 78 and (2, 4) 108 / 62 (with 2047 70 / 56 and 76 / 49), with 8192 249 / 196 and 255 / 151
+        # and (2, 3) 60 / 34, 384 with 3100 101 / 78 and (2, 4) 108 / 62 (with 2047 70 / 56 and 76 / 49), with 8192 249 / 196 and 255 / 151.  Heads
+        # of 256 read twice as much a key: 256 with 4096 keys 173 and 206 where they are equal
         return (2, 3) if units < pairs and 3 * pairs <= simds else (2, 4)
     if pairs >= units:
         # a wave a SIMD, the waves of a pair in one block where they are two or four (64 requests of an 8B model, 512 pairs, with 768 keys 35.6 ->
         # 32.5 and no second kernel, 384 with 512 26.7 -> 22.3, 256 with 512 23.0 -> 15.2); three make blocks of their own
         # (288 with 512 23.8 -> 19.1), short contexts two (256 keys 14.3 -> 12.3)
         n = simds // pairs
-        if n == 2 and tiles >= 30 and 2 * pairs <= 3 * units:
-            return 1, 2                                    # 384 with 1400 keys 48.1, in one block 50.7; 408 1.00 and 0.93
+        if n == 2 and tiles >= 30 and (2 * pairs <= 3 * units or hd > 128):
+            # 384 with 1400 keys 48.1, in one block 50.7; 408 1.00 and 0.93, but heads of 256 with 1000 keys that spread 58 and 63
+            return 1, 2
         return (1, 1) if tiles <= 2 else (4, 1) if n == 4 else (1, 3) if n == 3 and tiles > 8 else (2, 1)
-    if 2 * pairs > units and 2 < tiles <= 16:
-        # short contexts: no second kernel (192 pairs with 256 keys 12.7 -> 9.9, 248 with 512 18.0 -> 15.3; 192 with 512 18.4 -> 14.2)
+    if hd <= 128 and 2 * pairs > units and 2 < tiles <= 16:
+        # short contexts: no second kernel (192 pairs with 256 keys 12.7 -> 9.9, 248 with 512 18.0 -> 15.3; 192 with 512 18.4 -> 14.2; heads of
+        # 256, 144 with 256 keys 13.8 and in one block 16.3)
         if tiles <= 8 or 8 * pairs >= 7 * units:
             return 4, 1
         if 4 * pairs >= 3 * units:
