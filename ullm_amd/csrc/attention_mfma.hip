@@ -1869,7 +1869,7 @@ static int prefill_any(
   // 13.7, 12.7 and 13.8, windows of 128 / 200 / 256 keys 12.4, 11.5, 12.5 / 13.3, 12.5, 12.2 / 15.9, 14.3, 13.9; 2048 tokens behind windows of
   // 256 / 512 17.5 / 28.5 in one, 24.8 / 34.3 in four)
   const int walk = keys_max <= 0 ? reach : keys_max < reach ? keys_max : reach;
-  const bool cut = walk == reach, few = walk <= 352;
+  const bool cut = window != 0 && walk == reach, few = walk <= 352;
   if (halves == 0 && hd == 128 && keys_max > 0 && walk <= (cut ? 128 : 224)) halves = 1;
   if (halves == 0 && two_heads)
     halves = wide && enough(n_wide, wide_total, wide_max)              ? PREFILL_WIDE
