@@ -1836,6 +1836,45 @@ static int compute_units() {
 // keys, 5: two halves of them; else by 32 tokens, the keys in four parts (3), or in one or two where a tile walks few of them.  16 heads over 8, us before (1 or 2) and in the ways 3 / 5 / 4:
 // 700 tokens behind 2100 57 and 40 / 59 / 87, 2048 53 and 43 / 47 / 66, 3000 92 and 83 / 63 / 93, 4000 156 and 126 / 95 / 120, 8000 523 and
 // 402 / 321 / 304, 11 000 980 and 711 / 589 / 536 (925 TFLOP/s).
+struct PrefillWork {
+  int n_tiles, keys_max;
+  long long keys_total;
+  int n_wide, wide_max;                                   // none: 0
+  long long wide_total;
+};
+static int prefill_way(const PrefillWork& work, int nq, int nkv, int hd, int window, bool two_heads, long long units) {
+  const int chunks = (nq / nkv + PREFILL_WAVES - 1) / PREFILL_WAVES;
+  const int reach = window == 0 ? 0x7fffffff : (window > 0 ? window : -window) + 32;      // keys a tile may see
+  // is there work for two blocks a unit to the end: `total` keys over the tiles, `most` of one
+  auto enough = [&](long long count, long long total, int most) {
+    if (total <= 0 || most <= 0) return count * nkv * chunks >= 3 * units;
+    if (most > reach) most = reach;
+    if (total > count * reach) total = count * reach;
+    return (double)total * nkv * chunks / (2.0 * units) >= 0.6 * most && count * nkv * chunks >= 2 * units;
+  };
+  const bool filled = enough(work.n_tiles, work.keys_total, work.keys_max);
+  // What a tile walks where it is known.  Few keys are walked sooner than parts of them are added, those that a window cuts, whose tiles are
+  // nearly all masked, fewer (us, few tiles of 32 heads over 8, one part and two: 130 keys 8.7 and 10.3; of 16 over 8, one, two and four: 320 keys
+  // 13.7, 12.7 and 13.8, windows of 128 / 200 / 256 keys 12.4, 11.5, 12.5 / 13.3, 12.5, 12.2 / 15.9, 14.3, 13.9; 2048 tokens behind windows of
+  // 256 / 512 17.5 / 28.5 in one, 24.8 / 34.3 in four)
+  const int walk = work.keys_max <= 0 ? reach : work.keys_max < reach ? work.keys_max : reach;
+  const bool cut = window != 0 && walk == reach, few = walk <= 352;
+  if (hd == 128 && work.keys_max > 0 && walk <= (cut ? 128 : 224)) return 1;
+  if (!two_heads) return filled ? 1 : 2;
+  if (work.n_wide > 0 && enough(work.n_wide, work.wide_total, work.wide_max)) return PREFILL_WIDE;
+  if (!few && (long long)work.n_wide * nkv > units) return PREFILL_WIDE_HALVES;
+  if ((few || cut) && filled) return 1;
+  return walk <= (cut ? 192 : 352) ? 2 : PREFILL_QUARTERS;
+}
+
+// The way a launch without a bias by distance goes on a device of `units` compute units (`halves` 0); n_wide 0: no wide tiles.
+extern "C" int ullm_attention_prefill_way(int n_tiles, long long keys_total, int keys_max, int n_wide, long long wide_total, int wide_max,
+                                          int nq, int nkv, int hd, int window, int units) {
+  if (hd > 128) return 1;
+  return prefill_way(PrefillWork{n_tiles, keys_max, keys_total, n_wide, wide_max, wide_total}, nq, nkv, hd, window, hd == 128 && nq / nkv <= 2,
+                     units);
+}
+
 static int prefill_any(
     const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
     const int* tiles, int n_tiles, const int* positions, const int* token_entry, const int* block_table,
@@ -1855,30 +1894,10 @@ static int prefill_any(
   const bool wide = two_heads && wide_tiles && n_wide > 0;
   if (halves < 0 || halves > (wide ? PREFILL_WIDE_HALVES : two_heads ? PREFILL_QUARTERS : 2)) return ULLM_ERR_SHAPE;
   const int chunks = (nq / nkv + PREFILL_WAVES - 1) / PREFILL_WAVES;
-  const long long units = compute_units();
-  const int reach = window == 0 ? 0x7fffffff : (window > 0 ? window : -window) + 32;      // keys a tile may see
-  // is there work for two blocks a unit to the end: `total` keys over the tiles, `most` of one
-  auto enough = [&](long long count, long long total, int most) {
-    if (total <= 0 || most <= 0) return count * nkv * chunks >= 3 * units;
-    if (most > reach) most = reach;
-    if (total > count * reach) total = count * reach;
-    return (double)total * nkv * chunks / (2.0 * units) >= 0.6 * most && count * nkv * chunks >= 2 * units;
-  };
-  // What a tile walks where it is known.  Few keys are walked sooner than parts of them are added, those that a window cuts, whose tiles are
-  // nearly all masked, fewer (us, few tiles of 32 heads over 8, one part and two: 130 keys 8.7 and 10.3; of 16 over 8, one, two and four: 320 keys
-  // 13.7, 12.7 and 13.8, windows of 128 / 200 / 256 keys 12.4, 11.5, 12.5 / 13.3, 12.5, 12.2 / 15.9, 14.3, 13.9; 2048 tokens behind windows of
-  // 256 / 512 17.5 / 28.5 in one, 24.8 / 34.3 in four)
-  const int walk = keys_max <= 0 ? reach : keys_max < reach ? keys_max : reach;
-  const bool cut = window != 0 && walk == reach, few = walk <= 352;
-  if (halves == 0 && hd == 128 && keys_max > 0 && walk <= (cut ? 128 : 224)) halves = 1;
-  if (halves == 0 && two_heads)
-    halves = wide && enough(n_wide, wide_total, wide_max)              ? PREFILL_WIDE
-             : !few && wide && (long long)n_wide * nkv > units         ? PREFILL_WIDE_HALVES
-             : (few || cut) && enough(n_tiles, keys_total, keys_max)   ? 1
-             : walk <= (cut ? 192 : 352)                               ? 2
-                                                                       : PREFILL_QUARTERS;
   if (hd > 128) halves = 1;                              // shared memory holds one half's tiles only
-  if (halves == 0) halves = enough(n_tiles, keys_total, keys_max) ? 1 : 2;
+  if (halves == 0)
+    halves = prefill_way(PrefillWork{n_tiles, keys_max, keys_total, wide ? n_wide : 0, wide_max, wide_total}, nq, nkv, hd, window, two_heads,
+                         compute_units());
   if (halves >= PREFILL_WIDE) tiles = wide_tiles, n_tiles = n_wide;
   const long long blocks = (long long)n_tiles * nkv * chunks;
   if (blocks > 0x7fffffffLL) return ULLM_ERR_SHAPE;
