@@ -1,0 +1,72 @@
+"""Decoded tokens beside prompt portions in one attention launch: every way against softmax in 64 bits, at teams without a token, tiles at their
+edges, windows, chunks and contexts of every remainder; and which steps go that way."""
+import ctypes
+
+import pytest
+import torch
+
+from gpu_util import DEV, paged_cache, table_tensor, tol
+from test_gpu_two_head_prompts import _attention
+
+
+# (new tokens, keys before them) of every request, heads, kv heads, window: pairs of tokens and kv heads that leave teams without one, kv heads that
+# are no multiple of the dies, groups of one to sixteen heads, contexts below, at and past a tile for each of four waves
+CASES = [([(1, 0), (33, 5), (1, 40), (1, 31)], 2, 1, 0), ([(1, 127), (70, 0), (1, 128), (1, 129), (31, 100), (1, 700)], 4, 2, 0),
+         ([(1, 300), (130, 400), (1, 49), (1, 50)], 6, 3, 50), ([(1, 200), (65, 63), (1, 64)], 8, 8, -64), ([(1, 15), (97, 60), (1, 500)], 10, 2, 0),
+         ([(1, 90), (40, 333), (1, 17)], 16, 1, 0), ([(1, 37 * i) for i in range(20)] + [(600, 17)], 16, 8, 0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entries,nq,nkv,window", CASES)
+def test_every_way_of_the_launch(entries, nq, nkv, window):
+    from ullm_amd.kernels import ops
+    from ullm_amd.parts import StepShape
+    from ullm_amd.parts.attention import plan_attention_step
+    g = torch.Generator().manual_seed(nq + window)
+    hd, P, dtype, scale = 128, 16, torch.bfloat16, 128 ** -0.5
+    ks, vs = ([torch.randn(n + s, nkv, hd, generator=g).to(dtype).float() for n, s in entries] for _ in range(2))
+    k_pool, v_pool, tables = paged_cache(ks, vs, P, dtype, DEV)
+    bt = table_tensor(tables, DEV)
+    plan = plan_attention_step(StepShape(tuple(n for n, _ in entries), tuple(s for _, s in entries)))
+    f, arrays = plan.facts, {k: torch.tensor(v, device=DEV) for k, v in plan.arrays.items()}
+    assert f["decode_keys"] == sum(s + 1 for n, s in entries if n == 1)
+    T = sum(n for n, _ in entries)
+    q = torch.randn(T, nq * hd, generator=g).to(dtype)
+    positions = torch.cat([torch.arange(s, s + n) for n, s in entries]).int().to(DEV)
+    entry = torch.cat([torch.full((n,), b) for b, (n, _) in enumerate(entries)]).int().to(DEV)
+    want = torch.cat([_attention(part.view(-1, nq, hd), k, v, window, scale)
+                      for part, k, v in zip(q.split([n for n, _ in entries]), ks, vs)])
+    for way in ((3, 4, 5) if nq // nkv <= 2 else (1, 2)):
+        out = torch.full((T, nq * hd), float("nan"), dtype=dtype, device=DEV)
+        assert ops.attention_mixed_mfma(
+            q.to(DEV), out, k_pool, v_pool, arrays["decode_tokens"], f["num_decode"], arrays["tiles"], f["num_tiles"], positions, entry, bt, P, nq,
+            nkv, hd, scale, window, f["decode_keys"], f["max_decode_kv"], wide_tiles=arrays["wide_tiles"], n_wide=f["num_wide"], way=way)
+        assert (out.float().cpu() - want.float()).abs().max() <= tol(dtype, want), way
+    with pytest.raises(ops.KernelError):
+        ops.attention_mixed_mfma(q.to(DEV), out, k_pool, v_pool, arrays["decode_tokens"], f["num_decode"], arrays["tiles"], f["num_tiles"], positions,
+                                 entry, bt, P, nq, nkv, hd, scale, window, f["decode_keys"], f["max_decode_kv"], way=6)
+
+
+# requests and keys of the longest (the others down to 0.58 of it), the portion and the keys before it, heads, kv heads: us of two launches (0) and of the ways
+MEASURED = [(4, 640, 700, 2100, 16, {0: 52.1, 3: 39.5, 5: 57.8, 4: 85.7}), (40, 640, 300, 600, 16, {0: 43.5, 3: 26.8, 5: 26.8, 4: 37.0}),
+            (100, 640, 300, 600, 16, {0: 66.8, 3: 44.2, 5: 45.0, 4: 41.7}), (100, 640, 700, 0, 16, {0: 64.0, 3: 54.0, 5: 45.2, 4: 43.0}),
+            (100, 640, 700, 2100, 16, {0: 88.6, 3: 65.5, 5: 60.3, 4: 93.0}), (100, 300, 1500, 3000, 16, {0: 123.7, 3: 98.2, 5: 88.8, 4: 136.5}),
+            (30, 2000, 300, 600, 16, {0: 62.1, 3: 66.0, 5: 66.7, 4: 41.5}), (8, 4000, 300, 600, 16, {0: 47.2, 3: 115.5, 5: 115.1, 4: 63.0}),
+            (100, 640, 700, 2100, 32, {0: 108.8, 1: 94.2, 2: 80.1}), (100, 640, 1900, 0, 32, {0: 102.6, 1: 77.9, 2: 100.2}),
+            (100, 64, 300, 600, 32, {0: 36.2, 1: 33.8, 2: 27.0}), (8, 4000, 700, 0, 32, {0: 50.4, 1: 64.6, 2: 117.0})]
+
+
+@pytest.mark.parametrize("case", range(len(MEASURED)))
+def test_near_the_best_of_those_measured(case):
+    """CPU: the way of a step."""
+    from ullm_amd.kernels import build
+    from ullm_amd.parts import StepShape
+    from ullm_amd.parts.attention import plan_attention_step
+    b, c, portion, behind, nq, times = MEASURED[case]
+    starts = [max(16, int(c * (1 - 0.45 * ((7 * i) % 16) / 16))) for i in range(b)]
+    f = plan_attention_step(StepShape((1,) * b + (portion,), tuple(starts) + (behind,))).facts
+    i, long = ctypes.c_int, ctypes.c_longlong
+    way = build.load("attention_mfma").ullm_attention_mixed_way(
+        i(f["num_decode"]), long(f["decode_keys"]), i(f["max_decode_kv"]), i(f["num_tiles"]), long(f["tile_keys_total"]), i(f["tile_keys_max"]),
+        i(f["num_wide"]), long(f["wide_keys_total"]), i(f["wide_keys_max"]), i(nq), i(8), i(0), i(256))
+    assert times[way] <= 1.07 * min(times.values())

@@ -305,11 +305,12 @@ __device__ __forceinline__ void attend_range(
 
 // Merge the waves of a block pairwise, lane by lane (a lane's values mean the same in every wave),
 // halving the number of live waves each round in a fixed order; wave 0 ends with the block's result.
-// `buf` holds (WAVES / 2) x (NG * (8 NQK + 2)) x 64 floats.  Every wave of the block must call this.
+// `buf` holds (WAVES / 2) x (NG * (8 NQK + 2)) x 64 floats.  Every wave of the block must call this; `wave`: which of the WAVES it is
+// (a block may be several teams of so many).
 template <int NQK, int NG, int WAVES>
-__device__ __forceinline__ void merge_waves(f32x4_t (&acc)[NG][2 * NQK], float (&m)[NG], float (&l)[NG], float* buf) {
+__device__ __forceinline__ void merge_waves(f32x4_t (&acc)[NG][2 * NQK], float (&m)[NG], float (&l)[NG], float* buf, int wave) {
   constexpr int PER_LANE = NG * (8 * NQK + 2);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int half = WAVES / 2; half >= 1; half >>= 1) {
     if (wave >= half && wave < 2 * half) {          // the upper half of the live waves hands over
@@ -594,7 +595,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
                                  scale_log2e, accs, ms, ls);
     }
   }
-  merge_waves<NQK, 1, WAVES>(accs, ms, ls, merge);
+  merge_waves<NQK, 1, WAVES>(accs, ms, ls, merge, wave);
   f32x4_t (&acc)[2 * NQK] = accs[0];
   float& m = ms[0];
   float& l = ls[0];
@@ -1331,28 +1332,38 @@ __device__ __forceinline__ void dma_tile_products(const unsigned char* __restric
   }
 }
 
-// EXTRA: a bias by distance (never null here; the waves' heads' rows are copied to dynamic shared memory
-// first, [PREFILL_WAVES][bias_rows] floats) and the gate per head, as in attention_prefill_kernel.
-template <int NQK, int HEADS, int KS, bool EXTRA = false>
-__global__ void __launch_bounds__(KS == 4 ? 512 : 64 * PREFILL_WAVES * KS, KS == 1 ? 2 : 1)
-attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
-                             const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
-                             const int* __restrict__ tiles, const int* __restrict__ positions,
-                             const int* __restrict__ token_entry, const int* __restrict__ block_table,
-                             int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
-                             int n_tiles, ScoreExtras extras) {
+// What a block of these takes: threads, and shared memory.
+template <int NQK, int HEADS, int KS>
+struct DmaBlock {
   static_assert(HEADS == 4 || HEADS == 2, "heads a block takes");
   static_assert(KS == 1 || KS == 2 || (KS == 4 && HEADS == 2), "parts of the keys");
-  constexpr int TEAM = KS == 4 ? HEADS : PREFILL_WAVES, SUBS = TEAM / HEADS, TILES = KS == 4 ? 2 : 4;
+  static constexpr int THREADS = KS == 4 ? 512 : 64 * PREFILL_WAVES * KS, PER_UNIT = KS == 1 ? 2 : 1;
+  static constexpr int TEAM = KS == 4 ? HEADS : PREFILL_WAVES, SUBS = TEAM / HEADS, TILES = KS == 4 ? 2 : 4;
   using T = DmaTile<NQK, TEAM>;
+  static constexpr int TABLE = 2 * (DMA_TABLE_TILES + 4);        // page ids in shared memory, one per 16-key sub-block
+  static constexpr int BYTES = KS * TILES * T::BYTES;            // [part][tile][keys | values]
+};
+
+// EXTRA: a bias by distance (never null here; the waves' heads' rows are copied to dynamic shared memory
+// first, [PREFILL_WAVES][bias_rows] floats) and the gate per head, as in attention_prefill_kernel.
+// `block`: which of the prompt's blocks.
+template <int NQK, int HEADS, int KS, bool EXTRA>
+__device__ __forceinline__ void
+prefill_dma_block(int block, unsigned char* lds, int (*page_ids)[DmaBlock<NQK, HEADS, KS>::TABLE],
+                  const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
+                  const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
+                  const int* __restrict__ tiles, const int* __restrict__ positions,
+                  const int* __restrict__ token_entry, const int* __restrict__ block_table,
+                  int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
+                  int n_tiles, const ScoreExtras& extras) {
+  using B = DmaBlock<NQK, HEADS, KS>;
+  constexpr int TEAM = B::TEAM, SUBS = B::SUBS, TILES = B::TILES, TABLE = B::TABLE;
+  using T = typename B::T;
   constexpr int HD = 32 * NQK;
   constexpr int NG = PREFILL_GROUPS;
   constexpr int PER_LANE = NG * (8 * NQK + 2);            // floats a lane hands over in the merge
   constexpr int PER = 2 * T::ROUNDS;                      // load instructions of a wave per tile
-  constexpr int TABLE = 2 * (DMA_TABLE_TILES + 4);        // page ids in shared memory, one per 16-key sub-block
-  static_assert((KS - 1) * TEAM * PER_LANE * 64 * 4 <= KS * TILES * T::BYTES, "the merge reuses the tiles' memory");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[KS * TILES * T::BYTES];   // [part][tile][keys | values]
-  __shared__ int page_ids[KS][TABLE];
+  static_assert((KS - 1) * TEAM * PER_LANE * 64 * 4 <= B::BYTES, "the merge reuses the tiles' memory");
   const int wave_id = (int)(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, wave = wave_id % TEAM, part = wave_id / TEAM;
   const int g = lane >> 4, c = lane & 15;
@@ -1361,12 +1372,12 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
   const int G = nq / nkv, chunks = (G + HEADS - 1) / HEADS, per_kv = n_tiles * chunks;
   int kvh, rest;
   if (nkv % 8 == 0) {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int xcd = block & 7, slot = block >> 3;
     kvh = (slot / per_kv) * 8 + xcd;
     rest = slot % per_kv;
   } else {
-    kvh = blockIdx.x / per_kv;
-    rest = blockIdx.x % per_kv;
+    kvh = block / per_kv;
+    rest = block % per_kv;
   }
   const int tile_idx = n_tiles - 1 - rest / chunks;
   const int head_in_group = (rest % chunks) * HEADS + wave % HEADS;
@@ -1543,6 +1554,76 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
           make_uint2(pack2_bf16(acc[qg][n][0] * inv, acc[qg][n][1] * inv),
                      pack2_bf16(acc[qg][n][2] * inv, acc[qg][n][3] * inv));
   }
+}
+
+template <int NQK, int HEADS, int KS, bool EXTRA = false>
+__global__ void __launch_bounds__((DmaBlock<NQK, HEADS, KS>::THREADS), (DmaBlock<NQK, HEADS, KS>::PER_UNIT))
+attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
+                             const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
+                             const int* __restrict__ tiles, const int* __restrict__ positions,
+                             const int* __restrict__ token_entry, const int* __restrict__ block_table,
+                             int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
+                             int n_tiles, ScoreExtras extras) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[DmaBlock<NQK, HEADS, KS>::BYTES];
+  __shared__ int page_ids[KS][DmaBlock<NQK, HEADS, KS>::TABLE];
+  prefill_dma_block<NQK, HEADS, KS, EXTRA>(blockIdx.x, lds, page_ids, q, q_stride, out, out_stride, k_pool, v_pool, tiles, positions, token_entry,
+                                           block_table, bt_stride, page_size, nq, nkv, scale_log2e, window, n_tiles, extras);
+}
+
+// ------------------------------------------------------------------------------- decoded tokens beside prompt portions
+// One launch for a step that holds both, head size 128, without extras: the prompt's blocks (the long ones first), and behind as many of them
+// as the chip takes at once, blocks that take decoded tokens: a (token, kv head) a team of four waves, which share its keys and merge.
+// What bounds the two alone: the decoded tokens' reads leave the matrix units idle, and the prompt's tiles, chains of steps over their keys, leave
+// most of the memory's rate and, where they are few, most of the units.  Two launches and one, us (rocprofv3 and graph replays, 16 heads over 8, 100
+// requests of 350 to 640 keys beside 700 tokens): behind no key 64 -> 43, behind 2100 89 -> 60; beside 300 behind 600 67 -> 42; 32 heads over 8 beside 700
+// behind 2100 109 -> 80; 4 requests of 64 keys beside 40 tokens 13 -> 7.
+template <int HEADS, int KS>
+__global__ void __launch_bounds__((DmaBlock<4, HEADS, KS>::THREADS), (DmaBlock<4, HEADS, KS>::PER_UNIT))
+attention_mixed_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
+                       const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
+                       const int* __restrict__ tiles, const int* __restrict__ positions,
+                       const int* __restrict__ token_entry, const int* __restrict__ block_table,
+                       int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
+                       int n_tiles, int prompt_blocks, int lead, const int* __restrict__ decode_tokens, int pairs) {
+  using B = DmaBlock<4, HEADS, KS>;
+  constexpr int NQK = 4, HD = 128, TEAMS = B::THREADS / 256;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[B::BYTES];
+  __shared__ int page_ids[KS][B::TABLE];
+  static_assert(TEAMS * 2 * (8 * NQK + 2) * 64 * 4 <= B::BYTES, "the teams' merges");
+  const int decode_blocks = (int)gridDim.x - prompt_blocks, at = (int)blockIdx.x;
+  if (at < lead || at >= lead + decode_blocks) {
+    prefill_dma_block<NQK, HEADS, KS, false>(at < lead ? at : at - decode_blocks, lds, page_ids, q, q_stride, out, out_stride, k_pool, v_pool, tiles, positions, token_entry,
+                                             block_table, bt_stride, page_size, nq, nkv, scale_log2e, window, n_tiles,
+                                             ScoreExtras{nullptr, 0, nullptr, 0});
+    return;
+  }
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  const int pair = (at - lead) * TEAMS + team;
+  const bool there = pair < pairs;                        // a team without work comes to the barriers
+  const int item = there ? pair / nkv : 0, kvh = there ? pair - item * nkv : 0, G = nq / nkv;
+  const int t = decode_tokens[item];
+  const bool col_ok = c < G;
+  const int head = kvh * G + (col_ok ? c : 0);
+  ReadyQueries<NQK> queries{col_ok ? q + (size_t)t * q_stride + (size_t)head * HD : nullptr, g};
+  queries.fetch_early();
+  const int pos = positions[t], lo = first_seen_key(pos, window), first = lo & ~31;
+  const int share = 32 * (((pos + 1 - first + 31) / 32 + 3) / 4);
+  const int begin = there ? first + wave * share : pos + 1, end = begin + share < pos + 1 ? begin + share : pos + 1;
+  const int* const bt = block_table + (size_t)token_entry[t] * bt_stride;
+  const int clo[1] = {lo}, chi[1] = {col_ok ? pos : -1};
+  f32x4_t acc[1][2 * NQK];
+  float m[1], l[1];
+  attend_range<NQK, 1, false>(queries, clo, chi, begin, end, pos, lo, k_pool, v_pool, bt, page_size, nkv, kvh, scale_log2e, acc, m, l);
+  merge_waves<NQK, 1, 4>(acc, m, l, reinterpret_cast<float*>(lds) + team * 2 * (8 * NQK + 2) * 64, wave);
+  if (wave != 0 || !there) return;
+  const float sum = sum_with_lane_xor32(sum_with_lane_xor16(l[0])), inv = sum > 0.f ? 1.f / sum : 0.f;
+  if (!col_ok) return;
+  bf16_t* op = out + (size_t)t * out_stride + (size_t)head * HD;
+#pragma unroll
+  for (int n = 0; n < 2 * NQK; ++n)
+    *reinterpret_cast<uint2*>(op + 16 * n + 4 * g) =
+        make_uint2(pack2_bf16(acc[0][n][0] * inv, acc[0][n][1] * inv), pack2_bf16(acc[0][n][2] * inv, acc[0][n][3] * inv));
 }
 
 // tokens of one request a prompt tile may hold
@@ -1927,6 +2008,118 @@ extern "C" int ullm_attention_prefill(
   return prefill_any(q, q_stride, out, out_stride, k_pool, v_pool, tiles, n_tiles, positions, token_entry, block_table,
                      bt_stride, page_size, nq, nkv, hd, scale, window, halves, keys_total, keys_max, wide_tiles, n_wide, wide_total,
                      wide_max, stream, nullptr);
+}
+
+// The way of a launch that takes decoded tokens and prompt tiles together (`keys`: of all decoded tokens, `longest`: of one), or 0: two launches are
+// expected to be ahead.  Times in us of what bounds each:
+//   a prompt block    a chain over its keys, 0.030 a key where a block takes them all (two blocks a unit), 0.021 in halves, 0.014 in quarters
+//   decoded tokens    their bytes at 5.3 TB/s and 4 at the head, or the longest context's walk by four waves, 0.0175 a key; 0.029 where two teams
+//                     share a unit that holds nothing else
+//   together          blocks that share units with prompt blocks (two a unit) hide under them and hold them up by a quarter of the shorter time;
+//                     where a prompt block has the unit for itself they run beside and behind it: both add up over the units
+//   apart             both, 6 for the second kernel of cut contexts or a coarser cut, 3 for the launch
+// Held against 288 steps (1 to 250 requests of 30 to 4000 keys, 17 to 1500 tokens behind 0 to 4500, 16, 32 and 40 heads over 8): 1.26 times as fast as two
+// launches in the geometric mean, nowhere slower by more than 5 %; over 84 of them with every way timed 1.05 times the time of the best way.  Longer contexts than a team walks in that time stay apart (8 requests of
+// 4000 keys beside 300 tokens 47 us, together 63).
+static int mixed_way(const PrefillWork& work, long long keys, int longest, int n_decode, int nq, int nkv, int window, long long units) {
+  if (keys <= 0 || longest <= 0 || work.keys_max <= 0 || work.keys_total <= 0) return 0;
+  const long long reach = window == 0 ? 0x7fffffffLL : (window > 0 ? window : -(long long)window) + 32;      // keys a query's tile may see
+  const bool two_heads = nq / nkv <= 2;
+  const int chunks = (nq / nkv + PREFILL_WAVES - 1) / PREFILL_WAVES;
+  auto least = [](double a, double b) { return a < b ? a : b; };
+  auto most = [](double a, double b) { return a > b ? a : b; };
+  const double walk = (double)(longest < reach ? longest : reach), read = least((double)keys, (double)n_decode * reach) * nkv * 512 / 5.3e6 + 4;
+  double apart = 1e30, together = 1e30;
+  int way = 0;
+  auto look = [&](int w, double a_key, long long count, long long total, int longest_tile, int per_unit) {
+    if (count <= 0 || total <= 0) return;
+    const double block = a_key * least(longest_tile, (double)reach);
+    const double even = a_key * least((double)total, (double)count * reach) * nkv * chunks / (double)(units * per_unit);
+    // more blocks than the chip holds: what the last ones leave idle
+    const long long blocks = count * nkv * chunks, slots = units * per_unit;
+    const double all = blocks > slots ? most(even + 0.3 * block, even * slots / blocks * ((blocks + slots - 1) / slots)) : even;
+    const double prompt = most(block, all);
+    apart = least(apart, prompt);
+    const double both = per_unit == 2 ? most(prompt + least(most(0.0175 * walk, read), prompt) / 4, most(0.0175 * walk, read))
+                                      : 2 + most(most(prompt, 0.029 * walk), all + read);
+    if (both < together) {
+      together = both;
+      way = w;
+    }
+  };
+  if (two_heads) {
+    look(PREFILL_QUARTERS, 0.014, work.n_tiles, work.keys_total, work.keys_max, 1);
+    look(PREFILL_WIDE_HALVES, 0.021, work.n_wide, work.wide_total, work.wide_max, 1);
+    look(PREFILL_WIDE, 0.030, work.n_wide, work.wide_total, work.wide_max, 2);
+  } else {
+    look(2, 0.021, work.n_tiles, work.keys_total, work.keys_max, 1);
+    look(1, 0.030, work.n_tiles, work.keys_total, work.keys_max, 2);
+  }
+  return together < 0.97 * (read + apart + 9) ? way : 0;
+}
+
+// How many of the prompt's blocks come before the decoded tokens', in a way that takes `per_unit` of them a unit.  Where the chip holds them all, every one.  Else
+// few decoded tokens with a long walk begin at once (a request of 900 keys beside 1200 tokens behind 400 49 -> 40 us); short ones
+// come last, beside the last prompt blocks (100 of 640 beside 1500 behind 4500, 40 heads over 8, 381 -> 349); the others behind the first round.
+static long long prompt_lead(long long blocks, long long prompt_keys, double a_key, long long decode_blocks, long long keys, int longest, int nkv,
+                             long long units, int per_unit) {
+  const long long slots = units * per_unit;
+  if (blocks <= slots) return blocks;
+  const double block = a_key * (double)prompt_keys / (double)blocks, walk = (per_unit == 2 ? 0.0175 : 0.029) * longest, read = (double)keys * nkv * 512 / 5.3e6;
+  if (walk > block && 2 * decode_blocks <= slots) return 0;
+  return walk <= block && read <= block ? blocks : slots / 8 * 8;
+}
+
+// 1 if ullm_attention_mixed takes such heads.
+extern "C" int ullm_attention_mixed_supports(int hd, int page_size, int nq, int nkv) {
+  return hd == 128 && nkv > 0 && nq / nkv <= 16 && ullm_attention_mfma_supports(hd, page_size, nq, nkv);
+}
+
+// The way ullm_attention_mixed goes on a device of `units` compute units, 0: two launches.
+extern "C" int ullm_attention_mixed_way(int n_decode, long long decode_keys, int decode_keys_max, int n_tiles, long long keys_total, int keys_max, int n_wide,
+                                        long long wide_total, int wide_max, int nq, int nkv, int window, int units) {
+  return mixed_way(PrefillWork{n_tiles, keys_max, keys_total, n_wide, wide_max, wide_total}, decode_keys, decode_keys_max, n_decode, nq, nkv, window, units);
+}
+
+// ullm_attention_decode over the tokens `decode_tokens` (the longest context first; `decode_keys` keys of all of them, `decode_keys_max` of one) and
+// ullm_attention_prefill over the tiles, in one launch.  way 0: chosen; ULLM_ERR_UNSUPPORTED where two launches are the better ones.
+extern "C" int ullm_attention_mixed(
+    const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool, const int* decode_tokens, int n_decode,
+    long long decode_keys, int decode_keys_max, const int* tiles, int n_tiles, const int* positions, const int* token_entry, const int* block_table,
+    int bt_stride, int page_size, int nq, int nkv, int hd, float scale, int window, long long keys_total, int keys_max, const int* wide_tiles,
+    int n_wide, long long wide_total, int wide_max, int way, hipStream_t stream) {
+  if (n_decode <= 0 || n_tiles <= 0) return ULLM_ERR_SHAPE;
+  if (!ullm_attention_mixed_supports(hd, page_size, nq, nkv)) return ULLM_ERR_UNSUPPORTED;
+  const bool two_heads = nq / nkv <= 2, wide = two_heads && wide_tiles && n_wide > 0;
+  if (way == 0)
+    way = mixed_way(PrefillWork{n_tiles, keys_max, keys_total, wide ? n_wide : 0, wide_max, wide_total}, decode_keys, decode_keys_max, n_decode, nq, nkv,
+                    window, compute_units());
+  if (way == 0) return ULLM_ERR_UNSUPPORTED;
+  if (way < 0 || way > (wide ? PREFILL_WIDE_HALVES : two_heads ? PREFILL_QUARTERS : 2) || (two_heads && way < PREFILL_QUARTERS)) return ULLM_ERR_SHAPE;
+  if (way >= PREFILL_WIDE) tiles = wide_tiles, n_tiles = n_wide;
+  const int chunks = (nq / nkv + PREFILL_WAVES - 1) / PREFILL_WAVES;
+  const long long blocks = (long long)n_tiles * nkv * chunks, pairs = (long long)n_decode * nkv, prompt_keys = way >= PREFILL_WIDE ? wide_total : keys_total;
+  if (blocks + pairs + 8 > 0x7fffffffLL || (long long)nkv * page_size * hd > 0x7fffffffLL) return ULLM_ERR_SHAPE;
+  const float sl = scale * 1.4426950408889634f;
+  // (a prompt block's id says which die it goes to: what lies between two of them is a multiple of the dies)
+#define GO(HEADS, KS) do {                                                                                                             \
+    using B = DmaBlock<4, HEADS, KS>;                                                                                                  \
+    constexpr int TEAMS = B::THREADS / 256;                                                                                            \
+    const long long decode_blocks = ((pairs + TEAMS - 1) / TEAMS + 7) / 8 * 8;                                                         \
+    const long long lead = prompt_lead(blocks, prompt_keys * nkv * chunks, KS == 4 ? 0.014 : KS == 2 ? 0.021 : 0.030, decode_blocks, decode_keys,      \
+                                       decode_keys_max, nkv, compute_units(), B::PER_UNIT);                                            \
+    hipLaunchKernelGGL((attention_mixed_kernel<HEADS, KS>), dim3((unsigned)(blocks + decode_blocks)), dim3(B::THREADS), 0, stream,     \
+                       (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, tiles,      \
+                       positions, token_entry, block_table, bt_stride, page_size, nq, nkv, sl, window, n_tiles, (int)blocks,           \
+                       (int)lead, decode_tokens, (int)pairs);                                                                          \
+  } while (0)
+  if (way == PREFILL_QUARTERS) GO(2, 4);
+  else if (way == PREFILL_WIDE) GO(2, 1);
+  else if (way == PREFILL_WIDE_HALVES) GO(2, 2);
+  else if (way == 2) GO(4, 2);
+  else GO(4, 1);
+#undef GO
+  ULLM_LAUNCH_CHECK();
 }
 
 // ullm_attention_prefill with a bias by distance on the scores and a gate per head on the outputs (as

@@ -30,16 +30,17 @@ struct DenseStep {
   decltype(&ullm_gemm_tiles) tiles;
   decltype(&ullm_attention_decode) decode;
   decltype(&ullm_attention_prefill) prefill;
+  decltype(&ullm_attention_mixed) mixed_attention;
   // the stream, and room for what lies between two launches (sums: q|k|v in slices; mixed, fed: what the two halves add to the stream)
   float* residual;
   void *normed, *qkv, *q, *attended, *act;
   float *sums, *decode_parts;
   void *mixed, *fed;
   const int *positions, *token_entry, *decode_tokens, *prompt_tiles, *wide_tiles;
-  long long tile_keys_total, wide_keys_total;
+  long long tile_keys_total, wide_keys_total, decode_keys_total;
   DenseProduct into, out, gate_up, down;
   int tokens, width, heads, kv_heads, head_dim, inner, table_rows, rot, style, page_size, window;
-  int num_decode, decode_splits, decode_waves, num_tiles, tile_keys_max, num_wide, wide_keys_max;
+  int num_decode, decode_splits, decode_waves, num_tiles, tile_keys_max, num_wide, wide_keys_max, decode_keys_max;
   float eps1, eps2, qk_eps, scale;
 };
 
@@ -88,11 +89,20 @@ extern "C" int ullm_dense_layers(const DenseStep* step, const DenseLayer* layers
     STEP(s.qk_norm_rope_write(s.qkv, qkv_width, s.q, q_width, l.q_gain, l.k_gain, s.qk_eps, l.cos_sin, s.table_rows, s.rot, s.style,
                               s.positions, s.token_entry, l.block_table, (int)l.bt_stride, l.k_pool, l.v_pool, s.page_size, T, s.heads,
                               s.kv_heads, s.head_dim, (int)l.write_kv, s.heads + s.kv_heads, s.head_dim, ULLM_BF16, stream));
-    if (s.num_decode > 0)
+    // both kinds of tokens in one launch, where that is the better way
+    int together = ULLM_ERR_UNSUPPORTED;
+    if (s.num_decode > 0 && s.num_tiles > 0) {
+      together = s.mixed_attention(s.q, q_width, s.attended, q_width, l.k_pool, l.v_pool, s.decode_tokens, s.num_decode, s.decode_keys_total,
+                                   s.decode_keys_max, s.prompt_tiles, s.num_tiles, s.positions, s.token_entry, l.block_table, (int)l.bt_stride,
+                                   s.page_size, s.heads, s.kv_heads, s.head_dim, s.scale, s.window, s.tile_keys_total, s.tile_keys_max,
+                                   s.wide_tiles, s.num_wide, s.wide_keys_total, s.wide_keys_max, 0, stream);
+      if (together != ULLM_ERR_UNSUPPORTED) STEP(together);
+    }
+    if (together != 0 && s.num_decode > 0)
       STEP(s.decode(s.q, q_width, s.attended, q_width, l.k_pool, l.v_pool, s.decode_tokens, s.num_decode, s.positions, s.token_entry,
                     l.block_table, (int)l.bt_stride, s.page_size, s.heads, s.kv_heads, s.head_dim, s.scale, s.window, s.decode_splits,
                     s.decode_waves, s.decode_parts, stream));
-    if (s.num_tiles > 0)
+    if (together != 0 && s.num_tiles > 0)
       STEP(s.prefill(s.q, q_width, s.attended, q_width, l.k_pool, l.v_pool, s.prompt_tiles, s.num_tiles, s.positions, s.token_entry,
                      l.block_table, (int)l.bt_stride, s.page_size, s.heads, s.kv_heads, s.head_dim, s.scale, s.window, 0,
                      s.tile_keys_total, s.tile_keys_max, s.wide_tiles, s.num_wide, s.wide_keys_total, s.wide_keys_max, stream));

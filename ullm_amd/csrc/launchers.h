@@ -24,4 +24,9 @@ int ullm_attention_prefill(const void* q, int q_stride, void* out, int out_strid
                            int bt_stride, int page_size, int nq, int nkv, int hd, float scale, int window, int halves,
                            long long keys_total, int keys_max, const int* wide_tiles, int n_wide, long long wide_total, int wide_max,
                            hipStream_t stream);
+int ullm_attention_mixed(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool, const int* decode_tokens,
+                         int n_decode, long long decode_keys, int decode_keys_max, const int* tiles, int n_tiles, const int* positions,
+                         const int* token_entry, const int* block_table, int bt_stride, int page_size, int nq, int nkv, int hd, float scale,
+                         int window, long long keys_total, int keys_max, const int* wide_tiles, int n_wide, long long wide_total, int wide_max,
+                         int way, hipStream_t stream);
 }

@@ -12,7 +12,7 @@ _ptr, _int, _float, _long = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctype
 # the entry points the run calls, in the order of the structure's first fields
 LAUNCHERS = (("elementwise", "ullm_add_rmsnorm"), ("elementwise", "ullm_sum_stacks"), ("elementwise", "ullm_qk_norm_rope_write"),
              ("gemm_panels", "ullm_gemm_panels"), ("gemm_tiles", "ullm_gemm_tiles"), ("attention_mfma", "ullm_attention_decode"),
-             ("attention_mfma", "ullm_attention_prefill"))
+             ("attention_mfma", "ullm_attention_prefill"), ("attention_mfma", "ullm_attention_mixed"))
 LAYER_FIELDS = ("norm1", "q_gain", "k_gain", "cos_sin", "b_qkv", "norm2", "w_qkv", "w_o", "w_gate_up", "w_down", "k_pool", "v_pool",
                 "block_table", "bt_stride", "write_kv")          # of 8 bytes each
 
@@ -26,11 +26,11 @@ class Step(ctypes.Structure):
     _fields_ = ([(name, _ptr) for _, name in LAUNCHERS]
                 + [(name, _ptr) for name in ("residual", "normed", "qkv", "q", "attended", "act", "sums", "decode_parts", "mixed", "fed",
                                              "positions", "token_entry", "decode_tokens", "prompt_tiles", "wide_tiles")]
-                + [("tile_keys_total", _long), ("wide_keys_total", _long)]
+                + [("tile_keys_total", _long), ("wide_keys_total", _long), ("decode_keys_total", _long)]
                 + [(name, Product) for name in ("into", "out", "gate_up", "down")]
                 + [(name, _int) for name in ("tokens", "width", "heads", "kv_heads", "head_dim", "inner",
                                              "table_rows", "rot", "style", "page_size", "window", "num_decode", "decode_splits",
-                                             "decode_waves", "num_tiles", "tile_keys_max", "num_wide", "wide_keys_max")]
+                                             "decode_waves", "num_tiles", "tile_keys_max", "num_wide", "wide_keys_max", "decode_keys_max")]
                 + [(name, _float) for name in ("eps1", "eps2", "qk_eps", "scale")])
 
 

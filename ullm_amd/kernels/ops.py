@@ -26,6 +26,9 @@ _ERR_NAMES = {-1: "unsupported dtype combination", -2: "operand shape outside wh
               -3: "unsupported argument combination", -4: "partial results exceed the fixed scratch array"}
 
 
+_UNSUPPORTED = -3
+
+
 def _check(rc: int, what: str) -> None:
     if rc != 0:
         reason = _ERR_NAMES.get(rc, f"HIP error {rc}")
@@ -1639,6 +1642,36 @@ def attention_prefill_mfma(q, out, k_pool, v_pool, tiles: torch.Tensor, n_tiles:
         ctypes.c_longlong(int(wide_keys_total)), _c_int(wide_keys_max), _stream()), "attention_prefill")
 
 
+def attention_mixed_mfma(q, out, k_pool, v_pool, decode_tokens: torch.Tensor, n_decode: int, tiles: torch.Tensor, n_tiles: int, positions,
+                         token_entry, block_table, page_size: int, nq: int, nkv: int, hd: int, scale: float, window: int, decode_keys: int,
+                         max_decode_kv: int, keys_total: int = 0, keys_max: int = 0, wide_tiles: Optional[torch.Tensor] = None, n_wide: int = 0,
+                         wide_keys_total: int = 0, wide_keys_max: int = 0, way: int = 0) -> bool:
+    """``attention_decode_mfma`` over ``decode_tokens`` (``decode_keys`` keys of all of them, ``max_decode_kv`` of one) and
+    ``attention_prefill_mfma`` over the tiles in one launch; False (and nothing done) where two are the better way.  ``way``: 0, chosen;
+    1 and 2 (groups of more than two heads), 3 to 5 as ``attention_prefill_mfma``'s ``halves``."""
+    _check_pools(k_pool, v_pool, nkv, page_size, hd, torch.bfloat16)
+    _need(q.dtype == torch.bfloat16 and q.stride(1) == 1 and q.shape[1] == nq * hd, "q must be bfloat16 [T, nq*hd]")
+    _need(out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.shape == q.shape, "bad attention output")
+    _i32(decode_tokens, "decode_tokens", n_decode)
+    _need(tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.numel() >= 2 * n_tiles, "tiles must be int32 [n, 2]")
+    _need(wide_tiles is None or (wide_tiles.dtype == torch.int32 and wide_tiles.is_contiguous() and wide_tiles.numel() >= 2 * n_wide),
+          "wide tiles must be int32 [n, 2]")
+    _i32(positions, "positions")
+    _i32(token_entry, "token_entry")
+    _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1, "block_table must be int32 [B, stride]")
+    _need(-(-max_decode_kv // page_size) <= block_table.shape[1], "block table narrower than the longest context")
+    err = build.load("attention_mfma").ullm_attention_mixed(
+        _p(q), _c_int(q.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(decode_tokens), _c_int(n_decode),
+        ctypes.c_longlong(int(decode_keys)), _c_int(max_decode_kv), _p(tiles), _c_int(n_tiles), _p(positions), _p(token_entry), _p(block_table),
+        _c_int(block_table.stride(0)), _c_int(page_size), _c_int(nq), _c_int(nkv), _c_int(hd), _c_float(scale), _c_int(window),
+        ctypes.c_longlong(int(keys_total)), _c_int(keys_max), _p(wide_tiles), _c_int(n_wide), ctypes.c_longlong(int(wide_keys_total)),
+        _c_int(wide_keys_max), _c_int(way), _stream())
+    if err == _UNSUPPORTED:
+        return False
+    _check(err, "attention_mixed")
+    return True
+
+
 _warned_general_attention = set()
 
 
@@ -1685,6 +1718,13 @@ def paged_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     _need(plan is not None, "the matrix-core attention kernels need the step's work lists (a step plan)")
     out = torch.empty((q.shape[0], nq * hd), dtype=q.dtype, device=q.device)
     n = plan.facts
+    if (n["num_decode"] and n["num_tiles"] and n.get("decode_keys") and bias is None and gate is None and sink is None
+            and attention_mixed_mfma(
+                q, out, k_pool, v_pool, plan.arrays["decode_tokens"], n["num_decode"], plan.arrays["tiles"], n["num_tiles"], ctx.positions,
+                ctx.token_entry, group.block_table, group.page_size, nq, nkv, hd, scale, window, n["decode_keys"], n["max_decode_kv"],
+                keys_total=n["tile_keys_total"], keys_max=n["tile_keys_max"], wide_tiles=plan.arrays.get("wide_tiles"),
+                n_wide=n.get("num_wide", 0), wide_keys_total=n.get("wide_keys_total", 0), wide_keys_max=n.get("wide_keys_max", 0))):
+        return out
     if n["num_decode"]:
         attention_decode_mfma(q, out, k_pool, v_pool, plan.arrays["decode_tokens"], n["num_decode"], ctx.positions,
                               ctx.token_entry, group.block_table, group.page_size, nq, nkv, hd, scale, window,

@@ -84,7 +84,9 @@ def plan_attention_step(shape: StepShape) -> StepPlan:
         arrays={"decode_tokens": np.asarray(decode_tokens, dtype=np.int32),
                 "tiles": np.asarray([x for _, first, count in tiles for x in (first, count)], dtype=np.int32),
                 "wide_tiles": np.asarray([x for _, first, count in wide for x in (first, count)], dtype=np.int32)},
+        # (of a captured launch's tokens nothing that changes from step to step)
         facts={"num_decode": len(decode_tokens), "max_decode_kv": max_decode_kv, "num_tiles": len(tiles),
+               "decode_keys": sum(1 - start for start, _ in dec) if shape.kv_bucket is None else 0,
                "tile_keys_total": sum(k for k, _, _ in tiles), "tile_keys_max": tiles[-1][0] if tiles else 0,
                "num_wide": len(wide), "wide_keys_total": sum(k for k, _, _ in wide), "wide_keys_max": wide[-1][0] if wide else 0})
 

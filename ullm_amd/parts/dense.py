@@ -185,6 +185,7 @@ def run_layers(blocks: List[Block], caches: List[LayerCache], residual: torch.Te
         heads=m.nq, kv_heads=m.nkv, head_dim=m.hd, inner=I, table_rows=table_rows, rot=rot, style=style, page_size=group.page_size,
         window=m.reach, num_decode=work["num_decode"], decode_splits=splits, decode_waves=4 if m.hd == 256 and waves == 8 else waves,
         num_tiles=work["num_tiles"], tile_keys_max=work["tile_keys_max"], num_wide=work["num_wide"], wide_keys_max=work["wide_keys_max"],
+        decode_keys_total=work.get("decode_keys", 0), decode_keys_max=work["max_decode_kv"],
         eps1=first.mixer_norm.eps, eps2=first.ffn_norm.eps,
         qk_eps=m.qk_norm_eps if m.qk_norm_eps is not None else 0.0, scale=m.scale)
     dense.dense_layers(step, layers)
