@@ -349,7 +349,8 @@ __device__ __forceinline__ void merge_waves(f32x4_t (&acc)[NG][2 * NQK], float (
 // ------------------------------------------------------------------------------- decode
 // grid (num_splits, nkv * col_groups, n_tokens), block 64 * WAVES.  The keys [lo, pos] of a token are
 // cut into num_splits * WAVES equal shares of whole 32-key tiles (so the cut depends on the token's
-// own length, not on the batch); block x takes shares x * WAVES ..., one per wave.  The waves then merge
+// own length, not on the batch); block x takes shares x * WAVES ..., one per wave (EVEN, of `even` items: EvenShares
+// says what block x takes, and the grid has no z).  The waves then merge
 // their (maximum, sum, output) pairwise through shared memory, lane by lane (a lane's values have the
 // same meaning in every wave), halving the number of waves each round in a fixed order.  Wave 0 ends
 // with the block's result: with one split that is the output; otherwise it goes to the workspace and
@@ -370,6 +371,47 @@ struct DecodeFuse {
   int table_rows;
   bf16_t* k_pool;         // the pools again, writable; null: this layer reads a cache that another layer writes
   bf16_t* v_pool;
+};
+
+// Which keys of which token a block takes when `blocks` of them (a kv head) share out all tokens' 32-key tiles evenly (at most 64
+// tokens, fewer than blocks): every share has as many tiles, a token's last one fewer, so that long contexts have more shares than
+// short ones and no block takes longer than the rest.  Every wave finds out by itself, lane i for the i-th token: a share's
+// tiles from the sum of all, tokens' shares from that, and where they begin from the sums of those before.
+// Bound by the longest share, for there is a wave a SIMD and each walks its tiles one after the other: 15 tokens of 8 kv heads, 8192 keys
+// the longest, in equal cuts a token 78 us where they spread from 0.55 of it, 66 from a tenth, 93 where they are equal; shared evenly 75, 58 and
+// 92 (224 pairs with 8180 keys 146, 121, 171 -> 132, 99, 168).  The sums cost every wave a microsecond before its first key.
+struct EvenShares {
+  int t, pos;             // lane's token and its position
+  int tiles, shares, end; // of its context; its shares, and those up to and with it
+  int share;              // tiles a share
+  __device__ __forceinline__ EvenShares(int blocks, const int* __restrict__ token_list, const int* __restrict__ positions, int n_items,
+                                        int window, int lane) {
+    const int i = lane < n_items ? lane : n_items - 1;
+    t = token_list ? token_list[i] : i;
+    pos = positions[t];
+    const int all = (pos + 1 - (first_seen_key(pos, window) & ~31) + 31) / 32;
+    tiles = lane >= n_items ? 0 : all > 1 ? all : 1;
+    const int sum = __builtin_amdgcn_readfirstlane((int)wave_pairs((unsigned)tiles, [](unsigned a, unsigned b) { return a + b; }));
+    // the fewest tiles a share with no more than `blocks` shares: not below the sum over the blocks, and
+    // the sum over (blocks - n_items) always does, for the last shares are n_items at most; five halvings between
+    unsigned least = ((unsigned)sum + blocks - 1) / (unsigned)blocks;
+    unsigned most = ((unsigned)sum + blocks - n_items - 1) / (unsigned)(blocks - n_items);
+    for (int step = 0; step < 5 && least < most; ++step) {
+      const unsigned mid = (least + most) / 2;
+      const unsigned need = __builtin_amdgcn_readfirstlane(wave_pairs(((unsigned)tiles + mid - 1) / mid, [](unsigned a, unsigned b) { return a + b; }));
+      if (need <= (unsigned)blocks) most = mid;
+      else least = mid + 1;
+    }
+    share = (int)most;
+    shares = end = (int)((unsigned)(tiles + share - 1) / (unsigned)share);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x111, 0xf, 0xf, true);      // row_shr:1, 2, 4, 8, then the rows before
+    end += __builtin_amdgcn_update_dpp(0, end, 0x112, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x114, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x118, 0xf, 0xf, true);
+    end += __builtin_amdgcn_update_dpp(0, end, 0x142, 0xa, 0xf, false);     // row_bcast:15 into rows 1 and 3
+    end += __builtin_amdgcn_update_dpp(0, end, 0x143, 0xc, 0xf, false);     // row_bcast:31 into rows 2 and 3
+  }
+  __device__ __forceinline__ int of(int value, int item) const { return __builtin_amdgcn_readlane(value, item); }
 };
 
 // Queries as the projection left them (bfloat16, normed and rotated by an earlier kernel).
@@ -526,25 +568,34 @@ struct RawQueries {
   }
 };
 
-template <int NQK, int WAVES, bool FUSE, bool EXTRA = false>
+template <int NQK, int WAVES, bool FUSE, bool EXTRA = false, bool EVEN = false>
 __global__ void __launch_bounds__(64 * WAVES)
 attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
                         const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
                         const int* __restrict__ token_list, const int* __restrict__ positions,
                         const int* __restrict__ token_entry, const int* __restrict__ block_table,
                         int bt_stride, int page_size, int nq, int nkv, float scale_log2e, int window,
-                        int num_splits, float* __restrict__ part, DecodeFuse fuse, ScoreExtras extras) {
+                        int num_splits, int even, float* __restrict__ part, DecodeFuse fuse, ScoreExtras extras) {
   constexpr int HD = 32 * NQK;
   constexpr int ROW = HD + 4;                       // output dims, then maximum and sum (rows stay 16-byte aligned)
   __shared__ float merge[(WAVES > 1 ? WAVES / 2 : 1) * (WAVES > 1 ? (8 * NQK + 2) * 64 : 1)];   // [writer][value][lane]: conflict-free
   __shared__ __attribute__((aligned(16))) bf16_t own_kv[FUSE ? 2 * HD : 8];   // the token's own key, then its value
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
-  const int split = blockIdx.x;
+  int split = blockIdx.x, item = blockIdx.z, t, pos, share;
   const int G = nq / nkv;
   const int groups = (G + 15) / 16;
   const int kvh = blockIdx.y / groups, cg = blockIdx.y % groups;
-  const int item = blockIdx.z;
-  const int t = token_list ? token_list[item] : item;
+  if constexpr (EVEN) {
+    const EvenShares all(num_splits, token_list, positions, even, window, lane);
+    item = __popcll(__ballot(lane < even && all.end <= split));
+    if (item >= even) return;                       // the last blocks may have no share
+    t = all.of(all.t, item);
+    pos = all.of(all.pos, item);
+    share = 32 * all.share;
+    split -= all.of(all.end, item) - all.of(all.shares, item);
+  } else {
+    t = token_list ? token_list[item] : item;
+  }
   const int head_in_group = cg * 16 + c;
   const bool col_ok = head_in_group < G;
   const int head = kvh * G + head_in_group;
@@ -559,11 +610,11 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
       return ReadyQueries<NQK>{col_ok ? row + (size_t)head * HD : nullptr, g};
   }();
   queries.fetch_early();
-  const int pos = positions[t];
+  if constexpr (!EVEN) pos = positions[t];
   const int lo = first_seen_key(pos, window);
   const int first = lo & ~31;
   const int tiles = (pos + 1 - first + 31) / 32;
-  const int share = 32 * ((tiles + num_splits * WAVES - 1) / (num_splits * WAVES));
+  if constexpr (!EVEN) share = 32 * ((tiles + num_splits * WAVES - 1) / (num_splits * WAVES));
   int begin = first + (split * WAVES + wave) * share, end = begin + share;
   if (end > pos + 1) end = pos + 1;
   f32x4_t accs[1][2 * NQK];
@@ -613,8 +664,8 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
           make_uint2(pack2_bf16(acc[n][0] * inv, acc[n][1] * inv), pack2_bf16(acc[n][2] * inv, acc[n][3] * inv));
     return;
   }
-  // partial of this block: [item][head][split][ROW]
-  float* pp = part + (((size_t)item * nq + head) * num_splits + split) * ROW;
+  // partial of this block: [item][head][split][ROW], or with even shares [head][block][ROW]
+  float* pp = part + (((size_t)(EVEN ? 0 : item) * nq + head) * num_splits + (EVEN ? blockIdx.x : split)) * ROW;
 #pragma unroll
   for (int n = 0; n < 2 * NQK; ++n)
     *reinterpret_cast<float4*>(pp + 16 * n + 4 * g) = make_float4(acc[n][0], acc[n][1], acc[n][2], acc[n][3]);
@@ -624,16 +675,22 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
   }
 }
 
-// Adds the splits' partials [item][head][split][head_dim + 4] in split order.  grid (n_items, nq),
+// Adds the splits' partials [item][head][split][head_dim + 4] (even shares, of `even` items: [head][share][head_dim + 4]) in their order.  grid (n_items, nq),
 // one wave: lane s first reads split s's maximum and sum (64 splits at a time), then every lane sums
 // its output dims over the splits with the splits' weights passed round by shuffles.
 __global__ void __launch_bounds__(64)
 attention_reduce_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int out_stride,
-                        const int* __restrict__ token_list, int nq, int hd, int num_splits, ScoreExtras extras) {
+                        const int* __restrict__ token_list, int nq, int hd, int num_splits, int even,
+                        const int* __restrict__ positions, int window, ScoreExtras extras) {
   const int item = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
   const int t = token_list ? token_list[item] : item;
   const int row = hd + 4;
-  const float* pp = part + ((size_t)item * nq + head) * num_splits * row;
+  const float* pp = part + ((size_t)(even > 0 ? 0 : item) * nq + head) * num_splits * row;
+  if (even > 0) {
+    const EvenShares all(num_splits, token_list, positions, even, window, lane);
+    num_splits = all.of(all.shares, item);
+    pp += (size_t)(all.of(all.end, item) - num_splits) * row;
+  }
   // Eight splits at a time: their loads are all queued before the first is used, and those of the first eight go
   // out before anything else (no load under a condition: an index past the end reads the last element), so that
   // the splits' maxima and their values come back in one round trip instead of two.
@@ -1646,6 +1703,10 @@ extern "C" int ullm_attention_mfma_supports(int hd, int page_size, int nq, int n
   return supported_hd(hd) && page_size > 0 && page_size % 16 == 0 && nkv > 0 && nq % nkv == 0;
 }
 
+// `waves` of a decode launch whose num_splits blocks (a kv head, of one wave) share out the keys of all its tokens evenly: heads of at most
+// 128, more blocks than tokens, of which there may be 64, and a workspace of nq * num_splits * (hd + 4) floats.
+#define ULLM_DECODE_EVEN (-1)
+
 // Workspace floats needed for `n_items` tokens split `num_splits` ways.
 extern "C" long long ullm_attention_decode_workspace(int n_items, int nq, int hd, int num_splits) {
   return num_splits <= 1 ? 0 : (long long)n_items * nq * num_splits * (hd + 4);
@@ -1660,6 +1721,9 @@ static int decode_launch(
   if (extras && fuse) return ULLM_ERR_UNSUPPORTED;
   if (extras && extras->bias && extras->bias_rows <= 0) return ULLM_ERR_SHAPE;
   if (!ullm_attention_mfma_supports(hd, page_size, nq, nkv)) return ULLM_ERR_UNSUPPORTED;
+  const int even = waves == ULLM_DECODE_EVEN ? n_items : 0;
+  if (even && (n_items > 64 || num_splits <= n_items || hd > 128)) return ULLM_ERR_SHAPE;
+  if (even) waves = 1;
   if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return ULLM_ERR_UNSUPPORTED;
   if (hd == 256 && waves == 8) waves = 4;                // shared memory of the merge
   if (num_splits < 1 || num_splits > 65535) return ULLM_ERR_SHAPE;
@@ -1667,19 +1731,21 @@ static int decode_launch(
   const int G = nq / nkv, groups = (G + 15) / 16;
   if (n_items > 65535 || nkv * groups > 65535) return ULLM_ERR_SHAPE;
   const float sl = scale * 1.4426950408889634f;
-  dim3 grid(num_splits, nkv * groups, n_items), block(64 * waves);
+  dim3 grid(num_splits, nkv * groups, even ? 1 : n_items), block(64 * waves);
   const DecodeFuse f = fuse ? *fuse : DecodeFuse{nullptr, nullptr, 0.f, nullptr, 0, nullptr, nullptr};
 #define ARGS (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, token_list, \
-    positions, token_entry, block_table, bt_stride, page_size, nq, nkv, sl, window, num_splits, workspace, f, x
+    positions, token_entry, block_table, bt_stride, page_size, nq, nkv, sl, window, num_splits, even, workspace, f, x
   const ScoreExtras x = extras ? *extras : ScoreExtras{nullptr, 0, nullptr, 0};
 #define CALL_AS(N, F) do {                                                                                     \
-    if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, F>), grid, block, 0, stream, ARGS);      \
+    if (even) { if constexpr (N <= 4) hipLaunchKernelGGL((attention_decode_kernel<N, 1, F, false, true>), grid, block, 0, stream, ARGS); } \
+    else if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, F>), grid, block, 0, stream, ARGS); \
     else if (waves == 4) hipLaunchKernelGGL((attention_decode_kernel<N, 4, F>), grid, block, 0, stream, ARGS); \
     else if (waves == 2) hipLaunchKernelGGL((attention_decode_kernel<N, 2, F>), grid, block, 0, stream, ARGS); \
     else hipLaunchKernelGGL((attention_decode_kernel<N, 1, F>), grid, block, 0, stream, ARGS);                 \
   } while (0)
 #define CALL_EXTRA(N) do {                                                                                               \
-    if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, false, true>), grid, block, 0, stream, ARGS);      \
+    if (even) { if constexpr (N <= 4) hipLaunchKernelGGL((attention_decode_kernel<N, 1, false, true, true>), grid, block, 0, stream, ARGS); } \
+    else if (waves == 8) hipLaunchKernelGGL((attention_decode_kernel<N, 8, false, true>), grid, block, 0, stream, ARGS); \
     else if (waves == 4) hipLaunchKernelGGL((attention_decode_kernel<N, 4, false, true>), grid, block, 0, stream, ARGS); \
     else if (waves == 2) hipLaunchKernelGGL((attention_decode_kernel<N, 2, false, true>), grid, block, 0, stream, ARGS); \
     else hipLaunchKernelGGL((attention_decode_kernel<N, 1, false, true>), grid, block, 0, stream, ARGS);                 \
@@ -1704,7 +1770,7 @@ static int decode_launch(
   int rc = (int)hipGetLastError();
   if (rc != 0 || num_splits == 1) return rc;
   hipLaunchKernelGGL(attention_reduce_kernel, dim3(n_items, nq), dim3(64), 0, stream, workspace, (bf16_t*)out,
-                     out_stride, token_list, nq, hd, num_splits, x);
+                     out_stride, token_list, nq, hd, num_splits, even, positions, window, x);
   ULLM_LAUNCH_CHECK();
 }
 
@@ -1808,6 +1874,7 @@ extern "C" int ullm_attention_decode_static(
     int num_splits, int waves, hipStream_t stream) {
   if (n_items <= 0) return 0;
   if (num_splits < 1 || nq < 1 || hd < 1) return ULLM_ERR_SHAPE;
+  if (waves == ULLM_DECODE_EVEN) return ULLM_ERR_UNSUPPORTED;
   if (ullm_attention_decode_workspace(n_items, nq, hd, num_splits) > (long long)ULLM_DECODE_SCRATCH_FLOATS)
     return ULLM_ERR_SCRATCH;
   int err = 0;

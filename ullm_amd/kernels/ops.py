@@ -1478,6 +1478,49 @@ def decode_split(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128
     return waves, splits
 
 
+DECODE_EVEN = -1       # "waves": one wave a block, and num_splits blocks (a kv head) share out all tokens' keys evenly
+
+
+def decode_cuts(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128, window: int = 0, units: int = 256):
+    """(waves, num_splits) as ``decode_split`` has them, or (``DECODE_EVEN``, blocks a kv head) where its single waves a block have long ways
+    and contexts of several lengths would leave some of them waiting for others.  It is told the longest context alone (in a graph the
+    power of two above it), so the line lies where equal contexts lose nothing by it either.  us in equal cuts / shared evenly, for
+    contexts that are equal, spread from 0.55 and from a tenth of the longest: 120 pairs with 8180 keys 93 / 92, 78 / 75, 66 / 58; 32 pairs
+    with 16000 52 / 52, 46 / 45, 40 / 40; 64 with 16000 92 / 93, 81 / 79, 70 / 63; 192 with 8180 138 / 139, 120 / 115, 103 / 87.  Half as long,
+    192 with 2040 keys 42 / 43, 37 / 38, 33 / 31; 64 with 8180 53 / 54, 45 / 45, 40 / 39; 32 with 4090 22 / 24, 21 / 22, 20 / 20.  Of 256 pairs
+    in (2, 4) 4090 keys 101 / 97, 80 / 81, 62 / 63 and 16000 342 / 337, 271 / 283, 201 / 211."""
+    waves, splits = decode_split(n_items, nkv, groups, max_kv, hd, window, units)
+    pairs = n_items * nkv * groups
+    if window != 0:
+        max_kv = min(max_kv, abs(window) + 31)
+    blocks = 4 * units // max(1, nkv * groups)
+    if (waves == 1 and splits > 1 and hd <= 128 and 4 <= n_items <= 64 and 8 * pairs >= units and blocks > n_items
+            and -(-max_kv // 32) >= (256 if 3 * pairs >= units else 512)):
+        return DECODE_EVEN, blocks
+    return waves, splits
+
+
+def _decode_launch(n_items: int, nq: int, nkv: int, max_kv: int, hd: int, window: int, splits: int, waves: int, device):
+    """(waves, num_splits, workspace) of a decode launch: those asked for, or chosen where they are 0."""
+    auto_waves, auto_splits = decode_cuts(n_items, nkv, -(-(nq // nkv) // 16), max_kv, hd, window, compute_units(device))
+    if waves == 0 and splits != 0 and auto_waves == DECODE_EVEN:
+        auto_waves = 1                                     # cuts of every token
+    if splits == 0 and waves not in (0, DECODE_EVEN) and auto_waves == DECODE_EVEN:
+        auto_splits = decode_split(n_items, nkv, -(-(nq // nkv) // 16), max_kv, hd, window, compute_units(device))[1]
+    waves = waves or auto_waves
+    if hd == 256 and waves == 8:
+        waves = 4
+    splits = splits or auto_splits
+    return waves, splits, decode_parts(n_items, nq, hd, splits, waves, device)
+
+
+def decode_parts(n_items: int, nq: int, hd: int, splits: int, waves: int, device) -> Optional[torch.Tensor]:
+    """The launch's partial results, where it has any."""
+    if splits <= 1:
+        return None
+    return torch.empty((1 if waves == DECODE_EVEN else n_items) * nq * splits * (hd + 4), dtype=torch.float32, device=device)
+
+
 def attention_decode_mfma(q, out, k_pool, v_pool, token_list: Optional[torch.Tensor], n_items: int,
                           positions, token_entry, block_table, page_size: int, nq: int, nkv: int, hd: int,
                           scale: float, window: int, max_kv: int, splits: int = 0, waves: int = 0,
@@ -1500,16 +1543,8 @@ def attention_decode_mfma(q, out, k_pool, v_pool, token_list: Optional[torch.Ten
     _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1,
           "block_table must be int32 [B, stride]")
     _need(-(-max_kv // page_size) <= block_table.shape[1], "block table narrower than the longest context")
-    groups = -(-(nq // nkv) // 16)
-    auto_waves, auto_splits = decode_split(n_items, nkv, groups, max_kv, hd, window, compute_units(q.device))
-    waves = waves or auto_waves
-    if hd == 256 and waves == 8:
-        waves = 4
-    splits = splits or auto_splits
+    waves, splits, ws = _decode_launch(n_items, nq, nkv, max_kv, hd, window, splits, waves, q.device)
     lib = build.load("attention_mfma")
-    ws = None
-    if splits > 1:
-        ws = torch.empty(n_items * nq * splits * (hd + 4), dtype=torch.float32, device=q.device)
     if bias_log2 is not None or gate is not None or sink_log2 is not None:
         _check_gate(gate, q.shape[0], nq)
         _check_sink(sink_log2, nq)
@@ -1571,20 +1606,13 @@ def attention_decode_fused(qkv, out, q_gain: Optional[torch.Tensor], k_gain: Opt
               and cos_sin.shape[1] == rotary_dim and cos_sin.is_contiguous(),
               "cos_sin must be float32 [positions, rotary_dim]")
         table_rows = cos_sin.shape[0]
-    groups = -(-(nq // nkv) // 16)
-    auto_waves, auto_splits = decode_split(n_items, nkv, groups, max_kv, hd, window, compute_units(qkv.device))
-    waves = waves or auto_waves
-    if hd == 256 and waves == 8:
-        waves = 4
-    splits = splits or auto_splits
+    waves, splits, ws = _decode_launch(n_items, nq, nkv, max_kv, hd, window, splits, waves, qkv.device)
     lib = build.load("attention_mfma")
-    ws = None
-    if splits > 1:
-        ws = torch.empty(n_items * nq * splits * (hd + 4), dtype=torch.float32, device=qkv.device)
     if entry_is_token:
         _need(n_items == qkv.shape[0] <= block_table.shape[0], "one token of every entry, nothing else")
         token_entry = None
-        if n_items * nkv * groups * splits * waves <= 2 * compute_units(qkv.device):
+        # nor do even shares care for it
+        if waves == DECODE_EVEN or n_items * nkv * -(-(nq // nkv) // 16) * splits * waves <= 2 * compute_units(qkv.device):
             token_list = None
     _check(lib.ullm_attention_decode_fused(
         _p(qkv), _c_int(qkv.stride(0)), _p(out), _c_int(out.stride(0)), _p(k_pool), _p(v_pool), _p(token_list),

@@ -171,10 +171,9 @@ def run_layers(blocks: List[Block], caches: List[LayerCache], residual: torch.Te
     sums = torch.empty((into.slices, T, qkv_width), dtype=torch.float32, device=device) if into.mode == dispatch.PANELS_FLOAT else None
     waves, splits, parts = 1, 1, None
     if work["num_decode"]:
-        waves, splits = ops.decode_split(work["num_decode"], m.nkv, -(-(m.nq // m.nkv) // 16), work["max_decode_kv"], m.hd, m.reach,
-                                         ops.compute_units(device))
-        if splits > 1:
-            parts = torch.empty(work["num_decode"] * m.nq * splits * (m.hd + 4), dtype=torch.float32, device=device)
+        waves, splits = ops.decode_cuts(work["num_decode"], m.nkv, -(-(m.nq // m.nkv) // 16), work["max_decode_kv"], m.hd, m.reach,
+                                        ops.compute_units(device))
+        parts = ops.decode_parts(work["num_decode"], m.nq, m.hd, splits, waves, device)
     address = lambda t: 0 if t is None else t.data_ptr()       # noqa: E731
     step = dense.Step(
         residual=residual.data_ptr(), normed=normed.data_ptr(), qkv=qkv.data_ptr(), q=q.data_ptr(), attended=attended.data_ptr(),
