@@ -8,24 +8,31 @@
 //
 // What bounds it: the matrix pipe (157 TFLOP/s in 32-bit) where the tiles fill the chip, the chain over K where they do
 // not (a 16 x 16 tile adds 4 k in 32 cycles).  Hence the tile sizes: large ones read shared memory and the second-level
-// cache less per product, small ones make more blocks.  Against a 64 x 64 tile of scalar multiply-adds whose operands came
-// one value a load: 500 rows, 4096 outputs, K = 1024 122 -> 49 us (85 TFLOP/s), 1024 outputs, K = 3072 407 -> 52 us; 2048
-// rows, 4096 outputs 272 -> 179 us; one row of 151 936 outputs 434 -> 115 us (5.4 TB/s).
+// cache less per product, small ones make more blocks.  A unit that has one block has one wave a SIMD: whatever is not
+// put between the products of that wave is time the pipe stands still.  So the next stage is written, and the one after the next
+// two fetched, piece by piece between the products, operands are read a chunk ahead, and the only wait a stage is its barrier.
+// In stages that were written in one go behind their products, with a condition on fetched values that waited for all of them:
+// 500 rows, 4096 outputs, K = 1024 43 -> 39 us (109 TFLOP/s), 6144 outputs 60 -> 56, 1024 outputs and K = 2048 34 -> 24, K = 3072
+// 49 -> 36; 40 rows 23 -> 16 and 33 -> 23; 2048 rows of 4096 outputs 156 -> 142.  Stages that are exchanged between lanes in
+// registers and written 16 bytes at a time, from rows read in half lines, are slower (43 us for 36, 56 for 44).
 #include "mfma_f32.h"
+
+#include <algorithm>
 
 // A block of four waves takes BM rows of A against BN rows of W, WGM waves side by side along M.  A stage is BK values of
 // K: rows in shared memory whose 16-byte piece c of row r lies at piece c ^ ((r >> 1) & 7) (the 16 lanes the hardware
-// serves together then read different bank groups); two stages take turns, and a stage is fetched into registers two
-// stages before its products.  A stage costs about 600 cycles of writing, barrier and reading beside its products, so the
-// smaller tiles take 64 values a stage.  Lane (r, g) of a wave reads k = g, 4 + g, 8 + g, 12 + g of its row's chunk at
+// serves together then read different bank groups); two stages take turns, and a stage is fetched into registers three
+// stages before its products.  A barrier costs the smaller tiles the more, so they
+// take 64 values a stage.  Lane (r, g) of a wave reads k = g, 4 + g, 8 + g, 12 + g of its row's chunk at
 // once (they are written side by side) and holds out[row r of A][columns 4g .. 4g + 3] of each 16 x 16 tile.  VEC: four values a load (K and the row lengths are
-// multiples of four values and the addresses of that alignment); else one by one.  No load stands under a condition: a
+// multiples of four values and the addresses of that alignment), 2 where also K is whole stages; 0: one by one.  No load stands under a condition: a
 // row past the end reads the last row, a piece past K the row's last piece (replaced by zeros); neither is stored.
-template <typename TA, typename TW, typename TC, int BM, int BN, int WGM, int BK, bool VEC>
+template <typename TA, typename TW, typename TC, int BM, int BN, int WGM, int BK, int VEC>
 __global__ void __launch_bounds__(256)
 gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, int ldw, const float* __restrict__ bias,
                    TC* __restrict__ C, int ldc, int M, int N, int K, int m_tiles, int n_tiles) {
-  constexpr int WGN = 4 / WGM, TM = BM / 16 / WGM, TN = BN / 16 / WGN, PR = BK / 4, STEP = 256 / PR;
+  constexpr int WGN = 4 / WGM, TM = BM / 16 / WGM, TN = BN / 16 / WGN, PR = BK / 4, STEP = 256 / PR, CHUNKS = BK / 16;
+  static_assert(CHUNKS % 2 == 0, "a stage's first chunk lies in the same registers every time");
   constexpr int AP = (BM + STEP - 1) / STEP, WP = (BN + STEP - 1) / STEP;  // pieces a thread fetches a stage
   __shared__ __attribute__((aligned(16))) unsigned char stages[2][(BM + BN) * BK * 4];
   // die d (blocks go to the 8 dies round-robin) takes the d-th eighth of the tiles, all rows of A for a strip of W before
@@ -52,24 +59,16 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
     wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw;
     wput[i] = (BM + row) * BK * 4 + (((pc & ~3) ^ ((row >> 1) & 4)) << 4) + 4 * (pc & 3), wlow[i] = (row >> 1) & 3;
   }
-  float4 areg[2][AP], wreg[2][WP];
-  auto fetch = [&](int set, int k0) __attribute__((always_inline)) {
+  // piece p of a stage (those of A first) on its way to registers
+  float4 reg[2][AP + WP];
+  auto fetch = [&](int set, int p, int k0) __attribute__((always_inline)) {
     const int k = k0 + 4 * pc;
     if (VEC) {
-      const bool in = k < K;
-      const int kk = in ? k : K - 4;
-#pragma unroll
-      for (int i = 0; i < AP; ++i) areg[set][i] = ld4_f32(asrc[i] + kk);
-#pragma unroll
-      for (int i = 0; i < WP; ++i) wreg[set][i] = ld4_f32(wsrc[i] + kk);
-      if (!in) {
-#pragma unroll
-        for (int i = 0; i < AP; ++i) areg[set][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int i = 0; i < WP; ++i) wreg[set][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+      const int kk = k < K ? k : K - 4;
+      if (p < AP) reg[set][p] = ld4_f32(asrc[p] + kk);
+      else reg[set][p] = ld4_f32(wsrc[p - AP] + kk);
     } else {
-      auto one = [&](auto* src) __attribute__((always_inline)) {
+      auto one = [&](auto src) __attribute__((always_inline)) {
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -78,70 +77,88 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
         }
         return make_float4(v[0], v[1], v[2], v[3]);
       };
-#pragma unroll
-      for (int i = 0; i < AP; ++i) areg[set][i] = one(asrc[i]);
-#pragma unroll
-      for (int i = 0; i < WP; ++i) wreg[set][i] = one(wsrc[i]);
+      if (p < AP) reg[set][p] = one(asrc[p]);
+      else reg[set][p] = one(wsrc[p - AP]);
     }
   };
   // value e of a piece goes to the chunk's piece e: a lane group's 16 bytes are then values g, 4 + g, 8 + g, 12 + g of the chunk
-  // (64 lanes write one value each to 64 different banks)
-  auto put = [&](int set, int buf) __attribute__((always_inline)) {
+  // (64 lanes write one value each to 64 different banks).  Zeros are put in here: a condition on a fetched value any earlier
+  // would wait for the fetch.
+  auto put = [&](int set, int p, int buf, int k0) __attribute__((always_inline)) {
+    float v[4] = {reg[set][p].x, reg[set][p].y, reg[set][p].z, reg[set][p].w};
+    if (VEC == 1) {
 #pragma unroll
-    for (int i = 0; i < AP; ++i) {
-      const float v[4] = {areg[set][i].x, areg[set][i].y, areg[set][i].z, areg[set][i].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(stages[buf] + aput[i] + ((e ^ alow[i]) << 4)) = v[e];
+      for (int e = 0; e < 4; ++e) v[e] = k0 + 4 * pc < K ? v[e] : 0.f;
     }
+    unsigned char* row = stages[buf] + (p < AP ? aput[p] : wput[p - AP]);
+    const int low = p < AP ? alow[p] : wlow[p - AP];
 #pragma unroll
-    for (int i = 0; i < WP; ++i) {
-      const float v[4] = {wreg[set][i].x, wreg[set][i].y, wreg[set][i].z, wreg[set][i].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(stages[buf] + wput[i] + ((e ^ wlow[i]) << 4)) = v[e];
-    }
+    for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(row + ((e ^ low) << 4)) = v[e];
   };
   f32x4_t acc[TN][TM];
 #pragma unroll
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto products = [&](int buf) __attribute__((always_inline)) {
+  f32x4_t a[2][TM], w[2][TN];
+  auto take = [&](int set, int buf, int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < BK / 16; ++c) {
-      f32x4_t a[TM], w[TN];
+    for (int m = 0; m < TM; ++m) {
+      const int row = wm + 16 * m + r;
+      a[set][m] = *reinterpret_cast<const f32x4_t*>(stages[buf] + row * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
+    }
 #pragma unroll
-      for (int m = 0; m < TM; ++m) {
-        const int row = wm + 16 * m + r;
-        a[m] = *reinterpret_cast<const f32x4_t*>(stages[buf] + row * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
-      }
+    for (int n = 0; n < TN; ++n) {
+      const int row = wn + 16 * n + r;
+      w[set][n] = *reinterpret_cast<const f32x4_t*>(stages[buf] + (BM + row) * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
+    }
+  };
+  // Stage k0 from its buffer, its first chunk taken already; `set` holds the next stage, the other set the one after it, both on
+  // their way.  A chunk is taken while the one before it is multiplied, over the barrier too: that stands ahead of the last
+  // chunk's products, when the last chunk has been taken (this buffer is free) and the next stage is written.  Between the
+  // products of the chunks before it the next stage is written, each piece's registers being fetched anew behind it.
+  auto stage = [&](int buf, int set, int k0) __attribute__((always_inline)) {
+    constexpr int P = AP + WP, SLOTS = 4 * (CHUNKS - 1);
 #pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const int row = wn + 16 * n + r;
-        w[n] = *reinterpret_cast<const f32x4_t*>(stages[buf] + (BM + row) * BK * 4 + (((4 * c + g) ^ ((row >> 1) & 7)) << 4));
-      }
+    for (int c = 0; c < CHUNKS; ++c) {
+      const bool last = c == CHUNKS - 1;
+      if (last) __syncthreads();
+      take((c + 1) & 1, last ? buf ^ 1 : buf, last ? 0 : c + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
 #pragma unroll
         for (int n = 0; n < TN; ++n)
 #pragma unroll
-          for (int m = 0; m < TM; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n][i], a[m][i], acc[n][m], 0, 0, 0);
+          for (int m = 0; m < TM; ++m)
+            acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[c & 1][n][i], a[c & 1][m][i], acc[n][m], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (!last && p * SLOTS / P == 4 * c + i) {
+            put(set, p, buf ^ 1, k0 + BK);
+            fetch(set, p, k0 + 3 * BK);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
-  fetch(0, 0);
-  put(0, 0);
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int p = 0; p < AP + WP; ++p) fetch(s, p, s * BK);
+#pragma unroll
+  for (int p = 0; p < AP + WP; ++p) {
+    put(0, p, 0, 0);
+    fetch(0, p, 2 * BK);
+  }
   __syncthreads();
-  fetch(0, BK);
-  for (int k0 = 0; k0 < K; k0 += 2 * BK) {
-    // stage k0 lies in buffer 0, set 0 holds stage k0 + BK (on its way)
-    fetch(1, k0 + 2 * BK);
-    products(0);
-    if (k0 + BK < K) put(0, 1);
-    __syncthreads();
+  take(0, 0, 0);
+  for (int k0 = 0;; k0 += 2 * BK) {
+    stage(0, 1, k0);
     if (k0 + BK >= K) break;
-    fetch(0, k0 + 3 * BK);
-    products(1);
-    if (k0 + 2 * BK < K) put(1, 0);
-    __syncthreads();
+    stage(1, 0, k0 + BK);
+    if (k0 + 2 * BK >= K) break;
   }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
@@ -168,19 +185,32 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
   }
 }
 
-template <typename TA, typename TW, typename TC, bool VEC>
+template <typename TA, typename TW, typename TC, int VEC>
 static void launch(const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
                    hipStream_t stream) {
 #define TILE(BM, BN, WGM, BK) do { \
     const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN; \
     hipLaunchKernelGGL((gemm_simple_kernel<TA, TW, TC, BM, BN, WGM, BK, VEC>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), 0, \
                        stream, (const TA*)A, lda, (const TW*)W, ldw, bias, (TC*)C, ldc, M, N, K, mt, nt); } while (0)
-  // 64 x 64 from where they give every compute unit a block and a half: 500 rows x 4096 outputs (512 tiles) 48 us against 64 in
-  // tiles of 32, 500 x 1024 (128 tiles) the other way round
-  auto tiles = [&](long long bm, long long bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  if (M <= 16) TILE(16, 64, 1, 64);
-  else if (tiles(64, 64) >= 400) TILE(64, 64, 2, 32);
-  else TILE(32, 32, 2, 64);
+  // How long each tile takes at K = 1024, in us: what begins and ends a launch and, for every tile that the fullest of 256 compute
+  // units takes, its products (blocks side by side on a unit share the matrix pipe).  Fitted to 15 numbers of rows by 12
+  // matrices, where the choice is within 5 % of the fastest tile; the constants grow alike with K.  Small tiles win while
+  // every unit has one at most (K = 3072, 250 rows of 1024 outputs: 25 us, 35 in tiles of 64 x 32, 57 of 64 x 64), 64 x 64 when
+  // units have many (500 rows of 4096: 50, 40, 39 us), stages of 32 values for 64 x 32 from two on; one to sixteen rows
+  // of many outputs are bound by the matrix's bytes (151 936: 110 us, 122 in tiles of 32 x 32).
+  auto time = [&](long long bm, long long bn, double once, double each) {
+    return once + each * (double)((((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256);
+  };
+  const double times[] = {time(32, 32, 5.0, 5.6), time(32, 64, 4.0, 9.9), time(64, 32, 4.0, 9.9), time(64, 32, 6.5, 9.0),
+                          time(64, 64, 4.0, 17.2), M <= 16 ? time(16, 64, 6.0, 5.0) : 1e30};
+  switch (std::min_element(times, times + 6) - times) {
+    case 0: TILE(32, 32, 2, 64); break;
+    case 1: TILE(32, 64, 2, 64); break;
+    case 2: TILE(64, 32, 2, 64); break;
+    case 3: TILE(64, 32, 2, 32); break;
+    case 4: TILE(64, 64, 2, 32); break;
+    default: TILE(16, 64, 1, 64);
+  }
 #undef TILE
 }
 
@@ -194,8 +224,9 @@ extern "C" int ullm_gemm_simple(const void* A, int lda, const void* W, int ldw, 
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && !((uintptr_t)A & (a_dtype == ULLM_F32 ? 15 : 7)) &&
                    !((uintptr_t)W & (w_dtype == ULLM_F32 ? 15 : 7));
 #define GO(TA, TW, TC) do { \
-    if (vec) launch<TA, TW, TC, true>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream); \
-    else launch<TA, TW, TC, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream); } while (0)
+    if (vec && K % 64 == 0) launch<TA, TW, TC, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream); \
+    else if (vec) launch<TA, TW, TC, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream); \
+    else launch<TA, TW, TC, 0>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream); } while (0)
   const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
   switch (key) {
     case 0: GO(float, float, float); break;
