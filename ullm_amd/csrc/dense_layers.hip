@@ -26,6 +26,7 @@ struct DenseStep {
   decltype(&ullm_add_rmsnorm) add_rmsnorm;
   decltype(&ullm_sum_stacks) sum_stacks;
   decltype(&ullm_qk_norm_rope_write) qk_norm_rope_write;
+  decltype(&ullm_qk_norm_rope_write_sums) qk_norm_rope_write_sums;
   decltype(&ullm_gemm_panels) panels;
   decltype(&ullm_gemm_tiles) tiles;
   decltype(&ullm_attention_decode) decode;
@@ -80,15 +81,22 @@ extern "C" int ullm_dense_layers(const DenseStep* step, const DenseLayer* layers
   for (int i = 0; i < n_layers; ++i) {
     const DenseLayer& l = layers[i];
     STEP(norm(l.norm1, s.eps1));
+    int written = ULLM_ERR_UNSUPPORTED;
     if (s.into.mode == FLOAT) {
       STEP(dense_product(s, s.into, s.normed, H, l.w_qkv, nullptr, s.sums, qkv_width, 0, stream));
-      STEP(s.sum_stacks(s.sums, s.into.slices, l.b_qkv, s.qkv, T, qkv_width, ULLM_BF16, stream));
+      // the heads' kernel adds the slices up, where it can
+      written = s.qk_norm_rope_write_sums(s.sums, s.into.slices, l.b_qkv, qkv_width, s.q, q_width, l.q_gain, l.k_gain, s.qk_eps, l.cos_sin,
+                                          s.table_rows, s.rot, s.style, s.positions, s.token_entry, l.block_table, (int)l.bt_stride, l.k_pool,
+                                          l.v_pool, s.page_size, T, s.heads, s.kv_heads, s.head_dim, (int)l.write_kv, stream);
+      if (written != ULLM_ERR_UNSUPPORTED) STEP(written);
+      else STEP(s.sum_stacks(s.sums, s.into.slices, l.b_qkv, s.qkv, T, qkv_width, ULLM_BF16, stream));
     } else {
       STEP(dense_product(s, s.into, s.normed, H, l.w_qkv, l.b_qkv, s.qkv, qkv_width, 0, stream));
     }
-    STEP(s.qk_norm_rope_write(s.qkv, qkv_width, s.q, q_width, l.q_gain, l.k_gain, s.qk_eps, l.cos_sin, s.table_rows, s.rot, s.style,
-                              s.positions, s.token_entry, l.block_table, (int)l.bt_stride, l.k_pool, l.v_pool, s.page_size, T, s.heads,
-                              s.kv_heads, s.head_dim, (int)l.write_kv, s.heads + s.kv_heads, s.head_dim, ULLM_BF16, stream));
+    if (written != 0)
+      STEP(s.qk_norm_rope_write(s.qkv, qkv_width, s.q, q_width, l.q_gain, l.k_gain, s.qk_eps, l.cos_sin, s.table_rows, s.rot, s.style,
+                                s.positions, s.token_entry, l.block_table, (int)l.bt_stride, l.k_pool, l.v_pool, s.page_size, T, s.heads,
+                                s.kv_heads, s.head_dim, (int)l.write_kv, s.heads + s.kv_heads, s.head_dim, ULLM_BF16, stream));
     // both kinds of tokens in one launch, where that is the better way
     int together = ULLM_ERR_UNSUPPORTED;
     if (s.num_decode > 0 && s.num_tiles > 0) {

@@ -779,9 +779,9 @@ __global__ void qk_norm_rope_write_kernel(
 // single elements; tokens that do not fill such a group are written one by one.
 #define VALUE_RUN_TOKENS 16
 #define VALUE_RUN_MAX_HD 256
-template <typename T>
+template <typename T, typename Row>
 __device__ __forceinline__ void value_runs_block(
-    const T* __restrict__ qkv, int qkv_stride, const int* __restrict__ positions, const int* __restrict__ token_entry,
+    const Row& rows, const int* __restrict__ positions, const int* __restrict__ token_entry,
     const int* __restrict__ block_table, int bt_stride, T* __restrict__ v_pool, int page_size, int v_head0, int nkv,
     int hd, int n_tokens, int block) {
   __shared__ __attribute__((aligned(16))) T tile[VALUE_RUN_TOKENS * VALUE_RUN_MAX_HD];
@@ -792,8 +792,7 @@ __device__ __forceinline__ void value_runs_block(
   const int pieces = hd / PER16;
   for (int c = threadIdx.x; c < n * pieces; c += blockDim.x) {
     const int tok = c / pieces, part = c % pieces;
-    *reinterpret_cast<uint4*>(tile + tok * hd + part * PER16) = *reinterpret_cast<const uint4*>(
-        qkv + (size_t)(tok0 + tok) * qkv_stride + (size_t)(v_head0 + kvh) * hd + part * PER16);
+    *reinterpret_cast<uint4*>(tile + tok * hd + part * PER16) = rows.piece(tok0 + tok, (v_head0 + kvh) * hd + part * PER16);
   }
   if (threadIdx.x < WAVE) {
     // a token leads a run if it is the block's first or does not continue its predecessor's group of 8; the run ends where the next
@@ -861,6 +860,58 @@ template <> struct EightValues<float> {
   }
 };
 
+// The projection's rows [T, qkv_stride] as a product has left them: finished values, or SLICES stacks of 32-bit sums
+// that are added here, in their order, with the bias behind them, and rounded (bit for bit what sum_stacks_kernel leaves).
+template <typename T>
+struct FinishedRows {
+  using Eight = EightValues<T>;
+  const T* qkv;
+  int stride;
+  __device__ __forceinline__ void fetch(Eight& e, int t, int column) const { e.fetch(qkv + (size_t)t * stride + column); }
+  __device__ __forceinline__ uint4 piece(int t, int column) const {
+    return *reinterpret_cast<const uint4*>(qkv + (size_t)t * stride + column);
+  }
+};
+template <int SLICES>
+struct SlicedRows {
+  const float *sums, *bias;
+  int stride;
+  size_t slice;
+  struct Eight {
+    EightValues<float> part[SLICES + 1];                    // the last: the bias
+    bool biased;
+    __device__ __forceinline__ unsigned two(const float (&x)[8], int i) const { return pack2_bf16(x[2 * i], x[2 * i + 1]); }
+    __device__ __forceinline__ uint4 rounded() const {
+      float x[8], y[8];
+      part[0].values(x);
+#pragma unroll
+      for (int s = 1; s <= SLICES; ++s) {
+        if (s == SLICES && !biased) break;
+        part[s].values(y);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] += y[j];
+      }
+      return make_uint4(two(x, 0), two(x, 1), two(x, 2), two(x, 3));
+    }
+    __device__ __forceinline__ void values(float (&x)[8]) const {
+      EightValues<bf16_t> e;
+      e.u = rounded();
+      e.values(x);
+    }
+  };
+  __device__ __forceinline__ void fetch(Eight& e, int t, int column) const {
+#pragma unroll
+    for (int s = 0; s < SLICES; ++s) e.part[s].fetch(sums + (size_t)s * slice + (size_t)t * stride + column);
+    e.biased = bias != nullptr;
+    if (bias) e.part[SLICES].fetch(bias + column);
+  }
+  __device__ __forceinline__ uint4 piece(int t, int column) const {
+    Eight e;
+    fetch(e, t, column);
+    return e.rounded();
+  }
+};
+
 // v of the lane N further back in its row of 16 lanes, the first behind the last
 template <int N>
 __device__ __forceinline__ float row_rotated(float v) {
@@ -881,10 +932,10 @@ __device__ __forceinline__ float row_rotated(float v) {
 // projection's bytes: so the heads of all passes are asked for before anything else, the page once, and value heads that blocks of
 // their own write are not read here.  32 heads over 8 of 128, us with a head's values and page asked for in its pass, eight bytes at a
 // time: 130 tokens 4.9 -> 3.5, 800 10.2 -> 7.1, 2048 18.6 -> 13.3, 12 000 83.6 -> 58.0 (5.0 TB/s).
-template <typename T, int PASSES>
+template <typename T, int PASSES, typename Rows>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_write_vec_kernel(
-    const T* __restrict__ qkv, int qkv_stride, T* __restrict__ q_out, int q_out_stride,
+    const Rows rows, T* __restrict__ q_out, int q_out_stride,
     const float* __restrict__ q_gain, const float* __restrict__ k_gain, float eps,
     const float* __restrict__ cos_sin, int table_rows, int rot, int style,
     const int* __restrict__ positions, const int* __restrict__ token_entry,
@@ -892,8 +943,8 @@ qk_norm_rope_write_vec_kernel(
     int page_size, int nq, int nkv, int hd, int write_kv, int n_tokens, int blocks_per_token,
     int v_head0, int norm_dim) {
   if (blockIdx.x >= (unsigned)(n_tokens * blocks_per_token)) {
-    value_runs_block<T>(qkv, qkv_stride, positions, token_entry, block_table, bt_stride, v_pool, page_size, v_head0, nkv,
-                        hd, n_tokens, (int)blockIdx.x - n_tokens * blocks_per_token);
+    value_runs_block<T>(rows, positions, token_entry, block_table, bt_stride, v_pool, page_size, v_head0, nkv, hd, n_tokens,
+                        (int)blockIdx.x - n_tokens * blocks_per_token);
     return;
   }
   const int lph = hd >> 3;                                  // lanes per head
@@ -901,13 +952,12 @@ qk_norm_rope_write_vec_kernel(
   const int part = threadIdx.x % lph, d0 = 8 * part;
   const int head0 = (blockIdx.x % blocks_per_token) * PASSES * (256 / lph) + threadIdx.x / lph;
   const int heads = write_kv & 2 ? nq + 2 * nkv : nq + nkv;     // those that this kernel reads
-  const T* const row = qkv + (size_t)t * qkv_stride;
-  EightValues<T> held[PASSES];
+  typename Rows::Eight held[PASSES];
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
     int head = head0 + pass * (256 / lph);
     if (head >= heads) head = 0;                            // no load under a condition; not used
-    held[pass].fetch(row + (size_t)(head < nq + nkv ? head : v_head0 + head - nq - nkv) * hd + d0);
+    rows.fetch(held[pass], t, (head < nq + nkv ? head : v_head0 + head - nq - nkv) * hd + d0);
   }
   const int pos = positions[t];
   const int entry = token_entry[t];
@@ -1003,8 +1053,9 @@ qk_norm_rope_write_vec_kernel(
   }
 }
 
-extern "C" int ullm_qk_norm_rope_write(
-    const void* qkv, int qkv_stride, void* q_out, int q_out_stride, const float* q_gain,
+// `slices` 0: qkv is finished rows of `dtype`; else stacks of 32-bit sums [slices, T, qkv_stride] of bfloat16 rows, with `bias`
+static int qk_norm_rope_write(
+    const void* qkv, int slices, const float* bias, int qkv_stride, void* q_out, int q_out_stride, const float* q_gain,
     const float* k_gain, float eps, const float* cos_sin, int table_rows, int rot, int style,
     const int* positions, const int* token_entry, const int* block_table, int bt_stride,
     void* k_pool, void* v_pool, int page_size, int T_, int nq, int nkv, int hd, int write_kv,
@@ -1032,7 +1083,7 @@ extern "C" int ullm_qk_norm_rope_write(
     const int heads_per_block = 256 / lph, read_heads = write_kv && !runs ? nq + 2 * nkv : nq + nkv;
     int blocks_per_token = (read_heads + heads_per_block - 1) / heads_per_block;
     int heads_per_thread = 1;
-    if (T_ >= (dtype == ULLM_F32 ? 1024 : 512)) {
+    if (!slices && T_ >= (dtype == ULLM_F32 ? 1024 : 512)) {
       const int few = (blocks_per_token + 3) / 4;          // blocks of up to four passes, as many in each
       heads_per_thread = (blocks_per_token + few - 1) / few;
       blocks_per_token = few;
@@ -1042,19 +1093,26 @@ extern "C" int ullm_qk_norm_rope_write(
     if (all_blocks > 0x7fffffffLL) return ULLM_ERR_SHAPE;
     const int kv_flags = !write_kv ? 0 : (runs ? 1 : 3);   // bit 0: keys, bit 1: values token by token
     dim3 vgrid((unsigned)all_blocks), vblock(256);
-#define GO(TT, PASSES) hipLaunchKernelGGL((qk_norm_rope_write_vec_kernel<TT, PASSES>), vgrid, vblock, 0, stream, \
-    (const TT*)qkv, qkv_stride, (TT*)q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, \
+#define GO_ROWS(TT, PASSES, ROWS, ...) hipLaunchKernelGGL((qk_norm_rope_write_vec_kernel<TT, PASSES, ROWS>), vgrid, vblock, 0, stream, \
+    (ROWS{__VA_ARGS__}), (TT*)q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, \
     rot, style, positions, token_entry, block_table, bt_stride, (TT*)k_pool, (TT*)v_pool, page_size, \
     nq, nkv, hd, kv_flags, T_, blocks_per_token, v_head0, norm_dim)
+#define GO(TT, PASSES) GO_ROWS(TT, PASSES, FinishedRows<TT>, (const TT*)qkv, qkv_stride)
+#define GO_SLICES(N) GO_ROWS(bf16_t, 1, SlicedRows<N>, (const float*)qkv, bias, qkv_stride, (size_t)T_ * qkv_stride)
 #define GOV(TT) do { if (heads_per_thread == 1) GO(TT, 1); else if (heads_per_thread == 2) GO(TT, 2); \
     else if (heads_per_thread == 3) GO(TT, 3); else GO(TT, 4); } while (0)
-    if (dtype == ULLM_F32) GOV(float);
+    if (slices == 2) GO_SLICES(2);
+    else if (slices == 4) GO_SLICES(4);
+    else if (dtype == ULLM_F32) GOV(float);
     else if (dtype == ULLM_BF16) GOV(bf16_t);
     else return ULLM_ERR_DTYPE;
 #undef GOV
+#undef GO_SLICES
 #undef GO
+#undef GO_ROWS
     ULLM_LAUNCH_CHECK();
   }
+  if (slices) return ULLM_ERR_UNSUPPORTED;
   dim3 grid(T_, nq + 2 * nkv), block(WAVE);
 #define GO(TT) hipLaunchKernelGGL(qk_norm_rope_write_kernel<TT>, grid, block, 0, stream, \
     (const TT*)qkv, qkv_stride, (TT*)q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, \
@@ -1065,6 +1123,33 @@ extern "C" int ullm_qk_norm_rope_write(
   else return ULLM_ERR_DTYPE;
 #undef GO
   ULLM_LAUNCH_CHECK();
+}
+
+extern "C" int ullm_qk_norm_rope_write(
+    const void* qkv, int qkv_stride, void* q_out, int q_out_stride, const float* q_gain,
+    const float* k_gain, float eps, const float* cos_sin, int table_rows, int rot, int style,
+    const int* positions, const int* token_entry, const int* block_table, int bt_stride,
+    void* k_pool, void* v_pool, int page_size, int T_, int nq, int nkv, int hd, int write_kv,
+    int v_head0, int norm_dim, int dtype, hipStream_t stream) {
+  return qk_norm_rope_write(qkv, 0, nullptr, qkv_stride, q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, rot, style, positions,
+                            token_entry, block_table, bt_stride, k_pool, v_pool, page_size, T_, nq, nkv, hd, write_kv, v_head0, norm_dim,
+                            dtype, stream);
+}
+
+// The same for bfloat16 rows that a product has left as 2 or 4 stacks of 32-bit sums [slices, T, stride] (v heads behind the k heads).  A
+// launch that adds them up, its write and this one's read are saved: 32 heads over 8 of 128, us for both launches -> this one: 65 tokens of 4
+// stacks 6.3 -> 4.3, 130 of 2 6.6 -> 4.3, 300 of 4 10.0 -> 8.4, 512 of 2 11.9 -> 7.9.  ULLM_ERR_UNSUPPORTED (and nothing launched): other
+// numbers of stacks, and head sizes and addresses that the kernel of one wave a head takes.
+extern "C" int ullm_qk_norm_rope_write_sums(
+    const float* sums, int slices, const float* bias, int stride, void* q_out, int q_out_stride, const float* q_gain,
+    const float* k_gain, float eps, const float* cos_sin, int table_rows, int rot, int style,
+    const int* positions, const int* token_entry, const int* block_table, int bt_stride,
+    void* k_pool, void* v_pool, int page_size, int T_, int nq, int nkv, int hd, int write_kv, hipStream_t stream) {
+  if (stride < (nq + 2 * nkv) * hd) return ULLM_ERR_SHAPE;
+  if ((slices != 2 && slices != 4) || ((uintptr_t)bias & 15)) return ULLM_ERR_UNSUPPORTED;
+  return qk_norm_rope_write(sums, slices, bias, stride, q_out, q_out_stride, q_gain, k_gain, eps, cos_sin, table_rows, rot, style, positions,
+                            token_entry, block_table, bt_stride, k_pool, v_pool, page_size, T_, nq, nkv, hd, write_kv, nq + nkv, hd,
+                            ULLM_BF16, stream);
 }
 
 // ------------------------------------------------------------------ x *= s

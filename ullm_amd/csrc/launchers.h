@@ -11,6 +11,10 @@ int ullm_qk_norm_rope_write(const void* qkv, int qkv_stride, void* q_out, int q_
                             float eps, const float* cos_sin, int table_rows, int rot, int style, const int* positions,
                             const int* token_entry, const int* block_table, int bt_stride, void* k_pool, void* v_pool, int page_size,
                             int T_, int nq, int nkv, int hd, int write_kv, int v_head0, int norm_dim, int dtype, hipStream_t stream);
+int ullm_qk_norm_rope_write_sums(const float* sums, int slices, const float* bias, int stride, void* q_out, int q_out_stride,
+                                 const float* q_gain, const float* k_gain, float eps, const float* cos_sin, int table_rows, int rot, int style,
+                                 const int* positions, const int* token_entry, const int* block_table, int bt_stride, void* k_pool,
+                                 void* v_pool, int page_size, int T_, int nq, int nkv, int hd, int write_kv, hipStream_t stream);
 int ullm_gemm_panels(const void* x, int ldx, const void* w, int ldw, const float* bias, void* out, int ldo, int M, int N, int K, int mode,
                      int shape, int slices, float limit, float alpha, int act, hipStream_t stream);
 int ullm_gemm_tiles(const void* x, int ldx, const void* w, int ldw, const float* bias, void* out, int ldo, int M, int N, int K, int mode,

@@ -11,8 +11,9 @@ from . import build, ops
 _ptr, _int, _float, _long = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_longlong
 # the entry points the run calls, in the order of the structure's first fields
 LAUNCHERS = (("elementwise", "ullm_add_rmsnorm"), ("elementwise", "ullm_sum_stacks"), ("elementwise", "ullm_qk_norm_rope_write"),
-             ("gemm_panels", "ullm_gemm_panels"), ("gemm_tiles", "ullm_gemm_tiles"), ("attention_mfma", "ullm_attention_decode"),
-             ("attention_mfma", "ullm_attention_prefill"), ("attention_mfma", "ullm_attention_mixed"))
+             ("elementwise", "ullm_qk_norm_rope_write_sums"), ("gemm_panels", "ullm_gemm_panels"), ("gemm_tiles", "ullm_gemm_tiles"),
+             ("attention_mfma", "ullm_attention_decode"), ("attention_mfma", "ullm_attention_prefill"),
+             ("attention_mfma", "ullm_attention_mixed"))
 LAYER_FIELDS = ("norm1", "q_gain", "k_gain", "cos_sin", "b_qkv", "norm2", "w_qkv", "w_o", "w_gate_up", "w_down", "k_pool", "v_pool",
                 "block_table", "bt_stride", "write_kv")          # of 8 bytes each
 
