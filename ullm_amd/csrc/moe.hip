@@ -167,55 +167,117 @@ extern "C" int ullm_moe_route(const float* logits, int ld, const float* correcti
   ULLM_LAUNCH_CHECK();
 }
 
-// The router's product and the routing in one kernel: a block takes TPB tokens; their rows lie in shared memory as
-// 32-bit values, every wave takes four router outputs at a time with four 16-byte pieces of each of their rows a
-// lane under way (the loop is a chain of trips to memory otherwise), and every piece fetched serves all the block's
-// tokens (four tokens and four waves a block for many tokens; one token and sixteen waves for few).  A lane adds a token's pieces in rising order, then the wave adds up: an order that depends on nothing but
-// the row.  Then wave v routes token v.  The router's matrix is 32-bit [n_router, H].
-template <typename T, int TPB>
-__global__ void __launch_bounds__(TPB == 1 ? 1024 : 256)
+// The router's product and the routing in one kernel: a block of WAVES waves takes TPB tokens, whose rows lie in shared memory as
+// they come; every wave takes U router outputs at a time with 16 / U 16-byte pieces of each of their rows a lane under way, and every
+// piece fetched serves all the block's tokens.  A lane adds a token's pieces in rising order, then the wave adds up: an order
+// that depends on nothing but the row.  Then wave v routes token v.  The router's matrix is 32-bit [n_router, H].
+//
+// What bounds it: few tokens by the chain of trips to memory, so the first pieces of the matrix are asked for behind the rows' first
+// and before anything waits, the corrections too, and eight or sixteen waves take up to 32 or 64 outputs in one round; many
+// tokens by the matrix's bytes from the second-level caches, 256 KB a block at 32 outputs of width 2048, and
+// by multiply-adds.  Rows read two bytes a load by four waves, and four of sixteen waves' outputs a round, the matrix asked for behind
+// them: 32 outputs of width 2048 for 48 / 512 / 1000 / 3000 tokens 12.0 -> 11.2, 25.8 -> 13.0, 26.2 -> 14.6, 28.2 -> 21.7 us, width 4096 13.3 -> 12.1,
+// 18 -> 14.7, 29 -> 16.2, 71 -> 29; level for one to 300 tokens of 64 outputs and more, slower by 2 % at 256 outputs of width 1024 and 8000 tokens and
+// at 300 of 640 and 5000; eight tokens a block 20.6 us at 2048 tokens of the first, 34 at 3000.
+template <typename S>
+__device__ __forceinline__ float4 router_values(const S* p);
+template <> __device__ __forceinline__ float4 router_values<float>(const float* p) { return *reinterpret_cast<const float4*>(p); }
+template <> __device__ __forceinline__ float4 router_values<bf16_t>(const bf16_t* p) {
+  const uint2 u = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                     __uint_as_float(u.y & 0xffff0000u));
+}
+typedef __attribute__((ext_vector_type(4))) unsigned router_u32x4;
+// 16 bytes of a row of T, kept as S: as they are or, bfloat16 values, widened
+template <typename T, typename S>
+__device__ __forceinline__ void keep_router_values(S* p, router_u32x4 v) {
+  if constexpr (sizeof(S) == sizeof(T)) {
+    *reinterpret_cast<router_u32x4*>(p) = v;
+  } else {
+    *reinterpret_cast<router_u32x4*>(p) = router_u32x4{v.x << 16, v.x & 0xffff0000u, v.y << 16, v.y & 0xffff0000u};
+    *reinterpret_cast<router_u32x4*>(p + 4) = router_u32x4{v.z << 16, v.z & 0xffff0000u, v.w << 16, v.w & 0xffff0000u};
+  }
+}
+
+template <typename T, typename S, int TPB, int WAVES, bool EARLY>
+__global__ void __launch_bounds__(64 * WAVES)
 moe_router_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ w, const float* __restrict__ correction,
                   int n_tokens, int H, int n_router, int top, int* __restrict__ ids, float* __restrict__ weights, int mode,
                   float weight_scale, int groups, int keep, int raw, int group_top) {
-  extern __shared__ __attribute__((aligned(16))) float xrow[];          // [TPB][H]
+  extern __shared__ __attribute__((aligned(16))) unsigned char router_rows[];
+  S* const xrow = reinterpret_cast<S*>(router_rows);                   // [TPB][H]
   constexpr int RCAP = TPB == 1 ? MOE_MAX_ROUTER : 256;                // router outputs the variant takes
-  __shared__ float z[TPB][RCAP], s_choice[TPB][RCAP];
+  constexpr int U = 4, PJ = 4, NT = 64 * WAVES, PER16 = 16 / (int)sizeof(T), AHEAD = TPB == 1 ? 1 : 4;
+  static_assert(WAVES >= TPB, "a wave routes a token");
+  __shared__ float z[TPB][RCAP], s_choice[TPB][RCAP], s_correction[RCAP];
   __shared__ float s_pick[TPB][MOE_MAX_TOP];
   const int t0 = blockIdx.x * TPB, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool vec = (H & 3) == 0 && (((uintptr_t)w) & 15) == 0;
+  const int pieces = H >> 2;
+  float4 wv[U][PJ];
+  // the wave's U rows of the matrix, the pieces p0 + 64 j of each
+  auto ask = [&](int e0, int p0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < TPB; ++q) {
-    const T* xr = x + (size_t)(t0 + q < n_tokens ? t0 + q : n_tokens - 1) * ldx;
-    for (int i = tid; i < H; i += (int)blockDim.x) xrow[q * H + i] = ld_f32(xr + i);
+    for (int j = 0; j < PJ; ++j) {
+      const int pj = p0 + 64 * j < pieces ? p0 + 64 * j : pieces - 1;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        wv[u][j] = *reinterpret_cast<const float4*>(w + (size_t)(e0 + u < n_router ? e0 + u : n_router - 1) * H + 4 * pj);
+    }
+  };
+  auto token = [&](int q) { return (size_t)(t0 + q < n_tokens ? t0 + q : n_tokens - 1) * ldx; };
+  const float own = correction && tid < n_router ? correction[tid] : 0.f;
+  if (H % PER16 == 0 && ldx % PER16 == 0 && ((uintptr_t)x & 15) == 0) {
+    const int row16 = H / PER16, all = TPB * row16;
+    router_u32x4 held[AHEAD];
+    auto rows = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) {
+        const int i = at + k * NT < all ? at + k * NT : all - 1;
+        const int q = TPB == 1 ? 0 : i / row16;
+        held[k] = *reinterpret_cast<const router_u32x4*>(x + token(q) + (size_t)(i - q * row16) * PER16);
+      }
+    };
+    rows(tid);
+    if (EARLY && vec) ask(U * wave, lane);
+    for (int at = tid;;) {
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k)
+        if (at + k * NT < all) keep_router_values<T, S>(xrow + (size_t)(at + k * NT) * PER16, held[k]);
+      at += AHEAD * NT;
+      if (at - tid >= all) break;
+      rows(at);
+    }
+  } else {
+    if (EARLY && vec) ask(U * wave, lane);
+    for (int q = 0; q < TPB; ++q)
+      for (int i = tid; i < H; i += NT) {
+        if constexpr (sizeof(S) == sizeof(T)) xrow[q * H + i] = x[token(q) + i];
+        else xrow[q * H + i] = ld_f32(x + token(q) + i);
+      }
+  }
+  if (correction) {
+    if (tid < n_router) s_correction[tid] = own;
+    for (int e = tid + NT; e < n_router; e += NT) s_correction[e] = correction[e];
   }
   __syncthreads();
-  const bool vec = (H & 3) == 0 && (((uintptr_t)w) & 15) == 0;
-  for (int e0 = 4 * wave; e0 < n_router; e0 += (int)(blockDim.x >> 4)) {
-    float a[TPB][4];
+  for (int e0 = U * wave; e0 < n_router; e0 += U * WAVES) {
+    float a[TPB][U];
 #pragma unroll
     for (int q = 0; q < TPB; ++q)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) a[q][u] = 0.f;
-    const float* we[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) we[u] = w + (size_t)(e0 + u < n_router ? e0 + u : n_router - 1) * H;
+      for (int u = 0; u < U; ++u) a[q][u] = 0.f;
     if (vec) {
-      const int pieces = H >> 2;
-      for (int p0 = lane; p0 < pieces; p0 += 256) {
-        float4 wv[4][4];
+      for (int p0 = lane; p0 < pieces; p0 += 64 * PJ) {
+        if (!EARLY || e0 != U * wave || p0 != lane) ask(e0, p0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int pj = p0 + 64 * j < pieces ? p0 + 64 * j : pieces - 1;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) wv[u][j] = *reinterpret_cast<const float4*>(we[u] + 4 * pj);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < PJ; ++j) {
           if (p0 + 64 * j >= pieces) break;
 #pragma unroll
           for (int q = 0; q < TPB; ++q) {
-            const float4 xv = *reinterpret_cast<const float4*>(xrow + q * H + 4 * (p0 + 64 * j));
+            const float4 xv = router_values<S>(xrow + q * H + 4 * (p0 + 64 * j));
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < U; ++u)
               a[q][u] = fmaf(xv.w, wv[u][j].w, fmaf(xv.z, wv[u][j].z, fmaf(xv.y, wv[u][j].y, fmaf(xv.x, wv[u][j].x, a[q][u]))));
           }
         }
@@ -225,20 +287,21 @@ moe_router_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ w,
 #pragma unroll
         for (int q = 0; q < TPB; ++q)
 #pragma unroll
-          for (int u = 0; u < 4; ++u) a[q][u] = fmaf(xrow[q * H + i], we[u][i], a[q][u]);
+          for (int u = 0; u < U; ++u)
+            a[q][u] = fmaf(ld_f32(xrow + q * H + i), w[(size_t)(e0 + u < n_router ? e0 + u : n_router - 1) * H + i], a[q][u]);
       }
     }
 #pragma unroll
     for (int q = 0; q < TPB; ++q)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         const float sum = wave_sum(a[q][u]);
         if (lane == 0 && e0 + u < n_router) z[q][e0 + u] = sum;
       }
   }
   __syncthreads();
   if (wave < TPB && t0 + wave < n_tokens)
-    route_from_logits(z[wave], s_choice[wave], s_pick[wave], correction, n_router, top, ids + (size_t)(t0 + wave) * top,
+    route_from_logits(z[wave], s_choice[wave], s_pick[wave], correction ? s_correction : nullptr, n_router, top, ids + (size_t)(t0 + wave) * top,
                       weights + (size_t)(t0 + wave) * top, lane, mode, weight_scale, groups, keep, raw, group_top);
 }
 
@@ -251,17 +314,33 @@ extern "C" int ullm_moe_router(const void* x, int ldx, const float* w, const flo
   if (n_router < 1 || n_router > MOE_MAX_ROUTER || top < 1 || top > MOE_MAX_TOP || top > n_router || H < 1 || ldx < H ||
       (size_t)H * sizeof(float) > 48 * 1024)
     return ULLM_ERR_SHAPE;
-  // many tokens: four a block, so that a piece of the router's matrix is fetched once for four rows (where their rows
-  // and four sets of scores fit shared memory); few: a block each
-  const bool four = T_ >= 512 && (size_t)H * sizeof(float) <= 8 * 1024 && n_router <= 256;
-  const size_t lds = (size_t)H * sizeof(float) * (four ? 4 : 1);
-  // a token a block: sixteen waves, so that up to 64 router outputs are summed in one round of trips to memory
-  dim3 grid(four ? (T_ + 3) / 4 : T_), block(four ? 256 : 1024);
-#define GO(TT, N) hipLaunchKernelGGL((moe_router_kernel<TT, N>), grid, block, lds, stream, (const TT*)x, ldx, w, correction, T_, H, \
-    n_router, top, ids, weights, mode, weight_scale, groups, keep, raw, group_top)
-  if (dtype == ULLM_F32) { if (four) GO(float, 4); else GO(float, 1); }
-  else if (dtype == ULLM_BF16) { if (four) GO(bf16_t, 4); else GO(bf16_t, 1); }
-  else return ULLM_ERR_DTYPE;
+  if (dtype != ULLM_F32 && dtype != ULLM_BF16) return ULLM_ERR_DTYPE;
+#define GO(TT, SS, TPB, WAVES, EARLY) hipLaunchKernelGGL((moe_router_kernel<TT, SS, TPB, WAVES, EARLY>), dim3((T_ + TPB - 1) / TPB), dim3(64 * WAVES), \
+    (size_t)H * sizeof(SS) * TPB, stream, (const TT*)x, ldx, w, correction, T_, H, n_router, top, ids, weights, mode, weight_scale, groups, \
+    keep, raw, group_top)
+#define GOT(TPB, WAVES, EARLY) do { \
+    if (dtype == ULLM_F32) GO(float, float, TPB, WAVES, EARLY); \
+    else if (TPB == 1 || H * TPB <= 8192) GO(bf16_t, float, TPB, WAVES, EARLY); \
+    else if constexpr (TPB > 1) GO(bf16_t, bf16_t, TPB, WAVES, EARLY); } while (0)
+  // Tokens a block, its waves, and whether the matrix is asked for before the rows are there (which takes the registers of two blocks'
+  // waves), by what fills the chip; several tokens where their rows fit 32 KB of shared memory, as 32-bit values if they do, and their scores
+  // beside them.  us on a matrix that is not cached, 1 token of 16 waves / 1 of 8 early / 1 of 8 / 2 of 8 early / 4 of 8 early / 4 of 4
+  // early / 4 of 4.  32 outputs of width 2048: 48 tokens 11.6 / 10.8 / 11.4 / 11.8 / 13.5 / 16.0 / 21.0, 400 13.3 / 13.8 / 13.1 / 12.5 / 13.3 /
+  // 15.5 / 20.4, 1000 22 / 22 / 20 / 18 / 14.3 / 16.5 / 21, 3000 46 / - / - / - / - / 21.5 / 22.8; 128 of 1024: 48 14.7 / 15.3 / 17.3 / 17.4 / 22 / 29 / 39,
+  // 400 21 / 20 / 20 / 18 / 21 / 28 / 38, 1000 36 / 34 / 32 / 27 / 22 / 29 / 39, 3000 75 / - / - / - / - / 42 / 44, 8000 172 / - / - / - / - / 92 / 84;
+  // 16 of 512: 48 7.5 / 8.2 / 7.6 / 9.2 / 10.1 / 10.2 / 9.2, 1000 11.2 / 13.1 / 8.3 / 12.1 / 9.7 / 9.2 / 9.4, 8000 56 / - / - / - / - / 21 / 17.  Width 5120,
+  // where two fit: 24 outputs, 1000 tokens 28 by ones, 18 by twos, 8000 152 and 87.
+  const int most = n_router > 256 ? 1 : 32768 / (H * (dtype == ULLM_F32 ? 4 : 2));
+  if (T_ > 1024 && most >= 4) {
+    if (H <= 512 || (H <= 1024 && T_ > 4096)) GOT(4, 4, false);
+    else GOT(4, 4, true);
+  } else if (T_ > 512 && most >= 4 && H >= 1024) GOT(4, 8, true);
+  else if (T_ > 512 && most >= 2 && H >= 1024) GOT(2, 8, false);
+  else if (T_ > 300 && most >= 2 && H >= 1024) GOT(2, 8, true);
+  else if (T_ > 300 && n_router <= 256) GOT(1, 8, false);
+  else if (n_router <= 32 && H >= 2048) GOT(1, 8, true);
+  else GOT(1, 16, false);
+#undef GOT
 #undef GO
   ULLM_LAUNCH_CHECK();
 }
