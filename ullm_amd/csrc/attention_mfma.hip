@@ -678,6 +678,7 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __re
 // Adds the splits' partials [item][head][split][head_dim + 4] (even shares, of `even` items: [head][share][head_dim + 4]) in their order.  grid (n_items, nq),
 // one wave: lane s first reads split s's maximum and sum (64 splits at a time), then every lane sums
 // its output dims over the splits with the splits' weights passed round by shuffles.
+template <bool EVEN>
 __global__ void __launch_bounds__(64)
 attention_reduce_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int out_stride,
                         const int* __restrict__ token_list, int nq, int hd, int num_splits, int even,
@@ -685,8 +686,8 @@ attention_reduce_kernel(const float* __restrict__ part, bf16_t* __restrict__ out
   const int item = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
   const int t = token_list ? token_list[item] : item;
   const int row = hd + 4;
-  const float* pp = part + ((size_t)(even > 0 ? 0 : item) * nq + head) * num_splits * row;
-  if (even > 0) {
+  const float* pp = part + ((size_t)(EVEN ? 0 : item) * nq + head) * num_splits * row;
+  if constexpr (EVEN) {
     const EvenShares all(num_splits, token_list, positions, even, window, lane);
     num_splits = all.of(all.shares, item);
     pp += (size_t)(all.of(all.end, item) - num_splits) * row;
@@ -1769,8 +1770,11 @@ static int decode_launch(
 #undef ARGS
   int rc = (int)hipGetLastError();
   if (rc != 0 || num_splits == 1) return rc;
-  hipLaunchKernelGGL(attention_reduce_kernel, dim3(n_items, nq), dim3(64), 0, stream, workspace, (bf16_t*)out,
-                     out_stride, token_list, nq, hd, num_splits, even, positions, window, x);
+#define REDUCE(E) hipLaunchKernelGGL((attention_reduce_kernel<E>), dim3(n_items, nq), dim3(64), 0, stream, workspace, (bf16_t*)out, out_stride, \
+    token_list, nq, hd, num_splits, even, positions, window, x)
+  if (even) REDUCE(true);
+  else REDUCE(false);
+#undef REDUCE
   ULLM_LAUNCH_CHECK();
 }
 
