@@ -2180,12 +2180,8 @@ def moe_rows(x: torch.Tensor, row_index: Optional[torch.Tensor], w: torch.Tensor
     return out
 
 
-def moe_combine(y: Optional[torch.Tensor], x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
-                slot_of_pair: torch.Tensor, n_experts: int, base: Optional[torch.Tensor] = None,
-                bias: Optional[torch.Tensor] = None, shared: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """float32 [T, H]: ``base`` + ``bias`` + ``shared`` + the sum over a token's chosen experts, in their order, of
-    weight times the expert's row of ``y`` (float32 [slots, H]) or, for an expert index >= ``n_experts``, times the
-    token's own row of ``x``."""
+def _check_combine(y, x, ids, weights, slot_of_pair, n_experts, base, bias, shared) -> int:
+    """The dtype code of ``base``, once everything is as the sums over experts take it."""
     T, H = x.shape
     top = ids.shape[1]
     _need(x.stride(1) == 1, "x must have unit stride along its rows")
@@ -2202,11 +2198,41 @@ def moe_combine(y: Optional[torch.Tensor], x: torch.Tensor, ids: torch.Tensor, w
         _need(bias.dtype == torch.float32 and bias.numel() == H and bias.is_contiguous(), "bias must be float32 [H]")
     if shared is not None:
         _need(shared.shape == (T, H) and shared.is_contiguous() and shared.dtype == x.dtype, "shared must be [T, H] of x's dtype")
+    return base_dt
+
+
+def moe_combine(y: Optional[torch.Tensor], x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
+                slot_of_pair: torch.Tensor, n_experts: int, base: Optional[torch.Tensor] = None,
+                bias: Optional[torch.Tensor] = None, shared: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """float32 [T, H]: ``base`` + ``bias`` + ``shared`` + the sum over a token's chosen experts, in their order, of
+    weight times the expert's row of ``y`` (float32 [slots, H]) or, for an expert index >= ``n_experts``, times the
+    token's own row of ``x``."""
+    T, H = x.shape
+    base_dt = _check_combine(y, x, ids, weights, slot_of_pair, n_experts, base, bias, shared)
     out = torch.empty((T, H), dtype=torch.float32, device=x.device)
     _check(build.load("moe").ullm_moe_combine(_p(y), _p(x), _c_int(x.stride(0)), _p(ids), _p(weights), _p(slot_of_pair),
-                                              _c_int(top), _c_int(n_experts), _p(base), _c_int(base_dt), _p(bias),
+                                              _c_int(ids.shape[1]), _c_int(n_experts), _p(base), _c_int(base_dt), _p(bias),
                                               _p(shared), _p(out), _c_int(T), _c_int(H), _c_int(_dt(x)), _stream()),
            "moe_combine")
+    return out
+
+
+def moe_combine_tanh(y: Optional[torch.Tensor], x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, slot_of_pair: torch.Tensor,
+                     n_experts: int, residual: torch.Tensor, alpha: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor, mult: float = 1.0,
+                     base: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
+                     shared: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`add_tanh` of what :func:`moe_combine` would return, in ``x``'s dtype and in one kernel: residual (float32
+    [T, H], in place) += mult * sum; returns tanh(alpha * residual) * gain + shift."""
+    T, H = x.shape
+    base_dt = _check_combine(y, x, ids, weights, slot_of_pair, n_experts, base, bias, shared)
+    _need(residual.dtype == torch.float32 and residual.shape == (T, H) and residual.is_contiguous(), "residual must be contiguous float32 [T, H]")
+    for g, n, nm in ((alpha, 1, "alpha"), (gain, H, "gain"), (shift, H, "shift")):
+        _need(g.dtype == torch.float32 and g.numel() == n and g.is_contiguous(), f"{nm} must be float32 with {n} values")
+    out = torch.empty((T, H), dtype=x.dtype, device=x.device)
+    _check(build.load("moe").ullm_moe_combine_tanh(
+        _p(y), _p(x), _c_int(x.stride(0)), _p(ids), _p(weights), _p(slot_of_pair), _c_int(ids.shape[1]), _c_int(n_experts), _p(base),
+        _c_int(base_dt), _p(bias), _p(shared), _c_float(mult), _p(residual), _p(alpha), _p(gain), _p(shift), _p(out), _c_int(T), _c_int(H),
+        _c_int(_dt(x)), _stream()), "moe_combine_tanh")
     return out
 
 

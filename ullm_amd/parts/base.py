@@ -345,6 +345,33 @@ class NormedBranch:
         return ops.weighted_sum(one_branch(self.branch), one_branch(self.second), self.a, self.b)
 
 
+class SummedBranch(NormedBranch):
+    """A branch without a norm behind it whose last kernel, a sum over experts, is still to run: a norm that looks at no other column makes
+    it part of its own kernel (``into``); for anyone else it runs when ``branch`` is first asked for."""
+    post = second = None
+    a = b = 1.0
+
+    def __init__(self, total: Callable[[], torch.Tensor], into: Callable[..., torch.Tensor], dtype: torch.dtype, mult: float = 1.0):
+        """``total()``: the sum, float32 [T, hidden].  ``into(residual, alpha, gain, shift, mult)``: added to the stream and squashed, in
+        ``dtype``."""
+        self._total, self._into, self._made = total, into, None
+        self.dtype, self.mult = dtype, mult
+
+    @property
+    def branch(self) -> torch.Tensor:
+        if self._made is None:
+            self._made, self._total, self._into = self._total(), None, None
+        return self._made
+
+    def added_and_squashed(self, residual: torch.Tensor, alpha: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
+                           out_dtype: torch.dtype) -> Optional[torch.Tensor]:
+        """The next sublayers' input, the stream being updated in place; None (and nothing done) where the sum is made already or the
+        input is wanted in another dtype."""
+        if self._into is None or out_dtype != self.dtype:
+            return None
+        return self._into(residual, alpha, gain, shift, self.mult)
+
+
 def one_branch(y: torch.Tensor) -> torch.Tensor:
     """A branch as one tensor [T, hidden]: a stack [S, T, hidden] of partial sums is added up."""
     from ..kernels import ops

@@ -14,6 +14,7 @@ import torch
 from ..kernels import ops
 from .base import (Block, FeedForward, LayerCache, Mixer, Norm, NormedBranch, PartEnv, PendingNorm, StateNeed, StepContext, StreamsBranch,
                    WeightDecl, one_branch, register_part, whole_branch)
+from .moe import RoutedExperts
 
 
 @register_part("block", "prenorm")
@@ -136,6 +137,8 @@ class ParallelBlock(Block):
             return residual, NormedBranch(whole_branch(self.mixer.forward, ctx, h, ctx, cache), None, self.mult)
         if hasattr(self.ffn, "forward_onto"):
             mixed = whole_branch(self.mixer.forward, ctx, h, ctx, cache)
+            if type(self.ffn) is RoutedExperts and "forward_onto" not in self.ffn.__dict__:
+                return residual, self.ffn.branch_onto(h, ctx, mixed, self.mult)
             return residual, NormedBranch(self.ffn.forward_onto(h, ctx, mixed), None, self.mult)
         # one kernel adds the two branches, whichever of them are stacks of partial sums
         mixed = self.mixer.forward(h, ctx, cache)

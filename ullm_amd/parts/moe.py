@@ -31,7 +31,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..kernels import ops
-from .base import FeedForward, PartEnv, StepContext, WeightDecl, register_part
+from .base import FeedForward, PartEnv, StepContext, SummedBranch, WeightDecl, register_part
 from .linear import gate_up, linear
 
 DEFAULT_NAMES = {"router": "router", "correction": "correction", "expert": "e{index}", "gate": "gate", "up": "up",
@@ -227,6 +227,18 @@ class RoutedExperts(FeedForward):
     def forward_onto(self, x: torch.Tensor, ctx: StepContext, base: Optional[torch.Tensor],
                      bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """float32 [T, hidden]: ``base`` (another branch's output, or None) + ``bias`` + this feed-forward of x."""
+        *products, shared = self._products(x, ctx)
+        return ops.moe_combine(*products, base=base, bias=bias, shared=shared)
+
+    def branch_onto(self, x: torch.Tensor, ctx: StepContext, base: Optional[torch.Tensor], mult: float) -> SummedBranch:
+        """``forward_onto`` whose last kernel is left to whoever adds the branch to the stream."""
+        *products, shared = self._products(x, ctx)
+        return SummedBranch(lambda: ops.moe_combine(*products, shared=shared, base=base),
+                            lambda residual, alpha, gain, shift, m: ops.moe_combine_tanh(*products, residual, alpha, gain, shift, m, base=base,
+                                                                                         shared=shared), x.dtype, mult)
+
+    def _products(self, x: torch.Tensor, ctx: StepContext) -> tuple:
+        """What the last kernel adds up: the experts' rows, x, ids, weights, every pair's slot, the experts' number, the shared expert's rows."""
         T = x.shape[0]
         ids, weights = self.route(x)
         y = None
@@ -243,4 +255,4 @@ class RoutedExperts(FeedForward):
             # gate | up with the unit on store where the few-rows kernels take the step, as the dense feed-forward's
             act = gate_up(x, self.w_shared_gate_up, self.shared_limit, self.alpha)
             shared = linear(act, self.w_shared_down)
-        return ops.moe_combine(y, x, ids, weights, slot_of_pair, self.experts, base=base, bias=bias, shared=shared)
+        return y, x, ids, weights, slot_of_pair, self.experts, shared

@@ -11,7 +11,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..kernels import ops
-from .base import Norm, NormedBranch, PartEnv, PendingNorm, WeightDecl, register_part
+from .base import Norm, NormedBranch, PartEnv, PendingNorm, SummedBranch, WeightDecl, register_part
 
 
 @register_part("norm", "rmsnorm")
@@ -123,6 +123,10 @@ class DynamicTanh(Norm):
             if branch.post is not None:
                 raise TypeError("dynamic_tanh adds a branch as it is: no norm can stand behind it")
             mult = branch.mult
+            if isinstance(branch, SummedBranch) and rows is None and out_dtype is not None:
+                y = branch.added_and_squashed(residual, self.alpha, self.gain, self.shift, out_dtype)
+                if y is not None:
+                    return y
             branch = branch.branch if branch.second is None else branch.joined()
         if out_dtype is None:
             out_dtype = branch.dtype if branch is not None and branch.dim() == 2 else torch.float32
