@@ -1063,6 +1063,20 @@ def gemm_simple(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return out
 
 
+def gemm_simple_silu(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(a G^T) * (a U^T) for float32 a [M, K] and w = G | U [2 I, K]: :func:`gemm_simple` and :func:`silu_mul` in one kernel."""
+    M, K = a.shape
+    N, K2 = w.shape
+    _need(a.dtype == w.dtype == torch.float32, "the gated 32-bit product takes float32")
+    _need(K == K2 and N % 2 == 0, f"a is [{M}, {K}], w must be [2 I, {K}], is [{N}, {K2}]")
+    _need(a.stride(1) == 1 and w.stride(1) == 1, "a and w must have unit stride along K")
+    out = torch.empty((M, N // 2), dtype=torch.float32, device=a.device)
+    _check(build.load("gemm_simple").ullm_gemm_simple_gated(
+        _p(a), _c_int(a.stride(0)), _p(w), _c_int(w.stride(0)), _p(out), _c_int(out.stride(0)), _c_int(M), _c_int(N // 2), _c_int(K),
+        _stream()), "gemm_simple_silu")
+    return out
+
+
 def _skinny_ok(M: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     return (w.dtype == torch.bfloat16 and 1 <= M <= 64 and K % 8 == 0 and K >= 8 and x.stride(1) == 1
             and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
