@@ -1562,7 +1562,8 @@ prefill_dma_block(int block, unsigned char* lds, int (*page_ids)[DmaBlock<NQK, H
   loads_left<0>();
   __syncthreads();
   if (KS > 1) {
-    // the parts behind the first hand (reference value, sum, output) over, which the first adds in their order
+    // The parts behind the first hand (reference value, sum, output) over, which the first adds in their order.  Which of a sum's two
+    // products is rounded by itself is written out: left to the compiler it differs between the kernels this is part of.
     float* const w = reinterpret_cast<float*>(lds) + (size_t)wave * PER_LANE * 64 + lane;
     constexpr int PART = TEAM * PER_LANE * 64;
     if (part > 0) {
@@ -1591,8 +1592,8 @@ prefill_dma_block(int block, unsigned char* lds, int (*page_ids)[DmaBlock<NQK, H
         for (int n = 0; n < 2 * NQK; ++n)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            acc[qg][n][e] = acc[qg][n][e] * fa + its[(qg * (8 * NQK + 2) + 4 * n + e) * 64] * fb;
-        l[qg] = l[qg] * fa + l_b * fb;
+            acc[qg][n][e] = fmaf(acc[qg][n][e], fa, its[(qg * (8 * NQK + 2) + 4 * n + e) * 64] * fb);
+        l[qg] = fmaf(l[qg], fa, l_b * fb);
         m[qg] = M;
       }
     }
