@@ -347,7 +347,8 @@ class NormedBranch:
 
 class SummedBranch(NormedBranch):
     """A branch without a norm behind it whose last kernel, a sum over experts, is still to run: a norm that looks at no other column makes
-    it part of its own kernel (``into``); for anyone else it runs when ``branch`` is first asked for."""
+    it part of its own kernel (``into``); for anyone else it runs when ``branch`` is first asked for.  What it sums is let go as soon as
+    the sum is made or added, for the branch itself lives on through the next block; once added it is used up."""
     post = second = None
     a = b = 1.0
 
@@ -357,19 +358,26 @@ class SummedBranch(NormedBranch):
         self._total, self._into, self._made = total, into, None
         self.dtype, self.mult = dtype, mult
 
+    def _taken(self, which: str) -> Callable[..., torch.Tensor]:
+        if self._total is None:
+            raise RuntimeError("this branch is in the stream already: adding it again would count it twice")
+        run = getattr(self, which)
+        self._total = self._into = None
+        return run
+
     @property
     def branch(self) -> torch.Tensor:
         if self._made is None:
-            self._made, self._total, self._into = self._total(), None, None
+            self._made = self._taken("_total")()
         return self._made
 
     def added_and_squashed(self, residual: torch.Tensor, alpha: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
                            out_dtype: torch.dtype) -> Optional[torch.Tensor]:
         """The next sublayers' input, the stream being updated in place; None (and nothing done) where the sum is made already or the
         input is wanted in another dtype."""
-        if self._into is None or out_dtype != self.dtype:
+        if self._made is not None or out_dtype != self.dtype:
             return None
-        return self._into(residual, alpha, gain, shift, self.mult)
+        return self._taken("_into")(residual, alpha, gain, shift, self.mult)
 
 
 def one_branch(y: torch.Tensor) -> torch.Tensor:
