@@ -290,7 +290,10 @@ class Mixer(Part):
 
 class FeedForward(Part):
     """``forward(x [T, hidden], ctx) -> [T, hidden]``; keeps nothing between steps.
-    ``fusable``, ``forward_fused(x, residual, ctx)``, ``folds_norm`` and ``hands_norm_ahead`` as for mixers."""
+    ``fusable``, ``forward_fused(x, residual, ctx)``, ``folds_norm`` and ``hands_norm_ahead`` as for mixers.
+    May offer ``forward_onto(x, ctx, base) -> [T, hidden]``, another branch's output and its own added up, and beside it
+    ``branch_onto(x, ctx, base, mult)``, the same times ``mult`` as a :class:`NormedBranch` whose last kernel may be left to a norm that
+    ``takes_sums``."""
     kind = "ffn"
     folds_norm = False
     hands_norm_ahead = False
@@ -419,9 +422,11 @@ class Norm(Part):
     ``pending(residual, out_dtype)``: a :class:`PendingNorm` of a stream with nothing left to add, for
     a consumer with ``folds_norm``, or None if this norm has no such form; with ``scaled`` and ``squares``
     where a product prepared them.  ``ahead_gain()``: the float32 gain [hidden] such a product multiplies
-    the stream by, or None if this norm is not a gain times rsqrt(mean of squares + eps)."""
+    the stream by, or None if this norm is not a gain times rsqrt(mean of squares + eps).
+    ``takes_sums``: the norm can make the sum of a :class:`SummedBranch` part of its own kernel."""
     kind = "norm"
     adds_stacks = False
+    takes_sums = False
 
     def kernel_form(self):
         """(gain float32 [hidden], eps, kind) with kind one of ``ops.NORM_RMS`` / ``ops.NORM_LAYER`` for a norm that

@@ -14,7 +14,6 @@ import torch
 from ..kernels import ops
 from .base import (Block, FeedForward, LayerCache, Mixer, Norm, NormedBranch, PartEnv, PendingNorm, StateNeed, StepContext, StreamsBranch,
                    WeightDecl, one_branch, register_part, whole_branch)
-from .moe import RoutedExperts
 
 
 @register_part("block", "prenorm")
@@ -115,7 +114,8 @@ class ParallelBlock(Block):
     h = norm(x); x += mult * (mixer(h) + ffn(h)).  A block without a feed-forward (``ffn`` None) adds the mixer
     alone.  The sum of the two branches is 32-bit and travels on as the pending branch; the next norm of the
     stream multiplies, adds and norms in one pass.  A feed-forward that offers ``forward_onto(x, ctx, base)`` adds
-    its result onto the mixer's in its own last kernel."""
+    its result onto the mixer's in its own last kernel; where it offers ``branch_onto`` too and the blocks' norm takes
+    sums, that kernel is left to the norm."""
 
     def __init__(self, norm: Norm, mixer: Mixer, ffn: Optional[FeedForward] = None, mult: float = 1.0):
         self.norm, self.mixer, self.ffn, self.mult = norm, mixer, ffn, float(mult)
@@ -137,7 +137,7 @@ class ParallelBlock(Block):
             return residual, NormedBranch(whole_branch(self.mixer.forward, ctx, h, ctx, cache), None, self.mult)
         if hasattr(self.ffn, "forward_onto"):
             mixed = whole_branch(self.mixer.forward, ctx, h, ctx, cache)
-            if type(self.ffn) is RoutedExperts and "forward_onto" not in self.ffn.__dict__:
+            if getattr(self.norm, "takes_sums", False) and hasattr(self.ffn, "branch_onto"):
                 return residual, self.ffn.branch_onto(h, ctx, mixed, self.mult)
             return residual, NormedBranch(self.ffn.forward_onto(h, ctx, mixed), None, self.mult)
         # one kernel adds the two branches, whichever of them are stacks of partial sums

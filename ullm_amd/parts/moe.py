@@ -31,7 +31,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..kernels import ops
-from .base import FeedForward, PartEnv, StepContext, SummedBranch, WeightDecl, register_part
+from .base import FeedForward, NormedBranch, PartEnv, StepContext, SummedBranch, WeightDecl, register_part
 from .linear import gate_up, linear
 
 DEFAULT_NAMES = {"router": "router", "correction": "correction", "expert": "e{index}", "gate": "gate", "up": "up",
@@ -230,8 +230,10 @@ class RoutedExperts(FeedForward):
         *products, shared = self._products(x, ctx)
         return ops.moe_combine(*products, base=base, bias=bias, shared=shared)
 
-    def branch_onto(self, x: torch.Tensor, ctx: StepContext, base: Optional[torch.Tensor], mult: float) -> SummedBranch:
+    def branch_onto(self, x: torch.Tensor, ctx: StepContext, base: Optional[torch.Tensor], mult: float) -> NormedBranch:
         """``forward_onto`` whose last kernel is left to whoever adds the branch to the stream."""
+        if type(self).forward_onto is not RoutedExperts.forward_onto:      # a subclass that changes the sum
+            return NormedBranch(self.forward_onto(x, ctx, base), None, mult)
         *products, shared = self._products(x, ctx)
         return SummedBranch(lambda: ops.moe_combine(*products, shared=shared, base=base),
                             lambda residual, alpha, gain, shift, m: ops.moe_combine_tanh(*products, residual, alpha, gain, shift, m, base=base,

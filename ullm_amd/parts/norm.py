@@ -101,6 +101,7 @@ class DynamicTanh(Norm):
     ``alpha`` is one learned number, ``gain`` and ``shift`` are as long as the row; the tensors are ``weight_name``,
     ``<weight_name>.alpha`` and ``<weight_name>.b`` (or what ``alpha_name`` and ``shift_name`` say)."""
     adds_stacks = True
+    takes_sums = True
 
     def __init__(self, size: int, weight_name: str, alpha_name: Optional[str] = None, shift_name: Optional[str] = None):
         self.size, self.weight_name = size, weight_name
