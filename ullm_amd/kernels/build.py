@@ -32,7 +32,7 @@ HIPCC_FLAGS = [
 ]
 HEADERS = ["common.h"]
 FAMILY_HEADERS = {"gemm_simple": ["mfma_f32.h"], "attention_generic": ["lds_load.h", "mfma_f32.h"],
-                  "attention_mfma": ["no_alloc.h", "lds_load.h", "launchers.h"], "moe": ["lds_load.h", "mfma_tiles.h"],
+                  "attention_mfma": ["no_alloc.h", "lds_load.h", "launchers.h", "prefill_dma_block.h"], "moe": ["lds_load.h", "mfma_tiles.h"],
                   "decay_scan": ["decay_inputs.h"], "decay_chunks": ["decay_inputs.h"],
                   "gemm_tiles": ["lds_load.h", "mfma_tiles.h", "launchers.h"],
                   "gemm_panels": ["lds_load.h", "mfma_tiles.h", "launchers.h"],
