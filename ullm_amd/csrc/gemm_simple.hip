@@ -210,6 +210,24 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
   }
 }
 
+// Compute units of the current device (asked once per device).
+static int simple_compute_units() {
+  static int units[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (units[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    units[dev] = n;
+  }
+  return units[dev];
+}
+
+// How many tiles the fullest unit takes.
+static long long fullest(long long M, long long N, int bm, int bn, int units) {
+  return (((M + bm - 1) / bm) * ((N + bn - 1) / bn) + units - 1) / units;
+}
+
 template <typename TA, typename TW, typename TC, int VEC>
 static void launch(const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
                    hipStream_t stream) {
@@ -217,15 +235,14 @@ static void launch(const void* A, int lda, const void* W, int ldw, const float* 
     const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN; \
     hipLaunchKernelGGL((gemm_simple_kernel<TA, TW, TC, BM, BN, WGM, BK, VEC>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), 0, \
                        stream, (const TA*)A, lda, (const TW*)W, ldw, bias, (TC*)C, ldc, M, N, K, mt, nt); } while (0)
-  // How long each tile takes at K = 1024, in us: what begins and ends a launch and, for every tile that the fullest of 256 compute
-  // units takes, its products (blocks side by side on a unit share the matrix pipe).  Fitted to 15 numbers of rows by 12
+  // How long each tile takes at K = 1024, in us: what begins and ends a launch and, for every tile that the fullest compute
+  // unit takes, its products (blocks side by side on a unit share the matrix pipe).  Fitted to 15 numbers of rows by 12
   // matrices, where the choice is within 5 % of the fastest tile; the constants grow alike with K.  Small tiles win while
   // every unit has one at most (K = 3072, 250 rows of 1024 outputs: 25 us, 35 in tiles of 64 x 32, 57 of 64 x 64), 64 x 64 when
   // units have many (500 rows of 4096: 50, 40, 39 us), stages of 32 values for 64 x 32 from two on; one to sixteen rows
   // of many outputs are bound by the matrix's bytes (151 936: 110 us, 122 in tiles of 32 x 32).
-  auto time = [&](long long bm, long long bn, double once, double each) {
-    return once + each * (double)((((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256);
-  };
+  const int units = simple_compute_units();
+  auto time = [&](int bm, int bn, double once, double each) { return once + each * (double)fullest(M, N, bm, bn, units); };
   const double times[] = {time(32, 32, 5.0, 5.6), time(32, 64, 4.0, 9.9), time(64, 32, 4.0, 9.9), time(64, 32, 6.5, 9.0),
                           time(64, 64, 4.0, 17.2), M <= 16 ? time(16, 64, 6.0, 5.0) : 1e30};
   switch (std::min_element(times, times + 6) - times) {
@@ -281,8 +298,8 @@ extern "C" int ullm_gemm_simple_gated(const float* A, int lda, const float* W, i
     hipLaunchKernelGGL((gemm_simple_kernel<float, float, float, BM, 64, 2, BK, VEC, true>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), \
                        0, stream, A, lda, W, ldw, (const float*)nullptr, out, ldo, M, N, K, mt, nt); } while (0)
 #define GO(VEC) do { if (small) TILE(32, 64, VEC); else TILE(64, 32, VEC); } while (0)
-  auto time = [&](long long bm, double each) { return each * (double)((((M + bm - 1) / bm) * nt + 255) / 256); };
-  const bool small = time(32, 9.9) <= time(64, 17.2);    // us a tile of the fullest unit, as in launch()
+  const int units = simple_compute_units();
+  const bool small = 9.9 * fullest(M, N, 32, 64, units) <= 17.2 * fullest(M, N, 64, 64, units);    // us a tile of the fullest unit, as in launch()
   if (vec && K % 64 == 0) GO(2);
   else if (vec) GO(1);
   else GO(0);
