@@ -228,6 +228,19 @@ static long long fullest(long long M, long long N, int bm, int bn, int units) {
   return (((M + bm - 1) / bm) * ((N + bn - 1) / bn) + units - 1) / units;
 }
 
+// How long each tile takes at K = 1024, in us: what begins and ends a launch and, for every tile that the fullest compute
+// unit takes, its products (blocks side by side on a unit share the matrix pipe).  Fitted to 15 numbers of rows by 12
+// matrices, where the choice is within 5 % of the fastest tile; the constants grow alike with K.  Small tiles win while
+// every unit has one at most (K = 3072, 250 rows of 1024 outputs: 25 us, 35 in tiles of 64 x 32, 57 of 64 x 64), 64 x 64 when
+// units have many (500 rows of 4096: 50, 40, 39 us), stages of 32 values for 64 x 32 from two on; one to sixteen rows
+// of many outputs are bound by the matrix's bytes (151 936: 110 us, 122 in tiles of 32 x 32).
+static int product_tile(int M, int N, int units) {
+  auto time = [&](int bm, int bn, double once, double each) { return once + each * (double)fullest(M, N, bm, bn, units); };
+  const double times[] = {time(32, 32, 5.0, 5.6), time(32, 64, 4.0, 9.9), time(64, 32, 4.0, 9.9), time(64, 32, 6.5, 9.0),
+                          time(64, 64, 4.0, 17.2), M <= 16 ? time(16, 64, 6.0, 5.0) : 1e30};
+  return (int)(std::min_element(times, times + 6) - times);
+}
+
 template <typename TA, typename TW, typename TC, int VEC>
 static void launch(const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
                    hipStream_t stream) {
@@ -235,17 +248,7 @@ static void launch(const void* A, int lda, const void* W, int ldw, const float* 
     const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN; \
     hipLaunchKernelGGL((gemm_simple_kernel<TA, TW, TC, BM, BN, WGM, BK, VEC>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), 0, \
                        stream, (const TA*)A, lda, (const TW*)W, ldw, bias, (TC*)C, ldc, M, N, K, mt, nt); } while (0)
-  // How long each tile takes at K = 1024, in us: what begins and ends a launch and, for every tile that the fullest compute
-  // unit takes, its products (blocks side by side on a unit share the matrix pipe).  Fitted to 15 numbers of rows by 12
-  // matrices, where the choice is within 5 % of the fastest tile; the constants grow alike with K.  Small tiles win while
-  // every unit has one at most (K = 3072, 250 rows of 1024 outputs: 25 us, 35 in tiles of 64 x 32, 57 of 64 x 64), 64 x 64 when
-  // units have many (500 rows of 4096: 50, 40, 39 us), stages of 32 values for 64 x 32 from two on; one to sixteen rows
-  // of many outputs are bound by the matrix's bytes (151 936: 110 us, 122 in tiles of 32 x 32).
-  const int units = simple_compute_units();
-  auto time = [&](int bm, int bn, double once, double each) { return once + each * (double)fullest(M, N, bm, bn, units); };
-  const double times[] = {time(32, 32, 5.0, 5.6), time(32, 64, 4.0, 9.9), time(64, 32, 4.0, 9.9), time(64, 32, 6.5, 9.0),
-                          time(64, 64, 4.0, 17.2), M <= 16 ? time(16, 64, 6.0, 5.0) : 1e30};
-  switch (std::min_element(times, times + 6) - times) {
+  switch (product_tile(M, N, simple_compute_units())) {
     case 0: TILE(32, 32, 2, 64); break;
     case 1: TILE(32, 64, 2, 64); break;
     case 2: TILE(64, 32, 2, 64); break;
@@ -282,6 +285,35 @@ extern "C" int ullm_gemm_simple(const void* A, int lda, const void* W, int ldw, 
   ULLM_LAUNCH_CHECK();
 }
 
+// Whether the gated product takes tiles of 32 rows, not of 64: us a tile of the fullest unit, as in product_tile.
+static bool gated_in_small_tiles(int M, int I, int units) {
+  return 9.9 * fullest(M, 2LL * I, 32, 64, units) <= 17.2 * fullest(M, 2LL * I, 64, 64, units);
+}
+
+// 1 where ullm_gemm_simple_gated is expected ahead of the product and the activation kernel behind it, on a device of `units` compute units.  It has
+// two tiles, those in which a wave holds pairs of gate and up; the product takes smaller or longer ones where these fill the chip better, most of
+// all where tiles of 32 x 32 are one a unit at most: 64 rows of 2 x 1408 columns, K = 2048, 19.7 us in two kernels and 24.6 in one, 17 of 2 x 3072,
+// K = 1024, 13.4 and 14.5, 192 of 2 x 5504, K = 2048, 95.0 and 98.7; but 65 of the first 27.6 and 24.7, 500 of the second 59.9 and 54.3.
+// Times in us of each tile, once and for every one that the fullest unit takes at K = 1024, and of the activation, by 390 pairs (17 to 2048
+// rows, 13 matrices): the choice is within 1.5 % of the better one in all; a tie is the gated product's.
+// Not `captured` (for a graph's replays): the host launches one after the other, and two launches take it 16 us (17 rows of 2 x 512 columns, K = 512: 8.3 and
+// 8.8 us in a graph, 15.2 and 8.3 without; prompts of 17 tokens of a 0.6B model 2.88 and 2.81 ms, decode of 17 requests the other way round).
+extern "C" int ullm_gemm_simple_gated_ahead(int M, int I, int K, int captured, int units) {
+  if (M <= 16 || I <= 0 || K <= 0 || units <= 0 || I > 0x3fffffff) return 0;
+  auto time = [&](int bm, int bn, double once, double each) { return once + each * K / 1024.0 * (double)fullest(M, 2LL * I, bm, bn, units); };
+  double two = 2.04 + 1.82e-6 * M * I;                     // the activation kernel
+  switch (product_tile(M, 2 * I, units)) {
+    case 0: two += time(32, 32, 3.67, 6.36); break;
+    case 1: two += time(32, 64, 4.6, 10.17); break;
+    case 2: two += time(64, 32, 4.6, 10.17); break;
+    case 3: two += time(64, 32, 3.47, 9.47); break;
+    default: two += time(64, 64, 6.0, 16.85);
+  }
+  if (!captured && two < 16.0) two = 16.0;
+  const double one = gated_in_small_tiles(M, I, units) ? time(32, 64, 4.06, 10.14) : time(64, 64, 5.63, 16.8);
+  return one <= 1.005 * two;
+}
+
 // silu(A G^T) * (A U^T) of 32-bit operands, W = G | U [2 I, K], out [M, I]: the product above with the gated unit on store, in the tiles in which a
 // wave holds gate and up of the same columns.  The bits are those of the product and the activation kernel behind it.  us for
 // both and for this one, 2 x 3072 columns, K = 1024: 40 rows 16.9, 14.3, 130 27.3, 23.9, 500 59.9, 54.3, 2048 227, 211; 2 x 6144, K = 2048: 40 rows 43, 40,
@@ -298,8 +330,7 @@ extern "C" int ullm_gemm_simple_gated(const float* A, int lda, const float* W, i
     hipLaunchKernelGGL((gemm_simple_kernel<float, float, float, BM, 64, 2, BK, VEC, true>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), \
                        0, stream, A, lda, W, ldw, (const float*)nullptr, out, ldo, M, N, K, mt, nt); } while (0)
 #define GO(VEC) do { if (small) TILE(32, 64, VEC); else TILE(64, 32, VEC); } while (0)
-  const int units = simple_compute_units();
-  const bool small = 9.9 * fullest(M, N, 32, 64, units) <= 17.2 * fullest(M, N, 64, 64, units);    // us a tile of the fullest unit, as in launch()
+  const bool small = gated_in_small_tiles(M, I, simple_compute_units());
   if (vec && K % 64 == 0) GO(2);
   else if (vec) GO(1);
   else GO(0);

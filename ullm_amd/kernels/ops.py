@@ -1063,6 +1063,13 @@ def gemm_simple(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] =
     return out
 
 
+@functools.lru_cache(maxsize=4096)      # asked for every layer of steps that wait for the host
+def gemm_simple_silu_ahead(rows: int, inner: int, K: int, captured: bool, units: int) -> bool:
+    """Whether :func:`gemm_simple_silu` is the faster way for so many rows and matrices of ``inner`` columns each, in a graph that is being
+    ``captured`` or launched as it is."""
+    return bool(build.load("gemm_simple").ullm_gemm_simple_gated_ahead(_c_int(rows), _c_int(inner), _c_int(K), _c_int(captured), _c_int(units)))
+
+
 def gemm_simple_silu(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(a G^T) * (a U^T) for float32 a [M, K] and w = G | U [2 I, K]: :func:`gemm_simple` and :func:`silu_mul` in one kernel."""
     M, K = a.shape

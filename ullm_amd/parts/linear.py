@@ -88,8 +88,7 @@ def gate_up(x: torch.Tensor, weight: torch.Tensor, limit: float = 0.0, alpha: fl
     fit one round (``dispatch.panels``), else by the few-rows kernel or the kernel for up
     to 128 rows with the activation on store, up to the row counts the matrix's limits name; beyond, by the large product with the
     activation on store where its tiles fill the chip (``dispatch.gated_tile_groups``); else by the
-    library product and the activation kernel (float32: the 32-bit product with the unit on store, up to 16 rows the activation kernel
-    behind it).  With
+    library product and the activation kernel (float32: the 32-bit product, with the unit on store where that is the faster way).  With
     ``limit`` > 0 the clamped gated unit (``ops.glu_clamped``) in place of silu(gate) * up, by the same kernels."""
     rows = x.shape[0]
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
@@ -108,9 +107,9 @@ def gate_up(x: torch.Tensor, weight: torch.Tensor, limit: float = 0.0, alpha: fl
             return ops.gemm_tiles(x, weight, gated=True, groups=groups, **unit)
     if limit > 0:
         return ops.glu_clamped(linear(x, weight), limit, alpha)
-    # one row of tiles that is more than the chip holds at once is ahead in smaller ones, which hold no pairs of gate and up (17 rows of
-    # 2 x 12288 columns, K = 4096: 82 us in two kernels, 89 in one; of 2 x 3072, K = 1024: 14.4 and 14.3)
-    if limit <= 0 and x.dtype == weight.dtype == torch.float32 and (rows > 32 or (rows > 16 and weight.shape[0] <= 16384)):
+    if (x.dtype == weight.dtype == torch.float32
+            and ops.gemm_simple_silu_ahead(rows, weight.shape[0] // 2, weight.shape[1], torch.cuda.is_current_stream_capturing(),
+                                           ops.compute_units(x.device))):
         return ops.gemm_simple_silu(x, weight)
     return ops.silu_mul(linear(x, weight))
 
