@@ -1691,6 +1691,12 @@ def attention_prefill_mfma(q, out, k_pool, v_pool, tiles: torch.Tensor, n_tiles:
         ctypes.c_longlong(int(wide_keys_total)), _c_int(wide_keys_max), _stream()), "attention_prefill")
 
 
+@functools.lru_cache(maxsize=256)
+def attention_mixed_supports(hd: int, page_size: int, nq: int, nkv: int) -> bool:
+    """True if :func:`attention_mixed_mfma` takes such heads."""
+    return bool(build.load("attention_mfma").ullm_attention_mixed_supports(_c_int(hd), _c_int(page_size), _c_int(nq), _c_int(nkv)))
+
+
 def attention_mixed_mfma(q, out, k_pool, v_pool, decode_tokens: torch.Tensor, n_decode: int, tiles: torch.Tensor, n_tiles: int, positions,
                          token_entry, block_table, page_size: int, nq: int, nkv: int, hd: int, scale: float, window: int, decode_keys: int,
                          max_decode_kv: int, keys_total: int = 0, keys_max: int = 0, wide_tiles: Optional[torch.Tensor] = None, n_wide: int = 0,
@@ -1768,7 +1774,7 @@ def paged_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     out = torch.empty((q.shape[0], nq * hd), dtype=q.dtype, device=q.device)
     n = plan.facts
     if (n["num_decode"] and n["num_tiles"] and n.get("decode_keys") and bias is None and gate is None and sink is None
-            and attention_mixed_mfma(
+            and attention_mixed_supports(hd, group.page_size, nq, nkv) and attention_mixed_mfma(
                 q, out, k_pool, v_pool, plan.arrays["decode_tokens"], n["num_decode"], plan.arrays["tiles"], n["num_tiles"], ctx.positions,
                 ctx.token_entry, group.block_table, group.page_size, nq, nkv, hd, scale, window, n["decode_keys"], n["max_decode_kv"],
                 keys_total=n["tile_keys_total"], keys_max=n["tile_keys_max"], wide_tiles=plan.arrays.get("wide_tiles"),
