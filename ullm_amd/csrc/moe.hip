@@ -199,8 +199,13 @@ __device__ __forceinline__ void keep_router_values(S* p, router_u32x4 v) {
   }
 }
 
+// Waves a SIMD that the registers are held to, where more blocks a unit are worth more than loads under way; 0: as they come.  (256 outputs of width
+// 1024, 8000 tokens by fours 148.6 -> 144.5 us, 32-bit rows 145.3 -> 147.3; 300 of width 640, 3000 32-bit rows by ones 95.2 -> 91.5.)
+constexpr int router_waves(int tpb, int waves, bool early, bool widened) {
+  return early ? 0 : tpb == 1 && waves == 8 ? 8 : tpb == 4 && waves == 4 && widened ? 6 : 0;
+}
 template <typename T, typename S, int TPB, int WAVES, bool EARLY>
-__global__ void __launch_bounds__(64 * WAVES)
+__global__ void __launch_bounds__(64 * WAVES, (router_waves(TPB, WAVES, EARLY, sizeof(T) < sizeof(S))))
 moe_router_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ w, const float* __restrict__ correction,
                   int n_tokens, int H, int n_router, int top, int* __restrict__ ids, float* __restrict__ weights, int mode,
                   float weight_scale, int groups, int keep, int raw, int group_top) {
@@ -330,15 +335,26 @@ extern "C" int ullm_moe_router(const void* x, int ldx, const float* w, const flo
   // 400 21 / 20 / 20 / 18 / 21 / 28 / 38, 1000 36 / 34 / 32 / 27 / 22 / 29 / 39, 3000 75 / - / - / - / - / 42 / 44, 8000 172 / - / - / - / - / 92 / 84;
   // 16 of 512: 48 7.5 / 8.2 / 7.6 / 9.2 / 10.1 / 10.2 / 9.2, 1000 11.2 / 13.1 / 8.3 / 12.1 / 9.7 / 9.2 / 9.4, 8000 56 / - / - / - / - / 21 / 17.  Width 5120,
   // where two fit: 24 outputs, 1000 tokens 28 by ones, 18 by twos, 8000 152 and 87.
+  // Rows that end inside a piece come one value a load, which many waves hide.  1 of 16 waves / 1 of 8 / 2 of 8 / 4 of 4: 200 outputs of width 1282, 400
+  // tokens 40 / 60 / 64 / 118, 700 58 / 60 / 65 / 118, 1500 95 / 93 / 68 / 120, 4000 203 / 193 / 157 / 123; 33 of 770, 1000 tokens 17 / 16 / 17 / 25,
+  // 1500 23 / 22 / 18 / 27, 3000 38 / 34 / 32 / 27; 60 of 6002, 700 62 / 69 / - / -, 1000 83 / 72 / - / -.
+  // One token a block because two do not fit: sixteen waves where outputs take many rounds (256 of width 7168 in 32 bits, 700 tokens 196 and in eight
+  // 203, but 400, where the chip holds all blocks of eight, 134 and 115); 300 outputs of width 640, 3000 tokens 94 and 91, 512 25.8 and 27.0, of width
+  // 2048 3000 tokens 242 and 250; 100 of width 600, 400 tokens 12.4 and 13.2.
   const int most = n_router > 256 ? 1 : 32768 / (H * (dtype == ULLM_F32 ? 4 : 2));
-  if (T_ > 1024 && most >= 4) {
+  if (H % 4 || ((uintptr_t)w & 15)) {
+    if (T_ > 1024 && most >= 4 && (T_ > 2048 || H <= 512)) GOT(4, 4, false);
+    else if (T_ > 1024 && most >= 2) GOT(2, 8, false);
+    else if (T_ > (H <= 2048 ? 512 : 800) && most >= 2) GOT(1, 8, false);
+    else GOT(1, 16, false);
+  } else if (T_ > 1024 && most >= 4) {
     if (H <= 512 || (H <= 1024 && T_ > 4096)) GOT(4, 4, false);
     else GOT(4, 4, true);
   } else if (T_ > 512 && most >= 4 && H >= 1024) GOT(4, 8, true);
   else if (T_ > 512 && most >= 2 && H >= 1024) GOT(2, 8, false);
-  else if (T_ > 300 && most >= 2 && H >= 1024) GOT(2, 8, true);
-  else if (T_ > 300 && n_router <= 256) GOT(1, 8, false);
-  else if (n_router <= 32 && H >= 2048) GOT(1, 8, true);
+  else if ((T_ > 300 || (T_ > 256 && H > 2048)) && most >= 2 && H >= 1024) GOT(2, 8, true);
+  else if (n_router > 256 ? T_ > 512 && H <= 1024 : T_ > 512 ? H < 1024 || n_router <= 64 : T_ > 300 && (H >= 1024 || n_router <= 32)) GOT(1, 8, false);
+  else if (T_ <= 300 && n_router <= 32 && H >= 2048) GOT(1, 8, true);
   else GOT(1, 16, false);
 #undef GOT
 #undef GO
