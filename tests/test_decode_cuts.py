@@ -1,7 +1,7 @@
 """How the keys of many requests are cut for decode: near the best for contexts that are equal and for contexts that are not, of those measured."""
 import pytest
 
-from ullm_amd.kernels.ops import decode_split
+from ullm_amd.kernels.ops import DECODE_EVEN, decode_cuts, decode_split
 
 # (pairs of token and kv head, longest context): us of (waves a block, blocks a pair), for equal contexts and for contexts that spread
 # from a tenth of the longest to it; 32 heads over 8, 256 compute units
@@ -57,3 +57,26 @@ def test_heads_of_256():
     assert decode_split(32, 8, 1, 4096) == (2, 4) and decode_split(32, 8, 1, 4096, 256) == (4, 1)
     assert decode_split(18, 8, 1, 256) == (4, 1) and decode_split(18, 8, 1, 256, 256)[0] == 1
     assert decode_split(51, 8, 1, 1000) == (2, 1) and decode_split(51, 8, 1, 1000, 256) == (1, 2)
+
+
+# pairs, what a captured step is told and the longest context: us in equal cuts and shared evenly, for contexts that are equal, that spread from 0.55
+# and from a tenth of the longest
+SHARED = {(88, 8192, 4174): ((37.3, 38.4), (33.2, 32.6), (29.1, 27.6)), (88, 8192, 8189): ((65.0, 65.8), (56.1, 52.7), (48.2, 41.3)),
+          (120, 8192, 4174): ((49.0, 50.0), (42.5, 40.7), (36.2, 32.4)), (144, 8192, 4174): ((54.0, 55.4), (47.2, 47.7), (40.3, 36.8)),
+          (192, 8192, 4174): ((70.8, 72.5), (61.5, 59.6), (52.1, 46.1)), (248, 8192, 4174): ((90.1, 90.3), (77.2, 74.0), (64.9, 56.7)),
+          (32, 16384, 8352): ((31.8, 32.8), (27.8, 27.5), (24.7, 24.1)), (32, 16384, 12285): ((40.8, 41.8), (34.6, 35.0), (30.0, 29.4)),
+          (40, 16384, 8352): ((37.7, 36.4), (35.4, 32.0), (31.4, 27.3)), (48, 16384, 8352): ((40.2, 41.2), (37.0, 34.7), (33.5, 28.5)),
+          (64, 16384, 8352): ((49.9, 50.5), (43.8, 42.8), (37.1, 35.0)), (32, 32768, 16708): ((50.9, 51.3), (44.1, 43.3), (37.7, 35.7)),
+          (32, 32768, 32765): ((89.3, 90.2), (75.2, 72.3), (61.1, 56.1))}
+
+
+@pytest.mark.parametrize("pairs,told,longest", sorted(SHARED))
+def test_shared_evenly_where_the_lower_half_of_a_range_gains_too(pairs, told, longest):
+    """A captured step is told the power of two above its longest context: equal contexts lose 3 % at most and the three kinds gain 1 % together, or
+    keys are cut as they were."""
+    ratio = 1.0
+    for cut, shared in SHARED[pairs, told, longest]:
+        ratio *= shared / cut
+    even = decode_cuts(pairs // 8, 8, 1, told)[0] == DECODE_EVEN
+    equal = SHARED[pairs, told, longest][0]
+    assert even == (equal[1] <= 1.031 * equal[0] and ratio ** (1 / 3) <= 0.99)

@@ -1504,19 +1504,23 @@ DECODE_EVEN = -1       # "waves": one wave a block, and num_splits blocks (a kv 
 
 def decode_cuts(n_items: int, nkv: int, groups: int, max_kv: int, hd: int = 128, window: int = 0, units: int = 256):
     """(waves, num_splits) as ``decode_split`` has them, or (``DECODE_EVEN``, blocks a kv head) where its single waves a block have long ways
-    and contexts of several lengths would leave some of them waiting for others.  It is told the longest context alone (in a graph the
-    power of two above it), so the line lies where equal contexts lose nothing by it either.  us in equal cuts / shared evenly, for
-    contexts that are equal, spread from 0.55 and from a tenth of the longest: 120 pairs with 8180 keys 93 / 92, 78 / 75, 66 / 58; 32 pairs
-    with 16000 52 / 52, 46 / 45, 40 / 40; 64 with 16000 92 / 93, 81 / 79, 70 / 63; 192 with 8180 138 / 139, 120 / 115, 103 / 87.  Half as long,
-    192 with 2040 keys 42 / 43, 37 / 38, 33 / 31; 64 with 8180 53 / 54, 45 / 45, 40 / 39; 32 with 4090 22 / 24, 21 / 22, 20 / 20.  Of 256 pairs
-    in (2, 4) 4090 keys 101 / 97, 80 / 81, 62 / 63 and 16000 342 / 337, 271 / 283, 201 / 211."""
+    and contexts of several lengths would leave some of them waiting for others.  It is told the longest context alone, in a graph the
+    power of two above it, which may be twice as long.  The line lies where the three kinds of contexts measured gain together in both halves of such a
+    range; contexts that are equal pay up to 1.5 us, 3 %, for shares that every wave works out.  us in equal cuts / shared evenly, for contexts that are
+    equal, spread from 0.55 and from a tenth of the longest.  Told 8192: 120 pairs with 4170 keys 49.0 / 50.0, 42.5 / 40.7, 36.2 / 32.4, with 8190
+    87.4 / 87.3, 73.7 / 68.6, 61.2 / 52.9; 88 with 4170 37.3 / 38.4, 33.2 / 32.6, 29.1 / 27.6; 144 with 4170 54.0 / 55.3, 47.3 / 47.7, 40.3 / 36.8, with
+    8190 97.8 / 99.2, 84.3 / 80.3, 71.1 / 61.0; 224 with 4170 86.7 / 85.6, 76.5 / 71.3, 65.8 / 58.6.  Told 16384: 40 with 8350 37.7 / 36.4, 35.4 / 32.0,
+    31.4 / 27.3; 64 with 8350 49.9 / 50.5, 43.8 / 42.8, 37.1 / 35.0, with 16380 89.0 / 89.5, 75.2 / 72.1, 62.3 / 55.0; 32 with 8350 31.8 / 32.8, 27.8 / 27.5,
+    24.7 / 24.1, with 12290 40.8 / 41.8, 34.6 / 35.0, 30.0 / 29.4, told 32768 with 16710 50.9 / 51.3, 44.1 / 43.3, 37.7 / 35.7.  Told less: 192 with 2040 keys
+    42 / 43, 37 / 38, 33 / 31; 64 with 8180 53 / 54, 45 / 45, 40 / 39; of 256 pairs in (2, 4) 4090 keys 101 / 97, 80 / 81, 62 / 63 and 16000 342 / 337, 271 / 283,
+    201 / 211."""
     waves, splits = decode_split(n_items, nkv, groups, max_kv, hd, window, units)
     pairs = n_items * nkv * groups
     if window != 0:
         max_kv = min(max_kv, abs(window) + 31)
     blocks = 4 * units // max(1, nkv * groups)
     if (waves == 1 and splits > 1 and hd <= 128 and 4 <= n_items <= 64 and 8 * pairs >= units and blocks > n_items
-            and -(-max_kv // 32) >= (256 if 3 * pairs >= units else 512)):
+            and -(-max_kv // 32) >= (256 if 3 * pairs >= units else 512 if 8 * pairs > units else 1024)):
         return DECODE_EVEN, blocks
     return waves, splits
 
