@@ -71,7 +71,7 @@ def decode_attention(args) -> None:
             out = torch.empty_like(q)
             ent = torch.arange(B, dtype=torch.int32, device=DEV)
             groups = -(-(nq // nkv) // 16)
-            auto = ops.decode_split(B, nkv, groups, ctx, hd)
+            auto = ops.decode_cuts(B, nkv, groups, ctx, hd)
             # all contexts equal, and (longest first, as a step lists them) from the longest to a tenth of it
             for shape, lens in (("equal", [ctx] * B), ("spread", [max(1, round(ctx * (1 - 0.9 * b / max(1, B - 1)))) for b in range(B)])):
                 if shape == "spread" and B == 1:
@@ -85,7 +85,8 @@ def decode_attention(args) -> None:
                                                                     nkv, hd, hd ** -0.5, 0, ctx, splits=splits, waves=waves))
                              for v in range(nv)]
                     t = graph_time(calls)
-                    name = f"chosen {auto[1]}x{auto[0]}" if splits == 0 else f"{splits}x{waves}"
+                    of = f"{auto[1]} shares" if auto[0] == ops.DECODE_EVEN else f"{auto[1]}x{auto[0]}"
+                    name = f"chosen {of}" if splits == 0 else f"{splits}x{waves}"
                     cells.append(f"{name}: {t:.1f}")
                 print(f"decode attention, batch {B}, {shape} contexts of {'' if shape == 'equal' else 'up to '}{ctx}, {nq}/{nkv} heads of {hd} "
                       f"({sum(lens) * nkv * hd * 4 / 1e6:.0f} MB of cache); us by splits x waves: " + "  ".join(cells), flush=True)
