@@ -47,6 +47,78 @@ def test_every_way_of_the_launch(entries, nq, nkv, window):
                                  entry, bt, P, nq, nkv, hd, scale, window, f["decode_keys"], f["max_decode_kv"], way=6)
 
 
+# keys of the decoded tokens, and where their blocks then stand among the prompt's: few with a long walk before them, many behind the first round, few
+# short ones behind all
+ORDERS = {"first": [3000, 2500], "between": [600, 520, 590] * 20, "last": [60, 31, 1, 47]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", ORDERS)
+@pytest.mark.parametrize("nq", [16, 64])
+def test_every_order_of_the_blocks(nq, order):
+    """More prompt blocks than the chip holds: the bits of the prompt's own launch, and softmax in 64 bits for the decoded tokens."""
+    from ullm_amd.kernels import build, ops
+    from ullm_amd.parts import StepShape
+    from ullm_amd.parts.attention import plan_attention_step
+    g = torch.Generator(DEV).manual_seed(nq)
+    nkv, hd, P, dtype, scale = 16, 128, 16, torch.bfloat16, 128 ** -0.5
+    entries = [(1, n - 1) for n in ORDERS[order]] + [(2133, 0)]
+    pages = [-(-(n + s) // P) for n, s in entries]
+    k_pool = torch.randn(sum(pages), nkv, P, hd, generator=g, device=DEV).to(dtype)
+    v_pool = torch.randn(sum(pages), nkv, hd, P, generator=g, device=DEV).to(dtype)
+    ids = torch.randperm(sum(pages), generator=g, device=DEV).int().split(pages)
+    bt = table_tensor([i.tolist() for i in ids], DEV)
+    plan = plan_attention_step(StepShape(tuple(n for n, _ in entries), tuple(s for _, s in entries)))
+    f, arrays = plan.facts, {k: torch.tensor(v, device=DEV) for k, v in plan.arrays.items()}
+    T = sum(n for n, _ in entries)
+    q = torch.randn(T, nq * hd, generator=g, device=DEV).to(dtype)
+    positions = torch.cat([torch.arange(s, s + n) for n, s in entries]).int().to(DEV)
+    entry = torch.cat([torch.full((n,), b) for b, (n, _) in enumerate(entries)]).int().to(DEV)
+    figures = dict(keys_total=f["tile_keys_total"], keys_max=f["tile_keys_max"], wide_tiles=arrays["wide_tiles"], n_wide=f["num_wide"],
+                   wide_keys_total=f["wide_keys_total"], wide_keys_max=f["wide_keys_max"])
+    want = []
+    for b, n in enumerate(ORDERS[order]):
+        k = k_pool[ids[b].long()].transpose(1, 2).reshape(-1, nkv, hd)[:n]
+        v = v_pool[ids[b].long()].permute(0, 3, 1, 2).reshape(-1, nkv, hd)[:n]
+        want.append(_attention(q[b:b + 1].view(1, nq, hd).cpu(), k.cpu(), v.cpu(), 0, scale))
+    want, decoded = torch.cat(want), len(ORDERS[order])
+    long, i = ctypes.c_longlong, ctypes.c_int
+    lead = build.load("attention_mfma").ullm_attention_mixed_lead
+    lead.restype = long
+    for way in ((3, 4, 5) if nq // nkv <= 2 else (1, 2)):
+        wide = way in (4, 5)
+        blocks = (f["num_wide"] if wide else f["num_tiles"]) * nkv * -(-nq // nkv // 4)
+        keys = f["wide_keys_total" if wide else "tile_keys_total"] * nkv * -(-nq // nkv // 4)
+        slots = ops.compute_units(DEV) * (2 if way in (1, 4) else 1)
+        assert blocks > slots
+        before = lead(i(way), long(blocks), long(keys), long(decoded * nkv), long(f["decode_keys"]), i(f["max_decode_kv"]), i(nkv),
+                      i(ops.compute_units(DEV)))
+        assert before == {"first": 0, "between": slots, "last": blocks}[order], way
+        out, alone = (torch.full((T, nq * hd), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+        assert ops.attention_mixed_mfma(
+            q, out, k_pool, v_pool, arrays["decode_tokens"], f["num_decode"], arrays["tiles"], f["num_tiles"], positions, entry, bt, P, nq, nkv, hd, scale,
+            0, f["decode_keys"], f["max_decode_kv"], way=way, **figures)
+        ops.attention_prefill_mfma(q, alone, k_pool, v_pool, arrays["tiles"], f["num_tiles"], positions, entry, bt, P, nq, nkv, hd, scale, 0, halves=way,
+                                   **figures)
+        assert torch.equal(out[decoded:], alone[decoded:]) and not torch.isnan(out).any(), way
+        assert (out[:decoded].float().cpu() - want.float()).abs().max() <= tol(dtype, want), way
+
+
+def test_orders_on_other_chips():
+    """CPU: what the chip holds at once is its units'; blocks between two of the prompt's are a multiple of the eight dies."""
+    from ullm_amd.kernels import build
+    long, i = ctypes.c_longlong, ctypes.c_int
+    f = build.load("attention_mfma").ullm_attention_mixed_lead
+    f.restype = long
+    for way, per_unit in ((1, 2), (2, 1), (3, 1), (4, 2), (5, 1)):
+        for units in (256, 250, 64):
+            slots = units * per_unit
+            lead = lambda blocks, pairs, keys, longest: f(i(way), long(blocks), long(1000 * blocks), long(pairs), long(keys), i(longest), i(8), i(units))  # noqa: E731
+            assert lead(slots, 8, 9000, 9000) == slots and lead(slots - 3, 800, 90000, 900) == slots - 3
+            assert lead(slots + 1, 8, 9000, 9000) == 0 and lead(slots + 5, 8, 40, 40) == slots + 5
+            assert lead(slots + 1, 2 * slots, 10 ** 6, 900) == slots // 8 * 8
+
+
 # requests and keys of the longest (the others down to 0.58 of it), the portion and the keys before it, heads, kv heads: us of two launches (0) and of the ways
 MEASURED = [(4, 640, 700, 2100, 16, {0: 52.1, 3: 39.5, 5: 57.8, 4: 85.7}), (40, 640, 300, 600, 16, {0: 43.5, 3: 26.8, 5: 26.8, 4: 37.0}),
             (100, 640, 300, 600, 16, {0: 66.8, 3: 44.2, 5: 45.0, 4: 41.7}), (100, 640, 700, 0, 16, {0: 64.0, 3: 54.0, 5: 45.2, 4: 43.0}),

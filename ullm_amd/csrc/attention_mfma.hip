@@ -1941,16 +1941,27 @@ static int mixed_way(const PrefillWork& work, long long keys, int longest, int n
   return together < 0.97 * (read + apart + 9) ? way : 0;
 }
 
-// How many of the prompt's blocks come before the decoded tokens', in a way that takes `per_unit` of them a unit.  Where the chip holds them all, every one.  Else
+// The blocks that take `pairs` of decoded token and kv head: a multiple of the dies, for a prompt block's id says which die it goes to.
+static long long decoded_blocks(int way, long long pairs) {
+  const int teams = way == 1 || way == PREFILL_WIDE ? 1 : 2;
+  return ((pairs + teams - 1) / teams + 7) / 8 * 8;
+}
+
+// How many of the prompt's `blocks` (which see `prompt_keys` keys together) come before the decoded tokens'.  Where the chip holds them all, every one.  Else
 // few decoded tokens with a long walk begin at once (a request of 900 keys beside 1200 tokens behind 400 49 -> 40 us); short ones
 // come last, beside the last prompt blocks (100 of 640 beside 1500 behind 4500, 40 heads over 8, 381 -> 349); the others behind the first round.
-static long long prompt_lead(long long blocks, long long prompt_keys, double a_key, long long decode_blocks, long long keys, int longest, int nkv,
-                             long long units, int per_unit) {
-  const long long slots = units * per_unit;
+static long long prompt_lead(int way, long long blocks, long long prompt_keys, long long pairs, long long keys, int longest, int nkv, long long units) {
+  const bool two_a_unit = way == 1 || way == PREFILL_WIDE;
+  const long long slots = units * (two_a_unit ? 2 : 1);
   if (blocks <= slots) return blocks;
-  const double block = a_key * (double)prompt_keys / (double)blocks, walk = (per_unit == 2 ? 0.0175 : 0.029) * longest, read = (double)keys * nkv * 512 / 5.3e6;
-  if (walk > block && 2 * decode_blocks <= slots) return 0;
+  const double block = (two_a_unit ? 0.030 : way == PREFILL_QUARTERS ? 0.014 : 0.021) * (double)prompt_keys / (double)blocks;
+  const double walk = (two_a_unit ? 0.0175 : 0.029) * longest, read = (double)keys * nkv * 512 / 5.3e6;
+  if (walk > block && 2 * decoded_blocks(way, pairs) <= slots) return 0;
   return walk <= block && read <= block ? blocks : slots / 8 * 8;
+}
+extern "C" long long ullm_attention_mixed_lead(int way, long long blocks, long long prompt_keys, long long pairs, long long keys, int longest, int nkv,
+                                               int units) {
+  return prompt_lead(way, blocks, prompt_keys, pairs, keys, longest, nkv, units);
 }
 
 // 1 if ullm_attention_mixed takes such heads.
@@ -1984,13 +1995,11 @@ extern "C" int ullm_attention_mixed(
   const long long blocks = (long long)n_tiles * nkv * chunks, pairs = (long long)n_decode * nkv, prompt_keys = way >= PREFILL_WIDE ? wide_total : keys_total;
   if (blocks + pairs + 8 > 0x7fffffffLL || (long long)nkv * page_size * hd > 0x7fffffffLL) return ULLM_ERR_SHAPE;
   const float sl = scale * 1.4426950408889634f;
-  // (a prompt block's id says which die it goes to: what lies between two of them is a multiple of the dies)
+  const long long decode_blocks = decoded_blocks(way, pairs);
+  const long long lead = prompt_lead(way, blocks, prompt_keys * nkv * chunks, pairs, decode_keys, decode_keys_max, nkv, compute_units());
 #define GO(HEADS, KS) do {                                                                                                             \
     using B = DmaBlock<4, HEADS, KS>;                                                                                                  \
-    constexpr int TEAMS = B::THREADS / 256;                                                                                            \
-    const long long decode_blocks = ((pairs + TEAMS - 1) / TEAMS + 7) / 8 * 8;                                                         \
-    const long long lead = prompt_lead(blocks, prompt_keys * nkv * chunks, KS == 4 ? 0.014 : KS == 2 ? 0.021 : 0.030, decode_blocks, decode_keys,      \
-                                       decode_keys_max, nkv, compute_units(), B::PER_UNIT);                                            \
+    static_assert(B::PER_UNIT == (B::THREADS == 256 ? 2 : 1), "what prompt_lead takes a way to be");                                   \
     hipLaunchKernelGGL((attention_mixed_kernel<HEADS, KS>), dim3((unsigned)(blocks + decode_blocks)), dim3(B::THREADS), 0, stream,     \
                        (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, tiles,      \
                        positions, token_entry, block_table, bt_stride, page_size, nq, nkv, sl, window, n_tiles, (unsigned)blocks,      \
