@@ -125,7 +125,10 @@ MEASURED = [(4, 640, 700, 2100, 16, {0: 52.1, 3: 39.5, 5: 57.8, 4: 85.7}), (40, 
             (100, 640, 700, 2100, 16, {0: 88.6, 3: 65.5, 5: 60.3, 4: 93.0}), (100, 300, 1500, 3000, 16, {0: 123.7, 3: 98.2, 5: 88.8, 4: 136.5}),
             (30, 2000, 300, 600, 16, {0: 62.1, 3: 66.0, 5: 66.7, 4: 41.5}), (8, 4000, 300, 600, 16, {0: 47.2, 3: 115.5, 5: 115.1, 4: 63.0}),
             (100, 640, 700, 2100, 32, {0: 108.8, 1: 94.2, 2: 80.1}), (100, 640, 1900, 0, 32, {0: 102.6, 1: 77.9, 2: 100.2}),
-            (100, 64, 300, 600, 32, {0: 36.2, 1: 33.8, 2: 27.0}), (8, 4000, 700, 0, 32, {0: 50.4, 1: 64.6, 2: 117.0})]
+            (100, 64, 300, 600, 32, {0: 36.2, 1: 33.8, 2: 27.0}), (8, 4000, 700, 0, 32, {0: 50.4, 1: 64.6, 2: 117.0}),
+            # what a walk waits for: another team's on its unit, the prompt's blocks, which take every slot, and its own beginning
+            (40, 2881, 35, 0, 16, {0: 74.2, 3: 96.3, 4: 86.7, 5: 96.8}), (37, 3175, 216, 25, 16, {0: 82.8, 3: 104.1, 4: 91.5, 5: 103.8}),
+            (1, 1906, 488, 3319, 40, {0: 89.4, 2: 126.7}), (2, 743, 43, 0, 16, {0: 16.0, 3: 27.0, 4: 17.7, 5: 27.4})]
 
 
 @pytest.mark.parametrize("case", range(len(MEASURED)))

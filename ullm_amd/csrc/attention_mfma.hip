@@ -1901,9 +1901,13 @@ extern "C" int ullm_attention_prefill(
 //   together          blocks that share units with prompt blocks (two a unit) hide under them and hold them up by a quarter of the shorter time;
 //                     where a prompt block has the unit for itself they run beside and behind it: both add up over the units
 //   apart             both, 6 for the second kernel of cut contexts or a coarser cut, 3 for the launch
-// Held against 288 steps (1 to 250 requests of 30 to 4000 keys, 17 to 1500 tokens behind 0 to 4500, 16, 32 and 40 heads over 8): 1.26 times as fast as two
-// launches in the geometric mean, nowhere slower by more than 5 %; over 84 of them with every way timed 1.05 times the time of the best way.  Longer contexts than a team walks in that time stay apart (8 requests of
-// 4000 keys beside 300 tokens 47 us, together 63).
+// The way that is expected to be the best is then held against two launches by what it waits for alone: the walk of the longest context and what
+// begins it, 2 or 3; where teams outnumber the units, two to a unit, a second walk behind it (33 requests of 2690 keys, 264 teams, beside 73 tokens: 82.5 apart, 94.9
+// together); where the prompt's blocks leave fewer slots than the decoded tokens take, the shortest of them first (a request of 1900 keys beside 488
+// tokens behind 3319, 40 heads, 256 blocks: 89 and 127).
+// Over 4000 steps (1 to 250 requests of 30 to 4000 keys that are equal or spread, 17 to 1500 tokens behind 0 to 4500, 16, 32 and 40 heads over 8):
+// 1.29 times as fast as two launches in the geometric mean (1.30 with the best way of each), 31 of them slower by more than 2 %, 12 % at most.  Longer contexts
+// than a team walks in that time stay apart (8 requests of 4000 keys beside 300 tokens 47 us, together 63).
 static int mixed_way(const PrefillWork& work, long long keys, int longest, int n_decode, int nq, int nkv, int window, long long units) {
   if (keys <= 0 || longest <= 0 || work.keys_max <= 0 || work.keys_total <= 0) return 0;
   const long long reach = window == 0 ? 0x7fffffffLL : (window > 0 ? window : -(long long)window) + 32;      // keys a query's tile may see
@@ -1912,7 +1916,8 @@ static int mixed_way(const PrefillWork& work, long long keys, int longest, int n
   auto least = [](double a, double b) { return a < b ? a : b; };
   auto most = [](double a, double b) { return a > b ? a : b; };
   const double walk = (double)(longest < reach ? longest : reach), read = least((double)keys, (double)n_decode * reach) * nkv * 512 / 5.3e6 + 4;
-  double apart = 1e30, together = 1e30;
+  const double mean = least((double)keys / n_decode, (double)reach), pairs = (double)n_decode * nkv;
+  double apart = 1e30, together = 1e30, sure = 1e30;
   int way = 0;
   auto look = [&](int w, double a_key, long long count, long long total, int longest_tile, int per_unit) {
     if (count <= 0 || total <= 0) return;
@@ -1928,6 +1933,11 @@ static int mixed_way(const PrefillWork& work, long long keys, int longest, int n
     if (both < together) {
       together = both;
       way = w;
+      const double shortest = 2 * least((double)total / count, (double)reach) - least(longest_tile, (double)reach);
+      const double teams = per_unit == 2 ? pairs : (pairs + 1) / 2;
+      const double late = blocks <= slots && blocks + teams > slots ? a_key * most(shortest, 0) : 0;
+      const double second = pairs > units && pairs <= 2.0 * units ? mean : 0;
+      sure = per_unit == 2 ? most(late + 0.0175 * (walk + second) + 2, read) : most(most(prompt, late + 0.029 * walk + 3), all + read);
     }
   };
   if (two_heads) {
@@ -1938,7 +1948,7 @@ static int mixed_way(const PrefillWork& work, long long keys, int longest, int n
     look(2, 0.021, work.n_tiles, work.keys_total, work.keys_max, 1);
     look(1, 0.030, work.n_tiles, work.keys_total, work.keys_max, 2);
   }
-  return together < 0.97 * (read + apart + 9) ? way : 0;
+  return together < 0.97 * (read + apart + 9) && sure < 0.95 * (read + apart + 9) ? way : 0;
 }
 
 // The blocks that take `pairs` of decoded token and kv head: a multiple of the dies, for a prompt block's id says which die it goes to.
