@@ -15,7 +15,7 @@ fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
 
 # tiles of 32 x 32, 32 x 64, 64 x 32 in stages of 64 and of 32, 64 x 64, 16 x 64; K of one stage, of two and of three, with and
 # without a last one that is not whole, and of rows that no 16-byte load takes
-@pytest.mark.parametrize("M,N", [(33, 1000), (150, 6100), (450, 1030), (380, 4100), (1000, 4097), (13, 9000)])
+@pytest.mark.parametrize("M,N", [(33, 1000), (150, 6100), (450, 1030), (192, 2720), (380, 4100), (1000, 4097), (13, 9000)])
 @pytest.mark.parametrize("K", [20, 64, 101, 128, 192, 196])
 @pytest.mark.parametrize("a_dtype", [torch.float32, torch.bfloat16])
 def test_a_tile_has_the_bits_of_a_loop_over_k(M, N, K, a_dtype):

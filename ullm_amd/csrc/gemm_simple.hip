@@ -76,10 +76,7 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
       auto one = [&](auto src) __attribute__((always_inline)) {
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float x = ld_f32(src + (k + j < K ? k + j : K - 1));
-          v[j] = k + j < K ? x : 0.f;
-        }
+        for (int j = 0; j < 4; ++j) v[j] = ld_f32(src + (k + j < K ? k + j : K - 1));
         return make_float4(v[0], v[1], v[2], v[3]);
       };
       if (p < AP) reg[set][p] = one(asrc[p]);
@@ -88,12 +85,12 @@ gemm_simple_kernel(const TA* __restrict__ A, int lda, const TW* __restrict__ W, 
   };
   // value e of a piece goes to the chunk's piece e: a lane group's 16 bytes are then values g, 4 + g, 8 + g, 12 + g of the chunk
   // (64 lanes write one value each to 64 different banks).  Zeros are put in here: a condition on a fetched value any earlier
-  // would wait for the fetch.
+  // would wait for the fetch (33 rows of 2048 outputs, K = 3001, whose values come one by one, 71 us, 46 so).
   auto put = [&](int set, int p, int buf, int k0) __attribute__((always_inline)) {
     float v[4] = {reg[set][p].x, reg[set][p].y, reg[set][p].z, reg[set][p].w};
-    if (VEC == 1) {
+    if (VEC < 2) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = k0 + 4 * pc < K ? v[e] : 0.f;
+      for (int e = 0; e < 4; ++e) v[e] = k0 + 4 * pc + (VEC ? 0 : e) < K ? v[e] : 0.f;
     }
     unsigned char* row = stages[buf] + (p < AP ? aput[p] : wput[p - AP]);
     const int low = p < AP ? alow[p] : wlow[p - AP];
@@ -248,7 +245,11 @@ static void launch(const void* A, int lda, const void* W, int ldw, const float* 
     const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN; \
     hipLaunchKernelGGL((gemm_simple_kernel<TA, TW, TC, BM, BN, WGM, BK, VEC>), dim3(8 * (((unsigned)mt * nt + 7) / 8)), dim3(256), 0, \
                        stream, (const TA*)A, lda, (const TW*)W, ldw, bias, (TC*)C, ldc, M, N, K, mt, nt); } while (0)
-  switch (product_tile(M, N, simple_compute_units())) {
+  // operands one by one: what is fetched counts, so large tiles where they give a unit one and a half (400 rows of 5000 outputs, K = 770: 75 us, 92 in tiles of
+  // 32 x 32)
+  const int units = simple_compute_units();
+  const bool large = VEC == 0 && ((M + 63) / 64) * ((N + 63LL) / 64) * 2 >= 3 * units;
+  switch (large ? 4 : product_tile(M, N, units)) {
     case 0: TILE(32, 32, 2, 64); break;
     case 1: TILE(32, 64, 2, 64); break;
     case 2: TILE(64, 32, 2, 64); break;
