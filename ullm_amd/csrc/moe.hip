@@ -1199,74 +1199,56 @@ extern "C" int ullm_moe_rows(const void* x, int ldx, const int* row_index, const
 // out[t][c] = base[t][c] + bias[c] + shared[t][c] + sum_k weights[t][k] * (ids[t][k] < n_experts ? y[slot][c] : x[t][c]);
 // base (float32 or TX), bias (float32), shared (TX) may be null.  grid (tokens, groups of columns): a thread takes
 // VEC consecutive columns, all its loads independent of each other.
-template <typename TX, typename TB>
-struct CombineArgs {
-  const float* y;
-  const TX* x;
-  int ldx;
-  const int* ids;
-  const float* weights;
-  const int* slot_of_pair;
-  int top, n_experts;
-  const TB* base;
-  const float* bias;
-  const TX* shared;
-  int H;
-};
-template <typename TX, typename TB, int VEC>
-__device__ __forceinline__ void combined(const CombineArgs<TX, TB>& s, int t, int c, float (&a)[VEC]) {
+//
+// TANH: on its way into the stream and through the squashing that the next sublayers read, which looks at no other column:
+// residual += mult * sum, squashed = tanh(alpha * residual) * gain + shift, as elementwise.hip's add_tanh_kernel does from a sum in memory.
+// What bounds it is bytes: without it the sum was written and read again by a launch of its own.  4 of 32 experts of width 2048, us for both
+// launches -> this one: 1 token 5.7 -> 4.3, 48 6.3 -> 4.4, 300 8.5 -> 5.5, 1000 18.5 -> 14.2, 3000 41.5 -> 33.8.
+// (One kernel with the sum in its body and its pointers one by one.  As a function of a structure's pointers, which may point anywhere, loads wait for each
+// other: 3000 tokens, 4 of width 2048, with a base and a shared expert 29.4 us and so 27.0, 48 tokens 3.86 and 3.64.)
+template <typename TX, typename TB, int VEC, bool TANH>
+__global__ void __launch_bounds__(256)
+moe_combine_kernel(const float* __restrict__ y, const TX* __restrict__ x, int ldx, const int* __restrict__ ids,
+                   const float* __restrict__ weights, const int* __restrict__ slot_of_pair, int top, int n_experts,
+                   const TB* __restrict__ base, const float* __restrict__ bias, const TX* __restrict__ shared,
+                   float* __restrict__ out, int H, float mult, float* __restrict__ residual, const float* __restrict__ alpha,
+                   const float* __restrict__ gain, const float* __restrict__ shift, TX* __restrict__ squashed) {
+  const int t = blockIdx.x, c = VEC * (blockIdx.y * 256 + threadIdx.x);
+  if (c >= H) return;
+  float r[VEC], g[VEC], h[VEC], by = 0.f;
+  if constexpr (TANH) {
+    by = *alpha;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) r[i] = residual[(size_t)t * H + c + i], g[i] = gain[c + i], h[i] = shift[c + i];
+  }
+  float a[VEC];
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
-    a[i] = s.base ? ld_f32(s.base + (size_t)t * s.H + c + i) : 0.f;
-    if (s.bias) a[i] += s.bias[c + i];
-    if (s.shared) a[i] += ld_f32(s.shared + (size_t)t * s.H + c + i);
+    a[i] = base ? ld_f32(base + (size_t)t * H + c + i) : 0.f;
+    if (bias) a[i] += bias[c + i];
+    if (shared) a[i] += ld_f32(shared + (size_t)t * H + c + i);
   }
-  for (int k = 0; k < s.top; ++k) {
-    const int e = s.ids[(size_t)t * s.top + k];
-    const float wk = s.weights[(size_t)t * s.top + k];
-    if (e < s.n_experts) {
-      const float* yr = s.y + (size_t)s.slot_of_pair[(size_t)t * s.top + k] * s.H + c;
+  for (int k = 0; k < top; ++k) {
+    const int e = ids[(size_t)t * top + k];
+    const float wk = weights[(size_t)t * top + k];
+    if (e < n_experts) {
+      const float* yr = y + (size_t)slot_of_pair[(size_t)t * top + k] * H + c;
 #pragma unroll
       for (int i = 0; i < VEC; ++i) a[i] = fmaf(wk, yr[i], a[i]);
     } else {
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) a[i] = fmaf(wk, ld_f32(s.x + (size_t)t * s.ldx + c + i), a[i]);
+      for (int i = 0; i < VEC; ++i) a[i] = fmaf(wk, ld_f32(x + (size_t)t * ldx + c + i), a[i]);
     }
   }
-}
-
-template <typename TX, typename TB, int VEC>
-__global__ void __launch_bounds__(256)
-moe_combine_kernel(const CombineArgs<TX, TB> s, float* __restrict__ out) {
-  const int t = blockIdx.x, c = VEC * (blockIdx.y * 256 + threadIdx.x);
-  if (c >= s.H) return;
-  float a[VEC];
-  combined<TX, TB, VEC>(s, t, c, a);
-#pragma unroll
-  for (int i = 0; i < VEC; ++i) out[(size_t)t * s.H + c + i] = a[i];
-}
-
-// The sum on its way into the stream and through the squashing that the next sublayers read, which looks at no other column:
-// residual += mult * sum, out = tanh(alpha * residual) * gain + shift, as elementwise.hip's add_tanh_kernel does from a sum in memory.
-// What bounds it is bytes: without it the sum was written and read again by a launch of its own.  4 of 32 experts of width 2048, us for both
-// launches -> this one: 1 token 5.7 -> 4.3, 48 6.3 -> 4.4, 300 8.5 -> 5.5, 1000 18.5 -> 14.2, 3000 41.5 -> 33.8.
-template <typename TX, typename TB, int VEC>
-__global__ void __launch_bounds__(256)
-moe_combine_tanh_kernel(const CombineArgs<TX, TB> s, float mult, float* __restrict__ residual, const float* __restrict__ alpha,
-                        const float* __restrict__ gain, const float* __restrict__ shift, TX* __restrict__ out) {
-  const int t = blockIdx.x, c = VEC * (blockIdx.y * 256 + threadIdx.x);
-  if (c >= s.H) return;
-  const size_t at = (size_t)t * s.H + c;
-  float r[VEC], g[VEC], h[VEC], a[VEC];
-  const float by = *alpha;
-#pragma unroll
-  for (int i = 0; i < VEC; ++i) r[i] = residual[at + i], g[i] = gain[c + i], h[i] = shift[c + i];
-  combined<TX, TB, VEC>(s, t, c, a);
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
-    r[i] += mult * a[i];
-    residual[at + i] = r[i];
-    st_f32(out + at + i, tanhf(by * r[i]) * g[i] + h[i]);
+    if constexpr (TANH) {
+      r[i] += mult * a[i];
+      residual[(size_t)t * H + c + i] = r[i];
+      st_f32(squashed + (size_t)t * H + c + i, tanhf(by * r[i]) * g[i] + h[i]);
+    } else {
+      out[(size_t)t * H + c + i] = a[i];
+    }
   }
 }
 
@@ -1281,8 +1263,7 @@ static int bad_combine(int top, int ldx, int T_, int H, const void* base, int ba
     if (dtype == ULLM_F32) { if (vec == 4) GO(float, float, 4); else GO(float, float, 1); } \
     else if (base && base_dtype == ULLM_BF16) { if (vec == 4) GO(bf16_t, bf16_t, 4); else GO(bf16_t, bf16_t, 1); } \
     else { if (vec == 4) GO(bf16_t, float, 4); else GO(bf16_t, float, 1); } } while (0)
-#define COMBINE_ARGS(TX, TB) (CombineArgs<TX, TB>{y, (const TX*)x, ldx, ids, weights, slot_of_pair, top, n_experts, (const TB*)base, bias, \
-    (const TX*)shared, H})
+#define COMBINE_ARGS(TX, TB) y, (const TX*)x, ldx, ids, weights, slot_of_pair, top, n_experts, (const TB*)base, bias, (const TX*)shared
 
 extern "C" int ullm_moe_combine(const float* y, const void* x, int ldx, const int* ids, const float* weights,
                                 const int* slot_of_pair, int top, int n_experts, const void* base, int base_dtype,
@@ -1292,7 +1273,8 @@ extern "C" int ullm_moe_combine(const float* y, const void* x, int ldx, const in
   if (const int bad = bad_combine(top, ldx, T_, H, base, base_dtype, dtype)) return bad;
   const int vec = H % 4 == 0 ? 4 : 1;
   dim3 grid(T_, (H / vec + 255) / 256), block(256);
-#define GO(TX, TB, V) hipLaunchKernelGGL((moe_combine_kernel<TX, TB, V>), grid, block, 0, stream, COMBINE_ARGS(TX, TB), out)
+#define GO(TX, TB, V) hipLaunchKernelGGL((moe_combine_kernel<TX, TB, V, false>), grid, block, 0, stream, COMBINE_ARGS(TX, TB), out, H, \
+    0.f, (float*)nullptr, (const float*)nullptr, (const float*)nullptr, (const float*)nullptr, (TX*)nullptr)
   COMBINE_BY_TYPES();
 #undef GO
   ULLM_LAUNCH_CHECK();
@@ -1307,8 +1289,8 @@ extern "C" int ullm_moe_combine_tanh(const float* y, const void* x, int ldx, con
   if (const int bad = bad_combine(top, ldx, T_, H, base, base_dtype, dtype)) return bad;
   const int vec = H % 4 == 0 ? 4 : 1;
   dim3 grid(T_, (H / vec + 255) / 256), block(256);
-#define GO(TX, TB, V) hipLaunchKernelGGL((moe_combine_tanh_kernel<TX, TB, V>), grid, block, 0, stream, COMBINE_ARGS(TX, TB), mult, residual, \
-    alpha, gain, shift, (TX*)out)
+#define GO(TX, TB, V) hipLaunchKernelGGL((moe_combine_kernel<TX, TB, V, true>), grid, block, 0, stream, COMBINE_ARGS(TX, TB), (float*)nullptr, H, \
+    mult, residual, alpha, gain, shift, (TX*)out)
   COMBINE_BY_TYPES();
 #undef GO
   ULLM_LAUNCH_CHECK();
