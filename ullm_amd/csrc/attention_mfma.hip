@@ -1427,11 +1427,12 @@ attention_prefill_dma_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t*
                              int n_tiles, ScoreExtras extras) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[DmaBlock<NQK, HEADS, KS>::BYTES];
   __shared__ int page_ids[KS][DmaBlock<NQK, HEADS, KS>::TABLE];
-  if constexpr (HEADS == 4 && KS == 1) {
+  if constexpr (KS == 1) {
     // A function is simplified by itself before it becomes part of a kernel, and the loop over all keys by four waves is laid out worse for it: 700
     // tokens of 32 heads over 8 behind 2100 84.5 us in the kernel's own body, 88.0 as a function, 330 tokens in each of three prompts 16.8 and
-    // 17.2, 2048 tokens 64.7 and 65.9.  The loops over parts of the keys and those of two heads gain (16 heads, 6000 tokens in quarters 239.6 and 234.4, in
-    // halves of two heads 203.5 and 199.5, 700 behind 2100 in quarters 40.1 and 39.5).
+    // 17.2, 2048 tokens 64.7 and 65.9; 16 heads by twos, 8000 tokens 300.7 and 308.4, three prompts of 3000 136.5 and 140.6 (but 6000 181.0 and
+    // 177.8).  The loops over parts of the keys gain (16 heads, 6000 tokens in quarters 239.6 and 234.4, in halves of two heads 203.5 and 199.5, 700
+    // behind 2100 in quarters 40.1 and 39.5).
     const unsigned block = blockIdx.x;
 #include "prefill_dma_block.h"
   } else {
